@@ -312,9 +312,12 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
  * over the 2^n - 1 non-empty column subsets, each subset's product of row
  * factors kept as a polynomial; here on the monomials that divide some e_q
  * (the reference keeps the box of the largest exponent per variable; the
- * kept coefficients are the same).  Rows with total degree above n give 0.
- * info (may be null, 6 entries): monomials, links, workgroups, 1 if the
- * polynomial was kept in LDS, algorithmic FP64 flops per subset, subsets.
+ * kept coefficients are the same).  Orders up to 12 expand the permanent row
+ * by row over the column subsets instead, without an alternating sum.  Rows
+ * with total degree above n give 0.
+ * info (may be null, 6 entries) describes the subset loop for these rows:
+ * monomials, links, workgroups, 1 if its polynomial fits LDS, algorithmic
+ * FP64 flops per subset, subsets.
  * n <= 24, at most 255 variables with a non-zero exponent, n x (those
  * variables + 1) <= 3072 and at most 2^23 monomials (PQP_ERR_RANGE beyond).
  */

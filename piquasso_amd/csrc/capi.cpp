@@ -1292,6 +1292,9 @@ struct PolyState {
   int64_t key_n = 0, key_vars = 0, key_out = 0;
   std::vector<int32_t> key_exps;
   PolyPlan plan;
+  std::vector<int16_t> subsets;        // poly_subsets of the plan's order (layer path)
+  std::vector<uint16_t> subset_bits;
+  std::vector<int64_t> subset_first;
 };
 
 PolyState &poly_state() {
@@ -1300,6 +1303,226 @@ PolyState &poly_state() {
 }
 
 size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
+
+// The layer path's subset tables for matrices of order n: the subsets of
+// 0 .. n - 1 columns by size, each size in increasing order of their bits
+// (`bits`), and for each subset and column j the place of the subset
+// without j in the next smaller size (`sub`; -1 when it does not hold j).
+// first[i]: subsets of sizes 0 .. i - 1.
+void poly_subsets(int n, std::vector<int16_t> &sub, std::vector<uint16_t> &bits,
+                  std::vector<int64_t> &first) {
+  std::vector<int16_t> place(size_t{1} << n, 0);
+  sub.clear();
+  bits.clear();
+  first.assign(static_cast<size_t>(n) + 1, 0);
+  for (int i = 0; i < n; ++i) {
+    int16_t at = 0;
+    first[i] = static_cast<int64_t>(bits.size());
+    for (uint32_t s = 0; s < (1u << n); ++s) {
+      if (__builtin_popcount(s) != i) continue;
+      place[s] = at++;
+      bits.push_back(static_cast<uint16_t>(s));
+      for (int j = 0; j < n; ++j)
+        sub.push_back((s >> j & 1u) ? place[s & ~(1u << j)] : static_cast<int16_t>(-1));
+    }
+  }
+}
+
+// Whether a polynomial permanent takes the layer path: the subsets of one
+// size fit a block's threads, a row's coefficients its LDS, and the two
+// largest layers 8 GiB.  `bytes` receives the size of one layer buffer.
+bool poly_layers_fit(const PolyPlan &p, size_t *bytes) {
+  if (p.n > kPolyLayerMaxN || static_cast<size_t>(p.n) * (p.M + 1) * sizeof(double2) > 16384) return false;
+  double most = 1.0, choose = 1.0;
+  for (int i = 1; i < p.n; ++i) {
+    choose = choose * (p.n - i + 1) / i;
+    most = std::max(most, choose * p.lvl_off[std::min(i, p.L) + 1]);
+  }
+  *bytes = static_cast<size_t>(most) * sizeof(double2);
+  return *bytes <= (size_t{4} << 30);
+}
+
+// The coefficients by the plan in S (PolyState::plan).  same(): whether the
+// plan belongs to the call's exponent rows; asked once, when the device has
+// its work.  If not, nothing is written to `out`.
+template <typename Same>
+int poly_run(PolyState &S, const double *b0, const double *bm, int64_t n_out, double *out, int64_t *info,
+             Same same) {
+  const PolyPlan &p = S.plan;
+  const int64_t n_keep = static_cast<int64_t>(p.out_index.size());
+  const int64_t n_subsets = (int64_t{1} << p.n) - 1;
+  if (info) {
+    info[0] = p.n_mono;
+    info[1] = static_cast<int64_t>(p.links.size());
+    info[2] = 0;
+    info[3] = 0;
+    info[4] = p.flops_per_subset;
+    info[5] = n_subsets;
+  }
+  if (n_keep == 0) {
+    std::fill(out, out + 2 * n_out, 0.0);
+    return PQP_OK;
+  }
+  if (n_keep > INT32_MAX / 2)
+    return fail(PQP_ERR_RANGE, std::to_string(n_keep) + " requested coefficients exceed the kernel's index range");
+  int st;
+  if ((st = require_device()) != PQP_OK) return st;
+  const DeviceState &dev = device_state();
+  const int cus = std::max(dev.cus, 1);
+  const int nn = p.n, M = p.M;
+  const size_t rs_bytes = static_cast<size_t>(nn) * (M + 1) * sizeof(double2);
+  const size_t poly_bytes = static_cast<size_t>(p.n_mono) * sizeof(double2);
+  // the polynomial stays in LDS up to 64 KiB per workgroup (two or more
+  // workgroups per CU), else in a global-memory slice per workgroup
+  if (rs_bytes > 49152)
+    return fail(PQP_ERR_RANGE, "n x (variables + 1) = " + std::to_string(nn * (M + 1)) +
+                                   " row sums exceed the 3072 kept in LDS");
+  const bool lds = rs_bytes + poly_bytes <= 65536;
+  if (!lds && poly_bytes > (size_t{8} << 30))
+    return fail(PQP_ERR_RANGE, "polynomial of " + std::to_string(p.n_mono) + " monomials is too large");
+  // in global memory, kPolyGroup subsets share a workgroup (coefficients
+  // interleaved) when their row sums fit in LDS and their slice in 8 GiB
+  const int group = (!lds && kPolyGroup * rs_bytes <= 49152 &&
+                     kPolyGroup * poly_bytes <= (size_t{8} << 30)) ? kPolyGroup : 1;
+  const size_t slice_bytes = poly_bytes * static_cast<size_t>(group);
+  const size_t lds_bytes = lds ? rs_bytes + poly_bytes : rs_bytes * static_cast<size_t>(group);
+  // global memory: two 1024-thread workgroups per CU (32 waves) hide the
+  // gather latency best (measured against one per CU and other groupings)
+  int64_t per_cu = lds ? std::min<int64_t>(8, std::max<int64_t>(1, 163840 / static_cast<int64_t>(lds_bytes))) : 2;
+  const int64_t n_groups = (n_subsets + group - 1) / group;
+  int64_t n_wg = std::min<int64_t>(n_groups, cus * per_cu);
+  // bound the per-workgroup slices: polynomials <= 8 GiB, accumulators <= 4 GiB
+  if (!lds) n_wg = std::min<int64_t>(n_wg, std::max<int64_t>(1, (int64_t{8} << 30) / static_cast<int64_t>(slice_bytes)));
+  n_wg = std::min<int64_t>(n_wg, std::max<int64_t>(1, (int64_t{4} << 30) / (n_keep * 16)));
+  if (info) {
+    info[2] = n_wg;
+    info[3] = lds ? 1 : 0;
+  }
+  size_t layer_bytes = 0;
+  const bool layers = poly_layers_fit(p, &layer_bytes);
+  // arena: the plan's tables (link_ptr, links, lvl_off, out_mono, subsets),
+  // then B_0 and the kept B_m (uploaded on every call)
+  const size_t mat = static_cast<size_t>(nn) * nn * sizeof(double2);
+  size_t off = 0;
+  const size_t o_lp = off;
+  off = align256(off + p.link_ptr.size() * sizeof(int32_t));
+  const size_t o_ln = off;
+  off = align256(off + std::max<size_t>(p.links.size(), 1) * sizeof(int32_t));
+  const size_t o_lv = off;
+  off = align256(off + p.lvl_off.size() * sizeof(int32_t));
+  const size_t o_om = off;
+  off = align256(off + p.out_mono.size() * sizeof(int32_t));
+  const size_t o_sb = off;
+  off = align256(off + S.subsets.size() * sizeof(int16_t));
+  const size_t o_bits = off;
+  off = align256(off + S.subset_bits.size() * sizeof(uint16_t));
+  const size_t o_b0 = off;
+  off = align256(off + mat);
+  const size_t o_bm = off;
+  off = align256(off + mat * static_cast<size_t>(M));
+  const size_t arena_bytes = off;
+  if (!S.init) {
+    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    S.init = true;
+  }
+  const void *arena_before = S.arena.p;
+  if ((st = S.arena.ensure(arena_bytes)) != PQP_OK) return st;
+  if (S.arena.p != arena_before) S.tables_on_device = false;
+  if ((st = S.stage.ensure(std::max(arena_bytes, static_cast<size_t>(n_keep) * 2 * sizeof(double)))) != PQP_OK)
+    return st;
+  if (layers) {
+    // layers alternate between the two halves
+    if ((st = S.scratch.ensure(2 * align256(layer_bytes))) != PQP_OK) return st;
+  } else if ((st = S.acc.ensure(static_cast<size_t>(n_wg) * static_cast<size_t>(n_keep) * sizeof(double2))) != PQP_OK) {
+    return st;
+  }
+  if ((st = S.out.ensure(static_cast<size_t>(n_keep) * 2 * sizeof(double))) != PQP_OK) return st;
+  if (!layers && !lds && (st = S.scratch.ensure(static_cast<size_t>(n_wg) * slice_bytes)) != PQP_OK) return st;
+  char *h = static_cast<char *>(S.stage.p);
+  const size_t first = S.tables_on_device ? o_b0 : 0;
+  if (!S.tables_on_device) {
+    std::memcpy(h + o_lp, p.link_ptr.data(), p.link_ptr.size() * sizeof(int32_t));
+    if (!p.links.empty()) std::memcpy(h + o_ln, p.links.data(), p.links.size() * sizeof(int32_t));
+    std::memcpy(h + o_lv, p.lvl_off.data(), p.lvl_off.size() * sizeof(int32_t));
+    std::memcpy(h + o_om, p.out_mono.data(), p.out_mono.size() * sizeof(int32_t));
+    if (!S.subsets.empty()) {
+      std::memcpy(h + o_sb, S.subsets.data(), S.subsets.size() * sizeof(int16_t));
+      std::memcpy(h + o_bits, S.subset_bits.data(), S.subset_bits.size() * sizeof(uint16_t));
+    }
+  }
+  std::memcpy(h + o_b0, b0, mat);
+  for (int v = 0; v < M; ++v)
+    std::memcpy(h + o_bm + mat * v, bm + static_cast<size_t>(p.vars[v]) * nn * nn * 2, mat);
+  PQP_HIP(hipMemcpyAsync(static_cast<char *>(S.arena.p) + first, h + first, arena_bytes - first,
+                         hipMemcpyHostToDevice, S.stream));
+  const char *d = static_cast<const char *>(S.arena.p);
+  if (layers) {
+    PolyLayerArgs la;
+    la.b0 = reinterpret_cast<const double2 *>(d + o_b0);
+    la.bm = reinterpret_cast<const double2 *>(d + o_bm);
+    la.link_ptr = reinterpret_cast<const int32_t *>(d + o_lp);
+    la.links = reinterpret_cast<const int32_t *>(d + o_ln);
+    la.out_mono = reinterpret_cast<const int32_t *>(d + o_om);
+    la.out = static_cast<double *>(S.out.p);
+    la.n = nn;
+    la.M = M;
+    la.n_out = static_cast<int32_t>(n_keep);
+    double2 *buf[2] = {static_cast<double2 *>(S.scratch.p),
+                       reinterpret_cast<double2 *>(static_cast<char *>(S.scratch.p) + align256(layer_bytes))};
+    la.n_dst = 1;
+    for (int i = 0; i < nn; ++i) {
+      la.row = i;
+      la.n_src = la.n_dst;
+      la.n_dst = la.n_src * (nn - i) / (i + 1);
+      la.n_src_mono = p.lvl_off[std::min(i, p.L) + 1];
+      la.n_dst_mono = p.lvl_off[std::min(i + 1, p.L) + 1];
+      la.src = i == 0 ? nullptr : buf[(i - 1) & 1];
+      la.dst = buf[i & 1];
+      const int64_t at = i + 1 < nn ? S.subset_first[i + 1] : 0;  // the last row reads no table
+      la.sub = reinterpret_cast<const int16_t *>(d + o_sb) + at * nn;
+      la.dst_bits = reinterpret_cast<const uint16_t *>(d + o_bits) + at;
+      la.src_bits = reinterpret_cast<const uint16_t *>(d + o_bits) + S.subset_first[i];
+      PQP_HIP(launch_poly_layer(la, S.stream));
+    }
+  } else {
+    PolyArgs a;
+    a.b0 = reinterpret_cast<const double2 *>(d + o_b0);
+    a.bm = reinterpret_cast<const double2 *>(d + o_bm);
+    a.link_ptr = reinterpret_cast<const int32_t *>(d + o_lp);
+    a.links = reinterpret_cast<const int32_t *>(d + o_ln);
+    a.lvl_off = reinterpret_cast<const int32_t *>(d + o_lv);
+    a.out_mono = reinterpret_cast<const int32_t *>(d + o_om);
+    a.scratch = lds ? nullptr : static_cast<double2 *>(S.scratch.p);
+    a.acc = static_cast<double2 *>(S.acc.p);
+    a.out = static_cast<double *>(S.out.p);
+    a.n = nn;
+    a.M = M;
+    a.L = p.L;
+    a.n_mono = static_cast<int32_t>(p.n_mono);
+    a.n_out = static_cast<int32_t>(n_keep);
+    a.n_wg = static_cast<int32_t>(n_wg);
+    PQP_HIP(launch_perm_poly(a, lds, group, lds_bytes, S.stream));
+  }
+  PQP_HIP(hipMemcpyAsync(S.stage.p, S.out.p, static_cast<size_t>(n_keep) * 2 * sizeof(double),
+                         hipMemcpyDeviceToHost, S.stream));
+  // a plan taken on trust is compared while the device works
+  const bool fresh = same();
+  PQP_HIP(hipStreamSynchronize(S.stream));
+  if (!fresh) return PQP_OK;
+  // the tables stay in the device arena for the next call with these rows
+  S.tables_on_device = true;
+  const double *r = static_cast<const double *>(S.stage.p);
+  if (n_keep == n_out) {  // every row kept, in order
+    std::memcpy(out, r, static_cast<size_t>(n_out) * 2 * sizeof(double));
+    return PQP_OK;
+  }
+  std::fill(out, out + 2 * n_out, 0.0);
+  for (int64_t q = 0; q < n_keep; ++q) {
+    out[2 * p.out_index[q]] = r[2 * q];
+    out[2 * p.out_index[q] + 1] = r[2 * q + 1];
+  }
+  return PQP_OK;
+}
 
 }  // namespace
 
@@ -1704,143 +1927,41 @@ int pqp_perm_poly_coefficients_c128(int64_t n, int64_t n_vars, const double *b0,
     return fail(PQP_ERR_INVALID, "invalid matrix polynomial arguments");
   PolyState &S = poly_state();
   std::lock_guard<std::mutex> lock(S.mu);
-  // the plan depends only on (n, the exponent rows): a call with the same
-  // rows as the previous one reuses it and the tables already on the device
+  // The plan depends only on (n, the exponent rows): a call with the same
+  // rows as the previous one reuses it and the tables already on the device.
+  // The rows can be larger than everything else the call reads (7.4 MB for
+  // 184756 outputs of 10 modes: 0.3 ms to compare), so a plan of the same
+  // sizes is tried at once and the rows compared while the device works;
+  // other rows start again with a plan of their own.
   const size_t n_ex = (n_out > 0 && n_vars > 0) ? static_cast<size_t>(n_out) * static_cast<size_t>(n_vars) : 0;
-  const bool hit = S.have_plan && S.key_n == n && S.key_vars == n_vars && S.key_out == n_out &&
-                   (n_ex == 0 || std::memcmp(S.key_exps.data(), exponents, n_ex * sizeof(int32_t)) == 0);
-  int st = PQP_OK;
-  if (!hit) {
-    S.have_plan = false;
-    S.tables_on_device = false;
-    std::string err;
-    st = poly_plan_build(n, n_vars, n_out, exponents, S.plan, err);
-    if (st != PQP_OK) return fail(st, err);
-    S.key_n = n;
-    S.key_vars = n_vars;
-    S.key_out = n_out;
-    S.key_exps.assign(exponents, exponents + n_ex);
-    S.have_plan = true;
+  int same = -1;  // not compared yet
+  auto compare = [&] {
+    if (same < 0)
+      same = n_ex == 0 || std::memcmp(S.key_exps.data(), exponents, n_ex * sizeof(int32_t)) == 0;
+    return same == 1;
+  };
+  if (S.have_plan && S.key_n == n && S.key_vars == n_vars && S.key_out == n_out) {
+    if (!S.tables_on_device) compare();
+    if (same != 0) {
+      const int st = poly_run(S, b0, bm, n_out, out, info, compare);
+      if (compare()) return st;
+      g_error.clear();
+    }
   }
-  const PolyPlan &p = S.plan;
-  for (int64_t q = 0; q < 2 * n_out; ++q) out[q] = 0.0;
-  const int64_t n_keep = static_cast<int64_t>(p.out_index.size());
-  const int64_t n_subsets = (int64_t{1} << p.n) - 1;
-  if (info) {
-    info[0] = p.n_mono;
-    info[1] = static_cast<int64_t>(p.links.size());
-    info[2] = 0;
-    info[3] = 0;
-    info[4] = p.flops_per_subset;
-    info[5] = n_subsets;
-  }
-  if (n_keep == 0) return PQP_OK;
-  if (n_keep > INT32_MAX / 2)
-    return fail(PQP_ERR_RANGE, std::to_string(n_keep) + " requested coefficients exceed the kernel's index range");
-  if ((st = require_device()) != PQP_OK) return st;
-  const DeviceState &dev = device_state();
-  const int cus = std::max(dev.cus, 1);
-  const int nn = p.n, M = p.M;
-  const size_t rs_bytes = static_cast<size_t>(nn) * (M + 1) * sizeof(double2);
-  const size_t poly_bytes = static_cast<size_t>(p.n_mono) * sizeof(double2);
-  // the polynomial stays in LDS up to 64 KiB per workgroup (two or more
-  // workgroups per CU), else in a global-memory slice per workgroup
-  if (rs_bytes > 49152)
-    return fail(PQP_ERR_RANGE, "n x (variables + 1) = " + std::to_string(nn * (M + 1)) +
-                                   " row sums exceed the 3072 kept in LDS");
-  const bool lds = rs_bytes + poly_bytes <= 65536;
-  if (!lds && poly_bytes > (size_t{8} << 30))
-    return fail(PQP_ERR_RANGE, "polynomial of " + std::to_string(p.n_mono) + " monomials is too large");
-  // in global memory, kPolyGroup subsets share a workgroup (coefficients
-  // interleaved) when their row sums fit in LDS and their slice in 8 GiB
-  const int group = (!lds && kPolyGroup * rs_bytes <= 49152 &&
-                     kPolyGroup * poly_bytes <= (size_t{8} << 30)) ? kPolyGroup : 1;
-  const size_t slice_bytes = poly_bytes * static_cast<size_t>(group);
-  const size_t lds_bytes = lds ? rs_bytes + poly_bytes : rs_bytes * static_cast<size_t>(group);
-  // global memory: two 1024-thread workgroups per CU (32 waves) hide the
-  // gather latency best (measured against one per CU and other groupings)
-  int64_t per_cu = lds ? std::min<int64_t>(8, std::max<int64_t>(1, 163840 / static_cast<int64_t>(lds_bytes))) : 2;
-  const int64_t n_groups = (n_subsets + group - 1) / group;
-  int64_t n_wg = std::min<int64_t>(n_groups, cus * per_cu);
-  // bound the per-workgroup slices: polynomials <= 8 GiB, accumulators <= 4 GiB
-  if (!lds) n_wg = std::min<int64_t>(n_wg, std::max<int64_t>(1, (int64_t{8} << 30) / static_cast<int64_t>(slice_bytes)));
-  n_wg = std::min<int64_t>(n_wg, std::max<int64_t>(1, (int64_t{4} << 30) / (n_keep * 16)));
-  if (info) {
-    info[2] = n_wg;
-    info[3] = lds ? 1 : 0;
-  }
-  // arena: the plan's tables (link_ptr, links, lvl_off, out_mono), then
-  // B_0 and the kept B_m (uploaded on every call)
-  const size_t mat = static_cast<size_t>(nn) * nn * sizeof(double2);
-  size_t off = 0;
-  const size_t o_lp = off;
-  off = align256(off + p.link_ptr.size() * sizeof(int32_t));
-  const size_t o_ln = off;
-  off = align256(off + std::max<size_t>(p.links.size(), 1) * sizeof(int32_t));
-  const size_t o_lv = off;
-  off = align256(off + p.lvl_off.size() * sizeof(int32_t));
-  const size_t o_om = off;
-  off = align256(off + p.out_mono.size() * sizeof(int32_t));
-  const size_t o_b0 = off;
-  off = align256(off + mat);
-  const size_t o_bm = off;
-  off = align256(off + mat * static_cast<size_t>(M));
-  const size_t arena_bytes = off;
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
-    S.init = true;
-  }
-  const void *arena_before = S.arena.p;
-  if ((st = S.arena.ensure(arena_bytes)) != PQP_OK) return st;
-  if (S.arena.p != arena_before) S.tables_on_device = false;
-  if ((st = S.stage.ensure(std::max(arena_bytes, static_cast<size_t>(n_keep) * 2 * sizeof(double)))) != PQP_OK)
-    return st;
-  if ((st = S.acc.ensure(static_cast<size_t>(n_wg) * static_cast<size_t>(n_keep) * sizeof(double2))) != PQP_OK)
-    return st;
-  if ((st = S.out.ensure(static_cast<size_t>(n_keep) * 2 * sizeof(double))) != PQP_OK) return st;
-  if (!lds && (st = S.scratch.ensure(static_cast<size_t>(n_wg) * slice_bytes)) != PQP_OK) return st;
-  char *h = static_cast<char *>(S.stage.p);
-  const size_t first = S.tables_on_device ? o_b0 : 0;
-  if (!S.tables_on_device) {
-    std::memcpy(h + o_lp, p.link_ptr.data(), p.link_ptr.size() * sizeof(int32_t));
-    if (!p.links.empty()) std::memcpy(h + o_ln, p.links.data(), p.links.size() * sizeof(int32_t));
-    std::memcpy(h + o_lv, p.lvl_off.data(), p.lvl_off.size() * sizeof(int32_t));
-    std::memcpy(h + o_om, p.out_mono.data(), p.out_mono.size() * sizeof(int32_t));
-  }
-  std::memcpy(h + o_b0, b0, mat);
-  for (int v = 0; v < M; ++v)
-    std::memcpy(h + o_bm + mat * v, bm + static_cast<size_t>(p.vars[v]) * nn * nn * 2, mat);
-  PQP_HIP(hipMemcpyAsync(static_cast<char *>(S.arena.p) + first, h + first, arena_bytes - first,
-                         hipMemcpyHostToDevice, S.stream));
-  const char *d = static_cast<const char *>(S.arena.p);
-  PolyArgs a;
-  a.b0 = reinterpret_cast<const double2 *>(d + o_b0);
-  a.bm = reinterpret_cast<const double2 *>(d + o_bm);
-  a.link_ptr = reinterpret_cast<const int32_t *>(d + o_lp);
-  a.links = reinterpret_cast<const int32_t *>(d + o_ln);
-  a.lvl_off = reinterpret_cast<const int32_t *>(d + o_lv);
-  a.out_mono = reinterpret_cast<const int32_t *>(d + o_om);
-  a.scratch = lds ? nullptr : static_cast<double2 *>(S.scratch.p);
-  a.acc = static_cast<double2 *>(S.acc.p);
-  a.out = static_cast<double *>(S.out.p);
-  a.n = nn;
-  a.M = M;
-  a.L = p.L;
-  a.n_mono = static_cast<int32_t>(p.n_mono);
-  a.n_out = static_cast<int32_t>(n_keep);
-  a.n_wg = static_cast<int32_t>(n_wg);
-  PQP_HIP(launch_perm_poly(a, lds, group, lds_bytes, S.stream));
-  PQP_HIP(hipMemcpyAsync(S.stage.p, S.out.p, static_cast<size_t>(n_keep) * 2 * sizeof(double),
-                         hipMemcpyDeviceToHost, S.stream));
-  PQP_HIP(hipStreamSynchronize(S.stream));
-  // the tables stay in the device arena for the next call with these rows
-  S.tables_on_device = true;
-  const double *r = static_cast<const double *>(S.stage.p);
-  for (int64_t q = 0; q < n_keep; ++q) {
-    out[2 * p.out_index[q]] = r[2 * q];
-    out[2 * p.out_index[q] + 1] = r[2 * q + 1];
-  }
-  return PQP_OK;
+  S.have_plan = false;
+  S.tables_on_device = false;
+  std::string err;
+  const int st = poly_plan_build(n, n_vars, n_out, exponents, S.plan, err);
+  if (st != PQP_OK) return fail(st, err);
+  S.subsets.clear();
+  S.subset_bits.clear();
+  if (n <= kPolyLayerMaxN) poly_subsets(static_cast<int>(n), S.subsets, S.subset_bits, S.subset_first);
+  S.key_n = n;
+  S.key_vars = n_vars;
+  S.key_out = n_out;
+  S.key_exps.assign(exponents, exponents + n_ex);
+  S.have_plan = true;
+  return poly_run(S, b0, bm, n_out, out, info, [] { return true; });
 }
 
 int pqp_grad_batch_c128(int64_t count, const double *const *matrices, const int64_t *m_r,

@@ -97,6 +97,11 @@ hipError_t launch_tensor_p1(int n, const TensorArgs &a, int first_unit, int n_un
 hipError_t launch_tensor(int n, const TensorArgs &a, int first_unit, int n_units, hipStream_t s);
 hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream);
 
+// One row of the layer path of a matrix-polynomial permanent
+// (perm_poly.hip): layer a.row + 1 from layer a.row, or for the last row the
+// requested coefficients.
+hipError_t launch_poly_layer(const PolyLayerArgs &a, hipStream_t stream);
+
 // Matrix-polynomial permanent (perm_poly.hip): the subset sweep over
 // a.n_wg workgroups (the polynomial in LDS when `lds`; else in global memory
 // with `group` (1 or kPolyGroup) subsets interleaved; dynamic LDS of

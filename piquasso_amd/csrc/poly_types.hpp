@@ -31,4 +31,27 @@ struct PolyArgs {
   int32_t n, M, L, n_mono, n_out, n_wg;
 };
 
+// The layer path (perm_poly.hip): rows 0..i-1 expanded over the column
+// subsets S of i columns, f_i[e][S] = [x^e] of the sum over the ways to
+// match those rows with S.
+constexpr int kPolyLayerMaxN = 12;         // C(12, 6) = 924 subsets in the widest layer
+constexpr int kPolyLayerThreads = 256;
+constexpr int kPolyLayerLds = 40960;       // bytes of products a layer block keeps (four blocks per CU)
+constexpr int kPolyMissFactor = 2;         // multiply only the missing columns from 2 (n - i) <= n on
+constexpr int kPolyLayerAcc = 4;           // subsets per thread: ceil(924 / 256)
+
+struct PolyLayerArgs {
+  const double2 *b0, *bm;  // as in PolyArgs
+  const int32_t *link_ptr, *links, *out_mono;
+  const int16_t *sub;      // n_dst x n: place of S without column j in the source layer, -1 if j is not in S
+  const uint16_t *src_bits, *dst_bits;  // each subset's columns
+  const double2 *src;      // n_src_mono x n_src (null: the empty product 1)
+  double2 *dst;            // n_dst_mono x n_dst
+  double *out;             // last row: 2 per requested coefficient
+  int32_t n, M, row;
+  int32_t n_src, n_dst;            // subsets of `row` and of row + 1 columns
+  int32_t n_src_mono, n_dst_mono;  // monomials of degree <= row and <= row + 1 (and <= L)
+  int32_t n_out;
+};
+
 }  // namespace pqp

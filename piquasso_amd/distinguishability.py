@@ -165,7 +165,7 @@ def perm_poly_coefficients(b0, bms, exponents, with_info: bool = False):
         e = np.ascontiguousarray(e, dtype=np.int32)
     if e.ndim != 2 or e.shape[1] != bm.shape[0]:
         raise ValueError("one exponent per variable in every row")
-    out = np.zeros(2 * max(len(e), 1))
+    out = np.empty(2 * max(len(e), 1))  # the call writes every row
     info = np.zeros(6, dtype=np.int64)
     dp = ctypes.POINTER(ctypes.c_double)
     st = _capi.lib().pqp_perm_poly_coefficients_c128(
@@ -174,7 +174,7 @@ def perm_poly_coefficients(b0, bms, exponents, with_info: bool = False):
         e.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), out.ctypes.data_as(dp),
         info.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)))
     _capi.check(st)
-    coef = out[: 2 * len(e)].view(np.complex128).copy()
+    coef = out[: 2 * len(e)].view(np.complex128)
     if not with_info:
         return coef
     keys = ("monomials", "links", "workgroups", "lds", "flops_per_subset", "subsets")
