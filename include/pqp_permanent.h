@@ -302,6 +302,19 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
                                     double *abs_sum);
 
 /*
+ * Amplitudes <t_q| U |s> = perm(U; rows = t_q, cols = s) / sqrt(prod t_q! prod s!)
+ * (2 doubles each) of many output occupations t_q for one input occupation s
+ * (modes entries each; U modes x modes, row-major, interleaved complex), or
+ * with `probabilities` their squared moduli (1 double each): the quantity of
+ * piquasso/_simulators/passive/probabilities.py:26-54 for a table of outputs.
+ * outputs: count x modes, row-major.  Outputs of another particle number
+ * give 0.  1..16 particles and at most 64 modes (PQP_ERR_RANGE beyond; any
+ * batch of permanents takes pqp_batch_create).
+ */
+int pqp_output_table_c128(const double *matrix, int64_t modes, int64_t ld, const int32_t *input,
+                          int64_t count, const int64_t *outputs, int probabilities, double *out);
+
+/*
  * Coefficients of the permanent of a matrix polynomial,
  *   out[q] = [x^e_q] perm(B + sum_{m < n_vars} x_m C_m)   (2 doubles: re, im)
  * for n x n complex matrices B (b0) and C_0..C_{n_vars-1} (bm: n_vars

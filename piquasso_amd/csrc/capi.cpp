@@ -1342,6 +1342,39 @@ bool poly_layers_fit(const PolyPlan &p, size_t *bytes) {
   return *bytes <= (size_t{4} << 30);
 }
 
+// Buffers of the probability-table entry point, kept across calls (grown on
+// demand, bounded by kTableSegment rows), with their own stream and lock.
+struct TableState {
+  std::mutex mu;
+  bool init = false;
+  hipStream_t stream = nullptr;
+  DevBuf in, out;
+  HostBuf stage;
+};
+
+TableState &table_state() {
+  static TableState *s = new TableState();  // never destroyed: outlives atexit HIP teardown
+  return *s;
+}
+
+// Rows of a table in one pass over the buffers (64 modes: 64 MiB of
+// occupations), and rows packed before their copy and launch are issued: the
+// device works on a chunk while the host packs the next.
+constexpr int64_t kTableSegment = int64_t{1} << 20;
+constexpr int64_t kTableChunk = int64_t{1} << 14;
+
+// Occupations as bytes; values above 127 stay above every particle number.
+// Returns false if one is negative.
+bool pack_occupations(const int64_t *src, int64_t count, uint8_t *dst) {
+  int64_t all = 0;
+  for (int64_t k = 0; k < count; ++k) {
+    const int64_t v = src[k];
+    all |= v;
+    dst[k] = static_cast<uint8_t>(v > 127 ? 127 : v);
+  }
+  return all >= 0;
+}
+
 // The coefficients by the plan in S (PolyState::plan).  same(): whether the
 // plan belongs to the call's exponent rows; asked once, when the device has
 // its work.  If not, nothing is written to `out`.
@@ -1900,6 +1933,109 @@ int pqp_tensor_permanent_c128(const double *matrix, int64_t n, int64_t ld, doubl
                               double *out, double *abs_sum) {
   const double *m[1] = {matrix};
   return pqp_tensor_permanent_batch_c128(1, m, &n, &ld, &overlap, out, abs_sum);
+}
+
+int pqp_output_table_c128(const double *matrix, int64_t modes, int64_t ld, const int32_t *input,
+                          int64_t count, const int64_t *outputs, int probabilities, double *out) {
+  CallRange range_("pqp_output_table_c128");
+  if (modes < 1 || count < 0 || !matrix || ld < modes || !input || (count > 0 && (!outputs || !out)))
+    return fail(PQP_ERR_INVALID, "invalid output table arguments");
+  if (modes > kTableMaxModes)
+    return fail(PQP_ERR_RANGE, "output tables support at most " + std::to_string(kTableMaxModes) + " modes");
+  int64_t n = 0;
+  int width = 0;
+  bool ones = true;
+  double in_norm = 1.0;
+  for (int64_t j = 0; j < modes; ++j) {
+    if (input[j] < 0) return fail(PQP_ERR_INVALID, "occupation numbers must be non-negative");
+    n += input[j];
+    width += input[j] > 0;
+    ones = ones && input[j] <= 1;
+  }
+  if (n < 1 || n > kTableMaxN)
+    return fail(PQP_ERR_RANGE, "output tables support 1.." + std::to_string(kTableMaxN) + " particles");
+  for (int64_t j = 0; j < modes; ++j)
+    for (int32_t q = 2; q <= input[j]; ++q) in_norm *= q;
+  const int per = probabilities ? 1 : 2;
+  const DeviceState &dev = device_state();
+  if (!dev.ok) {
+    // argument errors first, and a table without a matching row needs no device
+    bool any = false;
+    for (int64_t r = 0; r < count; ++r) {
+      int64_t sum = 0;
+      for (int64_t j = 0; j < modes; ++j) {
+        const int64_t v = outputs[r * modes + j];
+        if (v < 0) return fail(PQP_ERR_INVALID, "occupation numbers must be non-negative");
+        sum += v;
+      }
+      any = any || sum == n;
+    }
+    if (any) return fail(PQP_ERR_DEVICE, dev.error);
+    std::fill(out, out + per * count, 0.0);
+    return PQP_OK;
+  }
+  TableState &S = table_state();
+  std::lock_guard<std::mutex> lock(S.mu);
+  if (!S.init) {
+    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    S.init = true;
+  }
+  // input buffer: the occupied columns, their occupations, the outputs
+  const size_t o_mult = static_cast<size_t>(modes) * width * 2 * sizeof(double);
+  const size_t o_outs = align256(o_mult + static_cast<size_t>(width) * sizeof(int32_t));
+  const int64_t most = std::min(count, kTableSegment);
+  const size_t in_bytes = o_outs + static_cast<size_t>(most) * static_cast<size_t>(modes);
+  const size_t out_bytes = static_cast<size_t>(most) * per * sizeof(double);
+  int st;
+  if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
+  if ((st = S.out.ensure(out_bytes)) != PQP_OK) return st;
+  if ((st = S.stage.ensure(align256(in_bytes) + out_bytes)) != PQP_OK) return st;
+  char *h = static_cast<char *>(S.stage.p);
+  char *d = static_cast<char *>(S.in.p);
+  double *hrows = reinterpret_cast<double *>(h);
+  int32_t *hmult = reinterpret_cast<int32_t *>(h + o_mult);
+  int at = 0;
+  for (int64_t j = 0; j < modes; ++j) {
+    if (input[j] == 0) continue;
+    hmult[at] = input[j];
+    for (int64_t i = 0; i < modes; ++i) {
+      hrows[2 * (i * width + at)] = matrix[2 * (i * ld + j)];
+      hrows[2 * (i * width + at) + 1] = matrix[2 * (i * ld + j) + 1];
+    }
+    ++at;
+  }
+  TableArgs a;
+  a.rows = reinterpret_cast<const double *>(d);
+  a.mult = reinterpret_cast<const int32_t *>(d + o_mult);
+  a.in_norm = in_norm;
+  a.modes = static_cast<int32_t>(modes);
+  a.n = static_cast<int32_t>(n);
+  a.prob = probabilities ? 1 : 0;
+  double *hout = reinterpret_cast<double *>(h + align256(in_bytes));
+  for (int64_t s0 = 0; s0 < count; s0 += kTableSegment) {
+    const int64_t rows = std::min(count - s0, kTableSegment);
+    for (int64_t c0 = 0; c0 < rows; c0 += kTableChunk) {
+      const int64_t c = std::min(rows - c0, kTableChunk);
+      // the first copy also brings the columns
+      const size_t to = o_outs + static_cast<size_t>(c0 * modes);
+      const size_t from = c0 == 0 ? 0 : to;
+      if (!pack_occupations(outputs + (s0 + c0) * modes, c * modes, reinterpret_cast<uint8_t *>(h + to))) {
+        PQP_HIP(hipStreamSynchronize(S.stream));  // copies out of the staging buffer
+        return fail(PQP_ERR_INVALID, "occupation numbers must be non-negative");
+      }
+      PQP_HIP(hipMemcpyAsync(d + from, h + from, to + static_cast<size_t>(c * modes) - from,
+                             hipMemcpyHostToDevice, S.stream));
+      a.outs = reinterpret_cast<const uint8_t *>(d + to);
+      a.out = static_cast<double *>(S.out.p) + per * c0;
+      a.count = c;
+      PQP_HIP(launch_table(width, ones, a, S.stream));
+    }
+    PQP_HIP(hipMemcpyAsync(hout, S.out.p, static_cast<size_t>(rows) * per * sizeof(double),
+                           hipMemcpyDeviceToHost, S.stream));
+    PQP_HIP(hipStreamSynchronize(S.stream));
+    std::memcpy(out + per * s0, hout, static_cast<size_t>(rows) * per * sizeof(double));
+  }
+  return PQP_OK;
 }
 
 int pqp_perm_poly_plan_info(int64_t n, int64_t n_vars, int64_t n_out, const int32_t *exponents,

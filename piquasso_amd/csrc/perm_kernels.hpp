@@ -9,6 +9,7 @@
 #include "pqp_types.hpp"
 #include "tensor_types.hpp"
 #include "poly_types.hpp"
+#include "table_types.hpp"
 
 namespace pqp {
 
@@ -96,6 +97,10 @@ hipError_t launch_tensor_p0(int n, const TensorArgs &a, int first_unit, int n_un
 hipError_t launch_tensor_p1(int n, const TensorArgs &a, int first_unit, int n_units, hipStream_t s);
 hipError_t launch_tensor(int n, const TensorArgs &a, int first_unit, int n_units, hipStream_t s);
 hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream);
+
+// Probability tables (perm_table.hip): `width` occupied input modes, `ones`:
+// one particle in each.
+hipError_t launch_table(int width, bool ones, const TableArgs &a, hipStream_t stream);
 
 // One row of the layer path of a matrix-polynomial permanent
 // (perm_poly.hip): layer a.row + 1 from layer a.row, or for the last row the

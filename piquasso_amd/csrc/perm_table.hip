@@ -1,0 +1,265 @@
+// Probability tables on gfx950: the amplitudes
+//
+//   <t| U |s> = perm(U; rows = t, cols = s) / sqrt(prod t! prod s!)
+//
+// (or their squared moduli) of many output occupations t for one
+// interferometer U and input s (piquasso/_simulators/passive/
+// probabilities.py:26-54, one permanent after another there), n <= 16
+// particles.  Such permanents are small (at most 2^(n-1) Gray terms), and
+// planning each on the host costs far more than its sum: 1.4 us against
+// 2 ns for 7 particles.  So the kernel gets the occupations, a byte per
+// mode, and every wave plans its own item: lane i holds t_i, ballots give
+// the rows of multiplicity 1 and of more, and the first smallest row is
+// prepended as in src/permanent.cpp:54-95.  The binary digits come first:
+// the lowest k are swept by all lanes in Gray order, the others and the
+// digits of larger radix are the lane's, read off its index.  U's occupied
+// columns (at most 16 KB for every item alike) are read with scalar loads,
+// a row at a time, so no table is built or loaded per item.
+//
+// Sums as in perm_fwd.hip: FP64 row sums and products, FP64 runs of at most
+// 64 terms folded into double-double, the lanes' and waves' sums added in
+// double-double in a fixed order, exact integer weights.
+//
+// Bound by the per-item work of one wave (the plan, D row updates, a product
+// or a few, the double-double reduction), eight waves per SIMD hiding each
+// other's latency: 77 520 outputs of 7 particles in 14 modes take 126 us of
+// kernels, 1.6 ns an item, and 457 us a call, most of it the host packing
+// the occupations to bytes (the planned batch: 110 ms).  One wave per item
+// up to n = 9 (at most 256 terms, four per lane); 4 up to n = 12, 16 beyond,
+// so that a lane sweeps at most 32 states and a table of few items still
+// spreads (10 outputs of 16 particles: 49 us for 465 us planned; 1000: 128
+// us for 4.1 ms).
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "dd.hpp"
+#include "perm_kernels.hpp"
+#include "sweep_common.hpp"
+#include "table_types.hpp"
+
+namespace pqp {
+
+namespace {
+
+__constant__ double kFactorial[kTableMaxN + 1] = {
+    1.0,       1.0,        2.0,         6.0,          24.0,          120.0,
+    720.0,     5040.0,     40320.0,     362880.0,     3628800.0,     39916800.0,
+    479001600.0, 6227020800.0, 87178291200.0, 1307674368000.0, 20922789888000.0};
+
+// The product over the columns of one state's row sums.
+template <int W, bool ONES>
+__device__ __forceinline__ void table_product(const double (&cr)[W], const double (&ci)[W],
+                                              cptr<int32_t> mult, double &pr, double &pi) {
+  double ar = cr[0], ai = ci[0];
+  if constexpr (W > 1) {
+    double br = cr[1], bi = ci[1];
+#pragma unroll
+    for (int j = 2; j + 1 < W; j += 2) {
+      cmul(ar, ai, cr[j], ci[j]);
+      cmul(br, bi, cr[j + 1], ci[j + 1]);
+    }
+    if constexpr (W % 2 == 1 && W > 2) cmul(ar, ai, cr[W - 1], ci[W - 1]);
+    cmul(ar, ai, br, bi);
+  }
+  if constexpr (!ONES) {
+#pragma unroll
+    for (int j = 0; j < W; ++j)
+      for (int q = mult[j]; q > 1; --q) cmul(ar, ai, cr[j], ci[j]);
+  }
+  pr = ar;
+  pi = ai;
+}
+
+// NW waves per item, 4 / NW items per block (NW <= 4) or one.
+template <int W, bool ONES, int NW>
+__global__ __launch_bounds__(NW > 4 ? NW * kWave : 4 * kWave)
+__attribute__((amdgpu_waves_per_eu(W <= 8 ? 7 : W <= 12 ? 5 : 4, 8))) void perm_table_kernel(TableArgs a) {
+  constexpr int kPerBlock = NW < 4 ? 4 / NW : 1;
+  __shared__ double part[NW > 1 ? NW : 1][4];
+  const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+  const int bw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int wave = NW > 1 ? bw % NW : 0;
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * kPerBlock + bw / NW;
+  if (item >= a.count) return;  // whole blocks where NW > 1
+  const int occ = lane < a.modes ? a.outs[item * a.modes + lane] : 0;
+
+  // the item's plan: rows by multiplicity, the prepended row
+  int total = 0;
+  int i0 = 0, least = 0;
+  for (int v = 1; v <= a.n; ++v) {
+    const uint64_t at = __ballot(occ == v);
+    total += v * __builtin_popcountll(at);
+    if (at && !least) {
+      least = v;
+      i0 = __builtin_ctzll(at);
+    }
+  }
+  const bool match = total == a.n && !__ballot(occ > a.n);
+  double *out = a.out + (a.prob ? 1 : 2) * item;
+  if (!match) {  // another particle number: amplitude 0
+    if (lane == 0 && wave == 0) {
+      out[0] = 0.0;
+      if (!a.prob) out[1] = 0.0;
+    }
+    return;
+  }
+  const int rho = occ - (lane == i0 ? 1 : 0);
+  uint64_t bin = __ballot(rho == 1);
+  const uint64_t multi = __ballot(rho > 1);
+  const uint64_t rows_in = bin | multi;
+  const int nb = __builtin_popcountll(bin);
+  int states = 1;  // of the digits of larger radix
+  for (uint64_t m = multi; m; m &= m - 1)
+    states *= __builtin_amdgcn_readlane(rho, __builtin_ctzll(m)) + 1;
+  // inner digits: as many of the binary ones as leave the lanes a state each
+  int k = 0;
+  while (k < 6 && k < nb && ((states << (nb - k - 1)) >= NW * kWave)) ++k;
+  uint64_t inner = 0;  // the inner rows, a byte each
+  for (int p = 0; p < k; ++p) {
+    inner |= static_cast<uint64_t>(__builtin_ctzll(bin)) << (8 * p);
+    bin &= bin - 1;
+  }
+  const int S = 1 << k;
+  const int U = states << (nb - k);
+  const cptr<double> rows = as_const<double>(a.rows);
+  const cptr<int32_t> mult = as_const<int32_t>(a.mult);
+
+  cdd sum = cdd_zero();
+  for (int u0 = wave * kWave; u0 < U; u0 += NW * kWave) {
+    const bool active = u0 + lane < U;
+    const int u = active ? u0 + lane : 0;
+    // row sums of the lane's first state
+    double cr[W], ci[W];
+    {
+      // an opaque index: the row is loop-invariant, and hoisting it would
+      // hold a second set of row sums in registers
+      int r0 = i0;
+      __asm__ volatile("" : "+s"(r0));
+      const cptr<double> b = rows + r0 * (2 * W);
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        cr[j] = b[2 * j];
+        ci[j] = b[2 * j + 1];
+      }
+    }
+    auto add_row = [&](int r, double al) {
+      const cptr<double> b = rows + r * (2 * W);
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        cr[j] = fmaR(al, b[2 * j], cr[j]);
+        ci[j] = fmaR(al, b[2 * j + 1], ci[j]);
+      }
+    };
+    int rest = u, parity = 0;
+    double w = 1.0;
+    for (uint64_t m = rows_in; m; m &= m - 1) {  // one loop for all digits: one block of row sums
+      const int r = __builtin_ctzll(m);
+      const int rr = __builtin_amdgcn_readlane(rho, r);
+      double al = in_vgpr(1.0);  // inner digits start at 0
+      if (rr > 1) {
+        // u < 2^16: the quotient by a radix <= 17 is exact this way
+        const int q = static_cast<int>((static_cast<double>(rest) + 0.5) * (1.0 / (rr + 1)));
+        const int g = rest - q * (rr + 1);
+        rest = q;
+        parity ^= g & 1;
+        w *= lane_binomial(rr, g);
+        al = static_cast<double>(rr - 2 * g);
+      } else if ((bin >> r) & 1) {
+        al = (rest & 1) ? -1.0 : 1.0;
+        parity ^= rest & 1;
+        rest >>= 1;
+      }
+      add_row(r, al);
+    }
+    w = active ? (parity ? -w : w) : 0.0;
+    // the inner states in Gray order
+    double sr = 0.0, si = 0.0;
+    for (int v = 0; v < S; ++v) {
+      double pr, pi;
+      table_product<W, ONES>(cr, ci, mult, pr, pi);
+      sr += (v & 1) ? -pr : pr;
+      si += (v & 1) ? -pi : pi;
+      // the update after the last state (digit k: row 0) is never read
+      const int b = __builtin_ctz(v + 1);
+      const int up = (v + 1) ^ ((v + 1) >> 1);
+      add_row(static_cast<int>((inner >> (8 * b)) & 255), in_vgpr((up >> b & 1) ? -2.0 : 2.0));
+    }
+    sum = cdd_add(sum, cdd{dd_mul_d(dd{sr, 0.0}, w), dd_mul_d(dd{si, 0.0}, w)});
+  }
+  sum = wave_reduce<0>(sum, lane);
+  if constexpr (NW > 1) {
+    if (lane == 0) {
+      part[wave][0] = sum.re.hi;
+      part[wave][1] = sum.re.lo;
+      part[wave][2] = sum.im.hi;
+      part[wave][3] = sum.im.lo;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    // fixed order: lane l holds wave l's sum, then a butterfly over 16 lanes
+    static_assert(NW <= 16, "one lane per wave of a 16-lane group");
+    sum = lane < NW ? cdd{{part[lane][0], part[lane][1]}, {part[lane][2], part[lane][3]}} : cdd_zero();
+    sum = wave_reduce<0, 4>(sum, lane);
+  }
+  double norm = 1.0;
+  for (uint64_t m = __ballot(occ > 1); m; m &= m - 1)
+    norm *= kFactorial[__builtin_amdgcn_readlane(occ, __builtin_ctzll(m))];
+  norm = sqrt(norm * a.in_norm);
+  if (lane == 0) {
+    const int e = -(a.n - 1);
+    const double re = (ldexp(sum.re.hi, e) + ldexp(sum.re.lo, e)) / norm;
+    const double im = (ldexp(sum.im.hi, e) + ldexp(sum.im.lo, e)) / norm;
+    if (a.prob) {
+      out[0] = fmaR(re, re, im * im);
+    } else {
+      out[0] = re;
+      out[1] = im;
+    }
+  }
+}
+
+template <int W, bool ONES>
+hipError_t table_launch(const TableArgs &a, hipStream_t stream) {
+  const unsigned n = static_cast<unsigned>(a.count);
+  if (a.n <= 9)
+    hipLaunchKernelGGL((perm_table_kernel<W, ONES, 1>), dim3((n + 3) / 4), dim3(4 * kWave), 0, stream, a);
+  else if (a.n <= 12)
+    hipLaunchKernelGGL((perm_table_kernel<W, ONES, 4>), dim3(n), dim3(4 * kWave), 0, stream, a);
+  else
+    hipLaunchKernelGGL((perm_table_kernel<W, ONES, 16>), dim3(n), dim3(16 * kWave), 0, stream, a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_table(int width, bool ones, const TableArgs &a, hipStream_t stream) {
+  if (a.count <= 0) return hipSuccess;
+  if (a.count > INT32_MAX || a.n < 1 || a.n > kTableMaxN || a.modes > kTableMaxModes) return hipErrorInvalidValue;
+  switch (width) {
+#define PQP_TABLE_CASE(W) \
+  case W:                 \
+    return ones ? table_launch<W, true>(a, stream) : table_launch<W, false>(a, stream);
+    PQP_TABLE_CASE(1)
+    PQP_TABLE_CASE(2)
+    PQP_TABLE_CASE(3)
+    PQP_TABLE_CASE(4)
+    PQP_TABLE_CASE(5)
+    PQP_TABLE_CASE(6)
+    PQP_TABLE_CASE(7)
+    PQP_TABLE_CASE(8)
+    PQP_TABLE_CASE(9)
+    PQP_TABLE_CASE(10)
+    PQP_TABLE_CASE(11)
+    PQP_TABLE_CASE(12)
+    PQP_TABLE_CASE(13)
+    PQP_TABLE_CASE(14)
+    PQP_TABLE_CASE(15)
+    PQP_TABLE_CASE(16)
+#undef PQP_TABLE_CASE
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace pqp

@@ -74,6 +74,19 @@ __constant__ double kInvSmall[65] = {
     1.0 / 64};
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// C(rho, g) for a wave-uniform rho and the lane's g: prod_{i=1..g}
+// (rho - g + i) / i; every partial product is an integer, recovered exactly
+// by rounding.
+__device__ __forceinline__ double lane_binomial(int rho, int g) {
+  double cb = 1.0;
+  for (int i = 1; i <= rho; ++i) {
+    const double f = (i <= g) ? static_cast<double>(rho - g + i) : 1.0;
+    const double inv_i = (i <= g) ? kInvSmall[i] : 1.0;
+    cb = __builtin_rint(cb * f * inv_i);
+  }
+  return cb;
+}
+
 // Entry v of an inner table (scalar loads).
 __device__ __forceinline__ InnerEntry inner_entry(cptr<InnerEntry> tab, int v) {
   InnerEntry e;
@@ -229,15 +242,7 @@ __device__ __forceinline__ void start_state(const LaunchArgs &a, const cptr<Item
         q_hi = q;
         const int g = parity ? static_cast<int>(radix) - 1 - c : c;
         parity ^= (g & 1);
-        // C(rho, g) = prod_{i=1..g} (rho - g + i) / i; every partial product
-        // is an integer, recovered exactly by rounding.
-        double cb = 1.0;
-        for (int i = 1; i <= rho; ++i) {
-          const double f = (i <= g) ? static_cast<double>(rho - g + i) : 1.0;
-          const double inv_i = (i <= g) ? kInvSmall[i] : 1.0;
-          cb = __builtin_rint(cb * f * inv_i);
-        }
-        w_top *= cb;
+        w_top *= lane_binomial(rho, g);
         al = static_cast<R>(rho - 2 * g);
       }
     } else {

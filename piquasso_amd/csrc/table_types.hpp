@@ -1,0 +1,23 @@
+// Kernel arguments of the probability tables (perm_table.hip): one
+// interferometer and input occupation, many output occupations.
+#pragma once
+
+#include <cstdint>
+
+namespace pqp {
+
+constexpr int kTableMaxN = 16;      // particles (and columns) of a table on the fused kernel
+constexpr int kTableMaxModes = 64;  // one lane per mode
+
+struct TableArgs {
+  const double *rows;   // modes x width complex: the columns of occupied input modes
+  const int32_t *mult;  // their occupations (width)
+  const uint8_t *outs;  // count x modes output occupations
+  double *out;          // 2 doubles per output (amplitude) or 1 (probability)
+  double in_norm;       // prod of the input occupations' factorials
+  int64_t count;
+  int32_t modes, n;
+  int32_t prob;         // 1: probabilities
+};
+
+}  // namespace pqp

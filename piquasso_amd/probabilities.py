@@ -6,16 +6,20 @@ amplitude is perm(U; rows=t, cols=s) / sqrt(prod t! prod s!) and the
 probability its squared modulus — the quantity piquasso's passive simulator
 evaluates one permanent at a time (piquasso/_simulators/passive/utils.py:131-138,
 piquasso/_simulators/passive/probabilities.py:26-54).  Here all requested
-output patterns go to the GPU as one batch (:class:`PermanentBatch`).
+output patterns go to the GPU in one call: tables of at most 16 particles as
+bare occupations, planned by the kernel itself (``pqp_output_table_c128``),
+larger ones as a planned batch (:class:`PermanentBatch`).
 """
 
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Sequence
 
 import numpy as np
 
+from . import _capi
 from .engine import PermanentBatch
 
 __all__ = ["output_amplitudes", "output_probabilities", "particle_number_probabilities",
@@ -26,10 +30,31 @@ def _norm(occupation) -> float:
     return float(np.prod([math.factorial(int(k)) for k in occupation]))
 
 
-def output_amplitudes(unitary, input_state: Sequence[int], output_states,
-                      precision: str = "fp64") -> np.ndarray:
-    """Amplitudes <t| U |s> for every output pattern t (rows of
-    `output_states`), as a complex128 array."""
+# Tables the library plans on the device (pqp_output_table_c128); larger ones
+# go through a planned batch.
+_TABLE_PARTICLES = 16
+_TABLE_MODES = 64
+
+
+def _table(u, s, outs, probabilities: bool):
+    """Amplitudes or probabilities of the outputs from one call that takes
+    the occupations as they are, or None when the table is too large for it."""
+    n, m = int(s.sum()), u.shape[0]
+    if not 1 <= n <= _TABLE_PARTICLES or m > _TABLE_MODES or (s < 0).any():
+        return None
+    outs = np.ascontiguousarray(outs)
+    s32 = np.ascontiguousarray(s, dtype=np.int32)
+    res = np.empty(len(outs), dtype=np.float64 if probabilities else np.complex128)
+    dp = ctypes.POINTER(ctypes.c_double)
+    _capi.check(_capi.lib().pqp_output_table_c128(
+        u.view(np.float64).ctypes.data_as(dp), m, m,
+        s32.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), len(outs),
+        outs.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), int(probabilities),
+        res.view(np.float64).ctypes.data_as(dp)))
+    return res
+
+
+def _checked(unitary, input_state, output_states):
     u = np.ascontiguousarray(np.asarray(unitary, dtype=np.complex128))
     if u.ndim != 2 or u.shape[0] != u.shape[1]:
         raise ValueError(f"unitary must be square, got shape {u.shape}")
@@ -40,6 +65,18 @@ def output_amplitudes(unitary, input_state: Sequence[int], output_states,
     m = u.shape[0]
     if s.shape[0] != m or outs.shape[1] != m:
         raise ValueError("occupation vectors must have one entry per mode")
+    return u, s, outs
+
+
+def output_amplitudes(unitary, input_state: Sequence[int], output_states,
+                      precision: str = "fp64") -> np.ndarray:
+    """Amplitudes <t| U |s> for every output pattern t (rows of
+    `output_states`), as a complex128 array."""
+    u, s, outs = _checked(unitary, input_state, output_states)
+    if precision == "fp64":
+        amps = _table(u, s, outs, False)
+        if amps is not None:
+            return amps
     if (s < 0).any() or (outs < 0).any():
         raise ValueError("occupation numbers must be non-negative")
     n = int(s.sum())
@@ -61,6 +98,10 @@ def output_amplitudes(unitary, input_state: Sequence[int], output_states,
 def output_probabilities(unitary, input_state: Sequence[int], output_states,
                          precision: str = "fp64") -> np.ndarray:
     """Probabilities |<t| U |s>|^2 for every output pattern t."""
+    if precision == "fp64":
+        probs = _table(*_checked(unitary, input_state, output_states), True)
+        if probs is not None:
+            return probs
     return np.abs(output_amplitudes(unitary, input_state, output_states, precision)) ** 2
 
 
