@@ -302,6 +302,21 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
                                     double *abs_sum);
 
 /*
+ * Clifford & Clifford boson sampling, all steps of all shots on the device
+ * (piquasso/_simulators/passive/sampling.py:208-236,711-753).  Shot s places
+ * steps[s] <= photons photons of its pool (pools: shots x photons input
+ * modes, uint8): photon p is the picks[p][s]-th of those left, in order
+ * (photons x shots), and leaves in the mode where draws[p][s] (photons x
+ * shots, uniform in [0, 1)) falls in the running sum of its distribution
+ * over the modes.  out: shots x modes counts.  At most 64 modes
+ * and 24 photons (PQP_ERR_RANGE beyond); PQP_ERR_INVALID when a distribution
+ * has no finite positive sum.
+ */
+int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64_t shots, int64_t photons,
+                          const uint8_t *pools, const int32_t *steps, const int32_t *picks, const double *draws,
+                          int32_t *out);
+
+/*
  * Amplitudes <t_q| U |s> = perm(U; rows = t_q, cols = s) / sqrt(prod t_q! prod s!)
  * (2 doubles each) of many output occupations t_q for one input occupation s
  * (modes entries each; U modes x modes, row-major, interleaved complex), or

@@ -125,6 +125,12 @@ constexpr int64_t kBatchUnitsPerCu = 32;
 // SIMD: about 8 units per CU over the batch measured best (256 gradients of
 // n = 12..20: 0.74 ms at 8 or 16 per CU, 0.91 ms at 32).
 constexpr int64_t kGradUnitsPerCu = 8;
+// Waves a lone column-minor problem is spread over before its waves sweep
+// more than one state a lane: two per SIMD of 256 CUs.
+constexpr int64_t kLaplaceWaves = 2048;
+// Shots of one pass of the sampler (its buffers: 64 partials of 48
+// components and 24 columns of 64 modes each, 200 MB at most).
+constexpr int64_t kSampleShots = 2048;
 
 int expand_mode(uint32_t flags) {
   if (flags & PQP_FLAG_EXPAND_COLS) return 1;
@@ -769,12 +775,12 @@ void single_key(const PermInput &in, uint32_t flags, std::vector<int64_t> &key) 
 // Wait for `seq` in the host-visible done slot a one-block launch publishes.
 // A kernel that never signals (a device error) is caught by synchronising
 // the stream after 10 s of polling.
-int wait_done(Exec &x, volatile uint64_t *done, uint64_t seq) {
+int wait_done(hipStream_t stream, volatile uint64_t *done, uint64_t seq) {
   const auto t0 = std::chrono::steady_clock::now();
   for (uint32_t spin = 1; *done != seq; ++spin) {
     if ((spin & 4095u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::seconds(10)) {
-      PQP_HIP(hipStreamSynchronize(x.stream));
-      if (*done != seq) return fail(PQP_ERR_DEVICE, "single-permanent kernel did not signal completion");
+      PQP_HIP(hipStreamSynchronize(stream));
+      if (*done != seq) return fail(PQP_ERR_DEVICE, "kernel did not signal completion");
       break;
     }
     __builtin_ia32_pause();
@@ -876,7 +882,7 @@ int run_single(const PermInput &in, uint32_t flags, double *out2, double *out_dd
     *done = 0;
     x.abs_valid = true;
     PQP_HIP(launch_single_block(bucket, fp32, args, x.stream));
-    if ((st = wait_done(x, done, args.seq)) != PQP_OK) return st;
+    if ((st = wait_done(x.stream, done, args.seq)) != PQP_OK) return st;
   } else if (!(flags & PQP_FLAG_PLAIN) && x.plan.ranges.size() == 1 && d.units > 0 &&
              d.mcp <= kLastFinalizeMaxWidth) {
     // one static launch over the device whose last block finalizes the
@@ -899,7 +905,7 @@ int run_single(const PermInput &in, uint32_t flags, double *out2, double *out_dd
     *done = 0;
     x.abs_valid = true;
     PQP_HIP(launch_fwd(b, l));
-    if ((st = wait_done(x, done, l.args.seq)) != PQP_OK) {
+    if ((st = wait_done(x.stream, done, l.args.seq)) != PQP_OK) {
       // a launch that did not finish its count leaves it behind: clear it so
       // that the next call's last block is recognised
       (void)hipMemsetAsync(l.args.last_counter, 0, sizeof(int), x.stream);
@@ -1340,6 +1346,127 @@ bool poly_layers_fit(const PolyPlan &p, size_t *bytes) {
   }
   *bytes = static_cast<size_t>(most) * sizeof(double2);
   return *bytes <= (size_t{4} << 30);
+}
+
+// Buffers of the device-planned column minors: a lone problem (`res` holds
+// its results and the done slot) and the sampler's steps, each with its own
+// stream, kept across calls.
+struct MinorsState {
+  std::mutex mu;
+  bool init = false;
+  hipStream_t stream = nullptr;
+  DevBuf in, work, counter;
+  HostBuf stage;
+  MappedBuf res;
+  uint64_t seq = 0;
+};
+
+MinorsState &laplace_state() {
+  static MinorsState *s = new MinorsState();  // never destroyed: outlives atexit HIP teardown
+  return *s;
+}
+
+MinorsState &sample_state() {
+  static MinorsState *s = new MinorsState();
+  return *s;
+}
+
+// Column minors of one problem whose columns all hold one particle, planned
+// by the kernel's waves: no tables, one copy (rows of non-zero multiplicity,
+// compacted), two launches, the result polled.  Other problems (columns of
+// other multiplicities, or wider) return false.
+bool laplace_wave_fits(const PermInput &in) {
+  if (in.m_r < 1 || in.m_c < 2 || in.m_c > kMinorsWaveMaxCols || !in.a || !in.rows || !in.cols || in.ld < in.m_c)
+    return false;
+  int64_t sr = 0;
+  for (int64_t i = 0; i < in.m_r; ++i) {
+    if (in.rows[i] < 0) return false;
+    sr += in.rows[i];
+  }
+  for (int64_t j = 0; j < in.m_c; ++j)
+    if (in.cols[j] != 1) return false;
+  return sr + 1 == in.m_c;
+}
+
+int laplace_wave(const PermInput &in, double *out) {
+  int st;
+  if ((st = require_device()) != PQP_OK) return st;
+  const int W = static_cast<int>(in.m_c);
+  MinorsState &S = laplace_state();
+  std::lock_guard<std::mutex> lock(S.mu);
+  if (!S.init) {
+    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    if ((st = S.counter.ensure(sizeof(int))) != PQP_OK) return st;
+    PQP_HIP(hipMemsetAsync(S.counter.p, 0, sizeof(int), S.stream));
+    S.init = true;
+  }
+  // the occupied rows, and the digits the waves will find in them
+  const size_t row_bytes = static_cast<size_t>(W) * 2 * sizeof(double);
+  const size_t o_occ = static_cast<size_t>(W - 1) * row_bytes;  // at most W - 1 occupied rows
+  const size_t in_bytes = o_occ + static_cast<size_t>(W);
+  if ((st = S.stage.ensure(in_bytes)) != PQP_OK) return st;
+  if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
+  char *h = static_cast<char *>(S.stage.p);
+  int m = 0, least = 0, ones = 0;
+  for (int64_t i = 0; i < in.m_r; ++i) {
+    const int r = in.rows[i];
+    if (r == 0) continue;
+    std::memcpy(h + m * row_bytes, static_cast<const double *>(in.a) + 2 * i * in.ld, row_bytes);
+    h[o_occ + m] = static_cast<char>(r);
+    if (!least || r < least) least = r;
+    ones += r == 1;
+    ++m;
+  }
+  int64_t states = 1;  // of the digits of larger radix
+  bool prepended = false;
+  int nb = ones;
+  for (int i = 0; i < m; ++i) {
+    int rho = h[o_occ + i];
+    if (!prepended && rho == least) {
+      prepended = true;
+      if (rho == 1) --nb;
+      --rho;
+      if (rho == 1) ++nb;
+    }
+    if (rho > 1) states *= rho + 1;
+  }
+  // Waves of one state per lane up to kLaplaceWaves of them (two per SIMD,
+  // what the widest kernels hold), longer ones beyond: a lone call waits for
+  // its slowest wave, and a state costs a fifth of the start and the sums.
+  MinorsWaveArgs a;
+  const int64_t terms = states << nb;
+  a.k_max = 0;
+  while (a.k_max < 7 && terms >> (6 + a.k_max) > kLaplaceWaves) ++a.k_max;
+  int k = 0;
+  while (k < a.k_max && k < nb && (states << (nb - k - 1)) >= 64) ++k;
+  a.waves = static_cast<int32_t>(std::min<int64_t>(((terms >> k) + 63) / 64, 16 * kLaplaceWaves));
+  if ((st = S.work.ensure(static_cast<size_t>(a.waves) * 4 * W * sizeof(double))) != PQP_OK) return st;
+  const size_t res_bytes = static_cast<size_t>(kMinorsWaveMaxCols) * 2 * sizeof(double);
+  if ((st = S.res.ensure(res_bytes + sizeof(uint64_t))) != PQP_OK) return st;
+  PQP_HIP(hipMemcpyAsync(S.in.p, h, in_bytes, hipMemcpyHostToDevice, S.stream));
+  a.rows = static_cast<const double *>(S.in.p);
+  a.occ = static_cast<const uint8_t *>(S.in.p) + o_occ;
+  a.units = nullptr;
+  a.partials = static_cast<double *>(S.work.p);
+  a.out = static_cast<double *>(S.res.dev);
+  a.item_stride = 0;
+  a.ld = W;
+  a.modes = m;
+  a.last_counter = static_cast<int *>(S.counter.p);
+  a.done = reinterpret_cast<uint64_t *>(static_cast<char *>(S.res.dev) + res_bytes);
+  a.seq = ++S.seq;
+  volatile uint64_t *done = reinterpret_cast<volatile uint64_t *>(static_cast<char *>(S.res.host) + res_bytes);
+  *done = 0;
+  PQP_HIP(launch_minors_wave(W, a, 1, S.stream));
+  PQP_HIP(launch_minors_sum(W, a, S.stream));
+  if ((st = wait_done(S.stream, done, a.seq)) != PQP_OK) {
+    // a launch that did not finish its count leaves it behind
+    (void)hipMemsetAsync(S.counter.p, 0, sizeof(int), S.stream);
+    (void)hipStreamSynchronize(S.stream);
+    return st;
+  }
+  std::memcpy(out, S.res.host, static_cast<size_t>(W) * 2 * sizeof(double));
+  return PQP_OK;
 }
 
 // Buffers of the probability-table entry point, kept across calls (grown on
@@ -1849,6 +1976,7 @@ int pqp_laplace_c128(const double *matrix, int64_t m_r, int64_t m_c, int64_t ld,
   CallRange range_("pqp_laplace_c128");
   if (!out && m_c > 0) return fail(PQP_ERR_INVALID, "out is null");
   PermInput in{matrix, false, m_r, m_c, ld, rows, cols};
+  if (laplace_wave_fits(in)) return laplace_wave(in, out);
   PlanOptions opt;
   const DeviceState &dev = device_state();
   opt.auto_units_cap = static_cast<int64_t>(std::max(dev.cus, 1)) * kSingleUnitsPerCu;
@@ -2034,6 +2162,141 @@ int pqp_output_table_c128(const double *matrix, int64_t modes, int64_t ld, const
                            hipMemcpyDeviceToHost, S.stream));
     PQP_HIP(hipStreamSynchronize(S.stream));
     std::memcpy(out + per * s0, hout, static_cast<size_t>(rows) * per * sizeof(double));
+  }
+  return PQP_OK;
+}
+
+int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64_t shots, int64_t photons,
+                          const uint8_t *pools, const int32_t *steps, const int32_t *picks, const double *draws,
+                          int32_t *out) {
+  CallRange range_("pqp_sample_shots_c128");
+  if (modes < 1 || shots < 0 || photons < 0 || !matrix || ld < modes ||
+      (shots > 0 && (!steps || !out || (photons > 0 && (!pools || !picks || !draws)))))
+    return fail(PQP_ERR_INVALID, "invalid sampling arguments");
+  if (modes > kMinorsWaveMaxModes || photons > kMinorsWaveMaxCols)
+    return fail(PQP_ERR_RANGE, "sampling on the device supports at most " + std::to_string(kMinorsWaveMaxModes) +
+                                   " modes and " + std::to_string(kMinorsWaveMaxCols) + " photons");
+  for (int64_t s = 0; s < shots; ++s) {
+    if (steps[s] < 0 || steps[s] > photons) return fail(PQP_ERR_INVALID, "a shot's photons exceed its pool");
+    for (int32_t p = 0; p < steps[s]; ++p)
+      if (picks[p * shots + s] < 0 || picks[p * shots + s] >= photons - p)
+        return fail(PQP_ERR_INVALID, "a pick is out of the pool");
+    for (int64_t p = 0; p < photons; ++p)
+      if (pools[s * photons + p] >= modes) return fail(PQP_ERR_INVALID, "an input mode is out of range");
+  }
+  if (shots == 0) return PQP_OK;
+  int st;
+  if ((st = require_device()) != PQP_OK) return st;
+  MinorsState &S = sample_state();
+  std::lock_guard<std::mutex> lock(S.mu);
+  if (!S.init) {
+    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    S.init = true;
+  }
+  const int64_t most = std::min(shots, kSampleShots);
+  // Inner digits and waves per shot of each step's minors.  Most shots have
+  // bunched outputs and need fewer waves than 2^(step - 1) terms would; those
+  // left over end at once.  8 states a lane at least (the start and the sums
+  // cost as much as a handful of states), 64 where that leaves 8192 waves.
+  auto digits = [](int64_t n, int64_t step) {
+    int k = 3;
+    while (k < 6 && n * (int64_t{1} << (step - 1)) >= (int64_t{64} * 8192) << (k + 1)) ++k;
+    return k;
+  };
+  auto waves = [&](int64_t n, int64_t step) {
+    return static_cast<int32_t>(
+        std::min<int64_t>(64, std::max<int64_t>(1, (int64_t{1} << (step - 1)) >> (6 + digits(n, step)))));
+  };
+  // input: matrix, columns, photons, draws; work: the shots' columns,
+  // outputs, wave counts, the failure flag, partials
+  const size_t m2 = static_cast<size_t>(modes) * modes * 2 * sizeof(double);
+  const size_t o_draws = align256(m2);
+  const size_t o_steps = align256(o_draws + static_cast<size_t>(photons * most) * sizeof(double));
+  const size_t o_cols = align256(o_steps + static_cast<size_t>(most) * sizeof(int32_t));
+  const size_t in_bytes = o_cols + static_cast<size_t>(most * photons) + 1;
+  const size_t w_occ = align256(static_cast<size_t>(most * modes * photons) * 2 * sizeof(double));
+  const size_t w_units = align256(w_occ + static_cast<size_t>(most * modes));
+  const size_t w_failed = align256(w_units + static_cast<size_t>(most) * sizeof(int32_t));
+  const size_t w_part = w_failed + 256;
+  size_t part = 0;
+  for (int64_t step = 1; step < photons; ++step)
+    part = std::max(part, static_cast<size_t>(most) * waves(most, step) * 4 * (step + 1) * sizeof(double));
+  if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
+  if ((st = S.work.ensure(w_part + part)) != PQP_OK) return st;
+  if ((st = S.stage.ensure(std::max(in_bytes, w_failed + 256 - w_occ))) != PQP_OK) return st;
+  char *h = static_cast<char *>(S.stage.p);
+  char *d = static_cast<char *>(S.in.p);
+  char *w = static_cast<char *>(S.work.p);
+  for (int64_t s0 = 0; s0 < shots; s0 += most) {
+    const int64_t n = std::min(most, shots - s0);
+    for (int64_t i = 0; i < modes; ++i)
+      std::memcpy(h + static_cast<size_t>(i * modes) * 16, matrix + 2 * i * ld, static_cast<size_t>(modes) * 16);
+    for (int64_t p = 0; p < photons; ++p)
+      std::memcpy(h + o_draws + static_cast<size_t>(p * n) * 8, draws + p * shots + s0, static_cast<size_t>(n) * 8);
+    std::memcpy(h + o_steps, steps + s0, static_cast<size_t>(n) * sizeof(int32_t));
+    for (int64_t s = 0; s < n; ++s) {  // the input modes in the order they join
+      uint8_t pool[kMinorsWaveMaxCols];
+      uint8_t *cols = reinterpret_cast<uint8_t *>(h + o_cols) + s * photons;
+      if (photons) std::memcpy(pool, pools + (s0 + s) * photons, static_cast<size_t>(photons));
+      for (int64_t p = 0; p < photons; ++p) {
+        if (p >= steps[s0 + s]) {
+          cols[p] = 0;
+          continue;
+        }
+        const int32_t at = picks[p * shots + s0 + s];
+        cols[p] = pool[at];
+        std::memmove(pool + at, pool + at + 1, static_cast<size_t>(photons - p - 1 - at));
+      }
+    }
+    PQP_HIP(hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, S.stream));
+    SampleArgs a;
+    a.u_t = reinterpret_cast<const double *>(d);
+    a.draws = reinterpret_cast<const double *>(d + o_draws);
+    a.steps = reinterpret_cast<const int32_t *>(d + o_steps);
+    a.cols = reinterpret_cast<const uint8_t *>(d + o_cols);
+    a.v = reinterpret_cast<double *>(w);
+    a.occ = reinterpret_cast<uint8_t *>(w + w_occ);
+    a.units = reinterpret_cast<int32_t *>(w + w_units);
+    a.failed = reinterpret_cast<int32_t *>(w + w_failed);
+    a.partials = reinterpret_cast<const double *>(w + w_part);
+    a.shots = static_cast<int32_t>(n);
+    a.modes = static_cast<int32_t>(modes);
+    a.photons = static_cast<int32_t>(photons);
+    a.waves = 1;
+    PQP_HIP(launch_sample_columns(a, S.stream));
+    int64_t last = 0;
+    for (int64_t s = 0; s < n; ++s) last = std::max<int64_t>(last, steps[s0 + s]);
+    for (int64_t step = 0; step < last; ++step) {
+      if (step > 0) {
+        MinorsWaveArgs m;
+        m.rows = a.v;
+        m.occ = a.occ;
+        m.units = a.units;
+        m.partials = reinterpret_cast<double *>(w + w_part);
+        m.out = nullptr;
+        m.item_stride = 2 * modes * photons;
+        m.ld = static_cast<int32_t>(photons);
+        m.modes = static_cast<int32_t>(modes);
+        m.waves = waves(n, step);
+        m.k_max = digits(n, step);
+        m.last_counter = nullptr;
+        m.done = nullptr;
+        m.seq = 0;
+        PQP_HIP(launch_minors_wave(static_cast<int>(step) + 1, m, static_cast<int>(n), S.stream));
+        a.waves = m.waves;
+      }
+      a.step = static_cast<int32_t>(step);
+      a.next_waves = waves(n, step + 1);
+      a.next_k_max = digits(n, step + 1);
+      PQP_HIP(launch_sample_step(a, S.stream));
+    }
+    PQP_HIP(hipMemcpyAsync(h, w + w_occ, w_failed + sizeof(int32_t) - w_occ, hipMemcpyDeviceToHost, S.stream));
+    PQP_HIP(hipStreamSynchronize(S.stream));
+    int32_t failed = 0;
+    std::memcpy(&failed, h + (w_failed - w_occ), sizeof(failed));
+    if (failed) return fail(PQP_ERR_INVALID, "probabilities contain NaN");
+    const uint8_t *occ = reinterpret_cast<const uint8_t *>(h);
+    for (int64_t t = 0; t < n * modes; ++t) out[s0 * modes + t] = occ[t];
   }
   return PQP_OK;
 }

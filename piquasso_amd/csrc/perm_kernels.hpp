@@ -10,6 +10,7 @@
 #include "tensor_types.hpp"
 #include "poly_types.hpp"
 #include "table_types.hpp"
+#include "minors_wave_types.hpp"
 
 namespace pqp {
 
@@ -68,6 +69,14 @@ hipError_t launch_minors(int bucket, const LaunchArgs &a, int first_unit, int n_
                          hipStream_t stream);
 hipError_t launch_minors_finalize(const LaunchArgs &a, int n_items, int max_units,
                                   hipStream_t stream);
+
+// Column minors planned on the device (perm_minors_wave.hip): one launch for
+// the items of one width, the sum of a lone item's partials, and the two
+// kernels of the sampler around them.
+hipError_t launch_minors_wave(int width, const MinorsWaveArgs &a, int items, hipStream_t stream);
+hipError_t launch_minors_sum(int width, const MinorsWaveArgs &a, hipStream_t stream);
+hipError_t launch_sample_columns(const SampleArgs &a, hipStream_t stream);
+hipError_t launch_sample_step(const SampleArgs &a, hipStream_t stream);
 
 // Gradient kernels (perm_grad.hip), unit column multiplicities: buckets for
 // widths 1-8, 9-16, 17-19, 20, 21-32.

@@ -8,11 +8,7 @@
 // particles.  Such permanents are small (at most 2^(n-1) Gray terms), and
 // planning each on the host costs far more than its sum: 1.4 us against
 // 2 ns for 7 particles.  So the kernel gets the occupations, a byte per
-// mode, and every wave plans its own item: lane i holds t_i, ballots give
-// the rows of multiplicity 1 and of more, and the first smallest row is
-// prepended as in src/permanent.cpp:54-95.  The binary digits come first:
-// the lowest k are swept by all lanes in Gray order, the others and the
-// digits of larger radix are the lane's, read off its index.  U's occupied
+// mode, and every wave plans its own item (wave_plan.hpp).  U's occupied
 // columns (at most 16 KB for every item alike) are read with scalar loads,
 // a row at a time, so no table is built or loaded per item.
 //
@@ -37,6 +33,7 @@
 #include "perm_kernels.hpp"
 #include "sweep_common.hpp"
 #include "table_types.hpp"
+#include "wave_plan.hpp"
 
 namespace pqp {
 
@@ -84,17 +81,8 @@ __attribute__((amdgpu_waves_per_eu(W <= 8 ? 7 : W <= 12 ? 5 : 4, 8))) void perm_
   if (item >= a.count) return;  // whole blocks where NW > 1
   const int occ = lane < a.modes ? a.outs[item * a.modes + lane] : 0;
 
-  // the item's plan: rows by multiplicity, the prepended row
   int total = 0;
-  int i0 = 0, least = 0;
-  for (int v = 1; v <= a.n; ++v) {
-    const uint64_t at = __ballot(occ == v);
-    total += v * __builtin_popcountll(at);
-    if (at && !least) {
-      least = v;
-      i0 = __builtin_ctzll(at);
-    }
-  }
+  for (int v = 1; v <= a.n; ++v) total += v * __builtin_popcountll(__ballot(occ == v));
   const bool match = total == a.n && !__ballot(occ > a.n);
   double *out = a.out + (a.prob ? 1 : 2) * item;
   if (!match) {  // another particle number: amplitude 0
@@ -104,75 +92,17 @@ __attribute__((amdgpu_waves_per_eu(W <= 8 ? 7 : W <= 12 ? 5 : 4, 8))) void perm_
     }
     return;
   }
-  const int rho = occ - (lane == i0 ? 1 : 0);
-  uint64_t bin = __ballot(rho == 1);
-  const uint64_t multi = __ballot(rho > 1);
-  const uint64_t rows_in = bin | multi;
-  const int nb = __builtin_popcountll(bin);
-  int states = 1;  // of the digits of larger radix
-  for (uint64_t m = multi; m; m &= m - 1)
-    states *= __builtin_amdgcn_readlane(rho, __builtin_ctzll(m)) + 1;
-  // inner digits: as many of the binary ones as leave the lanes a state each
-  int k = 0;
-  while (k < 6 && k < nb && ((states << (nb - k - 1)) >= NW * kWave)) ++k;
-  uint64_t inner = 0;  // the inner rows, a byte each
-  for (int p = 0; p < k; ++p) {
-    inner |= static_cast<uint64_t>(__builtin_ctzll(bin)) << (8 * p);
-    bin &= bin - 1;
-  }
-  const int S = 1 << k;
-  const int U = states << (nb - k);
+  const WavePlan p = wave_plan(occ, a.n, NW * kWave, 6);
+  const int S = 1 << p.k;
   const cptr<double> rows = as_const<double>(a.rows);
   const cptr<int32_t> mult = as_const<int32_t>(a.mult);
 
   cdd sum = cdd_zero();
-  for (int u0 = wave * kWave; u0 < U; u0 += NW * kWave) {
-    const bool active = u0 + lane < U;
-    const int u = active ? u0 + lane : 0;
-    // row sums of the lane's first state
+  for (int u0 = wave * kWave; u0 < p.U; u0 += NW * kWave) {
+    const bool active = u0 + lane < p.U;
     double cr[W], ci[W];
-    {
-      // an opaque index: the row is loop-invariant, and hoisting it would
-      // hold a second set of row sums in registers
-      int r0 = i0;
-      __asm__ volatile("" : "+s"(r0));
-      const cptr<double> b = rows + r0 * (2 * W);
-#pragma unroll
-      for (int j = 0; j < W; ++j) {
-        cr[j] = b[2 * j];
-        ci[j] = b[2 * j + 1];
-      }
-    }
-    auto add_row = [&](int r, double al) {
-      const cptr<double> b = rows + r * (2 * W);
-#pragma unroll
-      for (int j = 0; j < W; ++j) {
-        cr[j] = fmaR(al, b[2 * j], cr[j]);
-        ci[j] = fmaR(al, b[2 * j + 1], ci[j]);
-      }
-    };
-    int rest = u, parity = 0;
-    double w = 1.0;
-    for (uint64_t m = rows_in; m; m &= m - 1) {  // one loop for all digits: one block of row sums
-      const int r = __builtin_ctzll(m);
-      const int rr = __builtin_amdgcn_readlane(rho, r);
-      double al = in_vgpr(1.0);  // inner digits start at 0
-      if (rr > 1) {
-        // u < 2^16: the quotient by a radix <= 17 is exact this way
-        const int q = static_cast<int>((static_cast<double>(rest) + 0.5) * (1.0 / (rr + 1)));
-        const int g = rest - q * (rr + 1);
-        rest = q;
-        parity ^= g & 1;
-        w *= lane_binomial(rr, g);
-        al = static_cast<double>(rr - 2 * g);
-      } else if ((bin >> r) & 1) {
-        al = (rest & 1) ? -1.0 : 1.0;
-        parity ^= rest & 1;
-        rest >>= 1;
-      }
-      add_row(r, al);
-    }
-    w = active ? (parity ? -w : w) : 0.0;
+    const double w_top = wave_start<W>(p, active ? u0 + lane : 0, rows, 2 * W, cr, ci);
+    const double w = active ? w_top : 0.0;
     // the inner states in Gray order
     double sr = 0.0, si = 0.0;
     for (int v = 0; v < S; ++v) {
@@ -180,10 +110,13 @@ __attribute__((amdgpu_waves_per_eu(W <= 8 ? 7 : W <= 12 ? 5 : 4, 8))) void perm_
       table_product<W, ONES>(cr, ci, mult, pr, pi);
       sr += (v & 1) ? -pr : pr;
       si += (v & 1) ? -pi : pi;
-      // the update after the last state (digit k: row 0) is never read
-      const int b = __builtin_ctz(v + 1);
-      const int up = (v + 1) ^ ((v + 1) >> 1);
-      add_row(static_cast<int>((inner >> (8 * b)) & 255), in_vgpr((up >> b & 1) ? -2.0 : 2.0));
+      const cptr<double> b = rows + wave_step_row(p, v) * (2 * W);
+      const double s2 = in_vgpr(wave_step_factor(v));
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        cr[j] = fmaR(s2, b[2 * j], cr[j]);
+        ci[j] = fmaR(s2, b[2 * j + 1], ci[j]);
+      }
     }
     sum = cdd_add(sum, cdd{dd_mul_d(dd{sr, 0.0}, w), dd_mul_d(dd{si, 0.0}, w)});
   }

@@ -6,10 +6,13 @@ by photon, the next output mode is drawn from a distribution built from the
 column minors perm(U_sub; sample, input - e_l) of the interferometer
 (piquasso/_simulators/passive/sampling.py:197-236,711-753).  The reference
 runs the shots one after the other and calls ``permanent_laplace`` once per
-shot and photon.  Here every shot advances one photon per round and each
-round's minors of all shots come from ONE launch of the column-minor kernels
-(``pqp_laplace_batch_c128``); the bookkeeping around them (input growth,
-distributions, draws) is vectorised over the shots.
+shot and photon.  Here every shot advances one photon per round.  Without
+postselection (up to 24 photons in 64 modes) all draws are made first and
+every round of all shots runs on the device in one call
+(``pqp_sample_shots_c128``).  Otherwise each round's minors of all shots come
+from one launch of the column-minor kernels (``pqp_laplace_batch_c128``); the
+bookkeeping around them (input growth, distributions, draws) is vectorised
+over the shots.
 
 The samples equal the reference's for equal seeds.  Each shot draws from its
 own ``numpy.random.default_rng(seed + shot)`` (sampling.py:178-193) in the
@@ -56,9 +59,9 @@ __all__ = ["generate_samples", "generate_lossy_samples", "expanded_lossy_matrix"
 
 # Counters of the most recent generate_samples call in this process: rounds,
 # column-minor problems, the seconds spent in the batched minors calls
-# (planning, upload, kernels, download) and in total, and, when
-# ``count_flops`` is set, the minors' algorithmic FLOP (off by default: it
-# costs host time every round).
+# (planning, upload, kernels, download) or the device rounds and in total,
+# and, when ``count_flops`` is set, the minors' algorithmic FLOP (off by
+# default: the rounds then run in lockstep with the host).
 last_run: dict = {}
 count_flops = False
 
@@ -129,6 +132,28 @@ class _MinorsBatch:
         _capi.check(st)
         return out.view(np.complex128)
 
+    # sizes pqp_sample_shots_c128 takes; larger samplings run in lockstep
+    device_modes = 64
+    device_photons = 24
+
+    def sample(self, pools, steps, picks, draws) -> np.ndarray:
+        """Outputs of shots that place steps[s] photons of pools[s]: photon p
+        is the picks[p, s]-th of those left and goes where draws[p, s] falls."""
+        t0 = time.perf_counter()
+        shots, photons = pools.shape
+        out = np.empty((shots, self.d), dtype=np.int32)
+        pools = np.ascontiguousarray(pools, dtype=np.uint8)
+        steps = np.ascontiguousarray(steps, dtype=np.int32)
+        picks = np.ascontiguousarray(picks, dtype=np.int32)
+        draws = np.ascontiguousarray(draws, dtype=np.float64)
+        _capi.check(self.lib.pqp_sample_shots_c128(
+            self.u.view(np.float64).ctypes.data_as(self._dp), self.d, self.d, shots, photons,
+            pools.ctypes.data_as(ctypes.POINTER(ctypes.c_uint8)), steps.ctypes.data_as(self._i32p),
+            picks.ctypes.data_as(self._i32p), draws.ctypes.data_as(self._dp),
+            out.ctypes.data_as(self._i32p)))
+        self.seconds += time.perf_counter() - t0
+        return out
+
 
 _U32 = np.uint64(0xFFFFFFFF)
 
@@ -146,16 +171,17 @@ class _Draws:
     generators' states run ahead by the unused part of the blocks, so the
     engine must be the generators' last user."""
 
-    def __init__(self, rngs, block: int):
+    def __init__(self, rngs, block: int, fresh: bool = False):
         S = len(rngs)
-        self.bgs = [r.bit_generator for r in rngs]
+        self.bgs = [getattr(r, "bit_generator", r) for r in rngs]
         self.raw = np.empty((S, max(block, 1)), dtype=np.uint64)
         self.has32 = np.zeros(S, dtype=bool)
         self.cache = np.zeros(S, dtype=np.uint64)
         for k, bg in enumerate(self.bgs):
-            st = bg.state
-            self.has32[k] = bool(st["has_uint32"])
-            self.cache[k] = np.uint64(st["uinteger"])
+            if not fresh:  # a fresh generator holds no half
+                st = bg.state
+                self.has32[k] = bool(st["has_uint32"])
+                self.cache[k] = np.uint64(st["uinteger"])
             self.raw[k] = bg.random_raw(self.raw.shape[1])
         self.ptr = np.zeros(S, dtype=np.int64)
 
@@ -201,6 +227,43 @@ class _Draws:
             rej[i] = left[i] < thr[i]
         res[act] = (m >> np.uint64(32)).astype(np.int64)
         return res
+
+
+class _OnDevice:
+    """The shots of a sampling without postselection: which particles a shot
+    keeps and the order they join do not depend on the outputs, so every draw
+    is made here, in :class:`_Lockstep`'s order (per photon the particle, then
+    the number that places it), and the steps run on the device in one call."""
+
+    flops = 0.0
+
+    def __init__(self, minors: _MinorsBatch, rngs, pools, keep, fresh: bool):
+        S = len(pools)
+        self.minors = minors
+        n = np.array([len(p) for p in pools], dtype=np.int64)
+        width = max(int(n.max()), 1)
+        self.pools = np.zeros((S, width), dtype=np.uint8)
+        if all(p is pools[0] for p in pools):
+            self.pools[:] = pools[0] if len(pools[0]) else 0
+        else:
+            for s, p in enumerate(pools):
+                self.pools[s, : len(p)] = p
+        self.steps = n if keep is None else keep
+        most = int(self.steps.max())
+        draws = _Draws(rngs, most * 3 // 2 + 4, fresh)
+        self.picks = np.zeros((width, S), dtype=np.int32)
+        self.u = np.zeros((width, S))
+        for p in range(most):
+            live = np.flatnonzero(self.steps > p)
+            self.picks[p, live] = draws.integers(live, n[live] - p)
+            self.u[p, live] = draws.doubles(live)
+        self.rounds = most
+        self.problems = int(self.steps.sum())
+
+    def run(self) -> np.ndarray:
+        if self.rounds == 0:
+            return np.zeros((len(self.steps), self.minors.d), dtype=np.int32)
+        return self.minors.sample(self.pools, self.steps, self.picks, self.u)
 
 
 class _Lockstep:
@@ -445,7 +508,13 @@ def _sample_shots(minors, occ, shots, seed, reject_condition, ps_modes, ps_photo
     d = len(occ)
     n = int(occ.sum())
     postselected = len(ps_modes) > 0
-    rngs = [np.random.default_rng(seed=seed + s) for s in range(shots)]
+    on_device = (not postselected and not count_flops and d <= getattr(minors, "device_modes", 0)
+                 and n <= getattr(minors, "device_photons", 0))
+    if on_device and uniform_particle_overlap is None:
+        # default_rng(seed)'s bit generators alone: only raw outputs are drawn
+        rngs = [np.random.PCG64(seed + s) for s in range(shots)]
+    else:
+        rngs = [np.random.default_rng(seed=seed + s) for s in range(shots)]
 
     if postselected and uniform_particle_overlap is not None:
         # restarts depend on the draws: the shots run one after another
@@ -493,8 +562,17 @@ def _sample_shots(minors, occ, shots, seed, reject_condition, ps_modes, ps_photo
             indist, dist = _split_particles(occ, float(uniform_particle_overlap), rngs[s])
             dist_out[s] = _distinguishable(u, dist, rngs[s], lambda s=s: reject_one(s))
             pools.append(_first_quantized(indist))
-    eng = _Lockstep(minors, rngs, pools, reject_many if decisions is not None else None,
-                    (ps_modes, ps_photons, max_trials) if postselected else None, fast_draws=True)
+    if on_device:
+        keep = None
+        if decisions is not None:
+            # a shot takes one decision per particle of its pool, after those
+            # its distinguishable particles took
+            keep = np.array([len(p) - int(decisions[s, pointer[s]:pointer[s] + len(p)].sum())
+                             for s, p in enumerate(pools)], dtype=np.int64)
+        eng = _OnDevice(minors, rngs, pools, keep, fresh=dist_out is None)
+    else:
+        eng = _Lockstep(minors, rngs, pools, reject_many if decisions is not None else None,
+                        (ps_modes, ps_photons, max_trials) if postselected else None, fast_draws=True)
     engines.append(eng)
     smp = eng.run().astype(np.int64)
     if dist_out is not None:
