@@ -302,6 +302,18 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
                                     double *abs_sum);
 
 /*
+ * Permanents of `count` problems evaluated once: pqp_batch_create, an eager
+ * run and pqp_batch_results in one call, on buffers and streams the library
+ * keeps between calls (released after a call that grew them beyond 256 MiB).
+ * Arguments as in pqp_batch_create, complex128; flags PQP_FLAG_FP32,
+ * _STATIC, _EXPAND_COLS, _KEEP_COLS, _AS_GIVEN; out: 2 doubles per problem.
+ */
+int pqp_permanent_batch_c128(int64_t count, const double *const *matrices, const int64_t *m_r,
+                             const int64_t *m_c, const int64_t *ld, const int32_t *const *rows,
+                             const int32_t *const *cols, uint32_t flags, int64_t target_inner,
+                             int64_t total_units, double *out);
+
+/*
  * Clifford & Clifford boson sampling, all steps of all shots on the device
  * (piquasso/_simulators/passive/sampling.py:208-236,711-753).  Shot s places
  * steps[s] <= photons photons of its pool (pools: shots x photons input

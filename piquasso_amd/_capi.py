@@ -104,6 +104,11 @@ SIGNATURES = {
     "pqp_perm_poly_plan_info": (
         _c.c_int, [_c.c_int64, _c.c_int64, _c.c_int64, _i32p, _i64p],
     ),
+    "pqp_permanent_batch_c128": (
+        _c.c_int,
+        [_c.c_int64, _c.POINTER(_dp), _i64p, _i64p, _i64p, _c.POINTER(_i32p), _c.POINTER(_i32p),
+         _c.c_uint32, _c.c_int64, _c.c_int64, _dp],
+    ),
     "pqp_sample_shots_c128": (
         _c.c_int,
         [_dp, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.POINTER(_c.c_uint8), _i32p, _i32p, _dp, _i32p],

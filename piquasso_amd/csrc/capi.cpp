@@ -131,6 +131,8 @@ constexpr int64_t kLaplaceWaves = 2048;
 // Shots of one pass of the sampler (its buffers: 64 partials of 48
 // components and 24 columns of 64 modes each, 200 MB at most).
 constexpr int64_t kSampleShots = 2048;
+// Device buffers a one-shot batch may leave for the next one.
+constexpr size_t kKeptBytes = size_t{256} << 20;
 
 int expand_mode(uint32_t flags) {
   if (flags & PQP_FLAG_EXPAND_COLS) return 1;
@@ -2472,6 +2474,61 @@ int pqp_batch_create(int64_t count, const void *const *matrices, int is_c64, con
   }
   PQP_HIP(hipStreamSynchronize(b->x.stream));
   *out = b.release();
+  return PQP_OK;
+}
+
+int pqp_permanent_batch_c128(int64_t count, const double *const *matrices, const int64_t *m_r,
+                             const int64_t *m_c, const int64_t *ld, const int32_t *const *rows,
+                             const int32_t *const *cols, uint32_t flags, int64_t target_inner,
+                             int64_t total_units, double *out) {
+  CallRange range_("pqp_permanent_batch_c128");
+  if (count < 0 || (count > 0 && (!matrices || !m_r || !m_c || !ld || !rows || !cols || !out)))
+    return fail(PQP_ERR_INVALID, "invalid batch arguments");
+  if (count > INT32_MAX) return fail(PQP_ERR_RANGE, "too many items");
+  std::vector<PermInput> inputs(static_cast<size_t>(count));
+  for (int64_t k = 0; k < count; ++k)
+    inputs[k] = PermInput{matrices[k], false, m_r[k], m_c[k], ld[k], rows[k], cols[k]};
+  PlanOptions opt;
+  opt.fp32_products = (flags & PQP_FLAG_FP32) != 0;
+  opt.expand_cols = expand_mode(flags);
+  opt.orient = (flags & PQP_FLAG_AS_GIVEN) == 0;
+  opt.target_inner = target_inner;
+  opt.total_units = total_units > 0
+                        ? total_units
+                        : static_cast<int64_t>(std::max(device_state().cus, 1)) * kBatchUnitsPerCu;
+  Plan plan;
+  std::string err;
+  int st = plan_build(inputs, opt, plan, err);
+  if (st != PQP_OK) return fail(st, err);
+  if ((st = require_device()) != PQP_OK) return st;
+  if (count == 0) return PQP_OK;
+  SingleState &S = single_state();
+  std::lock_guard<std::mutex> lock(S.mu);
+  Exec &x = S.x;
+  if (!S.init) {
+    PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
+    x.own_stream = true;
+    S.init = true;
+  }
+  x.plan = std::move(plan);
+  index_units(x);
+  x.flags = flags;
+  const size_t out_bytes = static_cast<size_t>(count) * 2 * sizeof(double);
+  if ((st = x.stage.ensure(std::max(x.plan.arena.size(), out_bytes))) != PQP_OK) return st;
+  if ((st = upload(x)) != PQP_OK) return st;
+  if ((st = enqueue(x, PQP_RUN_EAGER, nullptr, nullptr)) != PQP_OK) return st;
+  // item k's value is result k; the copy follows the upload out of the
+  // staging buffer on the stream
+  PQP_HIP(hipMemcpyAsync(x.stage.p, x.results.p, out_bytes, hipMemcpyDeviceToHost, x.stream));
+  PQP_HIP(hipStreamSynchronize(x.stream));
+  std::memcpy(out, x.stage.p, out_bytes);
+  if (x.arena.bytes + x.partials.bytes > kKeptBytes) {
+    x.plan = Plan();
+    x.arena.release();
+    x.partials.release();
+    x.results.release();
+    x.stage.release();
+  }
   return PQP_OK;
 }
 

@@ -31,6 +31,7 @@ MODES = {
 
 _dp = ctypes.POINTER(ctypes.c_double)
 _i32p = ctypes.POINTER(ctypes.c_int32)
+_i64p = ctypes.POINTER(ctypes.c_int64)
 
 
 def _prep(matrix, rows, cols, dtype=np.complex128):
@@ -99,6 +100,51 @@ def _shared_marshal(matrices, rows, cols):
             np.full(n, m_c, dtype=np.int64))
 
 
+def _packed(matrices, rows, cols, terms: bool):
+    """Arguments of a batched C call from lists of arrays through the CPython
+    binding: (pointer arrays, m_r, m_c, buffers to keep, log2 of the mean Gray
+    terms); None when the binding is absent or an item has another form."""
+    from ._math.permanent import _fast_module
+
+    fast = _fast_module()
+    if not fast or len(matrices) == 0:
+        return None
+    sample = None
+    if terms:
+        from .tune import sampled_items
+
+        sample = sampled_items(len(matrices))
+    got = fast.pack(matrices, rows, cols, sample)
+    if got is None:
+        return None
+    mats, rp, cp, m_r, m_c, buf, mean = got
+    return ((mats, rp, cp), np.frombuffer(m_r, dtype=np.int64), np.frombuffer(m_c, dtype=np.int64),
+            (got, matrices), float(np.log2(mean)) if terms else None)
+
+
+def _tuned_launch(count, rows, persistent, target_inner, total_units, log2_terms=None):
+    """The caller's launch settings completed by the tuned ones."""
+    if persistent is None or not total_units:
+        from .tune import best_config, mean_log2_terms
+
+        try:
+            _, cus, arch = _capi.device_info()
+            if log2_terms is None:
+                log2_terms = mean_log2_terms(rows)
+            tuned = best_config(count, cus, arch, log2_terms=log2_terms)
+        except RuntimeError:  # no device: the call fails below with the C library's error
+            tuned = {}
+        if persistent is None:
+            persistent = bool(tuned.get("persistent", False))
+        if not total_units:
+            total_units = int(tuned.get("total_units", 0))
+            # a tuned inner-sweep length replaces the split total_units
+            # asks for, so it applies only where the caller gave neither
+            if not target_inner:
+                target_inner = int(tuned.get("target_inner", 0))
+    return persistent, target_inner, total_units
+
+
 class PermanentBatch:
     """A planned batch of permanents resident on the GPU.
 
@@ -157,33 +203,26 @@ class PermanentBatch:
             raise ValueError("precision must be 'fp64' or 'fp32'")
         self.count = len(matrices)
         self.precision = precision
+        n = self.count
+        shared = _shared_marshal(matrices, rows, cols)
+        packed = _packed(matrices, rows, cols, not gradient) if shared is None else None
         if gradient:
             # gradient sweeps: one block per work unit, the library's unit count
             if persistent is None:
                 persistent = False
-        elif persistent is None or not total_units:
-            from .tune import best_config, mean_log2_terms
-
-            try:
-                _, cus, arch = _capi.device_info()
-                tuned = best_config(len(matrices), cus, arch, log2_terms=mean_log2_terms(rows))
-            except RuntimeError:  # no device: creation fails below with the C library's error
-                tuned = {}
-            if persistent is None:
-                persistent = bool(tuned.get("persistent", False))
-            if not total_units:
-                total_units = int(tuned.get("total_units", 0))
-                # a tuned inner-sweep length replaces the split total_units
-                # asks for, so it applies only where the caller gave neither
-                if not target_inner:
-                    target_inner = int(tuned.get("target_inner", 0))
+        else:
+            persistent, target_inner, total_units = _tuned_launch(
+                n, rows, persistent, target_inner, total_units, packed[4] if packed else None)
         self.gradient = bool(gradient)
-        n = self.count
-        shared = _shared_marshal(matrices, rows, cols)
         if shared is not None:
             # one matrix for every item and multiplicities that stack into
             # two int32 arrays (probability tables): addresses by arithmetic
             self._keep, mat_arr, row_arr, col_arr, m_r, m_c = shared
+        elif packed is not None:
+            (mats, rp, cp), m_r, m_c, self._keep, _ = packed
+            mat_arr = ctypes.cast(mats, ctypes.POINTER(ctypes.c_void_p))
+            row_arr = ctypes.cast(rp, ctypes.POINTER(_i32p))
+            col_arr = ctypes.cast(cp, ctypes.POINTER(_i32p))
         else:
             self._keep = []
             mats, rws, cls = [], [], []
@@ -221,7 +260,7 @@ class PermanentBatch:
         )
         _capi.check(st)
         self._h = handle
-        self._shapes = [(int(m_r[k]), int(m_c[k])) for k in range(n)]
+        self._shapes = list(zip(m_r.tolist(), m_c.tolist()))[:n]
         self._keep = None  # inputs were copied into the plan
 
     # -- running ---------------------------------------------------------
@@ -328,7 +367,23 @@ class PermanentBatch:
 def permanent_batch(matrices, rows, cols, precision: str = "fp64",
                     target_inner: int = 0) -> np.ndarray:
     """Permanents of many (matrix, rows, cols) triples in one launch."""
-    with PermanentBatch(matrices, rows, cols, precision=precision,
-                        target_inner=target_inner) as b:
-        b.run("eager")
-        return b.results()
+    packed = None
+    if precision in ("fp64", "fp32") and len(matrices) == len(rows) == len(cols):
+        packed = _packed(matrices, rows, cols, True)
+    if packed is None:
+        with PermanentBatch(matrices, rows, cols, precision=precision,
+                            target_inner=target_inner) as b:
+            b.run("eager")
+            return b.results()
+    # inputs that are evaluated once: no handle, the library's own buffers
+    (mats, rp, cp), m_r, m_c, _keep, log2_terms = packed
+    n = len(matrices)
+    persistent, target_inner, total_units = _tuned_launch(n, rows, None, target_inner, 0, log2_terms)
+    flags = (_capi.PQP_FLAG_FP32 if precision == "fp32" else 0) | (0 if persistent else _capi.PQP_FLAG_STATIC)
+    out = np.empty(n, dtype=np.complex128)
+    shape = m_c.ctypes.data_as(_i64p)
+    _capi.check(_capi.lib().pqp_permanent_batch_c128(
+        n, ctypes.cast(mats, ctypes.POINTER(_dp)), m_r.ctypes.data_as(_i64p), shape, shape,
+        ctypes.cast(rp, ctypes.POINTER(_i32p)), ctypes.cast(cp, ctypes.POINTER(_i32p)), flags,
+        int(target_inner), int(total_units), out.view(np.float64).ctypes.data_as(_dp)))
+    return out

@@ -33,6 +33,7 @@ from typing import Sequence
 import numpy as np
 
 from . import _capi
+from .engine import _packed
 
 __all__ = ["permanent_grad", "permanent_grad_batch", "PermanentFunction", "torch_permanent",
            "PermanentBatchFunction", "torch_permanent_batch"]
@@ -62,27 +63,45 @@ def permanent_grad_batch(matrices: Sequence, rows: Sequence, cols: Sequence):
     list of complex128 arrays, ``grads[k]`` of the shape of ``matrices[k]``.
     Raises ``RuntimeError`` when an item's multiplicities do not sum to the
     same number (as ``permanent`` does)."""
+    perms, flat, shapes = _grad_batch(matrices, rows, cols)
+    grads, at = [], 0
+    for m_r, m_c in shapes:
+        grads.append(flat[at: at + m_r * m_c].reshape(m_r, m_c))
+        at += m_r * m_c
+    return perms, grads
+
+
+def _grad_batch(matrices, rows, cols):
+    """The permanents, all gradients one after another, and their shapes."""
     if not (len(matrices) == len(rows) == len(cols)):
         raise ValueError("matrices, rows and cols must have the same length")
-    items = [_prep(m, r, c) for m, r, c in zip(matrices, rows, cols)]
-    n = len(items)
-    grads = [np.zeros(a.shape, dtype=np.complex128) for a, _, _ in items]
-    perms = np.zeros(max(n, 1), dtype=np.complex128)
+    n = len(matrices)
     if n == 0:
-        return perms[:0], grads
-    mats = (_dp * n)(*[a.view(np.float64).ctypes.data_as(_dp) for a, _, _ in items])
-    rws = (_i32p * n)(*[r.ctypes.data_as(_i32p) for _, r, _ in items])
-    cls = (_i32p * n)(*[c.ctypes.data_as(_i32p) for _, _, c in items])
-    outs = (_dp * n)(*[g.view(np.float64).ctypes.data_as(_dp) for g in grads])
-    m_r = np.array([a.shape[0] for a, _, _ in items], dtype=np.int64)
-    m_c = np.array([a.shape[1] for a, _, _ in items], dtype=np.int64)
+        return np.zeros(0, dtype=np.complex128), np.zeros(0, dtype=np.complex128), []
+    packed = _packed(matrices, rows, cols, False)
+    if packed is not None:
+        (mats, rp, cp), m_r, m_c, _keep, _ = packed
+        mats = ctypes.cast(mats, ctypes.POINTER(_dp))
+        rws, cls = ctypes.cast(rp, ctypes.POINTER(_i32p)), ctypes.cast(cp, ctypes.POINTER(_i32p))
+    else:
+        items = [_prep(m, r, c) for m, r, c in zip(matrices, rows, cols)]
+        mats = (_dp * n)(*[a.view(np.float64).ctypes.data_as(_dp) for a, _, _ in items])
+        rws = (_i32p * n)(*[r.ctypes.data_as(_i32p) for _, r, _ in items])
+        cls = (_i32p * n)(*[c.ctypes.data_as(_i32p) for _, _, c in items])
+        m_r = np.array([a.shape[0] for a, _, _ in items], dtype=np.int64)
+        m_c = np.array([a.shape[1] for a, _, _ in items], dtype=np.int64)
+    ends = np.cumsum(m_r * m_c)
+    perms = np.zeros(n, dtype=np.complex128)
+    flat = np.empty(max(int(ends[-1]), 1), dtype=np.complex128)  # the call writes every entry
+    outs = (flat.ctypes.data + 16 * (ends - m_r * m_c)).astype(np.uint64)
     _capi.check(
         _capi.lib().pqp_grad_batch_c128(
             n, mats, m_r.ctypes.data_as(_i64p), m_c.ctypes.data_as(_i64p),
-            m_c.ctypes.data_as(_i64p), rws, cls, perms.view(np.float64).ctypes.data_as(_dp), outs,
+            m_c.ctypes.data_as(_i64p), rws, cls, perms.view(np.float64).ctypes.data_as(_dp),
+            outs.ctypes.data_as(ctypes.POINTER(_dp)),
         )
     )
-    return perms[:n], grads
+    return perms, flat, list(zip(m_r.tolist(), m_c.tolist()))
 
 
 def permanent_grad(matrix, rows, cols) -> np.ndarray:
@@ -182,8 +201,8 @@ class PermanentBatchFunction:
                     if r.shape != (B, a.shape[1]) or c.shape != (B, a.shape[2]):
                         raise ValueError("rows / cols must have shapes (B, m_r) / (B, m_c)")
                     if A.requires_grad:
-                        perms, grads = permanent_grad_batch(list(a), list(r), list(c))
-                        G = np.stack(grads) if B else np.zeros(a.shape, dtype=np.complex128)
+                        perms, flat, _ = _grad_batch(list(a), list(r), list(c))
+                        G = flat[: a.size].reshape(a.shape)
                         ctx.save_for_backward(torch.from_numpy(G).to(A.device, A.dtype))
                     else:
                         from .engine import permanent_batch

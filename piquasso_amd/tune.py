@@ -163,6 +163,11 @@ def best_config(count: int, cus: int, arch: str, path: str = None, log2_terms=No
     return {k: v for k, v in cfg.items() if k in ("total_units", "persistent", "target_inner")}
 
 
+def sampled_items(n: int, sample: int = 256) -> np.ndarray:
+    """Up to `sample` evenly spaced item indices of a batch of n."""
+    return np.unique(np.linspace(0, n - 1, min(n, sample)).astype(np.int64))
+
+
 def mean_log2_terms(rows, sample: int = 256) -> float:
     """log2 of the mean Gray term count over (up to `sample` evenly spaced)
     items' row multiplicities."""
@@ -171,7 +176,7 @@ def mean_log2_terms(rows, sample: int = 256) -> float:
     n = len(rows)
     if n == 0:
         return 0.0
-    idx = np.unique(np.linspace(0, n - 1, min(n, sample)).astype(int))
+    idx = sampled_items(n, sample)
     return float(np.log2(np.mean([float(glynn_terms(rows[k])) for k in idx])))
 
 
@@ -200,12 +205,23 @@ def tune(out: str = DEFAULT_TABLE, reps: int = 5, only=None, log=print) -> dict:
     return table
 
 
+_loaded: dict = {}  # path -> ((mtime, size), table)
+
+
 def load_tuning(path: str = DEFAULT_TABLE) -> dict:
-    """The tuned table, or {} when none has been written for this device."""
-    if not os.path.exists(path):
+    """The tuned table, or {} when none has been written for this device
+    (read again when the file changes)."""
+    try:
+        st = os.stat(path)
+    except OSError:
         return {}
-    with open(path) as f:
-        return json.load(f)
+    stamp = (st.st_mtime_ns, st.st_size)
+    held = _loaded.get(path)
+    if held is None or held[0] != stamp:
+        with open(path) as f:
+            held = (stamp, json.load(f))
+        _loaded[path] = held
+    return held[1]
 
 
 def main():
