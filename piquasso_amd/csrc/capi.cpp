@@ -131,6 +131,10 @@ constexpr int64_t kLaplaceWaves = 2048;
 // Shots of one pass of the sampler (its buffers: 64 partials of 48
 // components and 24 columns of 64 modes each, 200 MB at most).
 constexpr int64_t kSampleShots = 2048;
+// Waves of an exact permanent before its lanes sweep more states, and inner
+// digits at most.
+constexpr int64_t kIntWaves = 4096;
+constexpr int kIntInnerDigits = 7;
 // Device buffers a one-shot batch may leave for the next one.
 constexpr size_t kKeptBytes = size_t{256} << 20;
 
@@ -462,8 +466,6 @@ struct SingleState {
   std::mutex mu;
   Exec x;       // column minors, gradients, tensor permanents
   bool init = false;
-  Exec xi;      // exact integer permanents
-  bool init_i = false;
   Exec xs;      // single permanents: results in mapped host memory
   bool init_s = false;
   // the plan resident in xs and its key (shape, multiplicities, flags)
@@ -679,101 +681,6 @@ IntScan int_scan(const PermInput &in) {
   return sc;
 }
 
-// The exact permanent of an integral matrix (int_scan(in).integral) as
-// two's complement limbs: the multi-modular Glynn sweep of perm_int.hip and
-// Garner's reconstruction.  PQP_ERR_RANGE when the row sums or binomial
-// weights leave FP64's exact integers or the permanent may exceed the
-// product of the moduli / 4.
-int run_int(const PermInput &in, const IntScan &sc, uint64_t *v) {
-  // the matrix as contiguous complex128: the plan's B rows
-  std::vector<double> a(static_cast<size_t>(std::max<int64_t>(in.m_r * in.m_c, 1)) * 2, 0.0);
-  for (int64_t i = 0; i < in.m_r; ++i)
-    for (int64_t j = 0; j < in.m_c; ++j)
-      a[static_cast<size_t>(2 * (i * in.m_c + j))] =
-          in.a_is_float ? static_cast<const float *>(in.a)[2 * (i * in.ld + j)]
-                        : static_cast<const double *>(in.a)[2 * (i * in.ld + j)];
-  PlanOptions opt = single_plan_options(PQP_FLAG_AS_GIVEN, in);
-  opt.direct_out = false;
-  opt.expand_cols = 1;  // unit column multiplicities: the product is over n factors
-  opt.pad8 = true;
-  Plan plan;
-  std::string err;
-  const PermInput ind{a.data(), false, in.m_r, in.m_c, in.m_c, in.rows, in.cols};
-  int st = plan_build(std::vector<PermInput>{ind}, opt, plan, err);
-  if (st != PQP_OK) return fail(st, err);
-  if (!sc.integral)
-    return fail(PQP_ERR_RANGE, "matrix entries are not all integers of magnitude <= 2^47");
-  if (sc.rmax > std::ldexp(1.0, 48)) return fail(PQP_ERR_RANGE, "row sums of the matrix exceed 2^48");
-  if (sc.log2_weight > 52.0)
-    return fail(PQP_ERR_RANGE, "binomial weights of the row multiplicities exceed 2^52");
-  // products of G row sums stay below 2^49: exact in FP64 and valid
-  // inputs of the modular multiply
-  const double lr = sc.rmax > 1.0 ? std::log2(sc.rmax) : 0.0;
-  const int group = 4.0 * lr <= 49.0 ? 4 : (2.0 * lr <= 49.0 ? 2 : 1);
-  // moduli: their product (each prime > 2^48.99) must exceed 4 |perm|
-  const int K = std::max(1, static_cast<int>(std::ceil((std::max(sc.log2_perm, 0.0) + 2.0) / 48.99)));
-  if (K > kIntMaxPrimes)
-    return fail(PQP_ERR_RANGE, "the permanent may exceed 2^390 in magnitude: beyond the eight moduli");
-  const ItemDesc &d = plan.items[0];
-  if (d.n == 0) {  // empty selection: 1 (src/permanent.cpp:106-108)
-    std::memset(v, 0, kIntLimbs * sizeof(uint64_t));
-    v[0] = 1;
-    return PQP_OK;
-  }
-  // the moduli table: p, 1/p, 2^-(n-1) mod p
-  const int64_t mod_off = (static_cast<int64_t>(plan.arena.size()) + 63) / 64 * 64;
-  plan.arena.resize(static_cast<size_t>(mod_off) + 3 * kIntMaxPrimes * sizeof(double), 0);
-  double *mt = reinterpret_cast<double *>(plan.arena.data() + mod_off);
-  for (int k = 0; k < kIntMaxPrimes; ++k) {
-    const uint64_t p = kIntPrimes[k];
-    mt[k] = static_cast<double>(p);
-    mt[kIntMaxPrimes + k] = 1.0 / static_cast<double>(p);
-    const uint64_t inv2 = pow_mod((p + 1) / 2, static_cast<uint64_t>(d.n > 0 ? d.n - 1 : 0), p);
-    mt[2 * kIntMaxPrimes + k] = static_cast<double>(inv2);
-  }
-  if ((st = require_device()) != PQP_OK) return st;
-  SingleState &S = single_state();
-  std::lock_guard<std::mutex> lock(S.mu);
-  Exec &x = S.xi;
-  if (!S.init_i) {
-    PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-    x.own_stream = true;
-    S.init_i = true;
-  }
-  x.plan = std::move(plan);
-  index_units(x);
-  // 8 residues per unit and per item: twice the forward plan's partials
-  x.plan.n_partials = 2 * std::max<int64_t>(x.plan.n_partials, 1);
-  x.plan.n_out = 2 * std::max<int64_t>(x.plan.n_out, 1);
-  if ((st = upload(x)) != PQP_OK) return st;
-  const LaunchArgs la = x.args();
-  IntArgs ia;
-  ia.mod_off = mod_off;
-  ia.n_primes = K;
-  ia.group = group;
-  for (const Plan::Range &r : x.plan.ranges)
-    PQP_HIP(launch_int(x.plan.items[0].mcp, la, ia, r.first, r.count, x.stream));
-  PQP_HIP(launch_int_finalize(la, ia, 1, x.stream));
-  double res[kIntMaxPrimes];
-  PQP_HIP(hipMemcpyAsync(res, x.results.p, sizeof(res), hipMemcpyDeviceToHost, x.stream));
-  PQP_HIP(hipStreamSynchronize(x.stream));
-  crt_limbs(res, K, v);
-  return PQP_OK;
-}
-
-// Key of a single-permanent plan: everything the plan's tables depend on
-// (shape, multiplicities, flags, input precision); the matrix values only
-// fill the rows of B.
-void single_key(const PermInput &in, uint32_t flags, std::vector<int64_t> &key) {
-  key.clear();
-  key.push_back(in.m_r);
-  key.push_back(in.m_c);
-  key.push_back(static_cast<int64_t>(flags));
-  key.push_back(in.a_is_float ? 1 : 0);
-  for (int64_t i = 0; i < in.m_r; ++i) key.push_back(in.rows[i]);
-  for (int64_t j = 0; j < in.m_c; ++j) key.push_back(in.cols[j]);
-}
-
 // Wait for `seq` in the host-visible done slot a one-block launch publishes.
 // A kernel that never signals (a device error) is caught by synchronising
 // the stream after 10 s of polling.
@@ -789,6 +696,170 @@ int wait_done(hipStream_t stream, volatile uint64_t *done, uint64_t seq) {
   }
   std::atomic_thread_fence(std::memory_order_acquire);
   return PQP_OK;
+}
+
+// Buffers of exact integer permanents: `in` the moduli and rows, `work` the
+// waves' residues, `res` the permanent's and the done slot.
+struct IntState {
+  std::mutex mu;
+  bool init = false;
+  hipStream_t stream = nullptr;
+  DevBuf in, work;
+  HostBuf stage;
+  MappedBuf res;
+  uint64_t seq = 0;
+};
+
+IntState &int_state() {
+  static IntState *s = new IntState();  // never destroyed: outlives atexit HIP teardown
+  return *s;
+}
+
+// The exact permanent of an integral matrix (int_scan(in).integral) as
+// two's complement limbs: the multi-modular Glynn sweep of perm_int.hip and
+// Garner's reconstruction.  PQP_ERR_RANGE when the row sums or binomial
+// weights leave FP64's exact integers or the permanent may exceed the
+// product of the moduli / 4.
+int run_int(const PermInput &in, const IntScan &sc, uint64_t *v) {
+  if (in.m_r < 0 || in.m_c < 0 || (in.m_r * in.m_c > 0 && !in.a) || (in.m_r > 0 && !in.rows) ||
+      (in.m_c > 0 && !in.cols) || (in.m_r > 0 && in.ld < in.m_c))
+    return fail(PQP_ERR_INVALID, "item 0: invalid shape or null pointer");
+  int64_t sr = 0, sum_c = 0;
+  for (int64_t i = 0; i < in.m_r; ++i) {
+    if (in.rows[i] < 0) return fail(PQP_ERR_INVALID, "item 0: negative row multiplicity");
+    sr += in.rows[i];
+  }
+  for (int64_t j = 0; j < in.m_c; ++j) {
+    if (in.cols[j] < 0) return fail(PQP_ERR_INVALID, "item 0: negative column multiplicity");
+    sum_c += in.cols[j];
+  }
+  if (sr != sum_c) return fail(PQP_ERR_SUM_MISMATCH, "Number of input and output states should be equal");
+  if (sr > kMaxCols) return fail(PQP_ERR_RANGE, "item 0: more than 64 particles");
+  const int n = static_cast<int>(sr);
+  if (!sc.integral)
+    return fail(PQP_ERR_RANGE, "matrix entries are not all integers of magnitude <= 2^47");
+  if (sc.rmax > std::ldexp(1.0, 48)) return fail(PQP_ERR_RANGE, "row sums of the matrix exceed 2^48");
+  if (sc.log2_weight > 52.0)
+    return fail(PQP_ERR_RANGE, "binomial weights of the row multiplicities exceed 2^52");
+  // products of G row sums stay below 2^49: exact in FP64 and valid
+  // inputs of the modular multiply
+  const double lr = sc.rmax > 1.0 ? std::log2(sc.rmax) : 0.0;
+  int group = 1;
+  for (int g : {12, 8, 4, 2})
+    if (group == 1 && g * lr <= 49.0) group = g;
+  // moduli: their product (each prime > 2^48.99) must exceed 4 |perm|
+  const int K = std::max(1, static_cast<int>(std::ceil((std::max(sc.log2_perm, 0.0) + 2.0) / 48.99)));
+  if (K > kIntMaxPrimes)
+    return fail(PQP_ERR_RANGE, "the permanent may exceed 2^390 in magnitude: beyond the eight moduli");
+  if (n == 0) {  // empty selection: 1 (src/permanent.cpp:106-108)
+    std::memset(v, 0, kIntLimbs * sizeof(uint64_t));
+    v[0] = 1;
+    return PQP_OK;
+  }
+  // Gray terms, with the first smallest row one lower
+  int least = 0;
+  int64_t i0 = 0;
+  for (int64_t i = 0; i < in.m_r; ++i)
+    if (in.rows[i] > 0 && (!least || in.rows[i] < least)) {
+      least = in.rows[i];
+      i0 = i;
+    }
+  double states = 1.0;  // of the digits of larger radix
+  int nb = 0, m = 0;
+  for (int64_t i = 0; i < in.m_r; ++i) {
+    const int rho = in.rows[i] - (i == i0 ? 1 : 0);
+    m += in.rows[i] > 0;
+    if (rho == 1) ++nb;
+    if (rho > 1) states *= rho + 1;
+  }
+  const double terms = std::ldexp(states, nb);
+  if (terms > 0x1p62) return fail(PQP_ERR_RANGE, "item 0: Gray term count exceeds 2^62");
+  IntArgs a;
+  a.k_max = 0;
+  while (a.k_max < kIntInnerDigits && terms / 64.0 / (1 << a.k_max) > static_cast<double>(kIntWaves)) ++a.k_max;
+  int k = 0;
+  while (k < a.k_max && k < nb && std::ldexp(states, nb - k - 1) >= 64.0) ++k;
+  const double top = std::ldexp(states, nb - k);
+  if (top >= 0x1p50) return fail(PQP_ERR_RANGE, "item 0: too many top states");
+  a.waves = static_cast<int32_t>(std::min(std::ceil(top / 64.0), 8.0 * static_cast<double>(kIntWaves)));
+  int st;
+  if ((st = require_device()) != PQP_OK) return st;
+  IntState &S = int_state();
+  std::lock_guard<std::mutex> lock(S.mu);
+  if (!S.init) {
+    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    S.init = true;
+  }
+  // the moduli table: p, 1/p, 2^-(n-1) mod p; then the rows with each column
+  // repeated by its multiplicity, and their multiplicities
+  const int W = n <= 32 ? (n + 3) / 4 * 4 : (n + 7) / 8 * 8;
+  const size_t o_rows = 3 * kIntMaxPrimes * sizeof(double);
+  const size_t o_occ = o_rows + static_cast<size_t>(m + 1) * W * sizeof(double);
+  const size_t in_bytes = o_occ + static_cast<size_t>(m);
+  if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
+  if ((st = S.stage.ensure(in_bytes)) != PQP_OK) return st;
+  if ((st = S.work.ensure(static_cast<size_t>(K) * a.waves * sizeof(double))) != PQP_OK) return st;
+  if ((st = S.res.ensure((kIntMaxPrimes + 1) * sizeof(double))) != PQP_OK) return st;
+  char *h = static_cast<char *>(S.stage.p);
+  double *mt = reinterpret_cast<double *>(h);
+  for (int q = 0; q < kIntMaxPrimes; ++q) {
+    const uint64_t p = kIntPrimes[q];
+    mt[q] = static_cast<double>(p);
+    mt[kIntMaxPrimes + q] = 1.0 / static_cast<double>(p);
+    mt[2 * kIntMaxPrimes + q] = q < K ? static_cast<double>(pow_mod((p + 1) / 2, static_cast<uint64_t>(n - 1), p)) : 0.0;
+  }
+  double *rows = reinterpret_cast<double *>(h + o_rows);
+  auto fill = [&](int64_t i, double *dst, double pad) {
+    int at = 0;
+    for (int64_t j = 0; j < in.m_c; ++j) {
+      if (in.cols[j] == 0) continue;
+      const int64_t e = 2 * (i * in.ld + j);
+      const double x = in.a_is_float ? static_cast<const float *>(in.a)[e] : static_cast<const double *>(in.a)[e];
+      for (int32_t q = 0; q < in.cols[j]; ++q) dst[at++] = x;
+    }
+    while (at < W) dst[at++] = pad;
+  };
+  int at = 0;
+  for (int64_t i = 0; i < in.m_r; ++i) {
+    if (in.rows[i] == 0) continue;
+    fill(i, rows + static_cast<size_t>(at) * W, 0.0);
+    h[o_occ + at] = static_cast<char>(in.rows[i]);
+    ++at;
+  }
+  fill(i0, rows + static_cast<size_t>(m) * W, 1.0);
+  PQP_HIP(hipMemcpyAsync(S.in.p, h, in_bytes, hipMemcpyHostToDevice, S.stream));
+  const char *d = static_cast<const char *>(S.in.p);
+  a.mod = reinterpret_cast<const double *>(d);
+  a.rows = reinterpret_cast<const double *>(d + o_rows);
+  a.occ = reinterpret_cast<const uint8_t *>(d + o_occ);
+  a.partials = static_cast<double *>(S.work.p);
+  a.out = static_cast<double *>(S.res.dev);
+  a.modes = m;
+  a.n = n;
+  a.n_primes = K;
+  a.group = group;
+  a.done = static_cast<uint64_t *>(S.res.dev) + kIntMaxPrimes;
+  a.seq = ++S.seq;
+  volatile uint64_t *done = static_cast<uint64_t *>(S.res.host) + kIntMaxPrimes;
+  *done = 0;
+  PQP_HIP(launch_int(W, a, S.stream));
+  PQP_HIP(launch_int_sum(a, S.stream));
+  if ((st = wait_done(S.stream, done, a.seq)) != PQP_OK) return st;
+  crt_limbs(static_cast<const double *>(S.res.host), K, v);
+  return PQP_OK;
+}
+
+// Key of a single-permanent plan: everything the plan's tables depend on
+// (shape, multiplicities, flags, input precision); the matrix values only
+// fill the rows of B.
+void single_key(const PermInput &in, uint32_t flags, std::vector<int64_t> &key) {
+  key.clear();
+  key.push_back(in.m_r);
+  key.push_back(in.m_c);
+  key.push_back(static_cast<int64_t>(flags));
+  key.push_back(in.a_is_float ? 1 : 0);
+  for (int64_t i = 0; i < in.m_r; ++i) key.push_back(in.rows[i]);
+  for (int64_t j = 0; j < in.m_c; ++j) key.push_back(in.cols[j]);
 }
 
 int run_single(const PermInput &in, uint32_t flags, double *out2, double *out_dd4) {

@@ -93,4 +93,23 @@ hipError_t launch_tensor(int n, const TensorArgs &a, int first_unit, int n_units
   return hipErrorInvalidValue;
 }
 
+hipError_t launch_int(int width, const IntArgs &a, hipStream_t stream) {
+  if (a.waves < 1) return hipSuccess;
+  switch (width) {
+    case 4: return launch_int_w4(a, stream);
+    case 8: return launch_int_w8(a, stream);
+    case 12: return launch_int_w12(a, stream);
+    case 20: return launch_int_w20(a, stream);
+    case 28: return launch_int_w28(a, stream);
+    case 16: return launch_int_w16(a, stream);
+    case 24: return launch_int_w24(a, stream);
+    case 32: return launch_int_w32(a, stream);
+    case 40: return launch_int_w40(a, stream);
+    case 48: return launch_int_w48(a, stream);
+    case 56: return launch_int_w56(a, stream);
+    case 64: return launch_int_w64(a, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 }  // namespace pqp

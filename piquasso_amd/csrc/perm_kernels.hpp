@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "int_types.hpp"
 #include "pqp_types.hpp"
 #include "tensor_types.hpp"
 #include "poly_types.hpp"
@@ -93,12 +94,24 @@ hipError_t launch_grad(int bucket, const LaunchArgs &a, int first_unit, int n_un
 hipError_t launch_grad_finalize(const LaunchArgs &a, int n_items, int max_values,
                                 hipStream_t stream);
 
-// Exact integer permanents (perm_int.hip): one launch per padded width
-// (a multiple of 8), then the finalize; 8 residues per unit and per item.
-hipError_t launch_int(int mcp, const LaunchArgs &a, const IntArgs &ia, int first_unit,
-                      int n_units, hipStream_t stream);
-hipError_t launch_int_finalize(const LaunchArgs &a, const IntArgs &ia, int n_items,
-                               hipStream_t stream);
+// Exact integer permanents (perm_int.hip): the sweep of one padded width,
+// then the sum of its waves' residues.
+#define PQP_DECLARE_INT(w) hipError_t launch_int_w##w(const IntArgs &a, hipStream_t stream);
+PQP_DECLARE_INT(4)
+PQP_DECLARE_INT(8)
+PQP_DECLARE_INT(12)
+PQP_DECLARE_INT(16)
+PQP_DECLARE_INT(20)
+PQP_DECLARE_INT(24)
+PQP_DECLARE_INT(28)
+PQP_DECLARE_INT(32)
+PQP_DECLARE_INT(40)
+PQP_DECLARE_INT(48)
+PQP_DECLARE_INT(56)
+PQP_DECLARE_INT(64)
+#undef PQP_DECLARE_INT
+hipError_t launch_int(int width, const IntArgs &a, hipStream_t stream);
+hipError_t launch_int_sum(const IntArgs &a, hipStream_t stream);
 
 // Tensor permanents (tensor_perm.hip): one launch per matrix order n over
 // units [first_unit, first_unit + n_units), then one finalize for all items.

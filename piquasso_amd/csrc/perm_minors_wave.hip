@@ -121,7 +121,7 @@ __attribute__((amdgpu_waves_per_eu(minor_waves(W, true), 8))) void minors_wave_k
   for (int u0 = wave * kWave; u0 < p.U; u0 += a.waves * kWave) {
     const bool active = u0 + lane < p.U;
     double cr[W], ci[W];
-    const double w_top = wave_start<W>(p, active ? u0 + lane : 0, rows, stride, cr, ci);
+    const double w_top = wave_start<W>(p, active ? u0 + lane : 0, rows, stride, p.i0, cr, ci);
     const double w = active ? w_top : 0.0;
     for (int v = 0; v < S; ++v) {
       const cptr<double> row = rows + wave_step_row(p, v) * stride;

@@ -101,7 +101,7 @@ __attribute__((amdgpu_waves_per_eu(W <= 8 ? 7 : W <= 12 ? 5 : 4, 8))) void perm_
   for (int u0 = wave * kWave; u0 < p.U; u0 += NW * kWave) {
     const bool active = u0 + lane < p.U;
     double cr[W], ci[W];
-    const double w_top = wave_start<W>(p, active ? u0 + lane : 0, rows, 2 * W, cr, ci);
+    const double w_top = wave_start<W>(p, active ? u0 + lane : 0, rows, 2 * W, p.i0, cr, ci);
     const double w = active ? w_top : 0.0;
     // the inner states in Gray order
     double sr = 0.0, si = 0.0;

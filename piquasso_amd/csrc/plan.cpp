@@ -375,10 +375,6 @@ int plan_build(const std::vector<PermInput> &caller_inputs, const PlanOptions &o
     const int mc = static_cast<int>(colsrc.size());
     int mcp = 0;
     int bucket = bucket_for_width(mc, opt.fp32_products, &mcp);
-    if (opt.pad8 && bucket >= 0) {
-      mcp = static_cast<int>(align_up(mc, 8));
-      bucket = mcp / 8 - 1;  // one range per padded width
-    }
     if (opt.minors && mcp > 32) {
       err = "item " + std::to_string(k) + ": column minors support at most 32 columns";
       return kErrRange;

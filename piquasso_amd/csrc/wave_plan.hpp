@@ -17,20 +17,23 @@ namespace {
 
 constexpr int kMaxInnerDigits = 7;
 
-struct WavePlan {
+template <typename I>  // the type of a top state's index
+struct WavePlanOf {
   int rho;           // this lane's digit: its row's multiplicity, less the prepended one
   int i0;            // the prepended row
   uint64_t rows;     // rows that are digits
   uint64_t bin;      // binary digits that are not inner
   uint64_t inner;    // the inner rows, a byte each
   int k;             // inner digits
-  int U;             // top states
+  I U;               // top states
 };
+using WavePlan = WavePlanOf<int>;
 
 // occ: the lane's row multiplicity (n >= 1 in all).  At least `lanes` top
 // states are kept where the digits allow it, at most k_max inner digits.
-__device__ __forceinline__ WavePlan wave_plan(int occ, int n, int lanes, int k_max) {
-  WavePlan p;
+template <typename I = int>
+__device__ __forceinline__ WavePlanOf<I> wave_plan(int occ, int n, int lanes, int k_max) {
+  WavePlanOf<I> p;
   p.i0 = 0;
   for (int v = 1; v <= n; ++v) {
     const uint64_t at = __ballot(occ == v);
@@ -43,7 +46,7 @@ __device__ __forceinline__ WavePlan wave_plan(int occ, int n, int lanes, int k_m
   p.bin = __ballot(p.rho == 1);
   const uint64_t multi = __ballot(p.rho > 1);
   p.rows = p.bin | multi;
-  int states = 1;  // of the digits of larger radix
+  I states = 1;  // of the digits of larger radix
   for (uint64_t m = multi; m; m &= m - 1)
     states *= __builtin_amdgcn_readlane(p.rho, __builtin_ctzll(m)) + 1;
   const int nb = __builtin_popcountll(p.bin);
@@ -58,47 +61,49 @@ __device__ __forceinline__ WavePlan wave_plan(int occ, int n, int lanes, int k_m
   return p;
 }
 
-// The row sums of top state u with the inner digits at 0, from rows of W
-// complex values `stride` doubles apart, and its signed weight.
-template <int W>
-__device__ __forceinline__ double wave_start(const WavePlan &p, int u, cptr<double> rows, int stride,
-                                             double (&cr)[W], double (&ci)[W]) {
+// The row sums of top state u with the inner digits at 0, from rows of
+// values `stride` doubles apart (W complex ones, or W doubles into cr alone
+// when REAL), and its signed weight.  They start from row r0: the prepended
+// row, or a copy of it.
+template <int W, bool REAL = false, typename I>
+__device__ __forceinline__ double wave_start(const WavePlanOf<I> &p, I u, cptr<double> rows, int stride,
+                                             int r0, double (&cr)[W], double (&ci)[W]) {
   {
     // an opaque index: the row is the same for every chunk of top states,
     // and hoisting it would hold a second set of row sums in registers
-    int r0 = p.i0;
     __asm__ volatile("" : "+s"(r0));
     const cptr<double> b = rows + r0 * stride;
 #pragma unroll
     for (int j = 0; j < W; ++j) {
-      cr[j] = b[2 * j];
-      ci[j] = b[2 * j + 1];
+      cr[j] = b[REAL ? j : 2 * j];
+      if constexpr (!REAL) ci[j] = b[2 * j + 1];
     }
   }
-  int rest = u, parity = 0;
+  I rest = u;
+  int parity = 0;
   double w = 1.0;
   for (uint64_t m = p.rows; m; m &= m - 1) {  // one loop for all digits: one block of row sums
     const int r = __builtin_ctzll(m);
     const int rr = __builtin_amdgcn_readlane(p.rho, r);
     double al = in_vgpr(1.0);  // inner digits start at 0
     if (rr > 1) {
-      // u < 2^30: the quotient by a small radix is exact this way
-      const int q = static_cast<int>((static_cast<double>(rest) + 0.5) * (1.0 / (rr + 1)));
-      const int g = rest - q * (rr + 1);
+      // u < 2^50: the quotient by a small radix is exact this way
+      const I q = static_cast<I>((static_cast<double>(rest) + 0.5) * (1.0 / (rr + 1)));
+      const int g = static_cast<int>(rest - q * (rr + 1));
       rest = q;
       parity ^= g & 1;
       w *= lane_binomial(rr, g);
       al = static_cast<double>(rr - 2 * g);
     } else if ((p.bin >> r) & 1) {
       al = (rest & 1) ? -1.0 : 1.0;
-      parity ^= rest & 1;
+      parity ^= static_cast<int>(rest & 1);
       rest >>= 1;
     }
     const cptr<double> b = rows + r * stride;
 #pragma unroll
     for (int j = 0; j < W; ++j) {
-      cr[j] = fmaR(al, b[2 * j], cr[j]);
-      ci[j] = fmaR(al, b[2 * j + 1], ci[j]);
+      cr[j] = fmaR(al, b[REAL ? j : 2 * j], cr[j]);
+      if constexpr (!REAL) ci[j] = fmaR(al, b[2 * j + 1], ci[j]);
     }
   }
   return parity ? -w : w;
@@ -106,7 +111,8 @@ __device__ __forceinline__ double wave_start(const WavePlan &p, int u, cptr<doub
 
 // The inner row that moves after inner state v (Gray order) and its factor
 // +-2; after the last state (digit k) row 0, for an update that is not read.
-__device__ __forceinline__ int wave_step_row(const WavePlan &p, int v) {
+template <typename I>
+__device__ __forceinline__ int wave_step_row(const WavePlanOf<I> &p, int v) {
   return static_cast<int>((p.inner >> (8 * __builtin_ctz(v + 1))) & 255);
 }
 __device__ __forceinline__ double wave_step_factor(int v) {
