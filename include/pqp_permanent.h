@@ -302,6 +302,18 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
                                     double *abs_sum);
 
 /*
+ * Detection probabilities of many outputs for uniformly partially
+ * distinguishable photons (piquasso/_simulators/passive/probabilities.py:
+ * 156-190): the tensor permanent of U's rows by each output and columns by
+ * the input, over input_norm x prod t!.  outputs: count x modes, row-major;
+ * outputs of another particle number give 0.  At most 20 particles
+ * (PQP_ERR_RANGE beyond).
+ */
+int pqp_overlap_table_c128(const double *matrix, int64_t modes, int64_t ld, const int32_t *input,
+                           int64_t count, const int64_t *outputs, double overlap, double input_norm,
+                           double *out);
+
+/*
  * Permanents of `count` problems evaluated once: pqp_batch_create, an eager
  * run and pqp_batch_results in one call, on buffers and streams the library
  * keeps between calls (released after a call that grew them beyond 256 MiB).

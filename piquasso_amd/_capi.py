@@ -94,6 +94,10 @@ SIGNATURES = {
         [_c.c_int64, _c.POINTER(_dp), _i64p, _i64p, _i64p, _c.POINTER(_i32p),
          _c.POINTER(_i32p), _c.POINTER(_dp)],
     ),
+    "pqp_overlap_table_c128": (
+        _c.c_int,
+        [_dp, _c.c_int64, _c.c_int64, _i32p, _c.c_int64, _i64p, _c.c_double, _c.c_double, _dp],
+    ),
     "pqp_tensor_permanent_c128": (
         _c.c_int, [_dp, _c.c_int64, _c.c_int64, _c.c_double, _dp, _dp],
     ),

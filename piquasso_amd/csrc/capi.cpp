@@ -1223,123 +1223,87 @@ namespace {
 
 // ------------------------------------------------------- tensor permanents --
 
-// Host image of a batch of tensor permanents: items, work units (grouped by
-// matrix order, one launch per order) and per-item tables, laid out as one
-// arena (tensor_types.hpp).
-struct TensorPlan {
-  std::vector<char> arena;
-  int64_t items_off = 0, units_off = 0;
-  std::vector<TensorItem> items;
-  std::vector<TensorUnit> units;
-  std::vector<std::pair<int, std::pair<int, int>>> launches;  // (n, (first unit, count))
+// Buffers of tensor permanents, kept across calls (grown on demand): `in`
+// the work units and what the host sends, `work` the matrices, sign rows and
+// partials of a pass (kTensorBytes of sign rows, or one item's), `out` the
+// results.
+struct TensorState {
+  std::mutex mu;
+  bool init = false;
+  hipStream_t stream = nullptr;
+  DevBuf in, work, out;
+  HostBuf stage;
 };
 
-// Steps per unit 2^kt for sign vectors of nb free signs: about 2^20 units
-// at most (large n) and at least ~4096 where the pair count allows (small
-// n), so the grid fills the chip.
+TensorState &tensor_state() {
+  static TensorState *s = new TensorState();  // never destroyed: outlives atexit HIP teardown
+  return *s;
+}
+
+constexpr size_t kTensorBytes = size_t{512} << 20;
+
+// Steps per unit 2^kt for sign vectors of nb free signs, the same whatever
+// the number of items (a value does not depend on its company): at most 512
+// steps, or as many as keep the units near 2^20 (large n), fewer where that
+// leaves less than about 8192 units, at least 16 (a unit's start costs about
+// four).  Against 4096 units of up to 1024 steps: 15 particles, two outputs
+// 1468 -> 1330 us, 16 particles 3041 -> 2780 us (the last waves run alone
+// for less time); 32768 units cost one output of 14 particles 351 us
+// instead of 237.
 int tensor_walk_bits(int nb, int ls) {
   auto units = [&](int kt) {
     return std::ldexp(1.0, (nb - ls) + (nb - kt)) / 2.0;
   };
-  int kt = std::min(nb, 10);
+  int kt = std::min(nb, 9);
   while (kt < nb && units(kt) > 1048576.0) ++kt;
-  while (kt > 1 && units(kt) < 4096.0) --kt;
+  while (kt > 4 && units(kt) < 8192.0) --kt;
   return kt;
 }
 
-int tensor_plan(int64_t count, const double *const *matrices, const int64_t *n, const int64_t *ld,
-                const double *overlap, TensorPlan &tp, std::string &err) {
-  tp = TensorPlan();
-  std::vector<int64_t> order(static_cast<size_t>(count));
-  for (int64_t k = 0; k < count; ++k) {
-    const int64_t nk = n[k];
-    if (nk < 0 || nk > kTensorMaxN) {
-      err = "item " + std::to_string(k) + ": tensor permanents support matrices of order 0.." +
-            std::to_string(kTensorMaxN);
-      return nk < 0 ? PQP_ERR_INVALID : PQP_ERR_RANGE;
+// The work units of one item of order n >= 1, by eps block: neighbouring
+// units then read the same sign rows.
+void tensor_units(int n, int *ls, int *kt, std::vector<TensorUnit> &units) {
+  const int nb = n - 1;  // free signs of a sign vector
+  *ls = std::min(nb, 6);
+  *kt = tensor_walk_bits(nb, *ls);
+  const uint32_t n_s = 1u << (nb - *ls);
+  const uint32_t n_t = 1u << (nb - *kt);
+  units.clear();
+  for (uint32_t tb = 0; tb < n_t; ++tb)
+    for (uint32_t sh = 0; sh < n_s; ++sh) {
+      const uint64_t lo = static_cast<uint64_t>(tb) << *kt;
+      const uint64_t hi = lo + (1ull << *kt) - 1;
+      if ((hi >> *ls) < sh) continue;  // every pair below the diagonal block
+      units.push_back(TensorUnit{static_cast<int32_t>(sh), static_cast<int32_t>(tb), (lo >> *ls) <= sh ? 1 : 0});
     }
-    if (nk > 0 && (!matrices[k] || ld[k] < nk)) {
-      err = "item " + std::to_string(k) + ": invalid matrix pointer or leading dimension";
-      return PQP_ERR_INVALID;
-    }
-    if (!std::isfinite(overlap[k])) {
-      err = "item " + std::to_string(k) + ": particle overlap is not finite";
-      return PQP_ERR_INVALID;
-    }
-    order[k] = k;
-  }
-  // units grouped by matrix order (one launch each)
-  std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return n[a] < n[b]; });
-  tp.items.resize(static_cast<size_t>(count));
-  for (int64_t k : order) {
-    TensorItem &it = tp.items[k];
-    std::memset(&it, 0, sizeof(it));
-    const int nk = static_cast<int>(n[k]);
-    it.n = nk;
-    it.x = overlap[k];
-    it.unit0 = static_cast<int32_t>(tp.units.size());
-    if (nk == 0) continue;
-    const int nb = nk - 1;  // free signs of a sign vector
-    it.ls = std::min(nb, 6);
-    it.kt = tensor_walk_bits(nb, it.ls);
-    const uint32_t n_s = 1u << (nb - it.ls);
-    const uint32_t n_t = 1u << (nb - it.kt);
-    for (uint32_t sh = 0; sh < n_s; ++sh)
-      for (uint32_t tb = 0; tb < n_t; ++tb) {
-        const uint64_t lo = static_cast<uint64_t>(tb) << it.kt;
-        const uint64_t hi = lo + (1ull << it.kt) - 1;
-        if ((hi >> it.ls) < sh) continue;  // every pair below the diagonal block
-        TensorUnit u;
-        u.item = static_cast<int32_t>(k);
-        u.s_hi = static_cast<int32_t>(sh);
-        u.t_blk = static_cast<int32_t>(tb);
-        u.mixed = (lo >> it.ls) <= sh ? 1 : 0;
-        tp.units.push_back(u);
-      }
-    it.n_units = static_cast<int32_t>(tp.units.size()) - it.unit0;
-    if (tp.units.size() > static_cast<size_t>(INT32_MAX)) {
-      err = "too many work units";
-      return PQP_ERR_RANGE;
-    }
-    if (!tp.launches.empty() && tp.launches.back().first == nk)
-      tp.launches.back().second.second += it.n_units;
-    else
-      tp.launches.push_back({nk, {it.unit0, it.n_units}});
-  }
-  // arena: items | units | per item: columns (complex, [c][i]), (1 - x)|a|^2 ([c][i])
-  auto align = [](int64_t v) { return (v + 255) & ~int64_t(255); };
-  int64_t off = 0;
-  tp.items_off = off;
-  off = align(off + static_cast<int64_t>(tp.items.size() * sizeof(TensorItem)));
-  tp.units_off = off;
-  off = align(off + static_cast<int64_t>(tp.units.size() * sizeof(TensorUnit)));
-  for (int64_t k = 0; k < count; ++k) {
-    TensorItem &it = tp.items[k];
-    const int64_t nn = static_cast<int64_t>(it.n) * it.n;
-    it.cols_off = off;
-    off = align(off + nn * 16);
-    it.pw_off = off;
-    off = align(off + nn * 8);
-  }
-  tp.arena.assign(static_cast<size_t>(std::max<int64_t>(off, 256)), 0);
-  std::memcpy(tp.arena.data() + tp.items_off, tp.items.data(), tp.items.size() * sizeof(TensorItem));
-  std::memcpy(tp.arena.data() + tp.units_off, tp.units.data(), tp.units.size() * sizeof(TensorUnit));
-  for (int64_t k = 0; k < count; ++k) {
-    const TensorItem &it = tp.items[k];
-    const int nk = it.n;
-    double *colp = reinterpret_cast<double *>(tp.arena.data() + it.cols_off);
-    double *pwp = reinterpret_cast<double *>(tp.arena.data() + it.pw_off);
-    const double y = 1.0 - it.x;
-    for (int c = 0; c < nk; ++c)
-      for (int i = 0; i < nk; ++i) {
-        const double re = matrices[k][2 * (i * ld[k] + c)];
-        const double im = matrices[k][2 * (i * ld[k] + c) + 1];
-        colp[2 * (c * nk + i)] = re;
-        colp[2 * (c * nk + i) + 1] = im;
-        pwp[c * nk + i] = y * (re * re + im * im);
-      }
-  }
-  return PQP_OK;
+}
+
+// Items per pass, and the layout of the work buffer for them: matrices, (1 -
+// x)|A|^2, sign rows, partials.
+struct TensorPass {
+  int64_t items;
+  size_t pw, signs, partials, bytes;
+};
+
+TensorPass tensor_pass(int n, int64_t count, size_t n_units) {
+  TensorPass t;
+  const size_t sign_bytes = (static_cast<size_t>(n) << (n - 1)) * 16;
+  t.items = std::min<int64_t>(std::min<int64_t>(count, 32768),
+                              std::max<int64_t>(1, static_cast<int64_t>(kTensorBytes / sign_bytes)));
+  const size_t m = static_cast<size_t>(t.items), nn = static_cast<size_t>(n) * n;
+  auto align = [](size_t v) { return (v + 255) & ~size_t{255}; };
+  t.pw = align(m * nn * 16);
+  t.signs = align(t.pw + m * nn * 8);
+  t.partials = align(t.signs + m * sign_bytes);
+  t.bytes = t.partials + m * n_units * 3 * sizeof(double);
+  return t;
+}
+
+void tensor_buffers(TensorArgs &a, const TensorPass &t, char *work) {
+  a.cols = reinterpret_cast<double *>(work);
+  a.pw = reinterpret_cast<double *>(work + t.pw);
+  a.signs = reinterpret_cast<double *>(work + t.signs);
+  a.partials = reinterpret_cast<double *>(work + t.partials);
 }
 
 // One evaluation of a batch (gradient batches have no plain mode: their
@@ -2085,48 +2049,198 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
     return fail(PQP_ERR_INVALID, "invalid tensor permanent arguments");
   if (count > INT32_MAX) return fail(PQP_ERR_RANGE, "too many items");
   if (count == 0) return PQP_OK;
-  TensorPlan tp;
-  std::string err;
-  int st = tensor_plan(count, matrices, n, ld, overlap, tp, err);
-  if (st != PQP_OK) return fail(st, err);
+  std::vector<int64_t> order;  // items by matrix order, empty matrices left out
+  for (int64_t k = 0; k < count; ++k) {
+    const std::string item = "item " + std::to_string(k);
+    if (n[k] < 0 || n[k] > kTensorMaxN)
+      return fail(n[k] < 0 ? PQP_ERR_INVALID : PQP_ERR_RANGE,
+                  item + ": tensor permanents support matrices of order 0.." + std::to_string(kTensorMaxN));
+    if (n[k] > 0 && (!matrices[k] || ld[k] < n[k]))
+      return fail(PQP_ERR_INVALID, item + ": invalid matrix pointer or leading dimension");
+    if (!std::isfinite(overlap[k])) return fail(PQP_ERR_INVALID, item + ": particle overlap is not finite");
+    if (n[k] > 0) order.push_back(k);
+  }
+  std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return n[a] < n[b]; });
+  int st;
   if ((st = require_device()) != PQP_OK) return st;
-  SingleState &S = single_state();
+  TensorState &S = tensor_state();
   std::lock_guard<std::mutex> lock(S.mu);
-  Exec &x = S.x;
   if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-    x.own_stream = true;
+    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
     S.init = true;
   }
-  if ((st = x.arena.ensure(tp.arena.size())) != PQP_OK) return st;
-  if ((st = x.partials.ensure(std::max<size_t>(tp.units.size(), 1) * 3 * sizeof(double))) != PQP_OK)
-    return st;
-  if ((st = x.results.ensure(static_cast<size_t>(count) * 2 * sizeof(double))) != PQP_OK) return st;
-  if ((st = x.stage.ensure(std::max(tp.arena.size(), static_cast<size_t>(count) * 2 * sizeof(double)))) !=
-      PQP_OK)
-    return st;
-  // the plan arena of the single-call state is replaced: force its re-upload
-  x.plan = Plan();
-  std::memcpy(x.stage.p, tp.arena.data(), tp.arena.size());
-  PQP_HIP(hipMemcpyAsync(x.arena.p, x.stage.p, tp.arena.size(), hipMemcpyHostToDevice, x.stream));
-  TensorArgs a;
-  a.arena = static_cast<const char *>(x.arena.p);
-  a.items = reinterpret_cast<const TensorItem *>(static_cast<const char *>(x.arena.p) + tp.items_off);
-  a.units = reinterpret_cast<const TensorUnit *>(static_cast<const char *>(x.arena.p) + tp.units_off);
-  a.partials = static_cast<double *>(x.partials.p);
-  a.out = static_cast<double *>(x.results.p);
-  a.n_units = static_cast<int32_t>(tp.units.size());
-  a.n_items = static_cast<int32_t>(count);
-  for (const auto &l : tp.launches) PQP_HIP(launch_tensor(l.first, a, l.second.first, l.second.second, x.stream));
-  PQP_HIP(launch_tensor_finalize(a, x.stream));
-  PQP_HIP(hipMemcpyAsync(x.stage.p, x.results.p, static_cast<size_t>(count) * 2 * sizeof(double),
-                         hipMemcpyDeviceToHost, x.stream));
-  PQP_HIP(hipStreamSynchronize(x.stream));
-  const double *r = static_cast<const double *>(x.stage.p);
-  for (int64_t k = 0; k < count; ++k) {
-    out[k] = r[2 * k];
-    if (abs_sum) abs_sum[k] = r[2 * k + 1];
+  for (int64_t k = 0; k < count; ++k)
+    if (n[k] == 0) {  // the empty product (probabilities.py:197-198)
+      out[k] = 1.0;
+      if (abs_sum) abs_sum[k] = 1.0;
+    }
+  std::vector<TensorUnit> units;
+  for (size_t g0 = 0; g0 < order.size();) {
+    const int nk = static_cast<int>(n[order[g0]]);
+    size_t g1 = g0;
+    while (g1 < order.size() && n[order[g1]] == nk) ++g1;
+    TensorArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.n = nk;
+    tensor_units(nk, &a.ls, &a.kt, units);
+    a.n_units = static_cast<int32_t>(units.size());
+    const TensorPass t = tensor_pass(nk, static_cast<int64_t>(g1 - g0), units.size());
+    const size_t nn = static_cast<size_t>(nk) * nk, most = static_cast<size_t>(t.items);
+    // units, overlaps, then (as in the work buffer) matrices and |A|^2
+    const size_t o_x = align256(units.size() * sizeof(TensorUnit));
+    const size_t o_cols = align256(o_x + most * sizeof(double));
+    const size_t in_bytes = o_cols + t.signs;
+    if ((st = S.in.ensure(o_cols)) != PQP_OK) return st;
+    if ((st = S.work.ensure(t.bytes)) != PQP_OK) return st;
+    if ((st = S.out.ensure(most * 2 * sizeof(double))) != PQP_OK) return st;
+    if ((st = S.stage.ensure(std::max(in_bytes, most * 2 * sizeof(double)))) != PQP_OK) return st;
+    char *h = static_cast<char *>(S.stage.p);
+    char *d = static_cast<char *>(S.in.p);
+    tensor_buffers(a, t, static_cast<char *>(S.work.p));
+    a.units = reinterpret_cast<const TensorUnit *>(d);
+    a.x = reinterpret_cast<const double *>(d + o_x);
+    a.out = static_cast<double *>(S.out.p);
+    for (size_t p0 = g0; p0 < g1; p0 += most) {
+      const size_t m = std::min(most, g1 - p0);
+      std::memcpy(h, units.data(), units.size() * sizeof(TensorUnit));
+      for (size_t q = 0; q < m; ++q) {
+        const int64_t k = order[p0 + q];
+        reinterpret_cast<double *>(h + o_x)[q] = overlap[k];
+        double *colp = reinterpret_cast<double *>(h + o_cols) + q * nn * 2;
+        double *pwp = reinterpret_cast<double *>(h + o_cols + t.pw) + q * nn;
+        const double y = 1.0 - overlap[k];
+        for (int c = 0; c < nk; ++c)
+          for (int i = 0; i < nk; ++i) {
+            const double re = matrices[k][2 * (i * ld[k] + c)];
+            const double im = matrices[k][2 * (i * ld[k] + c) + 1];
+            colp[2 * (c * nk + i)] = re;
+            colp[2 * (c * nk + i) + 1] = im;
+            pwp[c * nk + i] = y * (re * re + im * im);
+          }
+      }
+      PQP_HIP(hipMemcpyAsync(d, h, o_cols, hipMemcpyHostToDevice, S.stream));
+      PQP_HIP(hipMemcpyAsync(S.work.p, h + o_cols, t.signs, hipMemcpyHostToDevice, S.stream));
+      a.n_items = static_cast<int32_t>(m);
+      PQP_HIP(launch_tensor_signs(a, S.stream));
+      PQP_HIP(launch_tensor(a, S.stream));
+      PQP_HIP(launch_tensor_finalize(a, S.stream));
+      PQP_HIP(hipMemcpyAsync(h, S.out.p, m * 2 * sizeof(double), hipMemcpyDeviceToHost, S.stream));
+      PQP_HIP(hipStreamSynchronize(S.stream));
+      const double *r = reinterpret_cast<const double *>(h);
+      for (size_t q = 0; q < m; ++q) {
+        out[order[p0 + q]] = r[2 * q];
+        if (abs_sum) abs_sum[order[p0 + q]] = r[2 * q + 1];
+      }
+    }
+    g0 = g1;
   }
+  return PQP_OK;
+}
+
+int pqp_overlap_table_c128(const double *matrix, int64_t modes, int64_t ld, const int32_t *input,
+                           int64_t count, const int64_t *outputs, double overlap, double input_norm,
+                           double *out) {
+  CallRange range_("pqp_overlap_table_c128");
+  if (modes < 1 || modes > 65535 || count < 0 || !matrix || ld < modes || !input ||
+      (count > 0 && (!outputs || !out)))
+    return fail(PQP_ERR_INVALID, "invalid overlap table arguments");
+  int64_t n64 = 0;
+  for (int64_t j = 0; j < modes; ++j) {
+    if (input[j] < 0) return fail(PQP_ERR_INVALID, "occupation numbers must be non-negative");
+    n64 += input[j];
+  }
+  if (n64 > kTensorMaxN)
+    return fail(PQP_ERR_RANGE, "overlap tables support at most " + std::to_string(kTensorMaxN) + " particles");
+  const int n = static_cast<int>(n64);
+  // the outputs of n particles: their rows in first-quantized order, and
+  // input norm x prod t!
+  std::vector<uint16_t> rows;
+  std::vector<double> norm;
+  std::vector<int64_t> kept;
+  rows.reserve(static_cast<size_t>(count * n));
+  norm.reserve(static_cast<size_t>(count));
+  kept.reserve(static_cast<size_t>(count));
+  for (int64_t q = 0; q < count; ++q) {
+    const int64_t *t = outputs + q * modes;
+    int64_t sum = 0;
+    for (int64_t j = 0; j < modes; ++j) {
+      if (t[j] < 0) return fail(PQP_ERR_INVALID, "occupation numbers must be non-negative");
+      sum += std::min<int64_t>(t[j], kTensorMaxN + 1);
+    }
+    out[q] = 0.0;
+    if (sum != n) continue;
+    double f = 1.0;
+    for (int64_t j = 0; j < modes; ++j)
+      for (int64_t k = 1; k <= t[j]; ++k) {
+        rows.push_back(static_cast<uint16_t>(j));
+        f *= static_cast<double>(k);
+      }
+    norm.push_back(input_norm * f);
+    kept.push_back(q);
+  }
+  if (kept.empty()) return PQP_OK;
+  if (!std::isfinite(overlap)) return fail(PQP_ERR_INVALID, "particle overlap is not finite");
+  int st;
+  if ((st = require_device()) != PQP_OK) return st;
+  if (n == 0) {
+    for (size_t q = 0; q < kept.size(); ++q) out[kept[q]] = 1.0 / norm[q];
+    return PQP_OK;
+  }
+  TensorState &S = tensor_state();
+  std::lock_guard<std::mutex> lock(S.mu);
+  if (!S.init) {
+    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    S.init = true;
+  }
+  TensorArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.n = n;
+  std::vector<TensorUnit> units;
+  tensor_units(n, &a.ls, &a.kt, units);
+  a.n_units = static_cast<int32_t>(units.size());
+  const TensorPass t = tensor_pass(n, static_cast<int64_t>(kept.size()), units.size());
+  const size_t most = static_cast<size_t>(t.items), all = kept.size();
+  const size_t o_x = align256(units.size() * sizeof(TensorUnit));
+  const size_t o_u = align256(o_x + most * sizeof(double));
+  const size_t o_rows = align256(o_u + static_cast<size_t>(modes) * n * 16);
+  const size_t o_norm = align256(o_rows + all * n * sizeof(uint16_t));
+  const size_t in_bytes = o_norm + all * sizeof(double);
+  if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
+  if ((st = S.work.ensure(t.bytes)) != PQP_OK) return st;
+  if ((st = S.out.ensure(all * sizeof(double))) != PQP_OK) return st;
+  if ((st = S.stage.ensure(std::max(in_bytes, all * sizeof(double)))) != PQP_OK) return st;
+  char *h = static_cast<char *>(S.stage.p);
+  char *d = static_cast<char *>(S.in.p);
+  std::memcpy(h, units.data(), units.size() * sizeof(TensorUnit));
+  for (size_t q = 0; q < most; ++q) reinterpret_cast<double *>(h + o_x)[q] = overlap;
+  double *hu = reinterpret_cast<double *>(h + o_u);
+  for (int64_t i = 0; i < modes; ++i)
+    for (int64_t j = 0; j < modes; ++j)
+      for (int32_t k = 0; k < input[j]; ++k) {
+        *hu++ = matrix[2 * (i * ld + j)];
+        *hu++ = matrix[2 * (i * ld + j) + 1];
+      }
+  std::memcpy(h + o_rows, rows.data(), rows.size() * sizeof(uint16_t));
+  std::memcpy(h + o_norm, norm.data(), norm.size() * sizeof(double));
+  PQP_HIP(hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, S.stream));
+  tensor_buffers(a, t, static_cast<char *>(S.work.p));
+  a.units = reinterpret_cast<const TensorUnit *>(d);
+  a.x = reinterpret_cast<const double *>(d + o_x);
+  a.u = reinterpret_cast<const double *>(d + o_u);
+  for (size_t p0 = 0; p0 < all; p0 += most) {
+    a.n_items = static_cast<int32_t>(std::min(most, all - p0));
+    a.rows = reinterpret_cast<const uint16_t *>(d + o_rows) + p0 * n;
+    a.norm = reinterpret_cast<const double *>(d + o_norm) + p0;
+    a.prob = static_cast<double *>(S.out.p) + p0;
+    PQP_HIP(launch_tensor_gather(a, S.stream));
+    PQP_HIP(launch_tensor_signs(a, S.stream));
+    PQP_HIP(launch_tensor(a, S.stream));
+    PQP_HIP(launch_tensor_finalize(a, S.stream));
+  }
+  PQP_HIP(hipMemcpyAsync(h, S.out.p, all * sizeof(double), hipMemcpyDeviceToHost, S.stream));
+  PQP_HIP(hipStreamSynchronize(S.stream));
+  const double *r = reinterpret_cast<const double *>(h);
+  for (size_t q = 0; q < all; ++q) out[kept[q]] = r[q];
   return PQP_OK;
 }
 

@@ -87,9 +87,9 @@ hipError_t launch_minors(int bucket, const LaunchArgs &a, int first_unit, int n_
   }
 }
 
-hipError_t launch_tensor(int n, const TensorArgs &a, int first_unit, int n_units, hipStream_t s) {
-  if (n >= 1 && n <= 12) return launch_tensor_p0(n, a, first_unit, n_units, s);
-  if (n >= 13 && n <= kTensorMaxN) return launch_tensor_p1(n, a, first_unit, n_units, s);
+hipError_t launch_tensor(const TensorArgs &a, hipStream_t s) {
+  if (a.n >= 1 && a.n <= 12) return launch_tensor_p0(a, s);
+  if (a.n >= 13 && a.n <= kTensorMaxN) return launch_tensor_p1(a, s);
   return hipErrorInvalidValue;
 }
 

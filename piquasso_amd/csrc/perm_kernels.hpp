@@ -113,11 +113,14 @@ PQP_DECLARE_INT(64)
 hipError_t launch_int(int width, const IntArgs &a, hipStream_t stream);
 hipError_t launch_int_sum(const IntArgs &a, hipStream_t stream);
 
-// Tensor permanents (tensor_perm.hip): one launch per matrix order n over
-// units [first_unit, first_unit + n_units), then one finalize for all items.
-hipError_t launch_tensor_p0(int n, const TensorArgs &a, int first_unit, int n_units, hipStream_t s);
-hipError_t launch_tensor_p1(int n, const TensorArgs &a, int first_unit, int n_units, hipStream_t s);
-hipError_t launch_tensor(int n, const TensorArgs &a, int first_unit, int n_units, hipStream_t s);
+// Tensor permanents (tensor_perm.hip) of items of one order: the matrices
+// of a table, the rows R_eps of every sign vector, the sweep, and the
+// items' sums.
+hipError_t launch_tensor_gather(const TensorArgs &a, hipStream_t stream);
+hipError_t launch_tensor_signs(const TensorArgs &a, hipStream_t stream);
+hipError_t launch_tensor_p0(const TensorArgs &a, hipStream_t stream);
+hipError_t launch_tensor_p1(const TensorArgs &a, hipStream_t stream);
+hipError_t launch_tensor(const TensorArgs &a, hipStream_t stream);
 hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream);
 
 // Probability tables (perm_table.hip): `width` occupied input modes, `ones`:

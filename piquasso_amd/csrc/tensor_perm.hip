@@ -19,21 +19,35 @@
 // n = 8).
 //
 // One wave per work unit (tensor_types.hpp: delta's bits as s, eps's as t).
-// Each lane owns one delta and keeps x R_delta (2n doubles) in registers;
-// the wave walks 2^kt eps in Gray order, so a step flips one sign eps_c:
-// R_eps -+= 2 A[:, c] (wave-uniform, A's column read with scalar loads) and
-// Q -+= 2 delta_c (1 - x)|A[:, c]|^2.  The term costs 8 VALU per row; only
-// its real part is accumulated (the (delta, eps) and (eps, delta) terms are
-// conjugate).  FP64 runs of 64 steps are folded into a double-double lane
-// sum; the wave and then the item's units are reduced in double-double in a
-// fixed order.  Each unit also sums |term| (times its weight) for a
-// forward-error bound of the result.
+// Each lane owns one delta and keeps x R_delta (2n doubles) and Q (n) in
+// registers; the wave walks 2^kt eps in Gray order.  R_eps is the same in
+// every lane, so it is not kept: tensor_signs_kernel writes it for every t
+// once (2^(n-1) rows, 1.8 MB at n = 14), a step reads its row with scalar
+// loads, as operands, and a lane its R_delta when it starts.  A step costs 9
+// VALU per row: the flip Q -+= 2 delta_c (1 - x)|A[:, c]|^2, the factor (4)
+// and the product (4); only the term's real part is accumulated (the
+// (delta, eps) and (eps, delta) terms are conjugate).  FP64 runs of 64 steps
+// are folded into a double-double lane sum; the wave and then the item's
+// units are reduced in double-double in a fixed order.  Each unit also sums
+// |term| for a forward-error bound of the result.
 //
-// Compiled twice: -DPQP_TENSOR_PART=0 instantiates n = 1..12 and the
-// finalize kernel, =1 instantiates n = 13..20.
+// Bound by FP64 issue: 114 VALU a step at n = 14, which the sweep issues at
+// about 0.8 of the rate of the card's clock under FP64 load.  With R_eps
+// updated in every lane a step cost 11 per row and 10 n VGPRs held the chip
+// to two or three waves per SIMD: 8 outputs of 14 particles 1650 -> 1195 us
+// a call, one of 16 particles 3570 -> 2780, of 18 55.6 -> 46 ms.
+//
+// Tables of many outputs (pqp_overlap_table_c128) send each output's rows
+// of the interferometer instead of its matrix, and tensor_gather_kernel lays
+// the matrices out: 500 outputs of 6 particles 4640 -> 56 us, 2000 of 3
+// 22 ms -> 113 us (the host laid out and sent every matrix).
+//
+// Compiled twice: -DPQP_TENSOR_PART=0 instantiates n = 1..12 and the other
+// kernels, =1 instantiates n = 13..20.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "dd.hpp"
 #include "sweep_common.hpp"
@@ -42,6 +56,9 @@
 namespace pqp {
 
 namespace {
+
+constexpr int kTensorFinal = 512;  // threads of a finalize block
+constexpr int kWaitScalar = 0xC07F;  // s_waitcnt lgkmcnt(0)
 
 __device__ __forceinline__ dd wave_reduce_dd(dd v) {
 #pragma unroll
@@ -54,20 +71,21 @@ __device__ __forceinline__ dd wave_reduce_dd(dd v) {
   return v;
 }
 
+// Grid (units, items).
 template <int N>
-__global__ __launch_bounds__(kWave) void tensor_perm_kernel(TensorArgs a, int first_unit) {
-  const int u_idx = first_unit + static_cast<int>(blockIdx.x);
-  const cptr<TensorUnit> up = as_const<TensorUnit>(a.units) + u_idx;
-  const int item = up->item;
+__global__ __launch_bounds__(kWave) void tensor_perm_kernel(TensorArgs a) {
+  const cptr<TensorUnit> up = as_const<TensorUnit>(a.units) + blockIdx.x;
+  const int item = static_cast<int>(blockIdx.y);
   const uint32_t s_hi = static_cast<uint32_t>(up->s_hi);
   const uint32_t t_blk = static_cast<uint32_t>(up->t_blk);
   const int mixed = up->mixed;
-  const cptr<TensorItem> it = as_const<TensorItem>(a.items) + item;
-  const int ls = it->ls;
-  const int kt = it->kt;
-  const double x = it->x;
-  const cptr<double> col = as_const<double>(a.arena, it->cols_off);  // [c][i] (re, im)
-  const cptr<double> pw = as_const<double>(a.arena, it->pw_off);     // [c][i]
+  const int ls = a.ls;
+  const int kt = a.kt;
+  const double x = as_const<double>(a.x)[item];
+  constexpr int64_t kStates = int64_t{1} << (N - 1);
+  const cptr<double> col = as_const<double>(a.cols, int64_t{16} * N * N * item);  // [c][i] (re, im)
+  const cptr<double> pw = as_const<double>(a.pw, int64_t{8} * N * N * item);      // [c][i]
+  const cptr<double> signs = as_const<double>(a.signs, 16 * N * kStates * item);  // [t][i] (re, im)
 
   const int lane = static_cast<int>(threadIdx.x);
   const bool active = lane < (1 << ls);
@@ -75,95 +93,116 @@ __global__ __launch_bounds__(kWave) void tensor_perm_kernel(TensorArgs a, int fi
   const uint32_t s = (s_hi << ls) | static_cast<uint32_t>(active ? lane : 0);
   const uint32_t t0 = t_blk << kt;
 
-  // x R_delta, R_eps at the walk's first eps, (1 - x) Q_{delta eps}
-  double xr[N], xi[N], rr[N], ri[N], q[N];
+  // x R_delta and (1 - x) Q_{delta eps} at the walk's first eps
+  double xr[N], xi[N], q[N];
+  {
+    const double2 *own = reinterpret_cast<const double2 *>(a.signs) + N * (kStates * item + s);
 #pragma unroll
-  for (int i = 0; i < N; ++i) xr[i] = xi[i] = rr[i] = ri[i] = q[i] = 0.0;
+    for (int i = 0; i < N; ++i) {
+      const double2 z = own[i];
+      xr[i] = x * z.x;
+      xi[i] = x * z.y;
+      q[i] = 0.0;
+    }
+  }
 #pragma unroll 1
   for (int c = 0; c < N; ++c) {
     const bool dneg = c > 0 && ((s >> (c - 1)) & 1u);
     const bool eneg = c > 0 && ((t0 >> (c - 1)) & 1u);  // wave-uniform
-    const double dx = dneg ? -x : x;
-    const double es = in_vgpr(eneg ? -1.0 : 1.0);
     const double de = (dneg != eneg) ? -1.0 : 1.0;
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      xr[i] = fmaR(dx, col[2 * (c * N + i)], xr[i]);
-      xi[i] = fmaR(dx, col[2 * (c * N + i) + 1], xi[i]);
-      rr[i] = fmaR(es, col[2 * (c * N + i)], rr[i]);
-      ri[i] = fmaR(es, col[2 * (c * N + i) + 1], ri[i]);
-      q[i] = fmaR(de, pw[c * N + i], q[i]);
-    }
+    for (int i = 0; i < N; ++i) q[i] = fmaR(de, pw[c * N + i], q[i]);
   }
-  const double lane_sign = (__builtin_popcount(s) & 1) ? -1.0 : 1.0;
-  int par_t = __builtin_popcount(t0) & 1;
+  double sign = ((__builtin_popcount(s) ^ __builtin_popcount(t0)) & 1) ? -1.0 : 1.0;
+
+  // The scalar operands of a step, its row of `signs` and the column it
+  // flips, are loaded in groups of four rows (one 64-byte load; a single row
+  // left over joins the last group): the next group's loads are issued
+  // when the current group's have arrived and wait out its products.
+  constexpr int kParts = N <= 4 ? 1 : N == 5 ? 2 : (N + 2) / 4;
+  double r[2 * N], flip[N];
+  auto request = [&](auto part, uint32_t t, int c) {
+    constexpr int kFrom = 4 * part, kTo = part + 1 < kParts ? kFrom + 4 : N;
+    const cptr<double> row = signs + static_cast<int64_t>(t) * (2 * N);
+    const cptr<double> column = pw + c * N;
+#pragma unroll
+    for (int i = 2 * kFrom; i < 2 * kTo; ++i) r[i] = row[i];
+#pragma unroll
+    for (int i = kFrom; i < kTo; ++i) flip[i] = column[i];
+  };
 
   dd acc_dd{0.0, 0.0};
   double acc = 0.0;
-  double aabs = 0.0;  // sum of |weight x term| (forward-error scale)
+  double aabs = 0.0;  // sum of |term| as counted (forward-error scale)
   const int steps = 1 << kt;
-  // The step after state k flips eps at column c = ctz(k + 1) + 1:
-  // R_eps -+= 2 A[:, c], Q -+= 2 delta_c (1 - x)|A[:, c]|^2.  A step's
-  // column is 3n doubles of scalar operands, more than the SGPR file holds
-  // at once for large n: the first PF rows of A's column are loaded before
-  // the product of state k (their latency hides behind it), the rest after.
-  constexpr int PF = N < 8 ? N : 8;
+  request(std::integral_constant<int, 0>{}, t0, steps > 1 ? 1 : 0);
+  uint32_t t = t0;
   for (int k = 0; k < steps; ++k) {
-    const bool more = k + 1 < steps;  // wave-uniform
+    // the step to state k + 1 flips eps at column ctz(k + 1) + 1; after the
+    // last state column 0, for a Q that is not read
     const int b = __builtin_ctz(static_cast<unsigned>(k + 1));
-    const int c = more ? b + 1 : 0;
-    double ur[PF], ui[PF];
+    const int c = k + 1 < steps ? b + 1 : 0;
+    const uint32_t g = static_cast<uint32_t>((k + 1) ^ ((k + 1) >> 1));
+    const int b_next = __builtin_ctz(static_cast<unsigned>(k + 2));
+    const int c_next = k + 2 < steps ? b_next + 1 : 0;
+    const uint32_t t_next = k + 1 < steps ? (t0 | g) : t0;
+    const double sd2 = in_vgpr(((g >> b) & 1u) ? -2.0 : 2.0);
+    const double sq2 = ((s >> b) & 1u) ? -sd2 : sd2;
+    double pr = 0.0, pi = 0.0;
+    auto part_of_step = [&](auto part) {
+      constexpr int kFrom = 4 * part, kTo = part + 1 < kParts ? kFrom + 4 : N;
+      __builtin_amdgcn_s_waitcnt(kWaitScalar);
+      __builtin_amdgcn_sched_barrier(0);
+      double mr[2 * (kTo - kFrom)], mf[kTo - kFrom];
 #pragma unroll
-    for (int i = 0; i < PF; ++i) {
-      ur[i] = col[2 * (c * N + i)];
-      ui[i] = col[2 * (c * N + i) + 1];
-    }
-    double w = 2.0;
-    if (mixed) {
-      const uint32_t tb = (t0 | static_cast<uint32_t>(k ^ (k >> 1))) >> ls;
-      w = tb > s_hi ? 2.0 : (tb == s_hi ? 1.0 : 0.0);
-    }
-    if (w != 0.0) {
-      // factor i: x R_delta[i] conj(R_eps[i]) + Q[i]
-      double pr = fmaR(xi[0], ri[0], fmaR(xr[0], rr[0], q[0]));
-      double pi = fmaR(xi[0], rr[0], -(xr[0] * ri[0]));
+      for (int i = kFrom; i < kTo; ++i) {
+        mr[2 * (i - kFrom)] = r[2 * i];
+        mr[2 * (i - kFrom) + 1] = r[2 * i + 1];
+        mf[i - kFrom] = flip[i];
+      }
+      if constexpr (part + 1 < kParts)
+        request(std::integral_constant<int, part + 1>{}, t, c);
+      else
+        request(std::integral_constant<int, 0>{}, t_next, c_next);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 1; i < N - 1; ++i) {
-        const double fr = fmaR(xi[i], ri[i], fmaR(xr[i], rr[i], q[i]));
-        const double fi = fmaR(xi[i], rr[i], -(xr[i] * ri[i]));
-        cmul(pr, pi, fr, fi);
+      for (int i = kFrom; i < kTo; ++i) {
+        // factor i: x R_delta[i] conj(R_eps[i]) + Q[i]
+        const double rr = mr[2 * (i - kFrom)], ri = mr[2 * (i - kFrom) + 1];
+        const double fr = fmaR(xi[i], ri, fmaR(xr[i], rr, q[i]));
+        const double fi = fmaR(xi[i], rr, -(xr[i] * ri));
+        if (i == 0) {
+          pr = fr;
+          pi = fi;
+        } else if (i < N - 1) {
+          cmul(pr, pi, fr, fi);
+        } else {
+          pr = fmaR(pr, fr, -(pi * fi));  // real part of the product
+        }
+        q[i] = fmaR(sq2, mf[i - kFrom], q[i]);
       }
-      if (N > 1) {
-        const double fr = fmaR(xi[N - 1], ri[N - 1], fmaR(xr[N - 1], rr[N - 1], q[N - 1]));
-        const double fi = fmaR(xi[N - 1], rr[N - 1], -(xr[N - 1] * ri[N - 1]));
-        pr = fmaR(pr, fr, -(pi * fi));  // real part of the product
-      }
-      const double coef = (par_t ? -w : w) * lane_sign;
-      acc = fmaR(coef, pr, acc);
-      aabs = fmaR(w, __builtin_fabs(pr), aabs);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    part_of_step(std::integral_constant<int, 0>{});
+    if constexpr (kParts > 1) part_of_step(std::integral_constant<int, 1>{});
+    if constexpr (kParts > 2) part_of_step(std::integral_constant<int, 2>{});
+    if constexpr (kParts > 3) part_of_step(std::integral_constant<int, 3>{});
+    if constexpr (kParts > 4) part_of_step(std::integral_constant<int, 4>{});
+    static_assert(kParts <= 5, "parts of a step");
+    // pairs below the diagonal block are not counted, pairs in it half
+    if (!mixed || (t >> ls) > s_hi) {
+      acc = fmaR(sign, pr, acc);
+      aabs += __builtin_fabs(pr);
+    } else if ((t >> ls) == s_hi) {
+      acc = fmaR(0.5 * sign, pr, acc);
+      aabs = fmaR(0.5, __builtin_fabs(pr), aabs);
     }
     if ((k & (kDdFold - 1)) == kDdFold - 1) {
       acc_dd = dd_add_d(acc_dd, acc);
       acc = 0.0;
     }
-    if (more) {
-      const uint32_t g = static_cast<uint32_t>((k + 1) ^ ((k + 1) >> 1));
-      const double sd2 = in_vgpr(((g >> b) & 1u) ? -2.0 : 2.0);
-      const double sq2 = ((s >> b) & 1u) ? -sd2 : sd2;
-#pragma unroll
-      for (int i = 0; i < PF; ++i) {
-        rr[i] = fmaR(sd2, ur[i], rr[i]);
-        ri[i] = fmaR(sd2, ui[i], ri[i]);
-      }
-#pragma unroll
-      for (int i = PF; i < N; ++i) {
-        rr[i] = fmaR(sd2, col[2 * (c * N + i)], rr[i]);
-        ri[i] = fmaR(sd2, col[2 * (c * N + i) + 1], ri[i]);
-      }
-#pragma unroll
-      for (int i = 0; i < N; ++i) q[i] = fmaR(sq2, pw[c * N + i], q[i]);
-      par_t ^= 1;
-    }
+    t = t_next;
+    sign = -sign;
   }
   acc_dd = dd_add_d(acc_dd, acc);
   if (!active) {
@@ -174,40 +213,92 @@ __global__ __launch_bounds__(kWave) void tensor_perm_kernel(TensorArgs a, int fi
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) aabs += __shfl_xor(aabs, off);
   if (lane == 0) {
-    a.partials[3 * u_idx] = acc_dd.hi;
-    a.partials[3 * u_idx + 1] = acc_dd.lo;
-    a.partials[3 * u_idx + 2] = aabs;
+    double *p = a.partials + 3 * (static_cast<int64_t>(item) * a.n_units + blockIdx.x);
+    // twice: the sum counts each pair with its conjugate
+    p[0] = 2.0 * acc_dd.hi;
+    p[1] = 2.0 * acc_dd.lo;
+    p[2] = 2.0 * aabs;
   }
 }
 
 #if PQP_TENSOR_PART == 0
-// One wave per item: the dd sum of the item's unit partials in unit order
-// (lane-strided, then a fixed butterfly), T = hi + lo, and the sum of the
-// units' |term| sums.
-__global__ __launch_bounds__(kWave) void tensor_finalize_kernel(TensorArgs a) {
+// Tables: item's matrix A[i, c] = u[rows[i], c], with (1 - x) |A|^2 rounded
+// as the host rounds it for single matrices.
+__global__ __launch_bounds__(256) void tensor_gather_kernel(TensorArgs a) {
+#pragma clang fp contract(off)
   const int item = static_cast<int>(blockIdx.x);
-  if (item >= a.n_items) return;
-  const cptr<TensorItem> it = as_const<TensorItem>(a.items) + item;
-  const int lane = static_cast<int>(threadIdx.x);
+  const int n = a.n, nn = n * n;
+  const double y = 1.0 - a.x[item];
+  const double2 *u = reinterpret_cast<const double2 *>(a.u);
+  for (int t = static_cast<int>(threadIdx.x); t < nn; t += 256) {
+    const int c = t / n, i = t - c * n;
+    const double2 z = u[static_cast<int64_t>(a.rows[static_cast<int64_t>(item) * n + i]) * n + c];
+    reinterpret_cast<double2 *>(a.cols)[static_cast<int64_t>(item) * nn + t] = z;
+    a.pw[static_cast<int64_t>(item) * nn + t] = y * (z.x * z.x + z.y * z.y);
+  }
+}
+
+// R_eps[i] = sum_c eps_c A[i, c] for every t and row i: a thread each.
+__global__ __launch_bounds__(256) void tensor_signs_kernel(TensorArgs a) {
+  const int item = static_cast<int>(blockIdx.y);
+  const int n = a.n;
+  const int64_t all = static_cast<int64_t>(n) << (n - 1);
+  const int64_t at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (at >= all) return;
+  const uint32_t t = static_cast<uint32_t>(at / n);
+  const int i = static_cast<int>(at - static_cast<int64_t>(t) * n);
+  const double2 *col = reinterpret_cast<const double2 *>(a.cols) + static_cast<int64_t>(item) * n * n;
+  double2 r = col[i];
+  for (int c = 1; c < n; ++c) {
+    const double2 z = col[c * n + i];
+    const bool neg = (t >> (c - 1)) & 1u;
+    r.x += neg ? -z.x : z.x;
+    r.y += neg ? -z.y : z.y;
+  }
+  reinterpret_cast<double2 *>(a.signs)[static_cast<int64_t>(item) * all + at] = r;
+}
+
+// One block per item: the dd sum of the item's unit partials (strided over
+// the threads, a fixed butterfly in each wave, then the waves in order),
+// T = hi + lo, and the sum of the units' |term| sums; for a table, the
+// probability.  Bound by the chain of loads and dd additions of one thread:
+// one wave took 21 us over the 4160 units of n = 14.
+__global__ __launch_bounds__(kTensorFinal) void tensor_finalize_kernel(TensorArgs a) {
+  constexpr int kWaves = kTensorFinal / kWave;
+  __shared__ double part[kWaves][3];
+  const int item = static_cast<int>(blockIdx.x);
   dd s{0.0, 0.0};
   double sa = 0.0;
-  if (it->n == 0) {
-    if (lane == 0) s.hi = sa = 1.0;  // the empty product (probabilities.py:197-198)
-  } else {
-    for (int u = lane; u < it->n_units; u += kWave) {
-      const double *p = a.partials + 3 * (static_cast<int64_t>(it->unit0) + u);
-      s = dd_add(s, dd{p[0], p[1]});
-      sa += p[2];
-    }
+#pragma unroll 4
+  for (int u = static_cast<int>(threadIdx.x); u < a.n_units; u += kTensorFinal) {
+    const double *p = a.partials + 3 * (static_cast<int64_t>(item) * a.n_units + u);
+    s = dd_add(s, dd{p[0], p[1]});
+    sa += p[2];
   }
   s = wave_reduce_dd(s);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) sa += __shfl_xor(sa, off);
-  if (lane == 0) {
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    double *p = part[threadIdx.x / kWave];
+    p[0] = s.hi;
+    p[1] = s.lo;
+    p[2] = sa;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kWaves; ++w) {
+      s = dd_add(s, dd{part[w][0], part[w][1]});
+      sa += part[w][2];
+    }
     // Glynn scale 4^-(n-1) (exact)
-    const int e = it->n > 0 ? -2 * (it->n - 1) : 0;
-    a.out[2 * item] = ldexp(s.hi + s.lo, e);
-    a.out[2 * item + 1] = ldexp(sa, e);
+    const int e = -2 * (a.n - 1);
+    const double t = ldexp(s.hi + s.lo, e);
+    if (a.prob) {
+      a.prob[item] = t / a.norm[item];
+    } else {
+      a.out[2 * item] = t;
+      a.out[2 * item + 1] = ldexp(sa, e);
+    }
   }
 }
 #endif
@@ -216,19 +307,15 @@ __global__ __launch_bounds__(kWave) void tensor_finalize_kernel(TensorArgs a) {
 
 #if PQP_TENSOR_PART == 0
 #define PQP_TENSOR_CASES X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
-hipError_t launch_tensor_p0(int n, const TensorArgs &a, int first_unit, int n_units,
-                            hipStream_t stream) {
+hipError_t launch_tensor_p0(const TensorArgs &a, hipStream_t stream) {
 #else
 #define PQP_TENSOR_CASES X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20)
-hipError_t launch_tensor_p1(int n, const TensorArgs &a, int first_unit, int n_units,
-                            hipStream_t stream) {
+hipError_t launch_tensor_p1(const TensorArgs &a, hipStream_t stream) {
 #endif
-  if (n_units <= 0) return hipSuccess;
-  switch (n) {
-#define X(k)                                                                              \
-  case k:                                                                                 \
-    hipLaunchKernelGGL(tensor_perm_kernel<k>, dim3(n_units), dim3(kWave), 0, stream, a,  \
-                       first_unit);                                                      \
+  switch (a.n) {
+#define X(k)                                                                                       \
+  case k:                                                                                          \
+    hipLaunchKernelGGL(tensor_perm_kernel<k>, dim3(a.n_units, a.n_items), dim3(kWave), 0, stream, a); \
     return hipGetLastError();
     PQP_TENSOR_CASES
 #undef X
@@ -238,9 +325,20 @@ hipError_t launch_tensor_p1(int n, const TensorArgs &a, int first_unit, int n_un
 }
 
 #if PQP_TENSOR_PART == 0
+hipError_t launch_tensor_gather(const TensorArgs &a, hipStream_t stream) {
+  hipLaunchKernelGGL(tensor_gather_kernel, dim3(a.n_items), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_tensor_signs(const TensorArgs &a, hipStream_t stream) {
+  const int64_t all = static_cast<int64_t>(a.n) << (a.n - 1);
+  hipLaunchKernelGGL(tensor_signs_kernel, dim3(static_cast<unsigned>((all + 255) / 256), a.n_items), dim3(256),
+                     0, stream, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream) {
-  if (a.n_items <= 0) return hipSuccess;
-  hipLaunchKernelGGL(tensor_finalize_kernel, dim3(a.n_items), dim3(kWave), 0, stream, a);
+  hipLaunchKernelGGL(tensor_finalize_kernel, dim3(a.n_items), dim3(kTensorFinal), 0, stream, a);
   return hipGetLastError();
 }
 #endif

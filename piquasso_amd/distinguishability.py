@@ -94,45 +94,38 @@ def uniform_input_norm(input_occupation, particle_overlap: float) -> float:
     return norm
 
 
-def _expand(interferometer, rows, cols) -> np.ndarray:
-    """Row i repeated rows[i] times, column j cols[j] times
-    (piquasso/_math/linalg.py:98-117)."""
-    ri = np.repeat(np.arange(len(rows)), rows)
-    ci = np.repeat(np.arange(len(cols)), cols)
-    return np.asarray(interferometer)[np.ix_(ri, ci)]
-
-
 def detection_probabilities(occupation_numbers, interferometer, input_occupation: Sequence[int],
                             uniform_particle_overlap: float) -> np.ndarray:
     """Probabilities of detecting each output occupation (rows of
     ``occupation_numbers``) for the input occupation with uniform particle
     overlap: tensor permanent / (input norm x prod of output factorials),
-    0 where the photon numbers differ (probabilities.py:156-190).  All
-    tensor permanents come from one batched call."""
-    u = np.asarray(interferometer, dtype=np.complex128)
+    0 where the photon numbers differ (probabilities.py:156-190), all from
+    one call that takes the occupations (``pqp_overlap_table_c128``)."""
+    u = np.ascontiguousarray(np.asarray(interferometer, dtype=np.complex128))
     inp = np.asarray(input_occupation, dtype=np.int64).reshape(-1)
-    outs = np.asarray(occupation_numbers, dtype=np.int64)
+    outs = np.ascontiguousarray(np.asarray(occupation_numbers, dtype=np.int64))
     if outs.ndim == 1:
         outs = outs[None, :]
     d = u.shape[0]
     if u.shape != (d, d) or inp.shape[0] != d or outs.shape[1] != d:
         raise ValueError("occupations must have one entry per mode of a square interferometer")
-    if (inp < 0).any() or (outs < 0).any():
+    if (inp < 0).any():
         raise ValueError("occupation numbers must be non-negative")
     n = int(inp.sum())
     if n > MAX_PARTICLES:
+        if (outs < 0).any():
+            raise ValueError("occupation numbers must be non-negative")
         raise ValueError(f"at most {MAX_PARTICLES} particles are supported, got {n}")
     x = float(uniform_particle_overlap)
     probs = np.zeros(outs.shape[0])
-    keep = np.flatnonzero(outs.sum(axis=1) == n)
-    if keep.size == 0:
-        return probs
-    mats = [_expand(u, outs[k], inp) for k in keep]
-    t = tensor_permanent_batch(mats, [x] * len(mats))
-    in_norm = uniform_input_norm(inp, x)
-    for j, k in enumerate(keep):
-        out_fact = float(np.prod([math.factorial(int(v)) for v in outs[k]]))
-        probs[k] = t[j] / (in_norm * out_fact)
+    if d == 0 or len(probs) == 0:
+        return probs + (1.0 if d == 0 else 0.0)
+    inp32 = np.ascontiguousarray(inp, dtype=np.int32)
+    dp = ctypes.POINTER(ctypes.c_double)
+    _capi.check(_capi.lib().pqp_overlap_table_c128(
+        u.view(np.float64).ctypes.data_as(dp), d, d, inp32.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)),
+        len(outs), outs.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), x, uniform_input_norm(inp, x),
+        probs.ctypes.data_as(dp)))
     return probs
 
 
