@@ -138,6 +138,17 @@ constexpr int kIntInnerDigits = 7;
 // Device buffers a one-shot batch may leave for the next one.
 constexpr size_t kKeptBytes = size_t{256} << 20;
 
+// Permanents without tables: one block up to kOneBlockTerms Gray terms (the
+// blocks' meeting costs about 3 us: 13 particles 17.0 us a call in one block
+// and 16.5 in four), else blocks for about kOneLaneStates states a lane, up
+// to a wave per SIMD, and two above kOneManyTerms terms (2^23 terms: 85 us
+// at one, 61 at two).  Above kOneMaxTerms the planned sweep, whose units
+// walk longer, is as fast.
+constexpr double kOneBlockTerms = 2048.0;
+constexpr double kOneLaneStates = 4.0;
+constexpr double kOneManyTerms = 2097152.0;
+constexpr double kOneMaxTerms = 16777216.0;
+
 int expand_mode(uint32_t flags) {
   if (flags & PQP_FLAG_EXPAND_COLS) return 1;
   if (flags & PQP_FLAG_KEEP_COLS) return 0;
@@ -301,8 +312,7 @@ int upload(Exec &x) {
   // partials: 4 doubles per slot, then 1 (term magnitudes) per slot
   if ((st = x.partials.ensure(std::max<int64_t>(p.n_partials, 1) * 5 * sizeof(double))) != PQP_OK) return st;
   if (x.mapped_results) {
-    // + one done slot per result for one-block launches
-    if ((st = x.results_m.ensure(n_out * 8 * sizeof(double))) != PQP_OK) return st;
+    if ((st = x.results_m.ensure(n_out * 7 * sizeof(double))) != PQP_OK) return st;
   } else if ((st = x.results.ensure(n_out * 7 * sizeof(double))) != PQP_OK) {
     return st;
   }
@@ -471,7 +481,12 @@ struct SingleState {
   // the plan resident in xs and its key (shape, multiplicities, flags)
   std::vector<int64_t> xs_key;
   bool xs_planned = false;
-  uint64_t xs_seq = 0;  // last value published by a one-block launch
+  // permanents without tables (perm_one.hip)
+  bool init_one = false;
+  hipStream_t one_stream = nullptr;
+  DevBuf one_work;
+  MappedBuf one_res;
+  uint64_t one_seq = 0;
 };
 
 SingleState &single_state() {
@@ -681,7 +696,7 @@ IntScan int_scan(const PermInput &in) {
   return sc;
 }
 
-// Wait for `seq` in the host-visible done slot a one-block launch publishes.
+// Wait for `seq` in the host-visible done slot a launch publishes.
 // A kernel that never signals (a device error) is caught by synchronising
 // the stream after 10 s of polling.
 int wait_done(hipStream_t stream, volatile uint64_t *done, uint64_t seq) {
@@ -862,6 +877,47 @@ void single_key(const PermInput &in, uint32_t flags, std::vector<int64_t> &key) 
   for (int64_t j = 0; j < in.m_c; ++j) key.push_back(in.cols[j]);
 }
 
+// A single permanent on perm_one.hip: one launch, polled.
+int run_one(OnePlan &p, double *out2, double *out_dd4) {
+  int st;
+  if ((st = require_device()) != PQP_OK) return st;
+  SingleState &S = single_state();
+  std::lock_guard<std::mutex> lock(S.mu);
+  constexpr size_t kPartials = 256;  // after the counter
+  if (!S.init_one) {
+    PQP_HIP(hipStreamCreateWithFlags(&S.one_stream, hipStreamNonBlocking));
+    if ((st = S.one_res.ensure(8 * sizeof(double))) != PQP_OK) return st;
+    if ((st = S.one_work.ensure(kPartials + static_cast<size_t>(kOneMaxBlocks) * 5 * sizeof(double))) != PQP_OK)
+      return st;
+    PQP_HIP(hipMemset(S.one_work.p, 0, kPartials));
+    S.init_one = true;
+  }
+  thread_local OneArgs a;
+  one_fill(p, a);
+  char *work = static_cast<char *>(S.one_work.p);
+  a.counter = reinterpret_cast<int *>(work);
+  a.partials = reinterpret_cast<double *>(work + kPartials);
+  a.out = static_cast<double *>(S.one_res.dev);
+  a.done = reinterpret_cast<uint64_t *>(a.out + 7);
+  a.seq = ++S.one_seq;
+  const double *res = static_cast<const double *>(S.one_res.host);
+  volatile uint64_t *done = static_cast<uint64_t *>(S.one_res.host) + 7;
+  *done = 0;
+  PQP_HIP(p.fp32 ? launch_one_f(p.width, p.ones, a, p.blocks, p.waves, S.one_stream)
+                 : launch_one_d(p.width, p.ones, a, p.blocks, p.waves, S.one_stream));
+  if ((st = wait_done(S.one_stream, done, a.seq)) != PQP_OK) {
+    // a launch that did not finish its count leaves it behind
+    (void)hipMemsetAsync(a.counter, 0, sizeof(int), S.one_stream);
+    (void)hipStreamSynchronize(S.one_stream);
+    return st;
+  }
+  out2[0] = res[0];
+  out2[1] = res[1];
+  if (out_dd4) std::memcpy(out_dd4, res + 2, 4 * sizeof(double));
+  g_last_bound = sweep_error_bound(p.n, p.fp32, res[6], res[0], res[1]);
+  return PQP_OK;
+}
+
 int run_single(const PermInput &in, uint32_t flags, double *out2, double *out_dd4) {
   const bool args_ok = in.m_r >= 0 && in.m_c >= 0 && (in.m_r * in.m_c == 0 || in.a) &&
                        (in.m_r == 0 || in.rows) && (in.m_c == 0 || in.cols) &&
@@ -896,6 +952,8 @@ int run_single(const PermInput &in, uint32_t flags, double *out2, double *out_dd
       g_error.clear();
     }
   }
+  OnePlan one;
+  if (args_ok && one_plan(in, flags, one)) return run_one(one, out2, out_dd4);
   SingleState &S = single_state();
   std::unique_lock<std::mutex> lock(S.mu);
   Exec &x = S.xs;
@@ -930,68 +988,21 @@ int run_single(const PermInput &in, uint32_t flags, double *out2, double *out_dd
   const int n = d.n;
   const bool fp32 = x.plan.fp32;
   double *res = static_cast<double *>(x.results_m.host);
-  int bucket = -1;
-  const bool one_block = single_block_eligible(x.plan, flags, &bucket);
   const size_t b_bytes = x.plan.info[0].rowsrc.size() * static_cast<size_t>(d.mcp) * 2 *
                          (fp32 ? sizeof(float) : sizeof(double));
-  const bool b_in_args = one_block && b_bytes <= static_cast<size_t>(kSingleArgBBytes);
   if (hit) {
     plan_refresh_matrix(x.plan, std::vector<PermInput>{in});
-    if (!x.plan.info[0].trivial_one && !b_in_args) {
+    if (!x.plan.info[0].trivial_one) {
       const size_t off = static_cast<size_t>(d.b_off);
       std::memcpy(static_cast<char *>(x.stage.p) + off, x.plan.arena.data() + off, b_bytes);
       PQP_HIP(hipMemcpyAsync(static_cast<char *>(x.arena.p) + off, static_cast<char *>(x.stage.p) + off,
                              b_bytes, hipMemcpyHostToDevice, x.stream));
     }
   }
-  if (one_block) {
-    // one launch: the block sweeps, sums and publishes the result; the rows
-    // of B travel in the kernel arguments when they fit
-    volatile uint64_t *done = reinterpret_cast<volatile uint64_t *>(res + 7 * x.n_results);
-    thread_local SingleArgs args;
-    single_block_args(x.plan, x.args(),
-                      reinterpret_cast<uint64_t *>(static_cast<double *>(x.results_m.dev) + 7 * x.n_results),
-                      ++S.xs_seq, args);
-    *done = 0;
-    x.abs_valid = true;
-    PQP_HIP(launch_single_block(bucket, fp32, args, x.stream));
-    if ((st = wait_done(x.stream, done, args.seq)) != PQP_OK) return st;
-  } else if (!(flags & PQP_FLAG_PLAIN) && x.plan.ranges.size() == 1 && d.units > 0 &&
-             d.mcp <= kLastFinalizeMaxWidth) {
-    // one static launch over the device whose last block finalizes the
-    // permanent and publishes the result (no finalize launch, no stream
-    // synchronisation)
-    volatile uint64_t *done = reinterpret_cast<volatile uint64_t *>(res + 7 * x.n_results);
-    FwdLaunch l;
-    l.args = x.args();
-    l.args.last_counter = static_cast<int *>(x.heads.p) + kLastCounterSlot;
-    l.args.done = reinterpret_cast<uint64_t *>(static_cast<double *>(x.results_m.dev) + 7 * x.n_results);
-    l.args.seq = ++S.xs_seq;
-    l.first_unit = 0;
-    l.n_units = d.units;
-    l.persistent = false;
-    l.fp32 = fp32;
-    l.comp = true;
-    l.stream = x.stream;
-    int mcp = 0;
-    const int b = bucket_for_width(d.mcp, fp32, &mcp);
-    *done = 0;
-    x.abs_valid = true;
-    PQP_HIP(launch_fwd(b, l));
-    if ((st = wait_done(x.stream, done, l.args.seq)) != PQP_OK) {
-      // a launch that did not finish its count leaves it behind: clear it so
-      // that the next call's last block is recognised
-      (void)hipMemsetAsync(l.args.last_counter, 0, sizeof(int), x.stream);
-      (void)hipStreamSynchronize(x.stream);
-      return st;
-    }
-  } else {
-    if ((st = enqueue(x, (flags & PQP_FLAG_PLAIN) ? PQP_RUN_PLAIN : PQP_RUN_EAGER, nullptr,
-                      nullptr)) != PQP_OK)
-      return st;
-    PQP_HIP(hipStreamSynchronize(x.stream));
-  }
-  // one item: results = [out (2)][out_dd (4)][term magnitudes (1)][done (1)],
+  if ((st = enqueue(x, (flags & PQP_FLAG_PLAIN) ? PQP_RUN_PLAIN : PQP_RUN_EAGER, nullptr, nullptr)) != PQP_OK)
+    return st;
+  PQP_HIP(hipStreamSynchronize(x.stream));
+  // one item: results = [out (2)][out_dd (4)][term magnitudes (1)],
   // written by the kernels into mapped host memory
   out2[0] = res[0];
   out2[1] = res[1];
@@ -1811,71 +1822,6 @@ namespace pqp {
 
 int capi_fail(int code, const std::string &msg) { return fail(code, msg); }
 
-bool single_block_eligible(const Plan &plan, uint32_t flags, int *bucket) {
-  if (plan.items.size() != 1 || (flags & PQP_FLAG_PLAIN)) return false;
-  const ItemDesc &d = plan.items[0];
-  int mcp = 0;
-  const int b = d.units > 0 ? bucket_for_width(d.mcp, plan.fp32, &mcp) : -1;
-  if (bucket) *bucket = b;
-  return d.units > 0 && b >= 0 && b <= 1 && d.units <= kSingleBlockThreads / kWave;
-}
-
-void single_block_args(const Plan &plan, const LaunchArgs &a, uint64_t *done, uint64_t seq,
-                       SingleArgs &args) {
-  const ItemDesc &d = plan.items[0];
-  const size_t rsz = plan.fp32 ? sizeof(float) : sizeof(double);
-  const size_t row_bytes = static_cast<size_t>(d.mcp) * 2 * rsz;
-  const size_t b_bytes = plan.info[0].rowsrc.size() * row_bytes;
-  args.a = a;
-  args.arena_lines = static_cast<int32_t>(plan.arena.size() / 64);  // whole lines only
-  args.b_in_args = b_bytes <= static_cast<size_t>(kSingleArgBBytes) ? 1 : 0;
-  args.base_in_args = 0;
-  args.base_off = 0;
-  // Binary top digits beyond the lane-dependent ones: each unit's start row
-  // without them, so that every lane adds kLaneDigits rows instead of all
-  // 1 + L + Dt (the start state is a chain of dependent row updates).  The
-  // kernel then reads rows 1 .. L + kLaneDigits of B only (the inner rows
-  // for the sweep, the lane digits' rows for the start), so the rows of the
-  // other top digits are left out of the arguments.
-  const int lane_rows = 1 + d.L + kLaneDigits;
-  const size_t base_off = (static_cast<size_t>(lane_rows) * row_bytes + 63) / 64 * 64;
-  const size_t base_bytes = static_cast<size_t>(d.units) * row_bytes;
-  if ((d.flags & kTopBinary) && d.Dt > kLaneDigits && d.units > 0 &&
-      d.units <= kSingleBlockThreads / kWave && base_off + base_bytes <= static_cast<size_t>(kSingleArgBBytes)) {
-    const int mcp = d.mcp, L = d.L;
-    const char *B = plan.arena.data() + d.b_off;
-    const double *alpha = reinterpret_cast<const double *>(plan.arena.data() + d.alpha_off);
-    auto row = [&](int r, int j, int c) -> double {  // component c of column j of row r of B
-      const size_t e = (static_cast<size_t>(r) * mcp + j) * 2 + c;
-      return plan.fp32 ? static_cast<double>(reinterpret_cast<const float *>(B)[e])
-                       : reinterpret_cast<const double *>(B)[e];
-    };
-    std::memcpy(args.b, B, static_cast<size_t>(lane_rows) * row_bytes);
-    for (int w = 0; w < d.units; ++w) {
-      const uint64_t u0 = static_cast<uint64_t>(w) * kWave;
-      const uint64_t g = u0 ^ (u0 >> 1);
-      for (int j = 0; j < mcp; ++j)
-        for (int c = 0; c < 2; ++c) {
-          double v = row(0, j, c);
-          for (int i = 1; i <= L; ++i) v += alpha[i - 1] * row(i, j, c);
-          for (int t = kLaneDigits; t < d.Dt; ++t) v += (((g >> t) & 1) ? -1.0 : 1.0) * row(L + 1 + t, j, c);
-          const size_t e = (static_cast<size_t>(w) * mcp + j) * 2 + c;
-          if (plan.fp32)
-            reinterpret_cast<float *>(args.b + base_off)[e] = static_cast<float>(v);
-          else
-            reinterpret_cast<double *>(args.b + base_off)[e] = v;
-        }
-    }
-    args.b_in_args = 1;
-    args.base_in_args = 1;
-    args.base_off = static_cast<int32_t>(base_off);
-  } else if (args.b_in_args) {
-    std::memcpy(args.b, plan.arena.data() + d.b_off, b_bytes);
-  }
-  args.done = done;
-  args.seq = seq;
-}
-
 double sweep_error_bound(int n, bool fp32, double m, double re, double im) {
   const double u = fp32 ? 0x1p-24 : 0x1p-53;
   return 4.0 * (std::max(n, 0) + 2) * u * m + 0x1p-53 * std::hypot(re, im);
@@ -1901,21 +1847,189 @@ double gray_terms(const PermInput &in) {
   return T;
 }
 
+namespace {
+int64_t first_smallest(const PermInput &in) {  // the prepended row
+  int64_t i0 = -1;
+  for (int64_t i = 0; i < in.m_r; ++i)
+    if (in.rows[i] > 0 && (i0 < 0 || in.rows[i] < in.rows[i0])) i0 = i;
+  return i0;
+}
+}  // namespace
+
+bool one_plan(const PermInput &given, uint32_t flags, OnePlan &p) {
+  if (flags & PQP_FLAG_PLAIN) return false;
+  const bool expand = (flags & PQP_FLAG_EXPAND_COLS) != 0;  // a column per particle
+  PermInput in = given;
+  if (in.m_r <= 0 || in.m_c <= 0 || !in.a || !in.rows || !in.cols || in.ld < in.m_c) return false;
+  if (!(flags & PQP_FLAG_AS_GIVEN)) plan_orient(in);
+  int64_t sr = 0, sc = 0;
+  int width = 0, cmax = 0;
+  for (int64_t i = 0; i < in.m_r; ++i) {
+    if (in.rows[i] < 0) return false;
+    sr += in.rows[i];
+  }
+  for (int64_t j = 0; j < in.m_c; ++j) {
+    if (in.cols[j] < 0) return false;
+    sc += in.cols[j];
+    width += expand ? std::min(in.cols[j], kOneMaxWidth + 1) : in.cols[j] > 0;
+    if (width > kOneMaxWidth) return false;
+    cmax = std::max(cmax, static_cast<int>(in.cols[j]));
+  }
+  if (sr != sc || sr < 1 || sr > kMaxCols) return false;
+  const double terms = gray_terms(in);
+  if (terms > kOneMaxTerms) return false;
+  p.in = in;
+  p.n = static_cast<int>(sr);
+  p.width = width;
+  p.ones = expand || cmax <= 1;
+  p.fp32 = (flags & PQP_FLAG_FP32) != 0;
+  p.terms = terms;
+  p.blocks = 1;
+  p.waves = kOneWaves;
+  if (terms > kOneBlockTerms) {
+    const double cap = terms > kOneManyTerms ? kOneMaxBlocks : kOneMaxBlocks / 2;
+    p.blocks = static_cast<int>(std::ceil(std::min(terms / (64.0 * kOneLaneStates * kOneWaves), cap)));
+  } else {
+    while (p.waves > 1 && terms <= 32.0 * kOneLaneStates * p.waves) p.waves /= 2;
+  }
+  return true;
+}
+
+void one_fill(OnePlan &p, OneArgs &a) {
+  const PermInput &in = p.in;
+  int64_t cols[kOneMaxWidth];
+  int width = 0;
+  a.cmax = 1;
+  std::memset(a.over, 0, sizeof(a.over));
+  for (int64_t j = 0; j < in.m_c; ++j) {
+    if (in.cols[j] == 0) continue;
+    const int64_t at = in.transposed ? j * in.ld : j;
+    if (p.ones) {
+      for (int r = 0; r < in.cols[j]; ++r) cols[width++] = at;
+      continue;
+    }
+    for (int r = 2; r <= in.cols[j]; ++r) a.over[r - 2] |= 1u << width;
+    a.cmax = std::max(a.cmax, in.cols[j]);
+    cols[width++] = at;
+  }
+  // the digits: every row, the first smallest one lower
+  const int64_t i0 = first_smallest(in);
+  auto rho = [&](int64_t i) { return in.rows[i] - (i == i0 ? 1 : 0); };
+  a.n = p.n;
+  int64_t digit[kOneMaxRows];  // binary ones first
+  int digits = 0, binary = 0;
+  for (int64_t i = 0; i < in.m_r; ++i)
+    if (rho(i) == 1) digit[digits++] = i;
+  binary = digits;
+  for (int64_t i = 0; i < in.m_r; ++i)
+    if (rho(i) > 1) digit[digits++] = i;
+  // the lanes' digits: six binary ones, or the largest product up to 64
+  uint32_t lane = 0;
+  if (binary >= kOneLaneDigits) {
+    lane = (1u << kOneLaneDigits) - 1;
+    a.lanes = kWave;
+  } else {
+    uint32_t best[kWave + 1] = {};  // digits of each product, and bit 31
+    best[1] = 1u << 31;
+    for (int d = 0; d < digits; ++d)
+      for (int v = kWave; v >= 1; --v)
+        if (best[v] && v * (rho(digit[d]) + 1) <= kWave && !best[v * (rho(digit[d]) + 1)])
+          best[v * (rho(digit[d]) + 1)] = best[v] | 1u << d;
+    a.lanes = kWave;
+    while (!best[a.lanes]) --a.lanes;
+    lane = best[a.lanes] & ~(1u << 31);
+  }
+  // inner digits until every wave has one state of the others; half as many
+  // waves more are added rather than a digit (radices above 2 leave waves
+  // without a state otherwise)
+  const double waves = (p.blocks > 1 ? 1.5 : 1.0) * p.waves * p.blocks;
+  double chunks = p.terms / a.lanes;
+  uint32_t inner = 0;
+  a.S = 1;
+  a.binary = 1;
+  for (int d = 0; d < digits && chunks > waves; ++d) {
+    const int radix = static_cast<int>(rho(digit[d])) + 1;
+    if ((lane >> d & 1u) || a.S * radix > kOneMaxStates) continue;
+    inner |= 1u << d;
+    a.S *= radix;
+    chunks /= radix;
+    if (d >= binary) a.binary = 0;
+  }
+  a.chunks = static_cast<int32_t>(std::llround(chunks));
+  if (p.blocks > 1) p.blocks = std::min((a.chunks + p.waves - 1) / p.waves, kOneMaxBlocks);
+  int64_t order[kOneMaxRows];
+  int rows = 0;
+  a.lane_digits = a.inner = a.rest = 0;
+  for (int d = 0; d < digits; ++d)
+    if (lane >> d & 1u) {
+      a.lane_rho[a.lane_digits++] = static_cast<int32_t>(rho(digit[d]));
+      order[rows++] = digit[d];
+    }
+  order[rows++] = i0;
+  for (int d = 0; d < digits; ++d)
+    if (inner >> d & 1u) {
+      a.rho[a.inner++] = static_cast<int32_t>(rho(digit[d]));
+      order[rows++] = digit[d];
+    }
+  for (int d = 0; d < digits; ++d)
+    if (!((lane | inner) >> d & 1u)) {
+      a.rho[a.inner + a.rest++] = static_cast<int32_t>(rho(digit[d]));
+      order[rows++] = digit[d];
+    }
+  if (!a.binary) {
+    // reflected mixed-radix Gray code of the inner digits
+    int g[kOneMaxRows] = {}, dir[kOneMaxRows];
+    double coef = 1.0;
+    std::fill(dir, dir + a.inner, 1);
+    for (int v = 0; v < a.S; ++v) {
+      a.step[v] = OneStep{coef, 0, 0};
+      if (v + 1 == a.S) break;
+      int i = 0;
+      for (; g[i] + dir[i] < 0 || g[i] + dir[i] > a.rho[i]; ++i) dir[i] = -dir[i];
+      // C(rho, g +- 1) from C(rho, g), exact
+      coef = dir[i] > 0 ? -coef * (a.rho[i] - g[i]) / (g[i] + 1) : -coef * g[i] / (a.rho[i] - g[i] + 1);
+      g[i] += dir[i];
+      a.step[v].factor = dir[i] > 0 ? -2 : 2;
+      a.step[v].row = 1 + i;
+    }
+  }
+  const int64_t step = in.transposed ? 1 : in.ld;
+  auto fill = [&](auto *dst, const auto *src) {
+    using R = std::remove_reference_t<decltype(*dst)>;
+    for (int r = 0; r < rows; ++r)
+      for (int j = 0; j < width; ++j, dst += 2) {
+        const auto *e = src + 2 * (order[r] * step + cols[j]);
+        dst[0] = static_cast<R>(e[0]);
+        dst[1] = static_cast<R>(e[1]);
+      }
+  };
+  if (in.a_is_float) {
+    if (p.fp32)
+      fill(reinterpret_cast<float *>(a.b), static_cast<const float *>(in.a));
+    else
+      fill(reinterpret_cast<double *>(a.b), static_cast<const float *>(in.a));
+  } else {
+    if (p.fp32)
+      fill(reinterpret_cast<float *>(a.b), static_cast<const double *>(in.a));
+    else
+      fill(reinterpret_cast<double *>(a.b), static_cast<const double *>(in.a));
+  }
+}
+
 PlanOptions single_plan_options(uint32_t flags, const PermInput &in) {
   PlanOptions opt;
   opt.fp32_products = (flags & PQP_FLAG_FP32) != 0;
   opt.expand_cols = expand_mode(flags);
   opt.orient = (flags & PQP_FLAG_AS_GIVEN) == 0;
   const DeviceState &dev = device_state();
-  // waves per permanent: ~1.4 sqrt(T), at most kSingleUnitsPerCu per CU
-  // (16 for the one-block form); a permanent of one wave writes its result
+  // waves per permanent: ~1.4 sqrt(T), at most kSingleUnitsPerCu per CU; a permanent of one wave writes its result
   // from the sweep kernel
   opt.auto_units_cap = static_cast<int64_t>(std::max(dev.cus, 1)) * kSingleUnitsPerCu;
   const bool rows_ok = in.m_r == 0 || (in.m_r > 0 && in.rows);
   if (!(flags & PQP_FLAG_PLAIN) && rows_ok) {
     const double t = gray_terms(in);
-    if (t <= kSingleBlockMaxTerms)
-      opt.auto_units_cap = t <= kSingleBlockSmallTerms ? kSingleBlockUnitsSmall : kSingleBlockUnits;
+    if (t <= kSingleFewTerms)
+      opt.auto_units_cap = t <= kSingleFewestTerms ? kSingleFewestUnits : kSingleFewUnits;
   }
   opt.direct_out = (flags & PQP_FLAG_PLAIN) == 0;
   return opt;

@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <string>
 
+#include "one_types.hpp"
 #include "plan.hpp"
 #include "pqp_types.hpp"
 
@@ -23,34 +24,38 @@ int capi_require_device();
 // `in.rows` must be valid (negative entries count as 0).
 double gray_terms(const PermInput &in);
 
-// Single permanents of at most this many Gray terms and at most 16 columns
-// run in one launch of one block (perm_single_block_kernel), planned for at
-// most kSingleBlockUnits waves, kSingleBlockUnitsSmall up to
-// kSingleBlockSmallTerms terms.  Each lane's start state costs about as much
-// as a few Gray steps and is latency-bound, so fewer, longer units finish
-// sooner (kernel time, MI355X: n = 12 at 4 / 8 / 16 waves 7.9 / 8.3 / 10.2
-// us; n = 14 14.2 / 13.6 / 15.4 us); larger ones spread over the device.
-constexpr double kSingleBlockMaxTerms = 16384.0;
-constexpr int kSingleBlockUnits = 8;
-constexpr double kSingleBlockSmallTerms = 2048.0;
-constexpr int kSingleBlockUnitsSmall = 4;
+// Planned single permanents of at most this many Gray terms are planned for
+// at most kSingleFewUnits waves, kSingleFewestUnits up to kSingleFewestTerms
+// terms: each lane's start state costs about as much as a few Gray steps, so
+// fewer, longer units finish sooner.
+constexpr double kSingleFewTerms = 16384.0;
+constexpr int kSingleFewUnits = 8;
+constexpr double kSingleFewestTerms = 2048.0;
+constexpr int kSingleFewestUnits = 4;
 
 // Planning options of a single-permanent call of `in` with these
-// PQP_FLAG_* flags: about 1.4 sqrt(T) waves, capped at 16 for the
-// one-block form and per compute unit otherwise; one-wave permanents write
-// their result from the sweep kernel.
+// PQP_FLAG_* flags: about 1.4 sqrt(T) waves, capped for few terms and per
+// compute unit otherwise; one-wave permanents write their result from the
+// sweep kernel.
 PlanOptions single_plan_options(uint32_t flags, const PermInput &in);
 
-// Whether the one-item plan runs as one block (perm_single_block_kernel):
-// compensated (no PQP_FLAG_PLAIN), at least one unit, at most 16 columns
-// and kSingleBlockThreads / 64 units; `bucket` receives its width bucket.
-bool single_block_eligible(const Plan &plan, uint32_t flags, int *bucket);
+// A single permanent without tables (perm_one.hip).
+struct OnePlan {
+  PermInput in;       // transposed where that sweep is clearly cheaper
+  int n, width;       // particles, distinct columns
+  bool ones, fp32;
+  int blocks, waves;  // waves of a block
+  double terms;       // Gray terms
+};
 
-// The one-block launch's arguments for the one-item plan: `a` with the
-// rows of B copied into the arguments when they fit (else read from the
-// arena), the arena's whole 64-byte lines, and the done slot and value.
-void single_block_args(const Plan &plan, const LaunchArgs &a, uint64_t *done, uint64_t seq,
-                       SingleArgs &args);
+// Whether a single-permanent call runs on perm_one.hip: 1 <= n <= 64
+// particles, at most kOneMaxWidth distinct columns and kOneMaxTerms Gray
+// terms, and not the plain baseline.  Arguments that are not valid are left
+// to the planner.
+bool one_plan(const PermInput &in, uint32_t flags, OnePlan &p);
+
+// The launch's arguments but for its buffers; fits the blocks to the digits.
+void one_fill(OnePlan &p, OneArgs &a);
 
 // Bound on |computed - perm| of a floating-point sweep from its term
 // magnitudes m = sum_t |term_t| / 2^(n-1) (as the kernels accumulate them):

@@ -79,17 +79,48 @@ int scratch_of_current_device(char **ptr) {
   return PQP_OK;
 }
 
-struct Range {
-  explicit Range(const char *name) { roctxRangePushA(name); }
-  ~Range() { roctxRangePop(); }
-};
-
 #define PQP_NA_HIP(expr)                                                                \
   do {                                                                                  \
     hipError_t e_ = (expr);                                                             \
     if (e_ != hipSuccess)                                                               \
       return capi_fail(PQP_ERR_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
+
+// A permanent that pqp_permanent_c128 runs on perm_one.hip, by the same
+// launch (same sums, same order: bit-identical results) on the scratch
+// array: [counter][results and done slot][partials].
+int one_noalloc(OnePlan &p, double *out, double *out_dd) {
+  int st;
+  if ((st = capi_require_device()) != PQP_OK) return st;
+  std::lock_guard<std::mutex> lock(g_mu);
+  char *base = nullptr;
+  if ((st = scratch_of_current_device(&base)) != PQP_OK) return st;
+  constexpr size_t kResults = 256, kPartials = 512;
+  static_assert(kPartials + 5 * sizeof(double) * kOneMaxBlocks <= kScratchBytes, "every such permanent fits");
+  static thread_local OneArgs a;
+  one_fill(p, a);
+  const int zero = 0;
+  PQP_NA_HIP(hipMemcpy(base, &zero, sizeof(zero), hipMemcpyHostToDevice));
+  a.counter = reinterpret_cast<int *>(base);
+  a.out = reinterpret_cast<double *>(base + kResults);
+  a.partials = reinterpret_cast<double *>(base + kPartials);
+  a.done = reinterpret_cast<uint64_t *>(a.out + 7);
+  a.seq = 0;
+  PQP_NA_HIP(p.fp32 ? launch_one_f(p.width, p.ones, a, p.blocks, p.waves, nullptr)
+                    : launch_one_d(p.width, p.ones, a, p.blocks, p.waves, nullptr));
+  double res[7];
+  PQP_NA_HIP(hipMemcpy(res, a.out, sizeof(res), hipMemcpyDeviceToHost));
+  out[0] = res[0];
+  out[1] = res[1];
+  if (out_dd) std::memcpy(out_dd, res + 2, 4 * sizeof(double));
+  capi_set_last_bound(sweep_error_bound(p.n, p.fp32, res[6], res[0], res[1]));
+  return PQP_OK;
+}
+
+struct Range {
+  explicit Range(const char *name) { roctxRangePushA(name); }
+  ~Range() { roctxRangePop(); }
+};
 
 }  // namespace
 
@@ -102,12 +133,13 @@ extern "C" int pqp_permanent_c128_noalloc(const double *matrix, int64_t m_r, int
   Plan plan;
   std::string err;
   if (m_r < 0 || (m_r > 0 && !rows)) return capi_fail(PQP_ERR_INVALID, "invalid shape or null pointer");
+  OnePlan one;
+  if (one_plan(in, flags, one)) return one_noalloc(one, out, out_dd);
   int st = plan_build(std::vector<PermInput>{in}, single_plan_options(flags, in), plan, err);
   if (st != PQP_OK) return capi_fail(st, err);
 
   // scratch layout: [arena][partials: 4 doubles per slot][term magnitudes:
-  // 1 double per slot][results: 2 + 4 + 1 doubles, then the done slot of a
-  // one-block launch]
+  // 1 double per slot][results: 2 + 4 + 1 doubles]
   const size_t arena_bytes = plan.arena.size();
   const size_t partials_off = align256(arena_bytes);
   const size_t n_slots = static_cast<size_t>(std::max<int64_t>(plan.n_partials, 1));
@@ -138,29 +170,19 @@ extern "C" int pqp_permanent_c128_noalloc(const double *matrix, int64_t m_r, int
   a.n_units = static_cast<int32_t>(plan.units.size());
   a.n_items = static_cast<int32_t>(plan.items.size());
   const bool comp = !(flags & PQP_FLAG_PLAIN) || plan.fp32;
-  int bucket = -1;
-  if (single_block_eligible(plan, flags, &bucket)) {
-    // the kernel pqp_permanent_c128 runs for this plan (same sums, same
-    // order: bit-identical results); its done slot is scratch here, and the
-    // synchronous copy below waits for the launch
-    static thread_local SingleArgs args;
-    single_block_args(plan, a, reinterpret_cast<uint64_t *>(a.out + 7), 0, args);
-    PQP_NA_HIP(launch_single_block(bucket, plan.fp32, args, nullptr));
-  } else {
-    for (const Plan::Range &r : plan.ranges) {
-      FwdLaunch l;
-      l.args = a;
-      l.first_unit = r.first;
-      l.n_units = r.count;
-      l.persistent = false;
-      l.fp32 = plan.fp32;
-      l.comp = comp;
-      l.stream = nullptr;
-      PQP_NA_HIP(launch_fwd(r.bucket, l));
-    }
-    if (!plan.all_direct)
-      PQP_NA_HIP(launch_finalize(comp, a, 0, a.n_items, 0, plan.max_units, nullptr));
+  for (const Plan::Range &r : plan.ranges) {
+    FwdLaunch l;
+    l.args = a;
+    l.first_unit = r.first;
+    l.n_units = r.count;
+    l.persistent = false;
+    l.fp32 = plan.fp32;
+    l.comp = comp;
+    l.stream = nullptr;
+    PQP_NA_HIP(launch_fwd(r.bucket, l));
   }
+  if (!plan.all_direct)
+    PQP_NA_HIP(launch_finalize(comp, a, 0, a.n_items, 0, plan.max_units, nullptr));
   double res[7];
   PQP_NA_HIP(hipMemcpy(res, base + results_off, sizeof(res), hipMemcpyDeviceToHost));
   out[0] = res[0];

@@ -137,19 +137,10 @@ __device__ __forceinline__ void column_product(const R (&cr)[MCP], const R (&ci)
   pi = ai;
 }
 
-// A unit's sum over its 64 lanes (every lane holds it after the butterfly)
-// and the magnitudes of its terms.
-struct WaveTotal {
-  cdd s;
-  double abs;
-};
-
 // One wave unit: top states [64*local, 64*local+64) of item `item`.  ABS
 // (compensated static launches): also sum the magnitudes of the terms.
-// `total`, when given, receives the unit's sum as well.
-template <int MCP, typename R, bool COMP, bool ABS, bool UNIT_BASE = false>
-__device__ __forceinline__ void sweep_unit(const LaunchArgs &a, int item, int local,
-                                           WaveTotal *total = nullptr) {
+template <int MCP, typename R, bool COMP, bool ABS>
+__device__ __forceinline__ void sweep_unit(const LaunchArgs &a, int item, int local) {
   const cptr<ItemDesc> it = as_const<ItemDesc>(a.items) + item;
   const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
   const int64_t U = it->U;
@@ -163,7 +154,7 @@ __device__ __forceinline__ void sweep_unit(const LaunchArgs &a, int item, int lo
   const bool active = u < U;
   if (!active) u = U - 1;
 
-  const cptr<R> Bin = b_rows<R>(a, it) + 2 * MCP;  // inner rows of B (after the prepended row)
+  const cptr<R> Bin = as_const<R>(a.arena, it->b_off) + 2 * MCP;  // inner rows of B (after the prepended row)
   const cptr<InnerEntry> tab = as_const<InnerEntry>(a.arena, it->step_off);
   const cptr<int32_t> cpow = as_const<int32_t>(a.arena, it->cpow_off + 24);
   PowState ps{0u, 0u, 0u, 0};
@@ -177,7 +168,7 @@ __device__ __forceinline__ void sweep_unit(const LaunchArgs &a, int item, int lo
 
   R cr[MCP], ci[MCP];
   double w_top;
-  start_state<MCP, R, UNIT_BASE>(a, it, u, L, Dt, flags, cr, ci, w_top);
+  start_state<MCP, R>(a, it, u, L, Dt, flags, cr, ci, w_top);
   // (-1)^{|g_top|} = (-1)^u: consecutive top states differ by one unit step.
   double lane_w = (u & 1) ? -w_top : w_top;
   if (!active) lane_w = 0.0;
@@ -253,10 +244,6 @@ __device__ __forceinline__ void sweep_unit(const LaunchArgs &a, int item, int lo
     lane_sum.re.hi = wave_sum(lane_sum.re.hi, lane);
     lane_sum.im.hi = wave_sum(lane_sum.im.hi, lane);
   }
-  if (total) {
-    total->s = lane_sum;
-    total->abs = abs_sum;
-  }
   if (lane == 0) {
     if (flags & kDirectOut) {
       // the item's only unit: scale by 2^-(n-1) and write the result
@@ -284,14 +271,13 @@ __device__ __forceinline__ void sweep_unit(const LaunchArgs &a, int item, int lo
   }
 }
 
-template <int LO, int HI, typename R, bool COMP, bool ABS, bool UNIT_BASE = false>
-__device__ __forceinline__ void dispatch(const LaunchArgs &a, int mcp, int item, int local,
-                                         WaveTotal *total = nullptr) {
+template <int LO, int HI, typename R, bool COMP, bool ABS>
+__device__ __forceinline__ void dispatch(const LaunchArgs &a, int mcp, int item, int local) {
   if constexpr (LO <= HI) {
     if (mcp == LO) {
-      sweep_unit<LO, R, COMP, ABS, UNIT_BASE>(a, item, local, total);
+      sweep_unit<LO, R, COMP, ABS>(a, item, local);
     } else {
-      dispatch<LO + 1, HI, R, COMP, ABS, UNIT_BASE>(a, mcp, item, local, total);
+      dispatch<LO + 1, HI, R, COMP, ABS>(a, mcp, item, local);
     }
   }
 }
@@ -406,14 +392,7 @@ __device__ __forceinline__ void finalize_item(const LaunchArgs &a, int item) {
 // One block of NT threads per item (finalize_item).  NT = 64 for batches of
 // small items, 1024 when an item has thousands of units.  Block 0 also
 // rewinds the work-queue heads for the next launch of the same plan.
-// Static launch: block b sweeps unit first_unit + b.  A one-item launch of a
-// single permanent (a.last_counter set) also finalizes the item in the block
-// that finishes last: every block makes its partial visible device-wide,
-// counts itself, and the block that counts last reads all partials (the
-// fences order the partial writes, on any XCD, before the count and the
-// count before the reads), writes the result to mapped host memory, resets
-// the counter for the next launch on the stream and publishes the sequence
-// number, so the caller polls instead of waiting for a finalize launch.
+// Static launch: block b sweeps unit first_unit + b.
 template <int LO, int HI, typename R, bool COMP>
 __global__ __launch_bounds__(kWave)
 __attribute__((amdgpu_waves_per_eu(waves_for(HI, sizeof(R) == 4), 8))) void perm_static_kernel(LaunchArgs a, int first_unit) {
@@ -422,25 +401,6 @@ __attribute__((amdgpu_waves_per_eu(waves_for(HI, sizeof(R) == 4), 8))) void perm
   const int local = uniform(wu->local);
   const int mcp = uniform(as_const<ItemDesc>(a.items)[item].mcp);
   dispatch<LO, HI, R, COMP, COMP>(a, mcp, item, local);
-  // widths up to 16 only (kLastFinalizeMaxWidth): in the wider kernels the
-  // finalize code took private memory
-  if constexpr (COMP && HI <= kLastFinalizeMaxWidth) {
-    if (a.last_counter) {
-      __threadfence();
-      int old = 0;
-      if (threadIdx.x == 0) old = atomicAdd(a.last_counter, 1);
-      old = __builtin_amdgcn_readfirstlane(old);
-      if (old == static_cast<int>(gridDim.x) - 1) {
-        __threadfence();
-        finalize_item<true, kWave>(a, item);
-        if (threadIdx.x == 0) {
-          *a.last_counter = 0;
-          __threadfence_system();
-          __hip_atomic_store(a.done, a.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-      }
-    }
-  }
 }
 
 template <bool COMP, int NT>
@@ -449,114 +409,6 @@ __global__ __launch_bounds__(NT) void perm_finalize_kernel(LaunchArgs a, int ite
   if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < n_heads) a.queue_head[threadIdx.x] = 0;
   if (item >= a.n_items) return;
   finalize_item<COMP, NT>(a, item);
-}
-
-// One small permanent (item 0 of a one-item plan) in one launch, for the
-// single-call path: the block's waves sweep the item's units (wave w: units
-// w, w + W, ...), the block adds their sums (a one-unit item has written
-// its result from the sweep), and thread 0 then publishes `seq` to `done`
-// (host-visible memory) after a system-scope fence, so the host can poll
-// for the result instead of synchronising the stream.
-//
-// A lone small sweep is latency-bound: every first touch of a table line
-// is a scalar-cache miss, and the sweep's loads depend on each other
-// (descriptor -> table -> row), so misses would queue up one after another.
-// The waves therefore first touch every 64-byte line of the plan's arena
-// (wave w: lines w, w + W, ..., four independent loads in flight per wave)
-// and meet at a barrier, after which the sweep's scalar loads hit.
-//
-// The rows of B may come in the kernel arguments (SingleArgs::b): the
-// argument struct is read through the kernel-argument segment pointer, as
-// scalar loads like the arena.
-template <int LO, int HI, typename R, bool UNIT_BASE>
-__global__ __launch_bounds__(kSingleBlockThreads) void perm_single_block_kernel(SingleArgs args) {
-  constexpr int W = kSingleBlockThreads / kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-  const uintptr_t b_addr = reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr()) +
-                           offsetof(SingleArgs, b);
-  LaunchArgs a = args.a;
-  const int arena_lines = args.arena_lines;
-  int b_lines = 0;
-  if (args.b_in_args) {
-    a.b_rows = reinterpret_cast<const char *>(b_addr);
-    b_lines = kSingleArgBBytes / 64;
-  }
-  if (UNIT_BASE) a.unit_base = reinterpret_cast<const char *>(b_addr + args.base_off);
-  {
-    const cptr<uint32_t> lines = as_const<uint32_t>(a.arena);
-    const cptr<uint32_t> blines = reinterpret_cast<cptr<uint32_t>>(b_addr);
-    // straight-line loads with indices clamped to the last line, consumed
-    // together by one asm statement, so all of them are in flight before
-    // a single wait (the first 4 W lines of the arena and the kernel
-    // arguments' rows of B; larger arenas continue in a loop)
-    const int la = arena_lines - 1, lb = b_lines > 0 ? b_lines - 1 : 0;
-    const cptr<uint32_t> bl = b_lines > 0 ? blines : lines;
-    const int lbx = b_lines > 0 ? lb : la;
-    const uint32_t v0 = lines[16 * min(wave, la)], v1 = lines[16 * min(wave + W, la)];
-    const uint32_t v2 = lines[16 * min(wave + 2 * W, la)], v3 = lines[16 * min(wave + 3 * W, la)];
-    const uint32_t v4 = bl[16 * min(wave, lbx)], v5 = bl[16 * min(wave + W, lbx)];
-    const uint32_t v6 = bl[16 * min(wave + 2 * W, lbx)], v7 = bl[16 * min(wave + 3 * W, lbx)];
-    __asm__ volatile("" ::"s"(v0), "s"(v1), "s"(v2), "s"(v3), "s"(v4), "s"(v5), "s"(v6), "s"(v7));
-    uint32_t t = 0;
-    for (int l = wave + 4 * W; l < arena_lines; l += W) t ^= lines[16 * l];
-    __asm__ volatile("" ::"s"(t));
-  }
-  __syncthreads();
-  const cptr<ItemDesc> it = as_const<ItemDesc>(a.items);
-  const int units = uniform(it->units);
-  const int mcp = uniform(it->mcp);
-  if (units <= W) {
-    // one unit per wave: the waves' totals meet in LDS and the first 16
-    // lanes of wave 0 add them with a fixed butterfly (a one-unit item has
-    // written its result itself)
-    __shared__ double part[W][5];
-    WaveTotal total{cdd_zero(), 0.0};
-    if (wave < units) dispatch<LO, HI, R, true, true, UNIT_BASE>(a, mcp, 0, wave, &total);
-    if ((threadIdx.x & (kWave - 1)) == 0 && wave < units) {
-      part[wave][0] = total.s.re.hi;
-      part[wave][1] = total.s.re.lo;
-      part[wave][2] = total.s.im.hi;
-      part[wave][3] = total.s.im.lo;
-      part[wave][4] = total.abs;
-    }
-    __syncthreads();
-    if (wave == 0 && !(uniform(it->flags) & kDirectOut)) {
-      // lane l < units holds unit l's total, the others zero; butterfly
-      // steps over lanes l ^ 1, l ^ 2, 7 - l and 15 - l leave the sum of
-      // lanes 0..15 (W = 16 waves) in every one of them, added in a fixed
-      // order; lane 0 writes the result
-      static_assert(W == 16, "the butterfly below covers 16 unit totals");
-      const int lane = static_cast<int>(threadIdx.x);
-      const bool has = lane < units;
-      cdd s = has ? cdd{{part[lane][0], part[lane][1]}, {part[lane][2], part[lane][3]}} : cdd_zero();
-      double abs_sum = has ? part[lane][4] : 0.0;
-      s = wave_reduce<0, 4>(s, lane);
-      abs_sum = wave_sum<0, 4>(abs_sum, lane);
-      if (lane == 0) {
-        const int e = -(it->n - 1);
-        const double re_hi = ldexp(s.re.hi, e), re_lo = ldexp(s.re.lo, e);
-        const double im_hi = ldexp(s.im.hi, e), im_lo = ldexp(s.im.lo, e);
-        const int o = it->out_index;
-        a.out[2 * o] = re_hi + re_lo;
-        a.out[2 * o + 1] = im_hi + im_lo;
-        if (a.out_dd) {
-          a.out_dd[4 * o] = re_hi;
-          a.out_dd[4 * o + 1] = re_lo;
-          a.out_dd[4 * o + 2] = im_hi;
-          a.out_dd[4 * o + 3] = im_lo;
-        }
-        if (a.out_abs) a.out_abs[o] = ldexp(abs_sum, e);
-      }
-    }
-  } else {
-    for (int u = wave; u < units; u += W) dispatch<LO, HI, R, true, true>(a, mcp, 0, u);
-    __syncthreads();
-    if (!(uniform(it->flags) & kDirectOut)) finalize_item<true, kSingleBlockThreads>(a, 0);
-  }
-  if (threadIdx.x == 0) {
-    __threadfence_system();
-    __hip_atomic_store(args.done, args.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
 }
 
 }  // namespace pqp
@@ -644,19 +496,6 @@ hipError_t PQP_NAME(occupancy_fwd_b)(bool persistent, int *blocks) {
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(
       blocks, perm_static_kernel<PQP_LO, PQP_HI, PQP_R, PQP_COMP>, kWave, 0);
 }
-
-#if PQP_BUCKET_ID <= 1 && PQP_VARIANT != 1
-hipError_t PQP_NAME(launch_single_block_b)(const SingleArgs &args, hipStream_t stream) {
-  // the instantiation with per-unit start rows only where the host made them
-  if (args.base_in_args)
-    hipLaunchKernelGGL((perm_single_block_kernel<PQP_LO, PQP_HI, PQP_R, true>), dim3(1),
-                       dim3(kSingleBlockThreads), 0, stream, args);
-  else
-    hipLaunchKernelGGL((perm_single_block_kernel<PQP_LO, PQP_HI, PQP_R, false>), dim3(1),
-                       dim3(kSingleBlockThreads), 0, stream, args);
-  return hipGetLastError();
-}
-#endif
 
 #if PQP_BUCKET_ID == 0 && PQP_VARIANT == 0
 hipError_t launch_finalize(bool comp, const LaunchArgs &a, int item0, int n_items,

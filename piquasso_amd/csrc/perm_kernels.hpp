@@ -12,6 +12,7 @@
 #include "poly_types.hpp"
 #include "table_types.hpp"
 #include "minors_wave_types.hpp"
+#include "one_types.hpp"
 
 namespace pqp {
 
@@ -44,13 +45,11 @@ PQP_DECLARE_BUCKET(7)
 #undef PQP_DECLARE_BUCKET
 #undef PQP_DECLARE
 
-// One-launch single permanents (perm_single_block_kernel), widths 1..16:
-// d = FP64 + dd, f = FP32 products + dd.
-hipError_t launch_single_block_b0_d(const SingleArgs &args, hipStream_t s);
-hipError_t launch_single_block_b0_f(const SingleArgs &args, hipStream_t s);
-hipError_t launch_single_block_b1_d(const SingleArgs &args, hipStream_t s);
-hipError_t launch_single_block_b1_f(const SingleArgs &args, hipStream_t s);
-hipError_t launch_single_block(int bucket, bool fp32, const SingleArgs &args, hipStream_t stream);
+// Single permanents planned by their own waves (perm_one.hip): one launch
+// of `blocks` blocks of `waves` waves for a permanent of `width` distinct columns (all of
+// multiplicity 1: ones).
+hipError_t launch_one_d(int width, bool ones, const OneArgs &a, int blocks, int waves, hipStream_t stream);
+hipError_t launch_one_f(int width, bool ones, const OneArgs &a, int blocks, int waves, hipStream_t stream);
 
 constexpr int kBuckets = 8;        // forward kernel width buckets
 constexpr int kMinorBuckets = 9;   // column-minor kernel buckets

@@ -1,0 +1,338 @@
+// One permanent of up to 2^24 Gray terms in one launch on gfx950, for the
+// single-call entry points (src/permanent.cpp:49-264 is the sum).  Nothing
+// is planned into tables, copied and loaded: the kernel arguments hold the
+// distinct rows, in the order of their digits, and the multiplicities.
+//
+// Sums as in perm_fwd.hip: row sums and products in Real (FP64, or FP32
+// where the caller chose it), FP64 runs of at most 64 terms folded into
+// double-double, exact integer weights, the lanes' and waves' sums added in
+// double-double in a fixed order (a value does not depend on scheduling).
+//
+// Bound by latency: 2^19 terms of 20 columns are 3 us of FP64 issue for the
+// whole chip.  What counts is the chain of one wave: its start, its inner
+// states, the double-double reductions, and the way to the host.  So
+//  * the lanes of a wave differ in a few digits only, six binary ones or as
+//    many states in at most 64 as the digits allow.  The rows of all other
+//    digits are summed once per wave, a lane per component (their loads are
+//    in flight together), and broadcast through the LDS; a lane then adds a
+//    few rows instead of all;
+//  * these rows and the inner ones are scalar operands, and the waves of
+//    a block touch their lines together first;
+//  * permanents of few terms stay in one block (no block waits for another),
+//    others take up to one wave per SIMD with few inner states.  Their
+//    blocks count themselves; the last one sums the partials and publishes
+//    the result to mapped host memory.
+//
+// A call with occupations not seen before, against the planned sweep: 8
+// particles 15.0 -> 11.7 us, 12 18.1 -> 14.5, 16 35.6 -> 17.6, 18 47 -> 19,
+// 20 45 -> 23, 24 98 -> 61 (of it 55 us of FP64 issue); 20 in 15 of 40
+// modes 49 -> 20.  The kernel takes 5.5 us at 8 particles (one wave) and
+// 12 at 18, of it about 3 for the blocks' meeting.
+//
+// Compiled once per type of the rows: -DPQP_ONE_FP32=0, 1.
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+
+#include "dd.hpp"
+#include "one_types.hpp"
+#include "perm_kernels.hpp"
+#include "sweep_common.hpp"
+
+namespace pqp {
+
+namespace {
+
+constexpr int kOneChunk = 8;  // common rows of a wave loaded at once
+
+#if PQP_ONE_FP32
+using Real = float;
+#else
+using Real = double;
+#endif
+
+// The product over the columns of one state's row sums.
+template <int W, bool ONES>
+__device__ __forceinline__ void one_product(const Real (&cr)[W], const Real (&ci)[W], cptr<uint32_t> over,
+                                            int cmax, Real &pr, Real &pi) {
+  Real ar = cr[0], ai = ci[0];
+  if constexpr (W > 1) {
+    Real br = cr[1], bi = ci[1];
+#pragma unroll
+    for (int j = 2; j + 1 < W; j += 2) {
+      cmul(ar, ai, cr[j], ci[j]);
+      cmul(br, bi, cr[j + 1], ci[j + 1]);
+    }
+    if constexpr (W % 2 == 1 && W > 2) cmul(ar, ai, cr[W - 1], ci[W - 1]);
+    cmul(ar, ai, br, bi);
+  }
+  if constexpr (!ONES) {
+    for (int r = 2; r <= cmax; ++r) {
+      const uint32_t cols = over[r - 2];
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        if ((cols >> j) & 1u) {
+          __asm__ volatile("");  // a branch, not a masked multiply at every column
+          cmul(ar, ai, cr[j], ci[j]);
+        }
+      }
+    }
+  }
+  pr = ar;
+  pi = ai;
+}
+
+// u's lowest digit of radix rho + 1, taken off u (u < 2^50: the quotient is
+// exact this way).
+__device__ __forceinline__ int one_digit(int &u, int rho) {
+  const int q = static_cast<int>((static_cast<double>(u) + 0.5) * kInvSmall[rho + 1]);
+  const int g = u - q * (rho + 1);
+  u = q;
+  return g;
+}
+
+// C(rho, g), the small ones without a loop.
+__device__ __forceinline__ double one_binomial(int rho, int g) {
+  if (rho <= 3) return (g == 0 || g == rho) ? 1.0 : static_cast<double>(rho);
+  return lane_binomial(rho, g);
+}
+
+// The sum over a block of nw waves, in the lanes 0..7 of wave 0.
+__device__ __forceinline__ void block_sum(cdd &s, double &mag, double (&part)[kOneWaves][5], int nw, int wave, int lane) {
+  s = wave_reduce<0>(s, lane);
+  mag = wave_sum(mag, lane);
+  if (nw == 1) return;
+  if (lane == 0) {
+    part[wave][0] = s.re.hi;
+    part[wave][1] = s.re.lo;
+    part[wave][2] = s.im.hi;
+    part[wave][3] = s.im.lo;
+    part[wave][4] = mag;
+  }
+  __syncthreads();
+  const int w = lane < nw ? lane : 0;
+  s = lane < nw ? cdd{{part[w][0], part[w][1]}, {part[w][2], part[w][3]}} : cdd_zero();
+  mag = lane < nw ? part[w][4] : 0.0;
+  static_assert(kOneWaves <= 8, "three butterfly steps");
+  s = wave_reduce<0, 3>(s, lane);
+  mag = wave_sum<0, 3>(mag, lane);
+}
+
+template <int W, bool ONES>
+__global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(OneArgs args) {
+  const int nw = static_cast<int>(blockDim.x) / kWave;
+  __shared__ double part[kOneWaves][5];
+  __shared__ Real base[kOneWaves][2 * W];
+  const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+  const int bw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
+  const int waves = nw * static_cast<int>(gridDim.x);
+  const int wave = nw * static_cast<int>(blockIdx.x) + bw;
+  const uintptr_t self = reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  const cptr<Real> rows = reinterpret_cast<cptr<Real>>(self + offsetof(OneArgs, b));
+  const Real *vrows = reinterpret_cast<const Real *>(self + offsetof(OneArgs, b));
+  const cptr<uint32_t> over = reinterpret_cast<cptr<uint32_t>>(self + offsetof(OneArgs, over));
+  const cptr<int32_t> lane_rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneArgs, lane_rho));
+  const cptr<int32_t> rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneArgs, rho));
+  const cptr<OneStep> step = reinterpret_cast<cptr<OneStep>>(self + offsetof(OneArgs, step));
+  const int n = args.n, k = args.inner, rest = args.rest, cmax = args.cmax;
+  const int L = args.lane_digits, S = args.S, chunks = args.chunks;
+  const bool active = lane < args.lanes;
+  const bool binary = args.binary;
+  // The first rows common to a wave's lanes, a component per lane: requested
+  // before the wave waits for anything else (a first touch costs about a
+  // microsecond, and one after another these were most of the start).
+  const int common = 1 + k + rest;
+  const int at = lane < 2 * W ? lane : 0;
+  Real first[kOneChunk];
+#pragma unroll
+  for (int i = 0; i < kOneChunk; ++i) first[i] = vrows[(L + min(i, common - 1)) * (2 * W) + at];
+  {
+    // every line of the rows read as scalars, eight loads of a wave in flight
+    const cptr<uint32_t> lines = reinterpret_cast<cptr<uint32_t>>(self + offsetof(OneArgs, b));
+    const int end = ((L + 1 + k) * 2 * W * static_cast<int>(sizeof(Real)) - 1) / 64;
+    for (int l = bw; l <= end; l += 8 * nw) {
+      const uint32_t v0 = lines[16 * l], v1 = lines[16 * min(l + nw, end)];
+      const uint32_t v2 = lines[16 * min(l + 2 * nw, end)], v3 = lines[16 * min(l + 3 * nw, end)];
+      const uint32_t v4 = lines[16 * min(l + 4 * nw, end)], v5 = lines[16 * min(l + 5 * nw, end)];
+      const uint32_t v6 = lines[16 * min(l + 6 * nw, end)], v7 = lines[16 * min(l + 7 * nw, end)];
+      __asm__ volatile("" ::"s"(v0), "s"(v1), "s"(v2), "s"(v3), "s"(v4), "s"(v5), "s"(v6), "s"(v7));
+    }
+  }
+  if (nw > 1) __syncthreads();
+
+  cdd sum = cdd_zero();
+  double mag = 0.0;  // of the terms: |Re| + |Im| each
+  for (int chunk = wave; chunk < chunks; chunk += waves) {
+    Real cr[W], ci[W];
+    double w = 1.0;
+    int parity = 0;
+    // the rows common to the lanes: the prepended one, the inner ones at
+    // their first state, then the rest digits
+    double b = 0.0;
+    int u = chunk;
+    for (int c0 = 0; c0 < common; c0 += kOneChunk) {
+      Real v[kOneChunk];
+#pragma unroll
+      for (int i = 0; i < kOneChunk; ++i)
+        v[i] = c0 == 0 ? first[i] : vrows[(L + min(c0 + i, common - 1)) * (2 * W) + at];
+#pragma unroll
+      for (int i = 0; i < kOneChunk; ++i) {
+        const int t = c0 + i - 1;
+        if (t < k + rest) {
+          double al = t < 0 ? 1.0 : rho[t];
+          if (t >= k) {
+            const int rr = rho[t];
+            const int g = one_digit(u, rr);
+            parity ^= g & 1;
+            w *= one_binomial(rr, g);
+            al = static_cast<double>(rr - 2 * g);
+          }
+          b = fmaR(al, static_cast<double>(v[i]), b);
+        }
+      }
+    }
+    if (lane < 2 * W) base[bw][lane] = static_cast<Real>(b);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+      cr[j] = base[bw][2 * j];
+      ci[j] = base[bw][2 * j + 1];
+    }
+    __builtin_amdgcn_wave_barrier();
+    u = lane;
+#pragma unroll 1
+    for (int t = 0; t < L; ++t) {
+      const int rr = lane_rho[t];
+      Real al;
+      if (rr == 1) {
+        al = (u & 1) ? Real(-1) : Real(1);
+        parity ^= u & 1;
+        u >>= 1;
+      } else {
+        const int g = one_digit(u, rr);
+        parity ^= g & 1;
+        w *= one_binomial(rr, g);
+        al = static_cast<Real>(rr - 2 * g);
+      }
+      const cptr<Real> row = rows + t * (2 * W);
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        cr[j] = fmaR(al, row[2 * j], cr[j]);
+        ci[j] = fmaR(al, row[2 * j + 1], ci[j]);
+      }
+    }
+    if (!active) w = 0.0;
+    if (parity) w = -w;
+    // the inner states in Gray order
+    double sr = 0.0, si = 0.0, sa = 0.0;
+    for (int v = 0; v < S; ++v) {
+      // the digit that moves after state v (after the last one any: an
+      // update that is not read)
+      const int move = __builtin_ctz(v + 1);
+      const int up = (v + 1) ^ ((v + 1) >> 1);
+      int row = move < k ? 1 + move : 0;
+      Real s2 = in_vgpr(((up >> move) & 1) ? Real(-2) : Real(2));
+      double coef = in_vgpr((v & 1) ? -1.0 : 1.0);
+      if (!binary) {
+        row = step[v].row;
+        s2 = in_vgpr(static_cast<Real>(step[v].factor));
+        coef = in_vgpr(step[v].coef);
+      }
+      const cptr<Real> b = rows + (L + row) * (2 * W);
+      Real pr, pi;
+      one_product<W, ONES>(cr, ci, over, cmax, pr, pi);
+      const double dr = static_cast<double>(pr), di = static_cast<double>(pi);
+      sr = fmaR(coef, dr, sr);
+      si = fmaR(coef, di, si);
+      sa = fmaR(__builtin_fabs(coef), __builtin_fabs(dr), sa);
+      sa = fmaR(__builtin_fabs(coef), __builtin_fabs(di), sa);
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        cr[j] = fmaR(s2, b[2 * j], cr[j]);
+        ci[j] = fmaR(s2, b[2 * j + 1], ci[j]);
+      }
+    }
+    sum = cdd_add(sum, cdd{dd_mul_d(dd{sr, 0.0}, w), dd_mul_d(dd{si, 0.0}, w)});
+    mag = fmaR(sa, __builtin_fabs(w), mag);
+  }
+  block_sum(sum, mag, part, nw, bw, lane);
+  if (bw != 0) return;
+  if (gridDim.x > 1) {
+    // The block that counts last sums the blocks' partials.  They are
+    // written and read at device scope, past the XCDs' own L2s, so that the
+    // count needs to wait for the block's own writes only (a device-wide
+    // fence writes a whole L2 back).
+    const int blocks = static_cast<int>(gridDim.x);
+    if (lane < 5) {
+      const double x = lane == 0   ? sum.re.hi
+                       : lane == 1 ? sum.re.lo
+                       : lane == 2 ? sum.im.hi
+                       : lane == 3 ? sum.im.lo
+                                   : mag;
+      __hip_atomic_store(args.partials + 5 * static_cast<int>(blockIdx.x) + lane, x, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    int old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(args.counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(old) != blocks - 1) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    sum = cdd_zero();
+    mag = 0.0;
+    for (int q0 = lane; q0 < blocks; q0 += kWave) {
+      double q[5];
+#pragma unroll
+      for (int i = 0; i < 5; ++i)
+        q[i] = __hip_atomic_load(args.partials + 5 * q0 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sum = cdd_add(sum, cdd{{q[0], q[1]}, {q[2], q[3]}});
+      mag += q[4];
+    }
+    sum = wave_reduce<0>(sum, lane);
+    mag = wave_sum(mag, lane);
+    if (lane == 0) __hip_atomic_store(args.counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (lane == 0) {
+    const int e = -(n - 1);
+    const double re_hi = ldexp(sum.re.hi, e), re_lo = ldexp(sum.re.lo, e);
+    const double im_hi = ldexp(sum.im.hi, e), im_lo = ldexp(sum.im.lo, e);
+    args.out[0] = re_hi + re_lo;
+    args.out[1] = im_hi + im_lo;
+    args.out[2] = re_hi;
+    args.out[3] = re_lo;
+    args.out[4] = im_hi;
+    args.out[5] = im_lo;
+    args.out[6] = ldexp(mag, e);
+    __threadfence_system();
+    __hip_atomic_store(args.done, args.seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+}  // namespace
+
+#if PQP_ONE_FP32
+hipError_t launch_one_f(int width, bool ones, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
+#else
+hipError_t launch_one_d(int width, bool ones, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
+#endif
+  if (blocks < 1 || waves < 1 || waves > kOneWaves || a.n < 1 || a.chunks < 1)
+    return hipErrorInvalidValue;
+  switch (width) {
+#define X(W)                                                                                              \
+  case W:                                                                                                 \
+    if (ones)                                                                                             \
+      hipLaunchKernelGGL((perm_one_kernel<W, true>), dim3(blocks), dim3(kWave * waves), 0, stream, a);    \
+    else                                                                                                  \
+      hipLaunchKernelGGL((perm_one_kernel<W, false>), dim3(blocks), dim3(kWave * waves), 0, stream, a);   \
+    return hipGetLastError();
+    X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
+    X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20) X(21) X(22) X(23) X(24)
+#undef X
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace pqp

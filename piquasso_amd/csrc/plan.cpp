@@ -156,34 +156,34 @@ double sweep_cost(const int32_t *rows, int64_t m_r, const int32_t *cols, int64_t
   return T * (2.0 * mc + 6.0 * mult + 4.0) * 1.25;
 }
 
-// Items whose transposed sweep costs less than 0.9 of the given one are
-// planned transposed: perm(A; r, c) = perm(A^T; c, r), the permanent of the
-// expanded matrix being invariant under transposition.  Invalid items are
-// left alone (the planner reports them).
+}  // namespace
+
+bool plan_orient(PermInput &v) {
+  if (v.col_excess || v.m_r <= 0 || v.m_c <= 0 || !v.a || !v.rows || !v.cols || !stride_ok(v)) return false;
+  int64_t sr = 0, sc = 0;
+  bool neg = false;
+  for (int64_t i = 0; i < v.m_r; ++i) {
+    neg = neg || v.rows[i] < 0;
+    sr += v.rows[i];
+  }
+  for (int64_t j = 0; j < v.m_c; ++j) {
+    neg = neg || v.cols[j] < 0;
+    sc += v.cols[j];
+  }
+  if (neg || sr != sc || sr == 0 || sr > kMaxCols) return false;
+  if (!(sweep_cost(v.cols, v.m_c, v.rows, v.m_r) < 0.9 * sweep_cost(v.rows, v.m_r, v.cols, v.m_c))) return false;
+  std::swap(v.m_r, v.m_c);
+  std::swap(v.rows, v.cols);
+  v.transposed = true;
+  return true;
+}
+
+namespace {
+
 void orient_items(const std::vector<PermInput> &in, std::vector<PermInput> &out, bool &any) {
   any = false;
   out = in;
-  for (PermInput &v : out) {
-    if (v.col_excess || v.m_r <= 0 || v.m_c <= 0 || !v.a || !v.rows || !v.cols || !stride_ok(v))
-      continue;
-    int64_t sr = 0, sc = 0;
-    bool neg = false;
-    for (int64_t i = 0; i < v.m_r; ++i) {
-      neg = neg || v.rows[i] < 0;
-      sr += v.rows[i];
-    }
-    for (int64_t j = 0; j < v.m_c; ++j) {
-      neg = neg || v.cols[j] < 0;
-      sc += v.cols[j];
-    }
-    if (neg || sr != sc || sr == 0 || sr > kMaxCols) continue;
-    if (sweep_cost(v.cols, v.m_c, v.rows, v.m_r) < 0.9 * sweep_cost(v.rows, v.m_r, v.cols, v.m_c)) {
-      std::swap(v.m_r, v.m_c);
-      std::swap(v.rows, v.cols);
-      v.transposed = true;
-      any = true;
-    }
-  }
+  for (PermInput &v : out) any = plan_orient(v) || any;
 }
 
 }  // namespace

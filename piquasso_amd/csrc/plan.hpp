@@ -114,6 +114,12 @@ int bucket_for_width(int mc, bool fp32, int *mcp_out);
 // [items[k].b_off, + info[k].rowsrc.size() * mcp * 2 * (4 or 8)).
 void plan_refresh_matrix(Plan &plan, const std::vector<PermInput> &inputs);
 
+// Transposes an item whose transposed sweep costs less than 0.9 of the given
+// one: perm(A; r, c) = perm(A^T; c, r), the permanent of the expanded matrix
+// being invariant under transposition.  Invalid items are left alone (the
+// planner reports them).  True when transposed.
+bool plan_orient(PermInput &in);
+
 int plan_build(const std::vector<PermInput> &inputs, const PlanOptions &opt,
                Plan &plan, std::string &err);
 

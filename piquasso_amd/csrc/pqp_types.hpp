@@ -23,7 +23,6 @@
 namespace pqp {
 
 constexpr int kWave = 64;          // CDNA wavefront width
-constexpr int kSingleBlockThreads = 1024;  // one-launch single permanents: 16 waves in one block
 constexpr int kMaxCols = 64;       // widest row-sum vector a kernel keeps in VGPRs
 constexpr int kMaxDigits = 63;     // Gray digits (rows) per permanent
 constexpr int kDdFold = 64;        // FP64 run length folded into dd accumulators
@@ -115,49 +114,6 @@ struct LaunchArgs {
   // permanent (out_abs).  Null where a launch does not keep them.
   double *part_abs = nullptr;
   double *out_abs = nullptr;
-  // One-item plans only: the rows of B of item 0 at this address instead of
-  // arena + b_off (the copy a one-block launch carries in its kernel
-  // arguments); null everywhere else.
-  const char *b_rows = nullptr;
-  // One-block launches of items whose top digits are all binary: per unit,
-  // the row sums of its first state less the lowest kLaneDigits top digits
-  // (the prepended row, the inner rows at their start coefficients and the
-  // top digits that are the same for all 64 lanes of the unit), m_cp values
-  // of the item's real type per unit, computed on the host; null elsewhere.
-  const char *unit_base = nullptr;
-  // One-item static launches of a single permanent: each block counts itself
-  // at last_counter after writing its partial; the block that counts last
-  // sums the item's partials, writes the result, resets the counter and
-  // publishes seq at done (mapped host memory).  Null elsewhere.
-  int *last_counter = nullptr;
-  uint64_t *done = nullptr;
-  uint64_t seq = 0;
-};
-
-// The queue-head slot that holds a single permanent's block counter, and
-// the widest kernel that finalizes in its last block.
-constexpr int kLastCounterSlot = 63;
-constexpr int kLastFinalizeMaxWidth = 16;
-
-// Top digits that differ between the 64 lanes of a unit (lane l of unit w
-// holds top state 64 w + l): the reflected binary digits 0..5.
-constexpr int kLaneDigits = 6;
-
-// Kernel arguments of the one-block single-permanent launch: the launch
-// arguments, the done slot it publishes to, and up to kSingleArgBBytes of
-// the rows of B (when they fit), which then need no copy to the device.
-// The whole struct is the kernel's only argument, so it sits at offset 0
-// of the kernel-argument segment (the first explicit argument's place).
-constexpr int kSingleArgBBytes = 3840;
-struct SingleArgs {
-  LaunchArgs a;
-  int32_t arena_lines;  // 64-byte lines of the arena the block touches first
-  int32_t b_in_args;    // 1: rows of B in b[] (a.b_rows is set in the kernel)
-  int32_t base_in_args; // 1: per-unit start rows in b[] at base_off (a.unit_base is set in the kernel)
-  int32_t base_off;     // byte offset of those rows in b[]
-  uint64_t *done;       // host-visible slot receiving seq
-  uint64_t seq;
-  alignas(64) char b[kSingleArgBBytes];
 };
 
 }  // namespace pqp

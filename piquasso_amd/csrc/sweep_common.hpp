@@ -168,18 +168,11 @@ constexpr int waves_for(int hi, bool fp32) {
 
 // Row sums of lane state u (top state u, inner digits all 0) and the lane's
 // top weight prod_top C(rho_t, g_t).
-// Rows of B of item `it`: in the arena, or in the kernel arguments of a
-// one-block single-permanent launch (a.b_rows).
-template <typename R>
-__device__ __forceinline__ cptr<R> b_rows(const LaunchArgs &a, const cptr<ItemDesc> it) {
-  return a.b_rows ? as_const<R>(a.b_rows) : as_const<R>(a.arena, it->b_off);
-}
-
-template <int MCP, typename R, bool UNIT_BASE = false>
+template <int MCP, typename R>
 __device__ __forceinline__ void start_state(const LaunchArgs &a, const cptr<ItemDesc> it,
                                             int64_t u, int L, int Dt, int flags,
                                             R (&cr)[MCP], R (&ci)[MCP], double &w_top) {
-  const cptr<R> B = b_rows<R>(a, it);
+  const cptr<R> B = as_const<R>(a.arena, it->b_off);
   const cptr<double> alpha = as_const<double>(a.arena, it->alpha_off);
   // Row sums at the lane's first state,
   //   b_0 + sum_inner rho_k b_k + sum_top (rho_t - 2 g_t(u)) b_t,
@@ -196,27 +189,6 @@ __device__ __forceinline__ void start_state(const LaunchArgs &a, const cptr<Item
   // u < 2^50 (the fraction stays >= 1/(2P) away from an integer).  For
   // all-binary top digits this is the reflected binary code u ^ (u >> 1).
   const uint64_t gbin = static_cast<uint64_t>(u) ^ (static_cast<uint64_t>(u) >> 1);
-  if (UNIT_BASE && a.unit_base) {
-    // one-block launch, binary top digits: the unit's start row (host sum of
-    // the rows common to its 64 lanes) plus the lane-dependent digits
-    const cptr<R> base = as_const<R>(a.unit_base) + (u / kWave) * 2 * MCP;
-#pragma unroll
-    for (int j = 0; j < MCP; ++j) {
-      cr[j] = base[2 * j];
-      ci[j] = base[2 * j + 1];
-    }
-    w_top = 1.0;
-    for (int t = (Dt < kLaneDigits ? Dt : kLaneDigits) - 1; t >= 0; --t) {
-      const R al = ((gbin >> t) & 1) ? R(-1) : R(1);
-      const cptr<R> row = B + static_cast<int64_t>(L + 1 + t) * 2 * MCP;
-#pragma unroll
-      for (int j = 0; j < MCP; ++j) {
-        cr[j] = fmaR(al, row[2 * j], cr[j]);
-        ci[j] = fmaR(al, row[2 * j + 1], ci[j]);
-      }
-    }
-    return;
-  }
 #pragma unroll
   for (int j = 0; j < MCP; ++j) {
     cr[j] = R(0);
