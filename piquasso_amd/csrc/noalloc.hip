@@ -18,9 +18,9 @@
 // this library serialise on a mutex; callers that drive the same array from
 // several threads through other means would race.
 //
-// The kernels are those of pqp_permanent_c128 for the same plan (the
-// one-block launch for small permanents, else static launches of one block
-// per work unit and the finalize kernel), on the null stream, so the
+// The kernels are those of pqp_permanent_c128 (perm_one.hip up to 2^24 Gray
+// terms, else static launches of one block per work unit of the same plan
+// and the finalize kernel), on the null stream, so the
 // results are bit-identical to that entry point's.
 #include <hip/hip_runtime.h>
 #include <rocprofiler-sdk-roctx/roctx.h>
