@@ -540,7 +540,7 @@ def _sampling_leg(pa, W, cpu):
         "minors_seconds": st["minors_seconds"],
         "minors_tflops": st["minors_flops"] / st["minors_seconds"] / 1e12 if st["minors_seconds"] else None,
         "what": "boson sampling (Clifford & Clifford B), 40-mode Haar unitary, one photon in each of "
-                "modes 0..19, shots in lockstep: one pqp_laplace_batch_c128 call per photon round",
+                "modes 0..19, every photon round of all shots on the device (pqp_sample_shots_c128)",
     }
     cs = (cpu or {}).get("sampling")
     if cs and cs.get("shots"):
