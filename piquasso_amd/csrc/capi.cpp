@@ -885,7 +885,7 @@ int run_one(OnePlan &p, double *out2, double *out_dd4) {
   std::lock_guard<std::mutex> lock(S.mu);
   constexpr size_t kPartials = 256;  // after the counter
   if (!S.init_one) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.one_stream, hipStreamNonBlocking));
+    if (!S.one_stream) PQP_HIP(hipStreamCreateWithFlags(&S.one_stream, hipStreamNonBlocking));
     if ((st = S.one_res.ensure(8 * sizeof(double))) != PQP_OK) return st;
     if ((st = S.one_work.ensure(kPartials + static_cast<size_t>(kOneMaxBlocks) * 5 * sizeof(double))) != PQP_OK)
       return st;
