@@ -341,6 +341,15 @@ int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64
                           int32_t *out);
 
 /*
+ * Planning only (no device involved): the pass of pqp_sample_shots_c128 that
+ * holds shot `first` of a call, for inspection by tests.  info (2 + 2 photons
+ * entries): its shots, the bytes of partial minors the call holds, then for
+ * each step its minors' inner digits and waves per shot.  No counterpart in
+ * the reference.
+ */
+int pqp_sample_plan_info(int64_t shots, int64_t photons, int64_t first, int64_t *info);
+
+/*
  * Amplitudes <t_q| U |s> = perm(U; rows = t_q, cols = s) / sqrt(prod t_q! prod s!)
  * (2 doubles each) of many output occupations t_q for one input occupation s
  * (modes entries each; U modes x modes, row-major, interleaved complex), or

@@ -117,6 +117,7 @@ SIGNATURES = {
         _c.c_int,
         [_dp, _c.c_int64, _c.c_int64, _c.c_int64, _c.c_int64, _c.POINTER(_c.c_uint8), _i32p, _i32p, _dp, _i32p],
     ),
+    "pqp_sample_plan_info": (_c.c_int, [_c.c_int64, _c.c_int64, _c.c_int64, _i64p]),
     "pqp_output_table_c128": (
         _c.c_int,
         [_dp, _c.c_int64, _c.c_int64, _i32p, _c.c_int64, _i64p, _c.c_int, _dp],

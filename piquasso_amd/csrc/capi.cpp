@@ -1517,6 +1517,37 @@ int laplace_wave(const PermInput &in, double *out) {
   return PQP_OK;
 }
 
+// Sizes of the sampler's passes over a call's shots.  Every pass, the short
+// last one too, takes the same inner digits and waves per shot at a step, so
+// the partials, sized for the longest pass, hold any of them.
+struct SamplePasses {
+  int64_t most;                       // shots of a pass at most
+  int32_t digits[kMinorsWaveMaxCols + 1], waves[kMinorsWaveMaxCols + 1];  // of each step's minors
+  size_t partials;                    // bytes
+};
+
+SamplePasses sample_passes(int64_t shots, int64_t photons) {
+  SamplePasses p;
+  const int64_t passes = std::max<int64_t>(1, (shots + kSampleShots - 1) / kSampleShots);
+  p.most = (shots + passes - 1) / passes;
+  p.partials = 0;
+  p.digits[0] = p.waves[0] = 0;  // no minors before the first photon
+  // Most shots have bunched outputs and need fewer waves than 2^(step - 1)
+  // terms would; those left over end at once.  8 states a lane at least (the
+  // start and the sums cost as much as a handful of states), 64 where that
+  // leaves 8192 waves.
+  for (int64_t step = 1; step <= photons; ++step) {
+    int k = 3;
+    while (k < 6 && p.most * (int64_t{1} << (step - 1)) >= (int64_t{64} * 8192) << (k + 1)) ++k;
+    p.digits[step] = k;
+    p.waves[step] = static_cast<int32_t>(
+        std::min<int64_t>(64, std::max<int64_t>(1, (int64_t{1} << (step - 1)) >> (6 + k))));
+    if (step < photons)
+      p.partials = std::max(p.partials, static_cast<size_t>(p.most) * p.waves[step] * 4 * (step + 1) * sizeof(double));
+  }
+  return p;
+}
+
 // Buffers of the probability-table entry point, kept across calls (grown on
 // demand, bounded by kTableSegment rows), with their own stream and lock.
 struct TableState {
@@ -2494,20 +2525,8 @@ int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64
     PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
     S.init = true;
   }
-  const int64_t most = std::min(shots, kSampleShots);
-  // Inner digits and waves per shot of each step's minors.  Most shots have
-  // bunched outputs and need fewer waves than 2^(step - 1) terms would; those
-  // left over end at once.  8 states a lane at least (the start and the sums
-  // cost as much as a handful of states), 64 where that leaves 8192 waves.
-  auto digits = [](int64_t n, int64_t step) {
-    int k = 3;
-    while (k < 6 && n * (int64_t{1} << (step - 1)) >= (int64_t{64} * 8192) << (k + 1)) ++k;
-    return k;
-  };
-  auto waves = [&](int64_t n, int64_t step) {
-    return static_cast<int32_t>(
-        std::min<int64_t>(64, std::max<int64_t>(1, (int64_t{1} << (step - 1)) >> (6 + digits(n, step)))));
-  };
+  const SamplePasses passes = sample_passes(shots, photons);
+  const int64_t most = passes.most;
   // input: matrix, columns, photons, draws; work: the shots' columns,
   // outputs, wave counts, the failure flag, partials
   const size_t m2 = static_cast<size_t>(modes) * modes * 2 * sizeof(double);
@@ -2519,11 +2538,8 @@ int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64
   const size_t w_units = align256(w_occ + static_cast<size_t>(most * modes));
   const size_t w_failed = align256(w_units + static_cast<size_t>(most) * sizeof(int32_t));
   const size_t w_part = w_failed + 256;
-  size_t part = 0;
-  for (int64_t step = 1; step < photons; ++step)
-    part = std::max(part, static_cast<size_t>(most) * waves(most, step) * 4 * (step + 1) * sizeof(double));
   if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
-  if ((st = S.work.ensure(w_part + part)) != PQP_OK) return st;
+  if ((st = S.work.ensure(w_part + passes.partials)) != PQP_OK) return st;
   if ((st = S.stage.ensure(std::max(in_bytes, w_failed + 256 - w_occ))) != PQP_OK) return st;
   char *h = static_cast<char *>(S.stage.p);
   char *d = static_cast<char *>(S.in.p);
@@ -2578,8 +2594,8 @@ int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64
         m.item_stride = 2 * modes * photons;
         m.ld = static_cast<int32_t>(photons);
         m.modes = static_cast<int32_t>(modes);
-        m.waves = waves(n, step);
-        m.k_max = digits(n, step);
+        m.waves = passes.waves[step];
+        m.k_max = passes.digits[step];
         m.last_counter = nullptr;
         m.done = nullptr;
         m.seq = 0;
@@ -2587,8 +2603,8 @@ int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64
         a.waves = m.waves;
       }
       a.step = static_cast<int32_t>(step);
-      a.next_waves = waves(n, step + 1);
-      a.next_k_max = digits(n, step + 1);
+      a.next_waves = passes.waves[step + 1];
+      a.next_k_max = passes.digits[step + 1];
       PQP_HIP(launch_sample_step(a, S.stream));
     }
     PQP_HIP(hipMemcpyAsync(h, w + w_occ, w_failed + sizeof(int32_t) - w_occ, hipMemcpyDeviceToHost, S.stream));
@@ -2598,6 +2614,20 @@ int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64
     if (failed) return fail(PQP_ERR_INVALID, "probabilities contain NaN");
     const uint8_t *occ = reinterpret_cast<const uint8_t *>(h);
     for (int64_t t = 0; t < n * modes; ++t) out[s0 * modes + t] = occ[t];
+  }
+  return PQP_OK;
+}
+
+int pqp_sample_plan_info(int64_t shots, int64_t photons, int64_t first, int64_t *info) {
+  if (!info || photons < 0 || first < 0 || first >= shots) return fail(PQP_ERR_INVALID, "invalid sampling plan arguments");
+  if (photons > kMinorsWaveMaxCols)
+    return fail(PQP_ERR_RANGE, "sampling on the device supports at most " + std::to_string(kMinorsWaveMaxCols) + " photons");
+  const SamplePasses p = sample_passes(shots, photons);
+  info[0] = std::min(p.most, shots - first / p.most * p.most);
+  info[1] = static_cast<int64_t>(p.partials);
+  for (int64_t step = 0; step < photons; ++step) {
+    info[2 + 2 * step] = p.digits[step];
+    info[3 + 2 * step] = p.waves[step];
   }
   return PQP_OK;
 }
