@@ -895,19 +895,20 @@ int run_one(OnePlan &p, double *out2, double *out_dd4) {
   thread_local OneArgs a;
   one_fill(p, a);
   char *work = static_cast<char *>(S.one_work.p);
-  a.counter = reinterpret_cast<int *>(work);
-  a.partials = reinterpret_cast<double *>(work + kPartials);
-  a.out = static_cast<double *>(S.one_res.dev);
-  a.done = reinterpret_cast<uint64_t *>(a.out + 7);
-  a.seq = ++S.one_seq;
+  OneHead &h = a.rows.h;
+  h.counter = reinterpret_cast<int *>(work);
+  h.partials = reinterpret_cast<double *>(work + kPartials);
+  h.out = static_cast<double *>(S.one_res.dev);
+  h.done = reinterpret_cast<uint64_t *>(h.out + 7);
+  h.seq = ++S.one_seq;
   const double *res = static_cast<const double *>(S.one_res.host);
   volatile uint64_t *done = static_cast<uint64_t *>(S.one_res.host) + 7;
   *done = 0;
-  PQP_HIP(p.fp32 ? launch_one_f(p.width, p.ones, a, p.blocks, p.waves, S.one_stream)
-                 : launch_one_d(p.width, p.ones, a, p.blocks, p.waves, S.one_stream));
-  if ((st = wait_done(S.one_stream, done, a.seq)) != PQP_OK) {
+  PQP_HIP(p.fp32 ? launch_one_f(p.width, p.ones, p.few, a, p.blocks, p.waves, S.one_stream)
+                 : launch_one_d(p.width, p.ones, p.few, a, p.blocks, p.waves, S.one_stream));
+  if ((st = wait_done(S.one_stream, done, h.seq)) != PQP_OK) {
     // a launch that did not finish its count leaves it behind
-    (void)hipMemsetAsync(a.counter, 0, sizeof(int), S.one_stream);
+    (void)hipMemsetAsync(h.counter, 0, sizeof(int), S.one_stream);
     (void)hipStreamSynchronize(S.one_stream);
     return st;
   }
@@ -1907,12 +1908,15 @@ bool one_plan(const PermInput &given, uint32_t flags, OnePlan &p) {
     cmax = std::max(cmax, static_cast<int>(in.cols[j]));
   }
   if (sr != sc || sr < 1 || sr > kMaxCols) return false;
+  int rmax = 0;
+  for (int64_t i = 0; i < in.m_r; ++i) rmax = std::max(rmax, static_cast<int>(in.rows[i]));
   const double terms = gray_terms(in);
   if (terms > kOneMaxTerms) return false;
   p.in = in;
   p.n = static_cast<int>(sr);
   p.width = width;
   p.ones = expand || cmax <= 1;
+  p.few = p.ones && rmax <= 1 && sr <= kOneFew;
   p.fp32 = (flags & PQP_FLAG_FP32) != 0;
   p.terms = terms;
   p.blocks = 1;
@@ -1926,12 +1930,14 @@ bool one_plan(const PermInput &given, uint32_t flags, OnePlan &p) {
   return true;
 }
 
-void one_fill(OnePlan &p, OneArgs &a) {
+void one_fill(OnePlan &p, OneArgs &args) {
+  OneTables &t = args.tables;
+  OneHead &a = args.rows.h;
   const PermInput &in = p.in;
   int64_t cols[kOneMaxWidth];
   int width = 0;
   a.cmax = 1;
-  std::memset(a.over, 0, sizeof(a.over));
+  if (!p.few) std::memset(t.over, 0, sizeof(t.over));
   for (int64_t j = 0; j < in.m_c; ++j) {
     if (in.cols[j] == 0) continue;
     const int64_t at = in.transposed ? j * in.ld : j;
@@ -1939,7 +1945,7 @@ void one_fill(OnePlan &p, OneArgs &a) {
       for (int r = 0; r < in.cols[j]; ++r) cols[width++] = at;
       continue;
     }
-    for (int r = 2; r <= in.cols[j]; ++r) a.over[r - 2] |= 1u << width;
+    for (int r = 2; r <= in.cols[j]; ++r) t.over[r - 2] |= 1u << width;
     a.cmax = std::max(a.cmax, in.cols[j]);
     cols[width++] = at;
   }
@@ -2013,15 +2019,15 @@ void one_fill(OnePlan &p, OneArgs &a) {
     double coef = 1.0;
     std::fill(dir, dir + a.inner, 1);
     for (int v = 0; v < a.S; ++v) {
-      a.step[v] = OneStep{coef, 0, 0};
+      t.step[v] = OneStep{coef, 0, 0};
       if (v + 1 == a.S) break;
       int i = 0;
       for (; g[i] + dir[i] < 0 || g[i] + dir[i] > a.rho[i]; ++i) dir[i] = -dir[i];
       // C(rho, g +- 1) from C(rho, g), exact
       coef = dir[i] > 0 ? -coef * (a.rho[i] - g[i]) / (g[i] + 1) : -coef * g[i] / (a.rho[i] - g[i] + 1);
       g[i] += dir[i];
-      a.step[v].factor = dir[i] > 0 ? -2 : 2;
-      a.step[v].row = 1 + i;
+      t.step[v].factor = dir[i] > 0 ? -2 : 2;
+      t.step[v].row = 1 + i;
     }
   }
   const int64_t step = in.transposed ? 1 : in.ld;
@@ -2036,14 +2042,14 @@ void one_fill(OnePlan &p, OneArgs &a) {
   };
   if (in.a_is_float) {
     if (p.fp32)
-      fill(reinterpret_cast<float *>(a.b), static_cast<const float *>(in.a));
+      fill(reinterpret_cast<float *>(args.rows.b), static_cast<const float *>(in.a));
     else
-      fill(reinterpret_cast<double *>(a.b), static_cast<const float *>(in.a));
+      fill(reinterpret_cast<double *>(args.rows.b), static_cast<const float *>(in.a));
   } else {
     if (p.fp32)
-      fill(reinterpret_cast<float *>(a.b), static_cast<const double *>(in.a));
+      fill(reinterpret_cast<float *>(args.rows.b), static_cast<const double *>(in.a));
     else
-      fill(reinterpret_cast<double *>(a.b), static_cast<const double *>(in.a));
+      fill(reinterpret_cast<double *>(args.rows.b), static_cast<const double *>(in.a));
   }
 }
 

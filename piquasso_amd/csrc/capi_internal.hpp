@@ -44,6 +44,7 @@ struct OnePlan {
   PermInput in;       // transposed where that sweep is clearly cheaper
   int n, width;       // particles, distinct columns
   bool ones, fp32;
+  bool few;           // up to kOneFew particles, one in each row and column
   int blocks, waves;  // waves of a block
   double terms;       // Gray terms
 };

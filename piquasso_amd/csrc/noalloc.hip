@@ -101,15 +101,16 @@ int one_noalloc(OnePlan &p, double *out, double *out_dd) {
   one_fill(p, a);
   const int zero = 0;
   PQP_NA_HIP(hipMemcpy(base, &zero, sizeof(zero), hipMemcpyHostToDevice));
-  a.counter = reinterpret_cast<int *>(base);
-  a.out = reinterpret_cast<double *>(base + kResults);
-  a.partials = reinterpret_cast<double *>(base + kPartials);
-  a.done = reinterpret_cast<uint64_t *>(a.out + 7);
-  a.seq = 0;
-  PQP_NA_HIP(p.fp32 ? launch_one_f(p.width, p.ones, a, p.blocks, p.waves, nullptr)
-                    : launch_one_d(p.width, p.ones, a, p.blocks, p.waves, nullptr));
+  OneHead &h = a.rows.h;
+  h.counter = reinterpret_cast<int *>(base);
+  h.out = reinterpret_cast<double *>(base + kResults);
+  h.partials = reinterpret_cast<double *>(base + kPartials);
+  h.done = reinterpret_cast<uint64_t *>(h.out + 7);
+  h.seq = 0;
+  PQP_NA_HIP(p.fp32 ? launch_one_f(p.width, p.ones, p.few, a, p.blocks, p.waves, nullptr)
+                    : launch_one_d(p.width, p.ones, p.few, a, p.blocks, p.waves, nullptr));
   double res[7];
-  PQP_NA_HIP(hipMemcpy(res, a.out, sizeof(res), hipMemcpyDeviceToHost));
+  PQP_NA_HIP(hipMemcpy(res, h.out, sizeof(res), hipMemcpyDeviceToHost));
   out[0] = res[0];
   out[1] = res[1];
   if (out_dd) std::memcpy(out_dd, res + 2, 4 * sizeof(double));

@@ -34,6 +34,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
 
 #include "dd.hpp"
 #include "one_types.hpp"
@@ -119,8 +120,16 @@ __device__ __forceinline__ void block_sum(cdd &s, double &mag, double (&part)[kO
   mag = wave_sum<0, 3>(mag, lane);
 }
 
-template <int W, bool ONES>
-__global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(OneArgs args) {
+using OneRowsHost = decltype(OneArgs::rows);
+
+// The kernel's part of the arguments.
+template <int W, bool FEW>
+using Rows = OneRows<one_row_bytes(FEW ? kOneFew : kOneMaxRows, W, sizeof(Real))>;
+template <int W, bool FEW>
+using Args = std::conditional_t<FEW, Rows<W, FEW>, OneArgsOf<sizeof(Rows<W, FEW>::b)>>;
+
+template <int W, bool ONES, bool FEW>
+__global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW> given) {
   const int nw = static_cast<int>(blockDim.x) / kWave;
   __shared__ double part[kOneWaves][5];
   __shared__ Real base[kOneWaves][2 * W];
@@ -128,17 +137,26 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(OneArgs arg
   const int bw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int waves = nw * static_cast<int>(gridDim.x);
   const int wave = nw * static_cast<int>(blockIdx.x) + bw;
-  const uintptr_t self = reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
-  const cptr<Real> rows = reinterpret_cast<cptr<Real>>(self + offsetof(OneArgs, b));
-  const Real *vrows = reinterpret_cast<const Real *>(self + offsetof(OneArgs, b));
-  const cptr<uint32_t> over = reinterpret_cast<cptr<uint32_t>>(self + offsetof(OneArgs, over));
-  const cptr<int32_t> lane_rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneArgs, lane_rho));
-  const cptr<int32_t> rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneArgs, rho));
-  const cptr<OneStep> step = reinterpret_cast<cptr<OneStep>>(self + offsetof(OneArgs, step));
+  const uintptr_t all = reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  uintptr_t self = all;  // the rows and their head
+  const OneHead *head;
+  if constexpr (FEW) {
+    head = &given.h;
+  } else {
+    head = &given.rows.h;
+    self += offsetof(OneArgs, rows);
+  }
+  const OneHead &args = *head;
+  const cptr<Real> rows = reinterpret_cast<cptr<Real>>(self + offsetof(OneRowsHost, b));
+  const Real *vrows = reinterpret_cast<const Real *>(self + offsetof(OneRowsHost, b));
+  const cptr<uint32_t> over = reinterpret_cast<cptr<uint32_t>>(all + offsetof(OneTables, over));
+  const cptr<int32_t> lane_rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneHead, lane_rho));
+  const cptr<int32_t> rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneHead, rho));
+  const cptr<OneStep> step = reinterpret_cast<cptr<OneStep>>(all + offsetof(OneTables, step));
   const int n = args.n, k = args.inner, rest = args.rest, cmax = args.cmax;
   const int L = args.lane_digits, S = args.S, chunks = args.chunks;
   const bool active = lane < args.lanes;
-  const bool binary = args.binary;
+  const bool binary = FEW || args.binary;
   // The first rows common to a wave's lanes, a component per lane: requested
   // before the wave waits for anything else (a first touch costs about a
   // microsecond, and one after another these were most of the start).
@@ -149,7 +167,7 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(OneArgs arg
   for (int i = 0; i < kOneChunk; ++i) first[i] = vrows[(L + min(i, common - 1)) * (2 * W) + at];
   {
     // every line of the rows read as scalars, eight loads of a wave in flight
-    const cptr<uint32_t> lines = reinterpret_cast<cptr<uint32_t>>(self + offsetof(OneArgs, b));
+    const cptr<uint32_t> lines = reinterpret_cast<cptr<uint32_t>>(self + offsetof(OneRowsHost, b));
     const int end = ((L + 1 + k) * 2 * W * static_cast<int>(sizeof(Real)) - 1) / 64;
     for (int l = bw; l <= end; l += 8 * nw) {
       const uint32_t v0 = lines[16 * l], v1 = lines[16 * min(l + nw, end)];
@@ -312,21 +330,40 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(OneArgs arg
 
 }  // namespace
 
+// The kernel copies its own length of the arguments: they begin alike for
+// every width.
+template <int W, bool ONES, bool FEW>
+static hipError_t one_launch(const OneArgs &a, dim3 grid, dim3 block, hipStream_t stream) {
+  using R = Rows<W, FEW>;
+  static_assert(offsetof(R, b) == offsetof(OneRowsHost, b) && sizeof(Args<W, FEW>) <= sizeof(OneArgs));
+  void *p[] = {const_cast<void *>(FEW ? static_cast<const void *>(&a.rows) : static_cast<const void *>(&a))};
+  return hipLaunchKernel(reinterpret_cast<const void *>(perm_one_kernel<W, ONES, FEW>), grid, block, p, 0, stream);
+}
+
 #if PQP_ONE_FP32
-hipError_t launch_one_f(int width, bool ones, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
+hipError_t launch_one_f(int width, bool ones, bool few, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
 #else
-hipError_t launch_one_d(int width, bool ones, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
+hipError_t launch_one_d(int width, bool ones, bool few, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
 #endif
-  if (blocks < 1 || waves < 1 || waves > kOneWaves || a.n < 1 || a.chunks < 1)
-    return hipErrorInvalidValue;
+  const OneHead &h = a.rows.h;
+  if (blocks < 1 || waves < 1 || waves > kOneWaves || h.n < 1 || h.chunks < 1) return hipErrorInvalidValue;
+  if (few && (!ones || !h.binary || 1 + h.lane_digits + h.inner + h.rest > kOneFew)) return hipErrorInvalidValue;
+  const dim3 grid(blocks), block(kWave * waves);
+  if (few) {
+    switch (width) {
+#define X(W) \
+  case W:    \
+    return one_launch<W, true, true>(a, grid, block, stream);
+      X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
+#undef X
+      default:
+        return hipErrorInvalidValue;
+    }
+  }
   switch (width) {
-#define X(W)                                                                                              \
-  case W:                                                                                                 \
-    if (ones)                                                                                             \
-      hipLaunchKernelGGL((perm_one_kernel<W, true>), dim3(blocks), dim3(kWave * waves), 0, stream, a);    \
-    else                                                                                                  \
-      hipLaunchKernelGGL((perm_one_kernel<W, false>), dim3(blocks), dim3(kWave * waves), 0, stream, a);   \
-    return hipGetLastError();
+#define X(W) \
+  case W:    \
+    return ones ? one_launch<W, true, false>(a, grid, block, stream) : one_launch<W, false, false>(a, grid, block, stream);
     X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
     X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20) X(21) X(22) X(23) X(24)
 #undef X
