@@ -889,7 +889,7 @@ int run_one(OnePlan &p, double *out2, double *out_dd4) {
     if ((st = S.one_res.ensure(8 * sizeof(double))) != PQP_OK) return st;
     if ((st = S.one_work.ensure(kPartials + static_cast<size_t>(kOneMaxBlocks) * 5 * sizeof(double))) != PQP_OK)
       return st;
-    PQP_HIP(hipMemset(S.one_work.p, 0, kPartials));
+    PQP_HIP(hipMemsetAsync(S.one_work.p, 0, kPartials, S.one_stream));
     S.init_one = true;
   }
   thread_local OneArgs a;
