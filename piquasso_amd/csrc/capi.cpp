@@ -257,6 +257,12 @@ struct MappedBuf {
   }
 };
 
+// A stream that is created once, also when what follows its creation fails.
+int ensure_stream(hipStream_t &stream) {
+  if (!stream) PQP_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+  return PQP_OK;
+}
+
 // Device image of one plan plus the stream it runs on.
 struct Exec {
   Plan plan;
@@ -270,7 +276,6 @@ struct Exec {
   bool heads_clean = false;  // queue heads zeroed since (re)allocation
   bool abs_valid = false;    // the last evaluation left term magnitudes
   hipStream_t stream = nullptr;
-  bool own_stream = false;
   uint32_t flags = 0;
   // side streams and events for running several width buckets concurrently
   hipStream_t side[kMaxRanges] = {};
@@ -337,9 +342,10 @@ int upload(Exec &x) {
 // Side streams (default priority) and fork/join events, created once per Exec.
 int ensure_side_streams(Exec &x) {
   if (x.ev_fork) return PQP_OK;
+  int st;
   for (int i = 1; i < kMaxRanges; ++i) {
-    PQP_HIP(hipStreamCreateWithFlags(&x.side[i], hipStreamNonBlocking));
-    PQP_HIP(hipEventCreateWithFlags(&x.ev_join[i], hipEventDisableTiming));
+    if ((st = ensure_stream(x.side[i])) != PQP_OK) return st;
+    if (!x.ev_join[i]) PQP_HIP(hipEventCreateWithFlags(&x.ev_join[i], hipEventDisableTiming));
   }
   PQP_HIP(hipEventCreateWithFlags(&x.ev_fork, hipEventDisableTiming));
   return PQP_OK;
@@ -475,9 +481,7 @@ namespace {
 struct SingleState {
   std::mutex mu;
   Exec x;       // column minors, gradients, tensor permanents
-  bool init = false;
   Exec xs;      // single permanents: results in mapped host memory
-  bool init_s = false;
   // the plan resident in xs and its key (shape, multiplicities, flags)
   std::vector<int64_t> xs_key;
   bool xs_planned = false;
@@ -717,7 +721,6 @@ int wait_done(hipStream_t stream, volatile uint64_t *done, uint64_t seq) {
 // waves' residues, `res` the permanent's and the done slot.
 struct IntState {
   std::mutex mu;
-  bool init = false;
   hipStream_t stream = nullptr;
   DevBuf in, work;
   HostBuf stage;
@@ -801,10 +804,7 @@ int run_int(const PermInput &in, const IntScan &sc, uint64_t *v) {
   if ((st = require_device()) != PQP_OK) return st;
   IntState &S = int_state();
   std::lock_guard<std::mutex> lock(S.mu);
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
-    S.init = true;
-  }
+  if ((st = ensure_stream(S.stream)) != PQP_OK) return st;
   // the moduli table: p, 1/p, 2^-(n-1) mod p; then the rows with each column
   // repeated by its multiplicity, and their multiplicities
   const int W = n <= 32 ? (n + 3) / 4 * 4 : (n + 7) / 8 * 8;
@@ -885,7 +885,7 @@ int run_one(OnePlan &p, double *out2, double *out_dd4) {
   std::lock_guard<std::mutex> lock(S.mu);
   constexpr size_t kPartials = 256;  // after the counter
   if (!S.init_one) {
-    if (!S.one_stream) PQP_HIP(hipStreamCreateWithFlags(&S.one_stream, hipStreamNonBlocking));
+    if ((st = ensure_stream(S.one_stream)) != PQP_OK) return st;
     if ((st = S.one_res.ensure(8 * sizeof(double))) != PQP_OK) return st;
     if ((st = S.one_work.ensure(kPartials + static_cast<size_t>(kOneMaxBlocks) * 5 * sizeof(double))) != PQP_OK)
       return st;
@@ -972,12 +972,8 @@ int run_single(const PermInput &in, uint32_t flags, double *out2, double *out_dd
     st = plan_build(std::vector<PermInput>{in}, single_plan_options(flags, in), plan, err);
     if (st != PQP_OK) return fail(st, err);
     if ((st = require_device()) != PQP_OK) return st;
-    if (!S.init_s) {
-      PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-      x.own_stream = true;
-      x.mapped_results = true;
-      S.init_s = true;
-    }
+    if ((st = ensure_stream(x.stream)) != PQP_OK) return st;
+    x.mapped_results = true;
     x.plan = std::move(plan);
     index_units(x);
     x.flags = (flags & PQP_FLAG_PLAIN) | PQP_FLAG_STATIC;
@@ -1241,7 +1237,6 @@ namespace {
 // results.
 struct TensorState {
   std::mutex mu;
-  bool init = false;
   hipStream_t stream = nullptr;
   DevBuf in, work, out;
   HostBuf stage;
@@ -1337,7 +1332,6 @@ namespace {
 // calls (grown on demand), with their own stream and lock.
 struct PolyState {
   std::mutex mu;
-  bool init = false;
   hipStream_t stream = nullptr;
   DevBuf arena, scratch, acc, out;
   HostBuf stage;
@@ -1444,7 +1438,7 @@ int laplace_wave(const PermInput &in, double *out) {
   MinorsState &S = laplace_state();
   std::lock_guard<std::mutex> lock(S.mu);
   if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
+    if ((st = ensure_stream(S.stream)) != PQP_OK) return st;
     if ((st = S.counter.ensure(sizeof(int))) != PQP_OK) return st;
     PQP_HIP(hipMemsetAsync(S.counter.p, 0, sizeof(int), S.stream));
     S.init = true;
@@ -1553,7 +1547,6 @@ SamplePasses sample_passes(int64_t shots, int64_t photons) {
 // demand, bounded by kTableSegment rows), with their own stream and lock.
 struct TableState {
   std::mutex mu;
-  bool init = false;
   hipStream_t stream = nullptr;
   DevBuf in, out;
   HostBuf stage;
@@ -1661,10 +1654,7 @@ int poly_run(PolyState &S, const double *b0, const double *bm, int64_t n_out, do
   const size_t o_bm = off;
   off = align256(off + mat * static_cast<size_t>(M));
   const size_t arena_bytes = off;
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
-    S.init = true;
-  }
+  if ((st = ensure_stream(S.stream)) != PQP_OK) return st;
   const void *arena_before = S.arena.p;
   if ((st = S.arena.ensure(arena_bytes)) != PQP_OK) return st;
   if (S.arena.p != arena_before) S.tables_on_device = false;
@@ -1780,11 +1770,7 @@ int run_minors(const std::vector<PermInput> &probs, const PlanOptions &opt, doub
   SingleState &S = single_state();
   std::lock_guard<std::mutex> lock(S.mu);
   Exec &x = S.x;
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-    x.own_stream = true;
-    S.init = true;
-  }
+  if ((st = ensure_stream(x.stream)) != PQP_OK) return st;
   x.plan = std::move(mp.plan);
   index_units(x);
   x.flags = PQP_FLAG_STATIC;
@@ -1821,11 +1807,7 @@ int grad_batch_minors(const std::vector<PermInput> &inputs, double *perms, doubl
   SingleState &S = single_state();
   std::lock_guard<std::mutex> lock(S.mu);
   Exec &x = S.x;
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-    x.own_stream = true;
-    S.init = true;
-  }
+  if ((st = ensure_stream(x.stream)) != PQP_OK) return st;
   std::vector<double> res;
   if (perms && !inputs.empty()) {
     x.plan = std::move(fwd);
@@ -2216,10 +2198,7 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
   if ((st = require_device()) != PQP_OK) return st;
   TensorState &S = tensor_state();
   std::lock_guard<std::mutex> lock(S.mu);
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
-    S.init = true;
-  }
+  if ((st = ensure_stream(S.stream)) != PQP_OK) return st;
   for (int64_t k = 0; k < count; ++k)
     if (n[k] == 0) {  // the empty product (probabilities.py:197-198)
       out[k] = 1.0;
@@ -2339,10 +2318,7 @@ int pqp_overlap_table_c128(const double *matrix, int64_t modes, int64_t ld, cons
   }
   TensorState &S = tensor_state();
   std::lock_guard<std::mutex> lock(S.mu);
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
-    S.init = true;
-  }
+  if ((st = ensure_stream(S.stream)) != PQP_OK) return st;
   TensorArgs a;
   std::memset(&a, 0, sizeof(a));
   a.n = n;
@@ -2442,17 +2418,14 @@ int pqp_output_table_c128(const double *matrix, int64_t modes, int64_t ld, const
   }
   TableState &S = table_state();
   std::lock_guard<std::mutex> lock(S.mu);
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
-    S.init = true;
-  }
+  int st;
+  if ((st = ensure_stream(S.stream)) != PQP_OK) return st;
   // input buffer: the occupied columns, their occupations, the outputs
   const size_t o_mult = static_cast<size_t>(modes) * width * 2 * sizeof(double);
   const size_t o_outs = align256(o_mult + static_cast<size_t>(width) * sizeof(int32_t));
   const int64_t most = std::min(count, kTableSegment);
   const size_t in_bytes = o_outs + static_cast<size_t>(most) * static_cast<size_t>(modes);
   const size_t out_bytes = static_cast<size_t>(most) * per * sizeof(double);
-  int st;
   if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
   if ((st = S.out.ensure(out_bytes)) != PQP_OK) return st;
   if ((st = S.stage.ensure(align256(in_bytes) + out_bytes)) != PQP_OK) return st;
@@ -2527,10 +2500,7 @@ int pqp_sample_shots_c128(const double *matrix, int64_t modes, int64_t ld, int64
   if ((st = require_device()) != PQP_OK) return st;
   MinorsState &S = sample_state();
   std::lock_guard<std::mutex> lock(S.mu);
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
-    S.init = true;
-  }
+  if ((st = ensure_stream(S.stream)) != PQP_OK) return st;
   const SamplePasses passes = sample_passes(shots, photons);
   const int64_t most = passes.most;
   // input: matrix, columns, photons, draws; work: the shots' columns,
@@ -2722,11 +2692,7 @@ int pqp_grad_batch_c128(int64_t count, const double *const *matrices, const int6
   SingleState &S = single_state();
   std::lock_guard<std::mutex> lock(S.mu);
   Exec &x = S.x;
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-    x.own_stream = true;
-    S.init = true;
-  }
+  if ((st = ensure_stream(x.stream)) != PQP_OK) return st;
   x.plan = std::move(plan);
   index_units(x);
   x.flags = PQP_FLAG_STATIC;
@@ -2797,14 +2763,12 @@ int pqp_batch_create(int64_t count, const void *const *matrices, int is_c64, con
   if ((st = require_device()) != PQP_OK) return st;
   index_units(b->x);
   b->x.flags = flags;
-  PQP_HIP(hipStreamCreateWithFlags(&b->x.stream, hipStreamNonBlocking));
-  b->x.own_stream = true;
+  if ((st = ensure_stream(b->x.stream)) != PQP_OK) return st;
   if ((st = upload(b->x)) != PQP_OK) return st;
   if (b->grad_minors) {
     index_units(b->xm);
     b->xm.flags = PQP_FLAG_STATIC;
     b->xm.stream = b->x.stream;  // shares the batch stream (and its graph)
-    b->xm.own_stream = false;
     if ((st = upload(b->xm)) != PQP_OK) return st;
   }
   PQP_HIP(hipStreamSynchronize(b->x.stream));
@@ -2840,11 +2804,7 @@ int pqp_permanent_batch_c128(int64_t count, const double *const *matrices, const
   SingleState &S = single_state();
   std::lock_guard<std::mutex> lock(S.mu);
   Exec &x = S.x;
-  if (!S.init) {
-    PQP_HIP(hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking));
-    x.own_stream = true;
-    S.init = true;
-  }
+  if ((st = ensure_stream(x.stream)) != PQP_OK) return st;
   x.plan = std::move(plan);
   index_units(x);
   x.flags = flags;
@@ -3107,7 +3067,7 @@ void pqp_batch_destroy(pqp_batch *b) {
     if (b->x.ev_join[i]) (void)hipEventDestroy(b->x.ev_join[i]);
   }
   if (b->x.ev_fork) (void)hipEventDestroy(b->x.ev_fork);
-  if (b->x.own_stream && b->x.stream) (void)hipStreamDestroy(b->x.stream);
+  if (b->x.stream) (void)hipStreamDestroy(b->x.stream);
   delete b;
 }
 
