@@ -22,9 +22,10 @@
  * multiplicities, one buffer request per array (about 0.5 us an item; numpy
  * and ctypes take 4 us).  Returns bytes objects (matrix pointers, row
  * pointers, column pointers, m_r, m_c as int64, the buffer the
- * multiplicities and widened matrices live in) and the mean Gray term count
- * of the items `sample` lists (int64 buffer; 0.0 when it is None).  Matrix
- * pointers refer to the caller's arrays, which must outlive their use.  None
+ * multiplicities and widened matrices live in), the mean Gray term count
+ * of the items `sample` lists (int64 buffer; 0.0 when it is None), and a
+ * capsule that holds the buffers of the matrices that the pointers refer to:
+ * they stay valid while it lives, whatever becomes of the list.  None
  * when an item has any other form: the caller's general path takes the
  * batch, and reports what is wrong with it.
  */
@@ -119,6 +120,21 @@ done:
   return result;
 }
 
+/* The buffers of a batch's matrices, released with the capsule around it. */
+typedef struct {
+  Py_ssize_t n;
+  Py_buffer view[];
+} Views;
+
+static void release_views(Views *v) {
+  for (Py_ssize_t k = 0; k < v->n; ++k) PyBuffer_Release(&v->view[k]);
+  free(v);
+}
+
+static void free_views(PyObject *capsule) {
+  release_views((Views *)PyCapsule_GetPointer(capsule, NULL));
+}
+
 typedef struct {
   const void *a, *r, *c;
   int64_t m_r, m_c;
@@ -175,25 +191,30 @@ static PyObject *pack(PyObject *self, PyObject *args) {
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(om);
   if (n < 1 || PySequence_Fast_GET_SIZE(orr) != n || PySequence_Fast_GET_SIZE(oc) != n) Py_RETURN_NONE;
   Item *items = (Item *)malloc((size_t)n * sizeof(Item));
-  if (!items) return PyErr_NoMemory();
+  Views *views = (Views *)malloc(sizeof(Views) + (size_t)n * sizeof(Py_buffer));
+  if (!items || !views) {
+    free(items);
+    free(views);
+    return PyErr_NoMemory();
+  }
+  views->n = 0;
   size_t widened = 0, mults = 0;
-  PyObject *res = NULL, *part[6] = {NULL, NULL, NULL, NULL, NULL, NULL};
+  PyObject *res = NULL, *part[7] = {NULL, NULL, NULL, NULL, NULL, NULL, NULL};
   for (Py_ssize_t k = 0; k < n; ++k) {
     Item *it = items + k;
-    Py_buffer b;
-    if (PyObject_GetBuffer(PySequence_Fast_GET_ITEM(om, k), &b, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) < 0) {
+    Py_buffer *b = &views->view[views->n];
+    if (PyObject_GetBuffer(PySequence_Fast_GET_ITEM(om, k), b, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) < 0) {
       PyErr_Clear();
       goto none;
     }
-    const char *f = b.format ? b.format : "B";
+    ++views->n;
+    const char *f = b->format ? b->format : "B";
     if (*f == '<' || *f == '=' || *f == '@') ++f;
-    it->wide = b.itemsize == 8 && strcmp(f, "Zf") == 0;
-    const int ok = b.ndim == 2 && (it->wide || (b.itemsize == 16 && strcmp(f, "Zd") == 0));
-    it->a = b.buf;
-    it->m_r = ok ? b.shape[0] : 0;
-    it->m_c = ok ? b.shape[1] : 0;
-    PyBuffer_Release(&b);
-    if (!ok) goto none;
+    it->wide = b->itemsize == 8 && strcmp(f, "Zf") == 0;
+    if (b->ndim != 2 || !(it->wide || (b->itemsize == 16 && strcmp(f, "Zd") == 0))) goto none;
+    it->a = b->buf;
+    it->m_r = b->shape[0];
+    it->m_c = b->shape[1];
     it->r = mult_buffer(PySequence_Fast_GET_ITEM(orr, k), it->m_r, &it->wr);
     it->c = it->r ? mult_buffer(PySequence_Fast_GET_ITEM(oc, k), it->m_c, &it->wc) : NULL;
     if (!it->c) goto none;
@@ -201,8 +222,8 @@ static PyObject *pack(PyObject *self, PyObject *args) {
     mults += (size_t)(it->m_r + it->m_c) * sizeof(int32_t);
   }
   for (int q = 0; q < 5; ++q)
-    if (!(part[q] = PyBytes_FromStringAndSize(NULL, n * 8))) goto fail;
-  if (!(part[5] = PyBytes_FromStringAndSize(NULL, (Py_ssize_t)(widened + mults + 16)))) goto fail;
+    if (!(part[q] = PyBytes_FromStringAndSize(NULL, n * 8))) goto out;
+  if (!(part[5] = PyBytes_FromStringAndSize(NULL, (Py_ssize_t)(widened + mults + 16)))) goto out;
   {
     int64_t *arr[5];
     for (int q = 0; q < 5; ++q) arr[q] = (int64_t *)PyBytes_AS_STRING(part[q]);
@@ -231,7 +252,7 @@ static PyObject *pack(PyObject *self, PyObject *args) {
     double terms = 0.0;
     if (os != Py_None) {
       Py_buffer b;
-      if (PyObject_GetBuffer(os, &b, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) < 0) goto fail;
+      if (PyObject_GetBuffer(os, &b, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) < 0) goto out;
       const int64_t *at = (const int64_t *)b.buf;
       const Py_ssize_t m = b.ndim == 1 && int_format(&b) == 8 ? b.shape[0] : 0;
       for (Py_ssize_t i = 0; i < m; ++i)
@@ -240,16 +261,19 @@ static PyObject *pack(PyObject *self, PyObject *args) {
       if (m > 0) terms /= (double)m;
       PyBuffer_Release(&b);
     }
-    res = Py_BuildValue("(OOOOOOd)", part[0], part[1], part[2], part[3], part[4], part[5], terms);
+    if (!(part[6] = PyCapsule_New(views, NULL, free_views))) goto out;
+    views = NULL;
+    res = Py_BuildValue("(OOOOOOdO)", part[0], part[1], part[2], part[3], part[4], part[5], terms, part[6]);
   }
-fail:
-  for (int q = 0; q < 6; ++q) Py_XDECREF(part[q]);
+  goto out;
+none:
+  Py_INCREF(Py_None);
+  res = Py_None;
+out:
+  for (int q = 0; q < 7; ++q) Py_XDECREF(part[q]);
+  if (views) release_views(views);
   free(items);
   return res;
-none:
-  for (int q = 0; q < 6; ++q) Py_XDECREF(part[q]);
-  free(items);
-  Py_RETURN_NONE;
 }
 
 static PyMethodDef methods[] = {

@@ -117,9 +117,9 @@ def _packed(matrices, rows, cols, terms: bool):
     got = fast.pack(matrices, rows, cols, sample)
     if got is None:
         return None
-    mats, rp, cp, m_r, m_c, buf, mean = got
+    mats, rp, cp, m_r, m_c, _, mean, _ = got
     return ((mats, rp, cp), np.frombuffer(m_r, dtype=np.int64), np.frombuffer(m_c, dtype=np.int64),
-            (got, matrices), float(np.log2(mean)) if terms else None)
+            got, float(np.log2(mean)) if terms else None)
 
 
 def _tuned_launch(count, rows, persistent, target_inner, total_units, log2_terms=None):
