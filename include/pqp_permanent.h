@@ -315,8 +315,9 @@ int pqp_overlap_table_c128(const double *matrix, int64_t modes, int64_t ld, cons
 
 /*
  * Permanents of `count` problems evaluated once: pqp_batch_create, an eager
- * run and pqp_batch_results in one call, on buffers and streams the library
- * keeps between calls (released after a call that grew them beyond 256 MiB).
+ * run and pqp_batch_results in one call.  Calls of several threads run side
+ * by side, each on buffers and streams of its own, which the library keeps
+ * for later calls (of at most four, 256 MiB of device memory in all).
  * Arguments as in pqp_batch_create, complex128; flags PQP_FLAG_FP32,
  * _STATIC, _EXPAND_COLS, _KEEP_COLS, _AS_GIVEN; out: 2 doubles per problem.
  */

@@ -135,8 +135,10 @@ constexpr int64_t kSampleShots = 2048;
 // digits at most.
 constexpr int64_t kIntWaves = 4096;
 constexpr int kIntInnerDigits = 7;
-// Device buffers a one-shot batch may leave for the next one.
+// Device buffers one-shot batches may leave for the next ones, and how many
+// calls' worth: as many threads find theirs ready.
 constexpr size_t kKeptBytes = size_t{256} << 20;
+constexpr size_t kKeptExecs = 4;
 
 // Permanents without tables: one block up to kOneBlockTerms Gray terms (the
 // blocks' meeting costs about 3 us: 13 particles 17.0 us a call in one block
@@ -351,6 +353,22 @@ int ensure_side_streams(Exec &x) {
   return PQP_OK;
 }
 
+// Everything an Exec holds, its stream too where it is the Exec's own.
+void release_exec(Exec &x, bool stream) {
+  x.arena.release();
+  x.partials.release();
+  x.results.release();
+  x.results_m.release();
+  x.stage.release();
+  x.heads.release();
+  for (int i = 1; i < kMaxRanges; ++i) {
+    if (x.side[i]) (void)hipStreamDestroy(x.side[i]);
+    if (x.ev_join[i]) (void)hipEventDestroy(x.ev_join[i]);
+  }
+  if (x.ev_fork) (void)hipEventDestroy(x.ev_fork);
+  if (stream && x.stream) (void)hipStreamDestroy(x.stream);
+}
+
 // Enqueue one evaluation.  ev_begin / ev_end (optional) bracket the sweep
 // kernels only when kernel_only is set, the whole evaluation otherwise.
 int enqueue(Exec &x, int mode, hipEvent_t ev_begin, hipEvent_t ev_end) {
@@ -497,6 +515,53 @@ SingleState &single_state() {
   static SingleState *s = new SingleState();  // never destroyed: outlives atexit HIP teardown
   return *s;
 }
+
+// One-shot batches: each call has an Exec (buffers and streams) to itself, so
+// calls of several threads run side by side.  What a call leaves is kept for
+// the next one, up to kKeptExecs of them and kKeptBytes in all.
+struct OneShotPool {
+  std::mutex mu;
+  std::vector<std::unique_ptr<Exec>> idle;
+};
+
+OneShotPool &one_shot_pool() {
+  static OneShotPool *p = new OneShotPool();  // never destroyed: outlives atexit HIP teardown
+  return *p;
+}
+
+struct OneShotLease {
+  std::unique_ptr<Exec> x;
+  bool finished = false;  // the call's work on the stream is done
+
+  OneShotLease() {
+    OneShotPool &pool = one_shot_pool();
+    std::lock_guard<std::mutex> lock(pool.mu);
+    if (pool.idle.empty()) {
+      x.reset(new Exec());
+    } else {
+      x = std::move(pool.idle.back());
+      pool.idle.pop_back();
+    }
+  }
+  ~OneShotLease() {
+    auto bytes = [](const Exec &e) { return e.arena.bytes + e.partials.bytes + e.results.bytes; };
+    x->plan = Plan();
+    if (finished) {
+      OneShotPool &pool = one_shot_pool();
+      std::lock_guard<std::mutex> lock(pool.mu);
+      size_t held = bytes(*x);
+      for (const auto &e : pool.idle) held += bytes(*e);
+      if (pool.idle.size() < kKeptExecs && held <= kKeptBytes) {
+        pool.idle.push_back(std::move(x));
+        return;
+      }
+    }
+    if (x->stream) (void)hipStreamSynchronize(x->stream);
+    release_exec(*x, true);
+  }
+  OneShotLease(const OneShotLease &) = delete;
+  OneShotLease &operator=(const OneShotLease &) = delete;
+};
 
 // ---------------------------------------------------- exact integers --
 
@@ -2801,9 +2866,8 @@ int pqp_permanent_batch_c128(int64_t count, const double *const *matrices, const
   if (st != PQP_OK) return fail(st, err);
   if ((st = require_device()) != PQP_OK) return st;
   if (count == 0) return PQP_OK;
-  SingleState &S = single_state();
-  std::lock_guard<std::mutex> lock(S.mu);
-  Exec &x = S.x;
+  OneShotLease lease;
+  Exec &x = *lease.x;
   if ((st = ensure_stream(x.stream)) != PQP_OK) return st;
   x.plan = std::move(plan);
   index_units(x);
@@ -2817,13 +2881,7 @@ int pqp_permanent_batch_c128(int64_t count, const double *const *matrices, const
   PQP_HIP(hipMemcpyAsync(x.stage.p, x.results.p, out_bytes, hipMemcpyDeviceToHost, x.stream));
   PQP_HIP(hipStreamSynchronize(x.stream));
   std::memcpy(out, x.stage.p, out_bytes);
-  if (x.arena.bytes + x.partials.bytes > kKeptBytes) {
-    x.plan = Plan();
-    x.arena.release();
-    x.partials.release();
-    x.results.release();
-    x.stage.release();
-  }
+  lease.finished = true;
   return PQP_OK;
 }
 
@@ -3045,29 +3103,8 @@ void pqp_batch_destroy(pqp_batch *b) {
   if (b->x.stream) (void)hipStreamSynchronize(b->x.stream);
   if (b->graph_exec) (void)hipGraphExecDestroy(b->graph_exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  b->xm.arena.release();
-  b->xm.partials.release();
-  b->xm.results.release();
-  b->xm.results_m.release();
-  b->xm.stage.release();
-  b->xm.heads.release();
-  for (int i = 1; i < kMaxRanges; ++i) {
-    if (b->xm.side[i]) (void)hipStreamDestroy(b->xm.side[i]);
-    if (b->xm.ev_join[i]) (void)hipEventDestroy(b->xm.ev_join[i]);
-  }
-  if (b->xm.ev_fork) (void)hipEventDestroy(b->xm.ev_fork);
-  b->x.arena.release();
-  b->x.partials.release();
-  b->x.results.release();
-  b->x.results_m.release();
-  b->x.stage.release();
-  b->x.heads.release();
-  for (int i = 1; i < kMaxRanges; ++i) {
-    if (b->x.side[i]) (void)hipStreamDestroy(b->x.side[i]);
-    if (b->x.ev_join[i]) (void)hipEventDestroy(b->x.ev_join[i]);
-  }
-  if (b->x.ev_fork) (void)hipEventDestroy(b->x.ev_fork);
-  if (b->x.stream) (void)hipStreamDestroy(b->x.stream);
+  release_exec(b->xm, false);  // shares b->x's stream
+  release_exec(b->x, true);
   delete b;
 }
 
