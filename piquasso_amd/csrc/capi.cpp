@@ -135,6 +135,9 @@ constexpr int64_t kSampleShots = 2048;
 // digits at most.
 constexpr int64_t kIntWaves = 4096;
 constexpr int kIntInnerDigits = 7;
+// Bytes of a polynomial permanent's exponent rows that are compared with the
+// kept plan's before anything runs (8 us).
+constexpr size_t kPolyCompareFirst = size_t{256} << 10;
 // Device buffers one-shot batches may leave for the next ones, and how many
 // calls' worth: as many threads find theirs ready.
 constexpr size_t kKeptBytes = size_t{256} << 20;
@@ -2700,22 +2703,26 @@ int pqp_perm_poly_coefficients_c128(int64_t n, int64_t n_vars, const double *b0,
   std::lock_guard<std::mutex> lock(S.mu);
   // The plan depends only on (n, the exponent rows): a call with the same
   // rows as the previous one reuses it and the tables already on the device.
-  // The rows can be larger than everything else the call reads (7.4 MB for
-  // 184756 outputs of 10 modes: 0.3 ms to compare), so a plan of the same
-  // sizes is tried at once and the rows compared while the device works;
-  // other rows start again with a plan of their own.
-  const size_t n_ex = (n_out > 0 && n_vars > 0) ? static_cast<size_t>(n_out) * static_cast<size_t>(n_vars) : 0;
-  int same = -1;  // not compared yet
-  auto compare = [&] {
-    if (same < 0)
-      same = n_ex == 0 || std::memcmp(S.key_exps.data(), exponents, n_ex * sizeof(int32_t)) == 0;
-    return same == 1;
-  };
+  // Other rows of the same sizes must not cost an evaluation, so the rows are
+  // compared before anything runs, of a long list on the layer path its first
+  // kPolyCompareFirst bytes, and the others while the device works (7.4 MB
+  // for 184756 outputs of 10 modes: 0.3 ms): lists that differ only there
+  // start again with a plan of their own, which takes ten times as long.
+  const size_t ex_bytes =
+      (n_out > 0 && n_vars > 0) ? static_cast<size_t>(n_out) * static_cast<size_t>(n_vars) * sizeof(int32_t) : 0;
+  const size_t n_ex = ex_bytes / sizeof(int32_t);
   if (S.have_plan && S.key_n == n && S.key_vars == n_vars && S.key_out == n_out) {
-    if (!S.tables_on_device) compare();
-    if (same != 0) {
-      const int st = poly_run(S, b0, bm, n_out, out, info, compare);
-      if (compare()) return st;
+    const char *key = reinterpret_cast<const char *>(S.key_exps.data());
+    const char *given = reinterpret_cast<const char *>(exponents);
+    size_t layer_bytes = 0;
+    const size_t first = S.tables_on_device && poly_layers_fit(S.plan, &layer_bytes)
+                             ? std::min(ex_bytes, kPolyCompareFirst) : ex_bytes;
+    bool same = first == 0 || std::memcmp(key, given, first) == 0;
+    if (same) {
+      auto rest = [&] { return same = first == ex_bytes || std::memcmp(key + first, given + first, ex_bytes - first) == 0; };
+      bool asked = false;
+      const int st = poly_run(S, b0, bm, n_out, out, info, [&] { asked = true; return rest(); });
+      if (asked ? same : rest()) return st;
       g_error.clear();
     }
   }
