@@ -138,6 +138,8 @@ constexpr int kIntInnerDigits = 7;
 // Bytes of a polynomial permanent's exponent rows that are compared with the
 // kept plan's before anything runs (8 us).
 constexpr size_t kPolyCompareFirst = size_t{256} << 10;
+// Outputs up to which 6 and 7 particles take the subset sum.
+constexpr size_t kPolyFew6 = 64, kPolyFew7 = 4;
 // Device buffers one-shot batches may leave for the next ones, and how many
 // calls' worth: as many threads find theirs ready.
 constexpr size_t kKeptBytes = size_t{256} << 20;
@@ -1447,9 +1449,17 @@ void poly_subsets(int n, std::vector<int16_t> &sub, std::vector<uint16_t> &bits,
 
 // Whether a polynomial permanent takes the layer path: the subsets of one
 // size fit a block's threads, a row's coefficients its LDS, and the two
-// largest layers 8 GiB.  `bytes` receives the size of one layer buffer.
+// largest layers 8 GiB.  Few outputs of 6 or 7 particles do not: their
+// layers are as many kernels one after another, where the subset sum is one
+// kernel and a reduction over outputs and workgroups (a call, layers against
+// subsets: 6 particles in 4 modes, one output 61 and 50 us, 64 outputs 61 and
+// 59, 210 outputs 57 and 61; 7 particles 62 and 59, 4 outputs 63 and 66; at 5
+// particles the layers take 41 against 41 or less, at 8 67 against 85).
+// `bytes` receives the size of one layer buffer.
 bool poly_layers_fit(const PolyPlan &p, size_t *bytes) {
+  if (p.out_index.empty()) return false;  // nothing to evaluate, no levels
   if (p.n > kPolyLayerMaxN || static_cast<size_t>(p.n) * (p.M + 1) * sizeof(double2) > 16384) return false;
+  if ((p.n == 6 && p.out_index.size() <= kPolyFew6) || (p.n == 7 && p.out_index.size() <= kPolyFew7)) return false;
   double most = 1.0, choose = 1.0;
   for (int i = 1; i < p.n; ++i) {
     choose = choose * (p.n - i + 1) / i;
@@ -2733,7 +2743,8 @@ int pqp_perm_poly_coefficients_c128(int64_t n, int64_t n_vars, const double *b0,
   if (st != PQP_OK) return fail(st, err);
   S.subsets.clear();
   S.subset_bits.clear();
-  if (n <= kPolyLayerMaxN) poly_subsets(static_cast<int>(n), S.subsets, S.subset_bits, S.subset_first);
+  size_t layer_bytes = 0;
+  if (poly_layers_fit(S.plan, &layer_bytes)) poly_subsets(S.plan.n, S.subsets, S.subset_bits, S.subset_first);
   S.key_n = n;
   S.key_vars = n_vars;
   S.key_out = n_out;
