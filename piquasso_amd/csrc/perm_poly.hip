@@ -17,12 +17,12 @@
 // of i columns.  It needs sum_i C(n, i) i times the monomials of degree <= i
 // times M + 1 products where the subset sum below needs 2^n - 1 times those
 // of every degree: 2.6e8 against 1.9e9 complex FMAs for 10 photons in 10
-// modes, since the wide layers have few subsets.  It has no alternating sum,
-// so its error is no larger (2.6e-16 against 3.9e-16 there).  Bound by the
-// reads of a layer through L2 and the Infinity Cache (31 MB for the largest)
-// and, in the middle layers, by the FMAs.  Measured, 10 photons in 10 modes:
-// ten launches, 0.32 ms, for 5.40 + 0.35 ms of the subset sum and its
-// reduction; 6 photons in 7 modes: the whole call 93 us for 101 us.
+// modes, since the wide layers have few subsets.  It has no alternating sum.
+// Bound by the reads of a layer through L2 and the Infinity Cache (31 MB for
+// the largest) and, in the middle layers, by the FMAs.  Measured, 10 photons
+// in 10 modes: ten launches, 0.32 ms, for 5.40 + 0.35 ms of the subset sum
+// and its reduction; 9 photons in 8 modes: the whole call 235 us for 615 us,
+// 6 in 7 104 for 103.
 //
 // Subset sum (larger orders, or coefficients or layers too large):
 //
@@ -346,7 +346,12 @@ __global__ __launch_bounds__(kPolyLayerThreads) void poly_layer_kernel(PolyLayer
 }
 
 // The last row: S is all n columns, S - j (place n - 1 - j of the source
-// layer) for every j, only the requested monomials.  One thread each.
+// layer) for every j, only the requested monomials.  One thread each.  The n
+// products of a link are an FP64 run and the links' sums are folded in
+// double-double, as the subset sum's workgroups are: bound by its gathers,
+// the kernel takes the same 26 us for 184756 outputs (10 photons in 10
+// modes) as in FP64 throughout, and the error of that table, the norm
+// against 64 bits, is 1.4e-16 for 3.4e-16 (the subset sum's: 3.5e-16).
 __global__ __launch_bounds__(kPolyLayerThreads) void poly_last_kernel(PolyLayerArgs a) {
   extern __shared__ double2 coef[];  // row n - 1 of every B_m, then of B_0
   const int n = a.n, M = a.M, row = a.row;
@@ -358,21 +363,23 @@ __global__ __launch_bounds__(kPolyLayerThreads) void poly_last_kernel(PolyLayerA
   const int p = static_cast<int>(blockIdx.x) * kPolyLayerThreads + static_cast<int>(threadIdx.x);
   if (p >= a.n_out) return;
   const int e = a.out_mono[p];
-  double2 v = make_double2(0.0, 0.0);
+  cdd v = cdd_zero();
   auto add = [&](int m, int mono) {
     const double2 *c = coef + m * n;
-    if (!a.src) {  // n = 1
-      v.x += c[0].x;
-      v.y += c[0].y;
-      return;
+    double2 t = c[0];  // n = 1: times the empty product
+    if (a.src) {
+      const double2 *f = a.src + static_cast<int64_t>(mono) * n;
+      t = make_double2(0.0, 0.0);
+      for (int j = 0; j < n; ++j) t = cfma(c[j], f[n - 1 - j], t);
     }
-    const double2 *f = a.src + static_cast<int64_t>(mono) * n;
-    for (int j = 0; j < n; ++j) v = cfma(c[j], f[n - 1 - j], v);
+    const dd re = dd_two_sum(v.re.hi, t.x), im = dd_two_sum(v.im.hi, t.y);
+    v.re = dd{re.hi, v.re.lo + re.lo};
+    v.im = dd{im.hi, v.im.lo + im.lo};
   };
   if (e < a.n_src_mono) add(M, e);
   for (int q = a.link_ptr[e]; q < a.link_ptr[e + 1]; ++q) add(a.links[q] & 0xff, a.links[q] >> 8);
-  a.out[2 * p] = v.x;
-  a.out[2 * p + 1] = v.y;
+  a.out[2 * p] = v.re.hi + v.re.lo;
+  a.out[2 * p + 1] = v.im.hi + v.im.lo;
 }
 
 }  // namespace
