@@ -1626,7 +1626,7 @@ SamplePasses sample_passes(int64_t shots, int64_t photons) {
 struct TableState {
   std::mutex mu;
   hipStream_t stream = nullptr;
-  DevBuf in, out;
+  DevBuf in, out, states;
   HostBuf stage;
 };
 
@@ -2528,6 +2528,27 @@ int pqp_output_table_c128(const double *matrix, int64_t modes, int64_t ld, const
   a.modes = static_cast<int32_t>(modes);
   a.n = static_cast<int32_t>(n);
   a.prob = probabilities ? 1 : 0;
+  a.states = 0;
+  a.width = width;
+  a.first = 0;
+  a.per_given = 0.0;
+  a.sums = nullptr;
+  a.weights = nullptr;
+  if (!ones) {
+    // the sweep over the input's digits: at most 3 2^13 states
+    int most_in = 0;
+    for (int q = 0; q < width; ++q) {
+      if (hmult[q] < hmult[a.first]) a.first = q;
+      most_in = std::max(most_in, static_cast<int>(hmult[q]));
+    }
+    a.states = 1;
+    for (int q = 0; q < width; ++q) a.states *= hmult[q] + (q == a.first ? 0 : 1);
+    a.per_given = sweep_term_cost(width, most_in, static_cast<int>(n));
+    const size_t sums = static_cast<size_t>(a.states) * modes * 2 * sizeof(double);
+    if ((st = S.states.ensure(sums + static_cast<size_t>(a.states) * sizeof(double))) != PQP_OK) return st;
+    a.sums = static_cast<double2 *>(S.states.p);
+    a.weights = reinterpret_cast<double *>(static_cast<char *>(S.states.p) + sums);
+  }
   double *hout = reinterpret_cast<double *>(h + align256(in_bytes));
   for (int64_t s0 = 0; s0 < count; s0 += kTableSegment) {
     const int64_t rows = std::min(count - s0, kTableSegment);
@@ -2545,6 +2566,7 @@ int pqp_output_table_c128(const double *matrix, int64_t modes, int64_t ld, const
       a.outs = reinterpret_cast<const uint8_t *>(d + to);
       a.out = static_cast<double *>(S.out.p) + per * c0;
       a.count = c;
+      if (!ones && s0 == 0 && c0 == 0) PQP_HIP(launch_table_states(a, S.stream));
       PQP_HIP(launch_table(width, ones, a, S.stream));
     }
     PQP_HIP(hipMemcpyAsync(hout, S.out.p, static_cast<size_t>(rows) * per * sizeof(double),

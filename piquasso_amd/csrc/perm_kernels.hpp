@@ -124,6 +124,7 @@ hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream);
 
 // Probability tables (perm_table.hip): `width` occupied input modes, `ones`:
 // one particle in each.
+hipError_t launch_table_states(const TableArgs &a, hipStream_t stream);
 hipError_t launch_table(int width, bool ones, const TableArgs &a, hipStream_t stream);
 
 // One row of the layer path of a matrix-polynomial permanent

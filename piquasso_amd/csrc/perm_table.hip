@@ -25,6 +25,14 @@
 // so that a lane sweeps at most 32 states and a table of few items still
 // spreads (10 outputs of 16 particles: 49 us for 465 us planned; 1000: 128
 // us for 4.1 ms).
+//
+// Inputs with several particles in a mode may have fewer digits than an
+// output: such outputs are summed over the input's digits, whose row sums are
+// the same for every output and are laid out once (table_states_kernel).  40
+// outputs of 12 particles from one mode: 6.4e-15 of error (norm) for 2.1e-14
+// by the output's digits, 44 us a call for 43; 5000 of 16 from two modes 138
+// us for 292; 2000 from [2, 1 x 14], whose 24576 states few outputs use, 300
+// for 280.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -68,6 +76,78 @@ __device__ __forceinline__ void table_product(const double (&cr)[W], const doubl
   pi = ai;
 }
 
+// Whether the sweep over the input's digits is the cheaper one for an output
+// of mc occupied modes, `most` in one, and `terms` terms of its own digits:
+// the planner's rule and cost of a term (plan.cpp, sweep_cost).  It is also
+// the more accurate one there.  Its terms carry the row sums to the powers of
+// the output, so an output mode of small amplitude scales every term, where
+// the other sweep's terms add it to the larger ones and cancel.
+__device__ __forceinline__ bool sweep_flips(int mc, int most, const TableArgs &a, double terms) {
+  const double mult = mc <= kPowGroupedMaxCols && most <= 4 ? mc + most - 2 : a.n - 1;
+  const double per = most <= 1 ? 8.0 * mc - 2.0 : (2.0 * mc + 6.0 * mult + 4.0) * 1.25;
+  return a.states * per < 0.9 * (terms * a.per_given);
+}
+
+// The lane's share of that sweep: states at, at + step, ... of the input.
+__device__ __forceinline__ cdd flipped_sum(const TableArgs &a, int occ, int at, int step) {
+  cdd sum = cdd_zero();
+  const uint64_t used = __ballot(occ > 0);
+  const int lane = lane_id();
+  for (int v0 = at - lane; v0 < a.states; v0 += step) {
+    const bool active = v0 + lane < a.states;
+    const int v = active ? v0 + lane : 0;
+    const double w = active ? a.weights[v] : 0.0;
+    double pr = 1.0, pi = 0.0;
+    for (uint64_t m = used; m;) {
+      // the loads of four modes together: a load waits longer than it multiplies
+      double2 z[4];
+      int power[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = __builtin_ctzll(m ? m : used);
+        power[k] = m ? __builtin_amdgcn_readlane(occ, i) : 0;
+        z[k] = a.sums[static_cast<int64_t>(i) * a.states + v];
+        m &= m - 1;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        for (int q = power[k]; q > 0; --q) cmul(pr, pi, z[k].x, z[k].y);
+    }
+    sum = cdd_add(sum, cdd{dd_mul_d(dd{pr, 0.0}, w), dd_mul_d(dd{pi, 0.0}, w)});
+  }
+  return sum;
+}
+
+// The row sums sum_j (rho_j - 2 g_j) U[i, j] (the prepended column with 1) of
+// every mode i at every state g of the input's digits, and the states' signed
+// weights.  Grid (states / 256, modes), a thread each.
+__global__ __launch_bounds__(256) void table_states_kernel(TableArgs a) {
+  const int v = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+  const int i = static_cast<int>(blockIdx.y);
+  if (v >= a.states) return;
+  const cptr<double> row = as_const<double>(a.rows, int64_t{16} * i * a.width);
+  const cptr<int32_t> mult = as_const<int32_t>(a.mult);
+  double2 s = make_double2(row[2 * a.first], row[2 * a.first + 1]);
+  double w = 1.0;
+  int rest = v;
+  for (int j = 0; j < a.width; ++j) {
+    const int rho = mult[j] - (j == a.first ? 1 : 0);
+    // the quotient by a small radix is exact this way
+    const int q = static_cast<int>((static_cast<double>(rest) + 0.5) * kInvSmall[rho + 1]);
+    const int g = rest - q * (rho + 1);
+    rest = q;
+    const double al = rho - 2 * g;
+    s.x = fmaR(al, row[2 * j], s.x);
+    s.y = fmaR(al, row[2 * j + 1], s.y);
+    if (i == 0) {
+      w *= lane_binomial(rho, g);
+      if (g & 1) w = -w;
+    }
+  }
+  a.sums[static_cast<int64_t>(i) * a.states + v] = s;
+  if (i == 0) a.weights[v] = w;
+}
+
 // NW waves per item, 4 / NW items per block (NW <= 4) or one.
 template <int W, bool ONES, int NW>
 __global__ __launch_bounds__(NW > 4 ? NW * kWave : 4 * kWave)
@@ -81,8 +161,12 @@ __attribute__((amdgpu_waves_per_eu(W <= 8 ? 7 : W <= 12 ? 5 : 4, 8))) void perm_
   if (item >= a.count) return;  // whole blocks where NW > 1
   const int occ = lane < a.modes ? a.outs[item * a.modes + lane] : 0;
 
-  int total = 0;
-  for (int v = 1; v <= a.n; ++v) total += v * __builtin_popcountll(__ballot(occ == v));
+  int total = 0, most = 0;
+  for (int v = 1; v <= a.n; ++v) {
+    const uint64_t at = __ballot(occ == v);
+    total += v * __builtin_popcountll(at);
+    if (at) most = v;
+  }
   const bool match = total == a.n && !__ballot(occ > a.n);
   double *out = a.out + (a.prob ? 1 : 2) * item;
   if (!match) {  // another particle number: amplitude 0
@@ -98,7 +182,12 @@ __attribute__((amdgpu_waves_per_eu(W <= 8 ? 7 : W <= 12 ? 5 : 4, 8))) void perm_
   const cptr<int32_t> mult = as_const<int32_t>(a.mult);
 
   cdd sum = cdd_zero();
-  for (int u0 = wave * kWave; u0 < p.U; u0 += NW * kWave) {
+  bool flipped = false;
+  if constexpr (!ONES) {
+    flipped = sweep_flips(__builtin_popcountll(__ballot(occ > 0)), most, a, static_cast<double>(p.U) * S);
+    if (flipped) sum = flipped_sum(a, occ, wave * kWave + lane, NW * kWave);
+  }
+  for (int u0 = flipped ? p.U : wave * kWave; u0 < p.U; u0 += NW * kWave) {
     const bool active = u0 + lane < p.U;
     double cr[W], ci[W];
     const double w_top = wave_start<W>(p, active ? u0 + lane : 0, rows, 2 * W, p.i0, cr, ci);
@@ -165,6 +254,12 @@ hipError_t table_launch(const TableArgs &a, hipStream_t stream) {
 }
 
 }  // namespace
+
+hipError_t launch_table_states(const TableArgs &a, hipStream_t stream) {
+  if (a.states < 1 || a.modes > kTableMaxModes || a.width < 1 || a.width > kTableMaxN) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(table_states_kernel, dim3((a.states + 255) / 256, a.modes), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
 
 hipError_t launch_table(int width, bool ones, const TableArgs &a, hipStream_t stream) {
   if (a.count <= 0) return hipSuccess;

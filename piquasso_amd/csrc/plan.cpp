@@ -116,6 +116,13 @@ void gray_steps(const std::vector<int> &radix, std::vector<int> &digit,
   }
 }
 
+double sweep_term_cost(int mc, int cmax, int n) {
+  if (cmax <= 1) return 2.0 * mc + 6.0 * std::max(mc - 1, 0) + 4.0;
+  const bool grouped = mc <= kPowGroupedMaxCols && cmax <= 4;
+  const double mult = grouped ? mc + cmax - 2 : n - 1;
+  return (2.0 * mc + 6.0 * mult + 4.0) * 1.25;
+}
+
 namespace {
 
 // The caller's row stride covers the view's rows (its columns when the
@@ -126,10 +133,7 @@ bool stride_ok(const PermInput &in) {
 
 // Modelled cost of the Glynn sweep with `rows` as Gray digits and `cols`
 // as the product side: T = prod (rho_i + 1) after the prepend, times the
-// work per term (row updates, column product with grouped powers or the
-// count form, accumulation), the grouped form weighted by the lower issue
-// rate of its per-column snapshot tests (about 76% VALU issue against 94%
-// for unit multiplicities, measured on MI355X).
+// work per term.
 double sweep_cost(const int32_t *rows, int64_t m_r, const int32_t *cols, int64_t m_c) {
   int minelem = 0;
   int64_t i0 = -1;
@@ -150,10 +154,7 @@ double sweep_cost(const int32_t *rows, int64_t m_r, const int32_t *cols, int64_t
       cmax = std::max(cmax, static_cast<int>(cols[j]));
       n += cols[j];
     }
-  if (cmax <= 1) return T * (2.0 * mc + 6.0 * std::max(mc - 1, 0) + 4.0);
-  const bool grouped = mc <= kPowGroupedMaxCols && cmax <= 4;
-  const double mult = grouped ? mc + cmax - 2 : n - 1;
-  return T * (2.0 * mc + 6.0 * mult + 4.0) * 1.25;
+  return T * sweep_term_cost(mc, cmax, n);
 }
 
 }  // namespace

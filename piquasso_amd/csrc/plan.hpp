@@ -114,6 +114,13 @@ int bucket_for_width(int mc, bool fp32, int *mcp_out);
 // [items[k].b_off, + info[k].rowsrc.size() * mcp * 2 * (4 or 8)).
 void plan_refresh_matrix(Plan &plan, const std::vector<PermInput> &inputs);
 
+// Modelled work of a Glynn term over mc columns of n particles, cmax in one
+// of them: row updates, column product with grouped powers or the count form,
+// accumulation, the grouped form weighted by the lower issue rate of its
+// per-column snapshot tests (about 76% VALU issue against 94% for unit
+// multiplicities, measured on MI355X).
+double sweep_term_cost(int mc, int cmax, int n);
+
 // Transposes an item whose transposed sweep costs less than 0.9 of the given
 // one: perm(A; r, c) = perm(A^T; c, r), the permanent of the expanded matrix
 // being invariant under transposition.  Invalid items are left alone (the

@@ -2,6 +2,8 @@
 // interferometer and input occupation, many output occupations.
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include <cstdint>
 
 namespace pqp {
@@ -18,6 +20,13 @@ struct TableArgs {
   int64_t count;
   int32_t modes, n;
   int32_t prob;         // 1: probabilities
+  // Inputs with more than one particle in a mode: the sweep over the input's
+  // digits (table_states_kernel), taken for the outputs where it is cheaper.
+  int32_t states, width;  // prod (rho_j + 1) after the prepend, and occupied columns
+  int32_t first;        // the prepended column: the first of the smallest occupation
+  double per_given;     // cost of a state of the sweep over the output's digits
+  double2 *sums;        // modes x states: the row sums of every output mode
+  double *weights;      // states: signed binomial weights
 };
 
 }  // namespace pqp
