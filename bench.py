@@ -456,12 +456,11 @@ def _probabilities_leg(pa, W, cpu):
 def _lossy_pd_leg(pa, W, cpu):
     """Lossy, partially distinguishable probability tables (every output with
     at most n photons; random Gram matrix; losses before a Haar unitary):
-    the matrix-polynomial permanent over all particle subsets in one call,
-    timed around the whole call (upload, kernels, download).  `ms` is the
+    the matrix-polynomial permanent of all outputs in one call, timed around the whole call (upload, kernels, download).  `ms` is the
     median over new Gram matrices for the same output set (the monomial plan
     is reused), `ms_first_call` a call that plans the closure afresh.
-    FLOP: the kernel's algorithmic count per subset (complex multiply 6, FMA
-    8 per link) times the subsets."""
+    FLOP: of the expansion by column subsets that these orders run
+    (workloads.lossy_layer_flops)."""
     from piquasso_amd import distinguishability as D
 
     recs = {}
@@ -482,7 +481,7 @@ def _lossy_pd_leg(pa, W, cpu):
             p = pa.lossy_detection_probabilities(outs, t, inp, gk)
             ts.append(time.perf_counter() - t0)
         sec = float(np.median(ts))
-        fl = float(info["flops_per_subset"]) * info["subsets"]
+        fl = W.lossy_layer_flops(d, n)
         rec = {
             "outputs": len(outs),
             "ms": sec * 1e3,
@@ -490,8 +489,6 @@ def _lossy_pd_leg(pa, W, cpu):
             "tflops": fl / sec / 1e12,
             "flops": fl,
             "monomials": info["monomials"],
-            "polynomial_in": "LDS" if info["lds"] else "global memory",
-            "workgroups": info["workgroups"],
             "sum_minus_one": float(p.sum() - 1.0),
             "what": f"lossy_detection_probabilities: all outputs with <= {n} photons in {d} modes, "
                     f"{n} photons, random {n} x {n} Gram matrix",
@@ -511,10 +508,9 @@ def _lossy_pd_leg(pa, W, cpu):
 
 
 def _sampling_leg(pa, W, cpu):
-    """Clifford & Clifford sampling of 20 photons in 40 modes, 1024 shots in
-    lockstep (20 rounds, each one batched column-minor launch over all
-    shots); samples/s over the whole call, host bookkeeping included.  The
-    shots the CPU leg also drew must come out identical."""
+    """Clifford & Clifford sampling of 20 photons in 40 modes, 1024 shots, all
+    20 rounds on the device in one call; samples/s over the whole call, host
+    bookkeeping included.  The shots the CPU leg also drew must come out identical."""
     from piquasso_amd import sampling as PS
 
     u, occ = W.sampling()

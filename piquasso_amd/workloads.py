@@ -26,6 +26,8 @@ Workloads (sizes from the engine's benchmark definition):
 
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 __all__ = [
@@ -39,6 +41,7 @@ __all__ = [
     "minors_flops",
     "tensor",
     "tensor_flops",
+    "lossy_layer_flops",
     "output_patterns",
     "glynn_terms",
     "glynn_flops",
@@ -203,11 +206,20 @@ def tensor_flops(n: int) -> float:
     """Algorithmic FLOP of one tensor permanent in the sign-vector form:
     4^(n-1) / 2 pairs (the conjugate half is not visited) of n factors
     x R conj(R') + Q (complex multiply 6, add 1), n - 1 complex products (6),
-    the Gray updates of R' (2 per row) and Q (1 per row) and the weighted
-    accumulation (2): 16 n - 4 per pair."""
+    the Gray update of Q (1 per row) and the weighted accumulation (2):
+    14 n - 4 per pair (R' is summed once per sign vector)."""
     if n <= 0:
         return 0.0
-    return 4.0 ** (n - 1) / 2.0 * (16.0 * n - 4.0)
+    return 4.0 ** (n - 1) / 2.0 * (14.0 * n - 4.0)
+
+
+def lossy_layer_flops(modes: int, photons: int) -> float:
+    """Algorithmic FLOP of a lossy table of all outputs expanded row by row
+    over the column subsets: row i takes every subset of i columns to each
+    column it lacks, for every monomial of degree <= i times the constant and
+    each variable, a complex FMA (8) each."""
+    return 8.0 * sum(math.comb(photons, i) * (photons - i) * math.comb(i + modes, modes) * (modes + 1)
+                     for i in range(photons))
 
 
 def output_patterns(modes: int = 14, photons: int = 7, seed: int = 8):
