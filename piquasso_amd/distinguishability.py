@@ -118,8 +118,10 @@ def detection_probabilities(occupation_numbers, interferometer, input_occupation
         raise ValueError(f"at most {MAX_PARTICLES} particles are supported, got {n}")
     x = float(uniform_particle_overlap)
     probs = np.zeros(outs.shape[0])
-    if d == 0 or len(probs) == 0:
-        return probs + (1.0 if d == 0 else 0.0)
+    if d == 0:  # empty products
+        return tensor_permanent_batch([u] * len(probs), [x] * len(probs))
+    if len(probs) == 0:
+        return probs
     inp32 = np.ascontiguousarray(inp, dtype=np.int32)
     dp = ctypes.POINTER(ctypes.c_double)
     _capi.check(_capi.lib().pqp_overlap_table_c128(
