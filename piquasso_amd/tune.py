@@ -17,6 +17,7 @@ CLI:  python -m piquasso_amd.tune [--out piquasso_amd/tuning/gfx950.json] [--rep
 from __future__ import annotations
 
 import argparse
+import copy
 import itertools
 import json
 import os
@@ -150,7 +151,7 @@ def best_config(count: int, cus: int, arch: str, path: str = None, log2_terms=No
     kwargs: total_units, persistent, target_inner), or {} when no table was written for
     it.  The entry is the tuned class of nearest size (choose_class); unit
     counts scale with the CU count of the table's device."""
-    table = load_tuning(path or DEFAULT_TABLE)
+    table = _held_table(path or DEFAULT_TABLE)
     if not table or not arch.split(":")[0] == str(table.get("device", "")).split(":")[0]:
         return {}
     name = choose_class(table, count, log2_terms)
@@ -205,17 +206,21 @@ def tune(out: str = DEFAULT_TABLE, reps: int = 5, only=None, log=print) -> dict:
     return table
 
 
-_loaded: dict = {}  # path -> ((mtime, size), table)
+_loaded: dict = {}  # path -> (stamp of the file, table)
 
 
 def load_tuning(path: str = DEFAULT_TABLE) -> dict:
-    """The tuned table, or {} when none has been written for this device
-    (read again when the file changes)."""
+    """The tuned table, or {} when none has been written for this device."""
+    return copy.deepcopy(_held_table(path))
+
+
+def _held_table(path: str) -> dict:
+    """The same, not to be changed: read again when the file is another."""
     try:
         st = os.stat(path)
     except OSError:
         return {}
-    stamp = (st.st_mtime_ns, st.st_size)
+    stamp = (st.st_ino, st.st_mtime_ns, st.st_size)
     held = _loaded.get(path)
     if held is None or held[0] != stamp:
         with open(path) as f:
