@@ -147,12 +147,13 @@ constexpr size_t kKeptExecs = 4;
 
 // Permanents without tables: one block up to kOneBlockTerms Gray terms (the
 // blocks' meeting costs about 3 us: 13 particles 17.0 us a call in one block
-// and 16.5 in four), else blocks for about kOneLaneStates states a lane, up
+// and 16.5 in four), else blocks for about kOneStates states a lane, up
 // to a wave per SIMD, and two above kOneManyTerms terms (2^23 terms: 85 us
 // at one, 61 at two).  Above kOneMaxTerms the planned sweep, whose units
 // walk longer, is as fast.
 constexpr double kOneBlockTerms = 2048.0;
-constexpr double kOneLaneStates = 4.0;
+constexpr double kOneStates = 4.0;
+constexpr int kOneBlockWaves = 4;  // one per SIMD
 constexpr double kOneManyTerms = 2097152.0;
 constexpr double kOneMaxTerms = 16777216.0;
 
@@ -974,8 +975,8 @@ int run_one(OnePlan &p, double *out2, double *out_dd4) {
   const double *res = static_cast<const double *>(S.one_res.host);
   volatile uint64_t *done = static_cast<uint64_t *>(S.one_res.host) + 7;
   *done = 0;
-  PQP_HIP(p.fp32 ? launch_one_f(p.width, p.ones, p.few, a, p.blocks, p.waves, S.one_stream)
-                 : launch_one_d(p.width, p.ones, p.few, a, p.blocks, p.waves, S.one_stream));
+  PQP_HIP(p.fp32 ? launch_one_f(p.width, p.kind, a, p.blocks, p.waves, S.one_stream)
+                 : launch_one_d(p.width, p.kind, a, p.blocks, p.waves, S.one_stream));
   if ((st = wait_done(S.one_stream, done, h.seq)) != PQP_OK) {
     // a launch that did not finish its count leaves it behind
     (void)hipMemsetAsync(h.counter, 0, sizeof(int), S.one_stream);
@@ -1975,20 +1976,60 @@ bool one_plan(const PermInput &given, uint32_t flags, OnePlan &p) {
   p.in = in;
   p.n = static_cast<int>(sr);
   p.width = width;
-  p.ones = expand || cmax <= 1;
-  p.few = p.ones && rmax <= 1 && sr <= kOneFew;
+  const bool ones = expand || cmax <= 1;
+  p.kind = !ones ? kOneAny : rmax <= 1 ? kOneUnit : kOneOnes;
   p.fp32 = (flags & PQP_FLAG_FP32) != 0;
   p.terms = terms;
-  p.blocks = 1;
-  p.waves = kOneWaves;
-  if (terms > kOneBlockTerms) {
-    const double cap = terms > kOneManyTerms ? kOneMaxBlocks : kOneMaxBlocks / 2;
-    p.blocks = static_cast<int>(std::ceil(std::min(terms / (64.0 * kOneLaneStates * kOneWaves), cap)));
-  } else {
-    while (p.waves > 1 && terms <= 32.0 * kOneLaneStates * p.waves) p.waves /= 2;
-  }
   return true;
 }
+
+namespace {
+
+// The lanes' digits: those whose states fill whole sets of 64 lanes best, few
+// of them (each is a row that every lane adds; the other digits' rows are
+// added once per wave).  radix[0 .. digits), equal ones side by side; the
+// search ends with the first set of digits that fills kOneFill of its lanes.
+struct LaneDigits {
+  const int *radix;
+  int digits;
+  uint32_t best;
+  int best_states;
+  double best_score;
+  int visits;
+};
+
+constexpr double kOneFill = 0.95;
+constexpr int kOneVisits = 400;
+
+OneDigit one_digit(int rho) {
+  OneDigit d{1.0 / (rho + 1), 0, rho, 0};
+  if (rho > 10) return d;
+  uint64_t c = 1;
+  for (int g = 0; g <= rho / 2; ++g) {
+    d.choose |= c << (8 * g);
+    c = c * static_cast<uint64_t>(rho - g) / static_cast<uint64_t>(g + 1);
+  }
+  return d;
+}
+
+bool lane_search(LaneDigits &s, int from, int used, uint32_t set, int states) {
+  const double fill = states / (64.0 * ((states + 63) / 64));
+  const double score = fill - 0.02 * used;
+  if (score > s.best_score) {
+    s.best = set;
+    s.best_states = states;
+    s.best_score = score;
+  }
+  if (fill >= kOneFill || ++s.visits > kOneVisits) return true;
+  for (int d = from; d < s.digits && used < kOneLaneDigits; ++d) {
+    if (d > from && s.radix[d] == s.radix[d - 1]) continue;  // one of equal digits is as good as another
+    if (states * s.radix[d] > kOneLaneStates) continue;
+    if (lane_search(s, d + 1, used + 1, set | 1u << d, states * s.radix[d])) return true;
+  }
+  return false;
+}
+
+}  // namespace
 
 void one_fill(OnePlan &p, OneArgs &args) {
   OneTables &t = args.tables;
@@ -1996,84 +2037,93 @@ void one_fill(OnePlan &p, OneArgs &args) {
   const PermInput &in = p.in;
   int64_t cols[kOneMaxWidth];
   int width = 0;
-  a.cmax = 1;
-  if (!p.few) std::memset(t.over, 0, sizeof(t.over));
+  if (p.kind == kOneAny) std::memset(t.more, 0, sizeof(t.more));
   for (int64_t j = 0; j < in.m_c; ++j) {
     if (in.cols[j] == 0) continue;
     const int64_t at = in.transposed ? j * in.ld : j;
-    if (p.ones) {
+    if (p.kind != kOneAny) {
       for (int r = 0; r < in.cols[j]; ++r) cols[width++] = at;
       continue;
     }
-    for (int r = 2; r <= in.cols[j]; ++r) t.over[r - 2] |= 1u << width;
-    a.cmax = std::max(a.cmax, in.cols[j]);
+    t.more[width / 4] |= static_cast<uint32_t>(in.cols[j] - 1) << (8 * (width % 4));
     cols[width++] = at;
   }
-  // the digits: every row, the first smallest one lower
+  // the digits: every row, the first smallest one lower; binary ones first,
+  // the others by radix
   const int64_t i0 = first_smallest(in);
   auto rho = [&](int64_t i) { return in.rows[i] - (i == i0 ? 1 : 0); };
   a.n = p.n;
-  int64_t digit[kOneMaxRows];  // binary ones first
+  int64_t digit[kOneMaxRows];
+  int radix[kOneMaxRows];
   int digits = 0, binary = 0;
   for (int64_t i = 0; i < in.m_r; ++i)
     if (rho(i) == 1) digit[digits++] = i;
   binary = digits;
   for (int64_t i = 0; i < in.m_r; ++i)
     if (rho(i) > 1) digit[digits++] = i;
-  // the lanes' digits: six binary ones, or the largest product up to 64
-  uint32_t lane = 0;
-  if (binary >= kOneLaneDigits) {
-    lane = (1u << kOneLaneDigits) - 1;
-    a.lanes = kWave;
-  } else {
-    uint32_t best[kWave + 1] = {};  // digits of each product, and bit 31
-    best[1] = 1u << 31;
-    for (int d = 0; d < digits; ++d)
-      for (int v = kWave; v >= 1; --v)
-        if (best[v] && v * (rho(digit[d]) + 1) <= kWave && !best[v * (rho(digit[d]) + 1)])
-          best[v * (rho(digit[d]) + 1)] = best[v] | 1u << d;
-    a.lanes = kWave;
-    while (!best[a.lanes]) --a.lanes;
-    lane = best[a.lanes] & ~(1u << 31);
+  std::stable_sort(digit + binary, digit + digits, [&](int64_t x, int64_t y) { return rho(x) < rho(y); });
+  for (int d = 0; d < digits; ++d) radix[d] = static_cast<int>(rho(digit[d])) + 1;
+  uint32_t lane = (1u << std::min(binary, kOneLaneDigits)) - 1;
+  a.lanes = 1 << std::min(binary, kOneLaneDigits);
+  t.lane_binary = 1;
+  if (binary < kOneLaneDigits && binary < digits) {
+    LaneDigits s{radix, digits, 0, 1, -1.0, 0};
+    lane_search(s, 0, 0, 0, 1);
+    lane = s.best;
+    a.lanes = s.best_states;
+    t.lane_binary = (lane >> binary) == 0;
   }
-  // inner digits until every wave has one state of the others; half as many
-  // waves more are added rather than a digit (radices above 2 leave waves
-  // without a state otherwise)
-  const double waves = (p.blocks > 1 ? 1.5 : 1.0) * p.waves * p.blocks;
-  double chunks = p.terms / a.lanes;
+  t.lane_chunks = (a.lanes + kWave - 1) / kWave;
+  t.lane_inv = 1.0 / t.lane_chunks;
+  // One block's waves, for two states a lane of single photons, one where a
+  // state is a longer product; or as many blocks as keep about kOneStates
+  // states a lane.  Inner digits as long as every wave keeps a chunk.
+  double chunks = p.terms / a.lanes;  // of the other digits
+  const double all = chunks * t.lane_chunks;
+  double waves;
+  if (p.terms > kOneBlockTerms) {
+    p.waves = kOneBlockWaves;
+    waves = std::min(all / kOneStates,
+                     static_cast<double>(kOneBlockWaves * (p.terms > kOneManyTerms ? kOneMaxBlocks : kOneMaxBlocks / 2)));
+  } else {
+    p.blocks = 1;
+    const double most = p.kind == kOneUnit ? std::min(all / 2.0, static_cast<double>(kOneBlockWaves))
+                                           : std::min(all, static_cast<double>(kOneWaves));
+    p.waves = std::max(1, static_cast<int>(most));
+    waves = p.waves;
+  }
   uint32_t inner = 0;
   a.S = 1;
-  a.binary = 1;
-  for (int d = 0; d < digits && chunks > waves; ++d) {
-    const int radix = static_cast<int>(rho(digit[d])) + 1;
-    if ((lane >> d & 1u) || a.S * radix > kOneMaxStates) continue;
+  t.binary = 1;
+  for (int d = 0; d < digits; ++d) {
+    if ((lane >> d & 1u) || a.S * radix[d] > kOneMaxStates || chunks * t.lane_chunks < waves * radix[d]) continue;
     inner |= 1u << d;
-    a.S *= radix;
-    chunks /= radix;
-    if (d >= binary) a.binary = 0;
+    a.S *= radix[d];
+    chunks /= radix[d];
+    if (d >= binary) t.binary = 0;
   }
-  a.chunks = static_cast<int32_t>(std::llround(chunks));
-  if (p.blocks > 1) p.blocks = std::min((a.chunks + p.waves - 1) / p.waves, kOneMaxBlocks);
+  a.chunks = static_cast<int32_t>(std::llround(chunks)) * t.lane_chunks;
+  if (p.terms > kOneBlockTerms) p.blocks = std::min((a.chunks + p.waves - 1) / p.waves, kOneMaxBlocks);
   int64_t order[kOneMaxRows];
   int rows = 0;
   a.lane_digits = a.inner = a.rest = 0;
   for (int d = 0; d < digits; ++d)
     if (lane >> d & 1u) {
-      a.lane_rho[a.lane_digits++] = static_cast<int32_t>(rho(digit[d]));
+      t.lane[a.lane_digits++] = one_digit(radix[d] - 1);
       order[rows++] = digit[d];
     }
   order[rows++] = i0;
   for (int d = 0; d < digits; ++d)
     if (inner >> d & 1u) {
-      a.rho[a.inner++] = static_cast<int32_t>(rho(digit[d]));
+      t.digit[a.inner++] = one_digit(radix[d] - 1);
       order[rows++] = digit[d];
     }
   for (int d = 0; d < digits; ++d)
     if (!((lane | inner) >> d & 1u)) {
-      a.rho[a.inner + a.rest++] = static_cast<int32_t>(rho(digit[d]));
+      t.digit[a.inner + a.rest++] = one_digit(radix[d] - 1);
       order[rows++] = digit[d];
     }
-  if (!a.binary) {
+  if (!t.binary) {
     // reflected mixed-radix Gray code of the inner digits
     int g[kOneMaxRows] = {}, dir[kOneMaxRows];
     double coef = 1.0;
@@ -2082,9 +2132,9 @@ void one_fill(OnePlan &p, OneArgs &args) {
       t.step[v] = OneStep{coef, 0, 0};
       if (v + 1 == a.S) break;
       int i = 0;
-      for (; g[i] + dir[i] < 0 || g[i] + dir[i] > a.rho[i]; ++i) dir[i] = -dir[i];
+      for (; g[i] + dir[i] < 0 || g[i] + dir[i] > t.digit[i].rho; ++i) dir[i] = -dir[i];
       // C(rho, g +- 1) from C(rho, g), exact
-      coef = dir[i] > 0 ? -coef * (a.rho[i] - g[i]) / (g[i] + 1) : -coef * g[i] / (a.rho[i] - g[i] + 1);
+      coef = dir[i] > 0 ? -coef * (t.digit[i].rho - g[i]) / (g[i] + 1) : -coef * g[i] / (t.digit[i].rho - g[i] + 1);
       g[i] += dir[i];
       t.step[v].factor = dir[i] > 0 ? -2 : 2;
       t.step[v].row = 1 + i;

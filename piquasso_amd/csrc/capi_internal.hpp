@@ -43,8 +43,8 @@ PlanOptions single_plan_options(uint32_t flags, const PermInput &in);
 struct OnePlan {
   PermInput in;       // transposed where that sweep is clearly cheaper
   int n, width;       // particles, distinct columns
-  bool ones, fp32;
-  bool few;           // up to kOneFew particles, one in each row and column
+  OneKind kind;
+  bool fp32;
   int blocks, waves;  // waves of a block
   double terms;       // Gray terms
 };

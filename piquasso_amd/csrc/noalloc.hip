@@ -107,8 +107,8 @@ int one_noalloc(OnePlan &p, double *out, double *out_dd) {
   h.partials = reinterpret_cast<double *>(base + kPartials);
   h.done = reinterpret_cast<uint64_t *>(h.out + 7);
   h.seq = 0;
-  PQP_NA_HIP(p.fp32 ? launch_one_f(p.width, p.ones, p.few, a, p.blocks, p.waves, nullptr)
-                    : launch_one_d(p.width, p.ones, p.few, a, p.blocks, p.waves, nullptr));
+  PQP_NA_HIP(p.fp32 ? launch_one_f(p.width, p.kind, a, p.blocks, p.waves, nullptr)
+                    : launch_one_d(p.width, p.kind, a, p.blocks, p.waves, nullptr));
   double res[7];
   PQP_NA_HIP(hipMemcpy(res, h.out, sizeof(res), hipMemcpyDeviceToHost));
   out[0] = res[0];

@@ -9,13 +9,18 @@ namespace pqp {
 
 constexpr int kOneMaxWidth = 24;         // distinct columns
 constexpr int kOneMaxRows = 25;          // the row the sums start from and the digits' rows (2^24 terms)
-constexpr int kOneFew = 12;              // rows and columns of the kernels for few of them
 constexpr int kOneMaxStates = 64;        // inner states of a lane: one FP64 run (kDdFold terms)
-constexpr int kOneLaneDigits = 6;        // binary digits that the 64 lanes of a wave differ in
-constexpr int kOneMaxMult = 64;          // largest multiplicity
+constexpr int kOneLaneDigits = 6;        // digits that the lanes of a wave differ in
+constexpr int kOneLaneStates = 4096;     // and their states: 64 chunks of lanes
 constexpr int kOneMaxBlocks = 512;
+constexpr int kOneWaves = 8;             // waves of a block at most
 
-constexpr int kOneWaves = 4;             // waves of a block at most: one per SIMD
+// What the kernel is compiled for.
+enum OneKind {
+  kOneUnit,  // one particle in each row and column: binary digits, as many rows as columns
+  kOneOnes,  // one particle in each column
+  kOneAny,
+};
 
 // Inner state v of a mixed-radix sweep: its signed weight, and the row that
 // is added, times factor, after it.
@@ -24,9 +29,23 @@ struct OneStep {
   int32_t factor, row;
 };
 
-// What only bunched rows or columns read.
+// A digit of values 0 .. rho: 1 / (rho + 1), and its binomials C(rho, g) for g
+// <= rho / 2, a byte each where the largest fits one (rho <= 10), else 0.
+struct OneDigit {
+  double inv;
+  uint64_t choose;
+  int32_t rho, pad;
+};
+
+// What a kOneUnit kernel has no use for.
 struct OneTables {
-  uint32_t over[kOneMaxMult];  // over[r - 2], r = 2 .. cmax: the columns of multiplicity >= r
+  uint32_t more[kOneMaxWidth / 4];  // a byte a column: its multiplicity less one
+  OneDigit lane[kOneLaneDigits];    // the lanes' digits
+  OneDigit digit[kOneMaxRows];      // the inner and the other ones
+  double lane_inv;      // 1 / lane_chunks
+  int32_t lane_chunks;  // sets of 64 of the lanes' states
+  int32_t lane_binary;  // the lanes' digits are binary
+  int32_t binary;       // the inner digits are: `step` is not used
   OneStep step[kOneMaxStates];
 };
 
@@ -39,16 +58,11 @@ struct alignas(64) OneHead {
   int32_t n;            // particles
   int32_t lane_digits, lanes;  // their states
   int32_t inner, rest;  // inner digits, and the others
-  int32_t S, chunks;    // states of the inner digits and of the others
-  int32_t binary;       // the inner digits are binary: `step` is not used
-  int32_t cmax;         // largest column multiplicity
-  int32_t lane_rho[kOneLaneDigits];  // largest values of the lanes' digits
-  int32_t rho[kOneMaxRows];          // and of the inner and the other ones
+  int32_t S, chunks;    // states of the inner digits; of the others, times the lane chunks
 };
 
-// The rows are in the order of their digits: the lanes' digits (six binary
-// ones, or as many states in at most 64 as the digits allow), the prepended
-// row, the inner digits, then the others.
+// The rows are in the order of their digits: the lanes', the prepended row,
+// the inner digits, then the others.
 template <size_t BYTES>
 struct OneRows {
   OneHead h;
@@ -56,10 +70,10 @@ struct OneRows {
 };
 
 // The arguments are written for every launch (about 0.1 us a KB), so a
-// kernel takes as many bytes of the host's OneArgs as its widths need: W
-// columns of kOneMaxRows rows, or, where rows and columns hold one particle
-// each and are few, of kOneFew rows without the tables, from `rows` on.
-// 12 particles: 11 KB 14.1 us a call, 6 KB 13.7, 2.5 KB 13.5.
+// kernel takes as many bytes of the host's OneArgs as it reads: W columns of
+// kOneMaxRows rows, or, of kind kOneUnit, of W rows without the tables, from
+// `rows` on.  12 particles: 11 KB 14.1 us a call, 6 KB 13.7, 2.5 KB 13.5 (12.5
+// with the kernel of this kind).
 template <size_t BYTES>
 struct OneArgsOf {
   OneTables tables;

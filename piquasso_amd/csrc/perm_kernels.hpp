@@ -48,8 +48,8 @@ PQP_DECLARE_BUCKET(7)
 // Single permanents planned by their own waves (perm_one.hip): one launch
 // of `blocks` blocks of `waves` waves for a permanent of `width` distinct columns (all of
 // multiplicity 1: ones).
-hipError_t launch_one_d(int width, bool ones, bool few, const OneArgs &a, int blocks, int waves, hipStream_t stream);
-hipError_t launch_one_f(int width, bool ones, bool few, const OneArgs &a, int blocks, int waves, hipStream_t stream);
+hipError_t launch_one_d(int width, OneKind kind, const OneArgs &a, int blocks, int waves, hipStream_t stream);
+hipError_t launch_one_f(int width, OneKind kind, const OneArgs &a, int blocks, int waves, hipStream_t stream);
 
 constexpr int kBuckets = 8;        // forward kernel width buckets
 constexpr int kMinorBuckets = 9;   // column-minor kernel buckets

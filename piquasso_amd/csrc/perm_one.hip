@@ -11,23 +11,30 @@
 // Bound by latency: 2^19 terms of 20 columns are 3 us of FP64 issue for the
 // whole chip.  What counts is the chain of one wave: its start, its inner
 // states, the double-double reductions, and the way to the host.  So
-//  * the lanes of a wave differ in a few digits only, six binary ones or as
-//    many states in at most 64 as the digits allow.  The rows of all other
-//    digits are summed once per wave, a lane per component (their loads are
-//    in flight together), and broadcast through the LDS; a lane then adds a
-//    few rows instead of all;
+//  * the lanes of a wave differ in a few digits only: six binary ones, or
+//    those whose states fill sets of 64 lanes best (one_fill).  The rows of
+//    all other digits are summed once per wave, a lane per component (their
+//    loads are in flight together), and broadcast through the LDS; a lane
+//    then adds a few rows instead of all;
 //  * these rows and the inner ones are scalar operands, and the waves of
-//    a block touch their lines together first;
+//    a block touch their lines, and the digits', together first;
 //  * permanents of few terms stay in one block (no block waits for another),
 //    others take up to one wave per SIMD with few inner states.  Their
 //    blocks count themselves; the last one sums the partials and publishes
-//    the result to mapped host memory.
+//    the result to mapped host memory;
+//  * permanents of one particle in each row and column have kernels of their
+//    own: all digits are binary, and no code of other digits is fetched.
 //
-// A call with occupations not seen before, against the planned sweep: 8
-// particles 15.0 -> 11.7 us, 12 18.1 -> 14.5, 16 35.6 -> 17.6, 18 47 -> 19,
-// 20 45 -> 23, 24 98 -> 61 (of it 55 us of FP64 issue); 20 in 15 of 40
-// modes 49 -> 20.  The kernel takes 5.5 us at 8 particles (one wave) and
-// 12 at 18, of it about 3 for the blocks' meeting.
+// A call, against the planned sweep with occupations not seen before and with
+// its plan kept: 8 particles 15.0 and 11.2 -> 10.3 us, 12 18.1 and 13.5 ->
+// 12.5, 16 35.6 and 30 -> 16.3, 24 98 and 95 -> 61 (of it 55 us of FP64
+// issue); 20 in 15 of 40 modes 49 and 43 -> 20.  Bunched on both sides, plan
+// kept: [20, 20] in both 15.7 -> 13.0 us, [8, 8, 8] 18.3 -> 13.4, 36 in 9 and
+// 18 modes 57 -> 42.  (With lanes of at most 64 states of whole digits, inner
+// digits that left waves idle, powers by a masked pass for every multiplicity
+// and binomials by a loop these took 47, 38 and 70.)  The kernel takes 4.7 us
+// at 8 particles (one wave) and 12 at 18, of it about 3 for the blocks'
+// meeting.
 //
 // Compiled once per type of the rows: -DPQP_ONE_FP32=0, 1.
 #include <hip/hip_runtime.h>
@@ -53,10 +60,12 @@ using Real = float;
 using Real = double;
 #endif
 
-// The product over the columns of one state's row sums.
-template <int W, bool ONES>
-__device__ __forceinline__ void one_product(const Real (&cr)[W], const Real (&ci)[W], cptr<uint32_t> over,
-                                            int cmax, Real &pr, Real &pi) {
+// The product over the columns of one state's row sums, in two chains of
+// multiplies (even and odd columns).  more: the columns' further powers, a
+// byte each.
+template <int W, OneKind KIND>
+__device__ __forceinline__ void one_product(const Real (&cr)[W], const Real (&ci)[W],
+                                            const uint32_t (&more)[kOneMaxWidth / 4], Real &pr, Real &pi) {
   Real ar = cr[0], ai = ci[0];
   if constexpr (W > 1) {
     Real br = cr[1], bi = ci[1];
@@ -66,37 +75,59 @@ __device__ __forceinline__ void one_product(const Real (&cr)[W], const Real (&ci
       cmul(br, bi, cr[j + 1], ci[j + 1]);
     }
     if constexpr (W % 2 == 1 && W > 2) cmul(ar, ai, cr[W - 1], ci[W - 1]);
-    cmul(ar, ai, br, bi);
-  }
-  if constexpr (!ONES) {
-    for (int r = 2; r <= cmax; ++r) {
-      const uint32_t cols = over[r - 2];
+    if constexpr (KIND == kOneAny) {
 #pragma unroll
-      for (int j = 0; j < W; ++j) {
-        if ((cols >> j) & 1u) {
-          __asm__ volatile("");  // a branch, not a masked multiply at every column
+      for (int j = 0; j < W; j += 2) {
+        int qa = (more[j / 4] >> (8 * (j % 4))) & 255;
+        int qb = 0;
+        if (j + 1 < W) qb = (more[(j + 1) / 4] >> (8 * ((j + 1) % 4))) & 255;
+        const int jb = j + 1 < W ? j + 1 : j;
+        for (; qa > 0 && qb > 0; --qa, --qb) {
           cmul(ar, ai, cr[j], ci[j]);
+          cmul(br, bi, cr[jb], ci[jb]);
         }
+        for (; qa > 0; --qa) cmul(ar, ai, cr[j], ci[j]);
+        for (; qb > 0; --qb) cmul(br, bi, cr[jb], ci[jb]);
       }
     }
+    cmul(ar, ai, br, bi);
+  } else if constexpr (KIND == kOneAny) {
+    for (int q = more[0] & 255; q > 0; --q) cmul(ar, ai, cr[0], ci[0]);
   }
   pr = ar;
   pi = ai;
 }
 
-// u's lowest digit of radix rho + 1, taken off u (u < 2^50: the quotient is
-// exact this way).
-__device__ __forceinline__ int one_digit(int &u, int rho) {
-  const int q = static_cast<int>((static_cast<double>(u) + 0.5) * kInvSmall[rho + 1]);
-  const int g = u - q * (rho + 1);
+// u's lowest digit of radix r (inv: 1 / r), taken off u (u < 2^50: the
+// quotient is exact this way).
+__device__ __forceinline__ int one_digit(int &u, int r, double inv) {
+  const int q = static_cast<int>((static_cast<double>(u) + 0.5) * inv);
+  const int g = u - q * r;
   u = q;
   return g;
 }
 
-// C(rho, g), the small ones without a loop.
-__device__ __forceinline__ double one_binomial(int rho, int g) {
-  if (rho <= 3) return (g == 0 || g == rho) ? 1.0 : static_cast<double>(rho);
-  return lane_binomial(rho, g);
+// C(rho, g), g <= rho <= 64, rounded once (exact up to 2^53), at rho (rho +
+// 1) / 2 + g: read where a loop of rho rounded quotients took 2 us for a digit
+// of 20 particles.
+struct Binomials {
+  double c[65 * 66 / 2];
+};
+constexpr Binomials binomials() {
+  Binomials t{};
+  uint64_t row[66] = {1};
+  for (int rho = 0; rho <= 64; ++rho) {
+    for (int g = 0; g <= rho; ++g) t.c[rho * (rho + 1) / 2 + g] = static_cast<double>(row[g]);
+    for (int g = rho + 1; g >= 1; --g) row[g] += row[g - 1];
+  }
+  return t;
+}
+__constant__ Binomials kBinomials = binomials();
+
+// The digit's C(rho, g), the small ones from its packed bytes.
+__device__ __forceinline__ double one_binomial(uint64_t choose, int rho, int g) {
+  if (choose) return static_cast<double>(static_cast<uint32_t>(choose >> (8 * min(g, rho - g))) & 255u);
+  return kBinomials.c[rho * (rho + 1) / 2 + g];
 }
 
 // The sum over a block of nw waves, in the lanes 0..7 of wave 0.
@@ -123,13 +154,14 @@ __device__ __forceinline__ void block_sum(cdd &s, double &mag, double (&part)[kO
 using OneRowsHost = decltype(OneArgs::rows);
 
 // The kernel's part of the arguments.
-template <int W, bool FEW>
-using Rows = OneRows<one_row_bytes(FEW ? kOneFew : kOneMaxRows, W, sizeof(Real))>;
-template <int W, bool FEW>
-using Args = std::conditional_t<FEW, Rows<W, FEW>, OneArgsOf<sizeof(Rows<W, FEW>::b)>>;
+template <int W, OneKind KIND>
+using Rows = OneRows<one_row_bytes(KIND == kOneUnit ? W : kOneMaxRows, W, sizeof(Real))>;
+template <int W, OneKind KIND>
+using Args = std::conditional_t<KIND == kOneUnit, Rows<W, KIND>, OneArgsOf<sizeof(Rows<W, KIND>::b)>>;
 
-template <int W, bool ONES, bool FEW>
-__global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW> given) {
+template <int W, OneKind KIND>
+__global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, KIND> given) {
+  constexpr bool kUnit = KIND == kOneUnit;
   const int nw = static_cast<int>(blockDim.x) / kWave;
   __shared__ double part[kOneWaves][5];
   __shared__ Real base[kOneWaves][2 * W];
@@ -140,7 +172,7 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
   const uintptr_t all = reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
   uintptr_t self = all;  // the rows and their head
   const OneHead *head;
-  if constexpr (FEW) {
+  if constexpr (kUnit) {
     head = &given.h;
   } else {
     head = &given.rows.h;
@@ -149,14 +181,23 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
   const OneHead &args = *head;
   const cptr<Real> rows = reinterpret_cast<cptr<Real>>(self + offsetof(OneRowsHost, b));
   const Real *vrows = reinterpret_cast<const Real *>(self + offsetof(OneRowsHost, b));
-  const cptr<uint32_t> over = reinterpret_cast<cptr<uint32_t>>(all + offsetof(OneTables, over));
-  const cptr<int32_t> lane_rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneHead, lane_rho));
-  const cptr<int32_t> rho = reinterpret_cast<cptr<int32_t>>(self + offsetof(OneHead, rho));
-  const cptr<OneStep> step = reinterpret_cast<cptr<OneStep>>(all + offsetof(OneTables, step));
-  const int n = args.n, k = args.inner, rest = args.rest, cmax = args.cmax;
-  const int L = args.lane_digits, S = args.S, chunks = args.chunks;
-  const bool active = lane < args.lanes;
-  const bool binary = FEW || args.binary;
+  // (of kind kOneUnit, not read)
+  const cptr<OneTables> tables = reinterpret_cast<cptr<OneTables>>(all);
+  const cptr<OneDigit> lane_digit = tables->lane, digit = tables->digit;
+  uint32_t more[kOneMaxWidth / 4] = {};
+  if constexpr (KIND == kOneAny) {
+#pragma unroll
+    for (int k = 0; k < (W + 3) / 4; ++k) more[k] = tables->more[k];
+  }
+  const int n = args.n, k = args.inner, rest = args.rest;
+  const int L = args.lane_digits, P = args.lanes, S = args.S, chunks = args.chunks;
+  bool binary = true, lane_binary = true;
+  int lane_chunks = 1;
+  if constexpr (!kUnit) {
+    binary = tables->binary;
+    lane_binary = tables->lane_binary;
+    lane_chunks = tables->lane_chunks;
+  }
   // The first rows common to a wave's lanes, a component per lane: requested
   // before the wave waits for anything else (a first touch costs about a
   // microsecond, and one after another these were most of the start).
@@ -166,29 +207,63 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
 #pragma unroll
   for (int i = 0; i < kOneChunk; ++i) first[i] = vrows[(L + min(i, common - 1)) * (2 * W) + at];
   {
-    // every line of the rows read as scalars, eight loads of a wave in flight
+    // every line of the rows read as scalars, eight loads of a wave in
+    // flight, and of the digits
     const cptr<uint32_t> lines = reinterpret_cast<cptr<uint32_t>>(self + offsetof(OneRowsHost, b));
     const int end = ((L + 1 + k) * 2 * W * static_cast<int>(sizeof(Real)) - 1) / 64;
-    for (int l = bw; l <= end; l += 8 * nw) {
-      const uint32_t v0 = lines[16 * l], v1 = lines[16 * min(l + nw, end)];
-      const uint32_t v2 = lines[16 * min(l + 2 * nw, end)], v3 = lines[16 * min(l + 3 * nw, end)];
-      const uint32_t v4 = lines[16 * min(l + 4 * nw, end)], v5 = lines[16 * min(l + 5 * nw, end)];
-      const uint32_t v6 = lines[16 * min(l + 6 * nw, end)], v7 = lines[16 * min(l + 7 * nw, end)];
-      __asm__ volatile("" ::"s"(v0), "s"(v1), "s"(v2), "s"(v3), "s"(v4), "s"(v5), "s"(v6), "s"(v7));
+    auto line = [&](int l) { return lines[16 * min(l, end)]; };
+    const uint32_t v0 = line(bw), v1 = line(bw + nw), v2 = line(bw + 2 * nw), v3 = line(bw + 3 * nw);
+    const uint32_t v4 = line(bw + 4 * nw), v5 = line(bw + 5 * nw), v6 = line(bw + 6 * nw), v7 = line(bw + 7 * nw);
+    if constexpr (!kUnit) {
+      const cptr<uint32_t> d = reinterpret_cast<cptr<uint32_t>>(tables);
+      const uint32_t d0 = d[0], d1 = d[16], d2 = d[32], d3 = d[48], d4 = d[64], d5 = d[80], d6 = d[96], d7 = d[112];
+      const uint32_t d8 = d[128], d9 = d[144], d10 = d[160], d11 = d[176], d12 = d[192];
+      static_assert(offsetof(OneTables, step) <= 13 * 64);
+      __asm__ volatile("" ::"s"(d0), "s"(d1), "s"(d2), "s"(d3), "s"(d4), "s"(d5), "s"(d6), "s"(d7), "s"(d8), "s"(d9),
+                       "s"(d10), "s"(d11), "s"(d12));
+    }
+    __asm__ volatile("" ::"s"(v0), "s"(v1), "s"(v2), "s"(v3), "s"(v4), "s"(v5), "s"(v6), "s"(v7));
+    for (int l = bw + 8 * nw; l <= end; l += 8 * nw) {
+      const uint32_t w0 = line(l), w1 = line(l + nw), w2 = line(l + 2 * nw), w3 = line(l + 3 * nw);
+      const uint32_t w4 = line(l + 4 * nw), w5 = line(l + 5 * nw), w6 = line(l + 6 * nw), w7 = line(l + 7 * nw);
+      __asm__ volatile("" ::"s"(w0), "s"(w1), "s"(w2), "s"(w3), "s"(w4), "s"(w5), "s"(w6), "s"(w7));
     }
   }
   if (nw > 1) __syncthreads();
 
   cdd sum = cdd_zero();
   double mag = 0.0;  // of the terms: |Re| + |Im| each
+  // the lane's signed weight in a set of lane states
+  auto lane_weight = [&](int at) {
+    if (lane_binary) return __builtin_popcount(at) & 1 ? -1.0 : 1.0;
+    double w = 1.0;
+    int u = at, parity = 0;
+    for (int t = 0; t < L; ++t) {
+      const int rr = lane_digit[t].rho;
+      const int g = one_digit(u, rr + 1, lane_digit[t].inv);
+      parity ^= g & 1;
+      w *= one_binomial(lane_digit[t].choose, rr, g);
+    }
+    return parity ? -w : w;
+  };
+  int held = 0;  // the set that lane_w belongs to
+  double lane_w = lane < P ? lane_weight(lane) : 0.0;
   for (int chunk = wave; chunk < chunks; chunk += waves) {
     Real cr[W], ci[W];
-    double w = 1.0;
+    int u = chunk, set = 0;
+    if (lane_chunks > 1) {
+      set = __builtin_amdgcn_readfirstlane(one_digit(u, lane_chunks, tables->lane_inv));
+      if (set != held) {
+        const int v = kWave * set + lane;
+        lane_w = v < P ? lane_weight(v) : 0.0;
+        held = set;
+      }
+    }
+    double w = lane_w;
     int parity = 0;
     // the rows common to the lanes: the prepended one, the inner ones at
     // their first state, then the rest digits
     double b = 0.0;
-    int u = chunk;
     for (int c0 = 0; c0 < common; c0 += kOneChunk) {
       Real v[kOneChunk];
 #pragma unroll
@@ -198,13 +273,21 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
       for (int i = 0; i < kOneChunk; ++i) {
         const int t = c0 + i - 1;
         if (t < k + rest) {
-          double al = t < 0 ? 1.0 : rho[t];
-          if (t >= k) {
-            const int rr = rho[t];
-            const int g = one_digit(u, rr);
+          double al = 1.0;
+          if constexpr (kUnit) {
+            if (t >= k) {
+              al = (u & 1) ? -1.0 : 1.0;
+              parity ^= u & 1;
+              u >>= 1;
+            }
+          } else if (t >= k) {
+            const int rr = digit[t].rho;
+            const int g = one_digit(u, rr + 1, digit[t].inv);
             parity ^= g & 1;
-            w *= one_binomial(rr, g);
+            w *= one_binomial(digit[t].choose, rr, g);
             al = static_cast<double>(rr - 2 * g);
+          } else if (t >= 0) {
+            al = digit[t].rho;
           }
           b = fmaR(al, static_cast<double>(v[i]), b);
         }
@@ -219,20 +302,17 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
       ci[j] = base[bw][2 * j + 1];
     }
     __builtin_amdgcn_wave_barrier();
-    u = lane;
+    u = kWave * set + lane;
 #pragma unroll 1
     for (int t = 0; t < L; ++t) {
-      const int rr = lane_rho[t];
       Real al;
+      int rr = 1;
+      if constexpr (!kUnit) rr = lane_digit[t].rho;
       if (rr == 1) {
         al = (u & 1) ? Real(-1) : Real(1);
-        parity ^= u & 1;
         u >>= 1;
       } else {
-        const int g = one_digit(u, rr);
-        parity ^= g & 1;
-        w *= one_binomial(rr, g);
-        al = static_cast<Real>(rr - 2 * g);
+        al = static_cast<Real>(rr - 2 * one_digit(u, rr + 1, lane_digit[t].inv));
       }
       const cptr<Real> row = rows + t * (2 * W);
 #pragma unroll
@@ -241,7 +321,6 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
         ci[j] = fmaR(al, row[2 * j + 1], ci[j]);
       }
     }
-    if (!active) w = 0.0;
     if (parity) w = -w;
     // the inner states in Gray order
     double sr = 0.0, si = 0.0, sa = 0.0;
@@ -254,13 +333,13 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
       Real s2 = in_vgpr(((up >> move) & 1) ? Real(-2) : Real(2));
       double coef = in_vgpr((v & 1) ? -1.0 : 1.0);
       if (!binary) {
-        row = step[v].row;
-        s2 = in_vgpr(static_cast<Real>(step[v].factor));
-        coef = in_vgpr(step[v].coef);
+        row = tables->step[v].row;
+        s2 = in_vgpr(static_cast<Real>(tables->step[v].factor));
+        coef = in_vgpr(tables->step[v].coef);
       }
       const cptr<Real> b = rows + (L + row) * (2 * W);
       Real pr, pi;
-      one_product<W, ONES>(cr, ci, over, cmax, pr, pi);
+      one_product<W, KIND>(cr, ci, more, pr, pi);
       const double dr = static_cast<double>(pr), di = static_cast<double>(pi);
       sr = fmaR(coef, dr, sr);
       si = fmaR(coef, di, si);
@@ -332,38 +411,36 @@ __global__ __launch_bounds__(kWave * kOneWaves) void perm_one_kernel(Args<W, FEW
 
 // The kernel copies its own length of the arguments: they begin alike for
 // every width.
-template <int W, bool ONES, bool FEW>
+template <int W, OneKind KIND>
 static hipError_t one_launch(const OneArgs &a, dim3 grid, dim3 block, hipStream_t stream) {
-  using R = Rows<W, FEW>;
-  static_assert(offsetof(R, b) == offsetof(OneRowsHost, b) && sizeof(Args<W, FEW>) <= sizeof(OneArgs));
-  void *p[] = {const_cast<void *>(FEW ? static_cast<const void *>(&a.rows) : static_cast<const void *>(&a))};
-  return hipLaunchKernel(reinterpret_cast<const void *>(perm_one_kernel<W, ONES, FEW>), grid, block, p, 0, stream);
+  using R = Rows<W, KIND>;
+  static_assert(offsetof(R, b) == offsetof(OneRowsHost, b) && sizeof(Args<W, KIND>) <= sizeof(OneArgs));
+  const void *given = KIND == kOneUnit ? static_cast<const void *>(&a.rows) : static_cast<const void *>(&a);
+  void *p[] = {const_cast<void *>(given)};
+  return hipLaunchKernel(reinterpret_cast<const void *>(perm_one_kernel<W, KIND>), grid, block, p, 0, stream);
+}
+
+template <int W>
+static hipError_t one_launch(OneKind kind, const OneArgs &a, dim3 grid, dim3 block, hipStream_t stream) {
+  if (kind == kOneUnit) return one_launch<W, kOneUnit>(a, grid, block, stream);
+  if (kind == kOneOnes) return one_launch<W, kOneOnes>(a, grid, block, stream);
+  return one_launch<W, kOneAny>(a, grid, block, stream);
 }
 
 #if PQP_ONE_FP32
-hipError_t launch_one_f(int width, bool ones, bool few, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
+hipError_t launch_one_f(int width, OneKind kind, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
 #else
-hipError_t launch_one_d(int width, bool ones, bool few, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
+hipError_t launch_one_d(int width, OneKind kind, const OneArgs &a, int blocks, int waves, hipStream_t stream) {
 #endif
   const OneHead &h = a.rows.h;
-  if (blocks < 1 || waves < 1 || waves > kOneWaves || h.n < 1 || h.chunks < 1) return hipErrorInvalidValue;
-  if (few && (!ones || !h.binary || 1 + h.lane_digits + h.inner + h.rest > kOneFew)) return hipErrorInvalidValue;
+  if (blocks < 1 || blocks > kOneMaxBlocks || waves < 1 || waves > kOneWaves || h.n < 1 || h.chunks < 1)
+    return hipErrorInvalidValue;
+  if (kind == kOneUnit && (width != h.n || 1 + h.lane_digits + h.inner + h.rest != width)) return hipErrorInvalidValue;
   const dim3 grid(blocks), block(kWave * waves);
-  if (few) {
-    switch (width) {
-#define X(W) \
-  case W:    \
-    return one_launch<W, true, true>(a, grid, block, stream);
-      X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
-#undef X
-      default:
-        return hipErrorInvalidValue;
-    }
-  }
   switch (width) {
 #define X(W) \
   case W:    \
-    return ones ? one_launch<W, true, false>(a, grid, block, stream) : one_launch<W, false, false>(a, grid, block, stream);
+    return one_launch<W>(kind, a, grid, block, stream);
     X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
     X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20) X(21) X(22) X(23) X(24)
 #undef X
