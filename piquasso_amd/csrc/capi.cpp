@@ -1311,7 +1311,12 @@ struct TensorState {
   hipStream_t stream = nullptr;
   DevBuf in, work, out;
   HostBuf stage;
+  MappedBuf res;  // results of few items
 };
+
+// Items whose results the kernel writes to host memory (a copy of a few would
+// cost a launch more than it moves: 5 us a call).
+constexpr size_t kTensorMapped = 4096;
 
 TensorState &tensor_state() {
   static TensorState *s = new TensorState();  // never destroyed: outlives atexit HIP teardown
@@ -1324,10 +1329,12 @@ constexpr size_t kTensorBytes = size_t{512} << 20;
 // the number of items (a value does not depend on its company): at most 512
 // steps, or as many as keep the units near 2^20 (large n), fewer where that
 // leaves less than about 8192 units, at least 16 (a unit's start costs about
-// four).  Against 4096 units of up to 1024 steps: 15 particles, two outputs
-// 1468 -> 1330 us, 16 particles 3041 -> 2780 us (the last waves run alone
-// for less time); 32768 units cost one output of 14 particles 351 us
-// instead of 237.
+// four), or 8 up to 9 particles, whose few units one output would wait for
+// (9 particles, one output 40 -> 38 us, 300 108; 10 particles, 2000 outputs
+// 1232 us by 16, 1460 by 8).  Against 4096 units of up to 1024 steps: 15
+// particles, two outputs 1468 -> 1330 us, 16 particles 3041 -> 2780 us (the
+// last waves run alone for less time); 32768 units cost one output of 14
+// particles 351 us instead of 237.
 int tensor_walk_bits(int nb, int ls) {
   auto units = [&](int kt) {
     return std::ldexp(1.0, (nb - ls) + (nb - kt)) / 2.0;
@@ -1335,6 +1342,7 @@ int tensor_walk_bits(int nb, int ls) {
   int kt = std::min(nb, 9);
   while (kt < nb && units(kt) > 1048576.0) ++kt;
   while (kt > 4 && units(kt) < 8192.0) --kt;
+  if (kt == 4 && units(kt) <= 32.0) kt = 3;
   return kt;
 }
 
@@ -2344,20 +2352,24 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
     a.n_units = static_cast<int32_t>(units.size());
     const TensorPass t = tensor_pass(nk, static_cast<int64_t>(g1 - g0), units.size());
     const size_t nn = static_cast<size_t>(nk) * nk, most = static_cast<size_t>(t.items);
-    // units, overlaps, then (as in the work buffer) matrices and |A|^2
+    // units, overlaps, matrices and |A|^2, in one copy
     const size_t o_x = align256(units.size() * sizeof(TensorUnit));
     const size_t o_cols = align256(o_x + most * sizeof(double));
     const size_t in_bytes = o_cols + t.signs;
-    if ((st = S.in.ensure(o_cols)) != PQP_OK) return st;
+    if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
     if ((st = S.work.ensure(t.bytes)) != PQP_OK) return st;
-    if ((st = S.out.ensure(most * 2 * sizeof(double))) != PQP_OK) return st;
-    if ((st = S.stage.ensure(std::max(in_bytes, most * 2 * sizeof(double)))) != PQP_OK) return st;
+    const size_t out_bytes = most * 2 * sizeof(double);
+    const bool mapped = most <= kTensorMapped;
+    if ((st = mapped ? S.res.ensure(out_bytes) : S.out.ensure(out_bytes)) != PQP_OK) return st;
+    if ((st = S.stage.ensure(std::max(in_bytes, out_bytes))) != PQP_OK) return st;
     char *h = static_cast<char *>(S.stage.p);
     char *d = static_cast<char *>(S.in.p);
     tensor_buffers(a, t, static_cast<char *>(S.work.p));
+    a.cols = reinterpret_cast<double *>(d + o_cols);
+    a.pw = reinterpret_cast<double *>(d + o_cols + t.pw);
     a.units = reinterpret_cast<const TensorUnit *>(d);
     a.x = reinterpret_cast<const double *>(d + o_x);
-    a.out = static_cast<double *>(S.out.p);
+    a.out = static_cast<double *>(mapped ? S.res.dev : S.out.p);
     for (size_t p0 = g0; p0 < g1; p0 += most) {
       const size_t m = std::min(most, g1 - p0);
       std::memcpy(h, units.data(), units.size() * sizeof(TensorUnit));
@@ -2376,15 +2388,15 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
             pwp[c * nk + i] = y * (re * re + im * im);
           }
       }
-      PQP_HIP(hipMemcpyAsync(d, h, o_cols, hipMemcpyHostToDevice, S.stream));
-      PQP_HIP(hipMemcpyAsync(S.work.p, h + o_cols, t.signs, hipMemcpyHostToDevice, S.stream));
+      PQP_HIP(hipMemcpyAsync(d, h, o_cols + t.pw + m * nn * sizeof(double), hipMemcpyHostToDevice, S.stream));
       a.n_items = static_cast<int32_t>(m);
       PQP_HIP(launch_tensor_signs(a, S.stream));
       PQP_HIP(launch_tensor(a, S.stream));
       PQP_HIP(launch_tensor_finalize(a, S.stream));
-      PQP_HIP(hipMemcpyAsync(h, S.out.p, m * 2 * sizeof(double), hipMemcpyDeviceToHost, S.stream));
+      if (!mapped)
+        PQP_HIP(hipMemcpyAsync(h, S.out.p, m * 2 * sizeof(double), hipMemcpyDeviceToHost, S.stream));
       PQP_HIP(hipStreamSynchronize(S.stream));
-      const double *r = reinterpret_cast<const double *>(h);
+      const double *r = static_cast<const double *>(mapped ? S.res.host : static_cast<void *>(h));
       for (size_t q = 0; q < m; ++q) {
         out[order[p0 + q]] = r[2 * q];
         if (abs_sum) abs_sum[order[p0 + q]] = r[2 * q + 1];

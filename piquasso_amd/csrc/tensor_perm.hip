@@ -39,13 +39,20 @@
 //
 // Tables of many outputs (pqp_overlap_table_c128) send each output's rows
 // of the interferometer instead of its matrix, and tensor_gather_kernel lays
-// the matrices out: 500 outputs of 6 particles 4640 -> 56 us, 2000 of 3
-// 22 ms -> 113 us (the host laid out and sent every matrix).
+// the matrices out: 500 outputs of 6 particles 4640 -> 50 us, 2000 of 3
+// 22 ms -> 59 us (the host laid out and sent every matrix).
+//
+// A lone small permanent is bound by latency: its matrix comes in one copy,
+// short walks touch their lines first, and results of few items are written
+// to host memory.  One of 9 particles, with R_eps in every lane 38.1 us a
+// call, by sign rows at first 49.8, now 38; of 3 30.9, 35.5, 31; 30 of 7
+// particles 92, 107, 91.
 //
 // Compiled twice: -DPQP_TENSOR_PART=0 instantiates n = 1..12 and the other
 // kernels, =1 instantiates n = 13..20.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -71,6 +78,20 @@ __device__ __forceinline__ dd wave_reduce_dd(dd v) {
   return v;
 }
 
+// Every line of `bytes` bytes read as scalars, sixteen loads in flight.
+__device__ __forceinline__ void touch(cptr<uint32_t> lines, int bytes) {
+  const int end = (bytes - 1) / 64;
+  auto line = [&](int l) { return lines[16 * (l < end ? l : end)]; };
+  for (int l = 0; l <= end; l += 16) {
+    const uint32_t v0 = line(l), v1 = line(l + 1), v2 = line(l + 2), v3 = line(l + 3), v4 = line(l + 4);
+    const uint32_t v5 = line(l + 5), v6 = line(l + 6), v7 = line(l + 7), v8 = line(l + 8), v9 = line(l + 9);
+    const uint32_t v10 = line(l + 10), v11 = line(l + 11), v12 = line(l + 12), v13 = line(l + 13);
+    const uint32_t v14 = line(l + 14), v15 = line(l + 15);
+    __asm__ volatile("" ::"s"(v0), "s"(v1), "s"(v2), "s"(v3), "s"(v4), "s"(v5), "s"(v6), "s"(v7), "s"(v8), "s"(v9),
+                     "s"(v10), "s"(v11), "s"(v12), "s"(v13), "s"(v14), "s"(v15));
+  }
+}
+
 // Grid (units, items).
 template <int N>
 __global__ __launch_bounds__(kWave) void tensor_perm_kernel(TensorArgs a) {
@@ -92,6 +113,19 @@ __global__ __launch_bounds__(kWave) void tensor_perm_kernel(TensorArgs a) {
   // sign vectors: column 0 fixed at +1, column b + 1 is -1 where bit b is set
   const uint32_t s = (s_hi << ls) | static_cast<uint32_t>(active ? lane : 0);
   const uint32_t t0 = t_blk << kt;
+
+  // A short walk first touches the lines of its rows of `signs` and of the
+  // columns, all in flight together (a lane each, then as scalars): in a
+  // launch of few waves every step would wait for its own.
+  if ((2 * N << kt) <= 8 * kWave) {
+    const int64_t from = 2 * N * (kStates * item + t0);
+    const int rows = 2 * N << kt, most = N * N;
+    const double v = a.signs[from + min(8 * lane, rows - 1)];
+    const double c = a.pw[static_cast<int64_t>(most) * item + min(8 * lane, most - 1)];
+    __asm__ volatile("" ::"v"(v), "v"(c));
+    touch(as_const<uint32_t>(a.pw, int64_t{8} * most * item), 8 * most);
+    touch(as_const<uint32_t>(a.signs, 8 * from), 8 * rows);
+  }
 
   // x R_delta and (1 - x) Q_{delta eps} at the walk's first eps
   double xr[N], xi[N], q[N];
@@ -249,6 +283,7 @@ __global__ __launch_bounds__(256) void tensor_signs_kernel(TensorArgs a) {
   const int i = static_cast<int>(at - static_cast<int64_t>(t) * n);
   const double2 *col = reinterpret_cast<const double2 *>(a.cols) + static_cast<int64_t>(item) * n * n;
   double2 r = col[i];
+#pragma unroll 4
   for (int c = 1; c < n; ++c) {
     const double2 z = col[c * n + i];
     const bool neg = (t >> (c - 1)) & 1u;
@@ -264,13 +299,13 @@ __global__ __launch_bounds__(256) void tensor_signs_kernel(TensorArgs a) {
 // probability.  Bound by the chain of loads and dd additions of one thread:
 // one wave took 21 us over the 4160 units of n = 14.
 __global__ __launch_bounds__(kTensorFinal) void tensor_finalize_kernel(TensorArgs a) {
-  constexpr int kWaves = kTensorFinal / kWave;
-  __shared__ double part[kWaves][3];
+  const int threads = static_cast<int>(blockDim.x), waves = threads / kWave;
+  __shared__ double part[kTensorFinal / kWave][3];
   const int item = static_cast<int>(blockIdx.x);
   dd s{0.0, 0.0};
   double sa = 0.0;
 #pragma unroll 4
-  for (int u = static_cast<int>(threadIdx.x); u < a.n_units; u += kTensorFinal) {
+  for (int u = static_cast<int>(threadIdx.x); u < a.n_units; u += threads) {
     const double *p = a.partials + 3 * (static_cast<int64_t>(item) * a.n_units + u);
     s = dd_add(s, dd{p[0], p[1]});
     sa += p[2];
@@ -286,7 +321,7 @@ __global__ __launch_bounds__(kTensorFinal) void tensor_finalize_kernel(TensorArg
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < kWaves; ++w) {
+    for (int w = 1; w < waves; ++w) {
       s = dd_add(s, dd{part[w][0], part[w][1]});
       sa += part[w][2];
     }
@@ -338,7 +373,8 @@ hipError_t launch_tensor_signs(const TensorArgs &a, hipStream_t stream) {
 }
 
 hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream) {
-  hipLaunchKernelGGL(tensor_finalize_kernel, dim3(a.n_items), dim3(kTensorFinal), 0, stream, a);
+  const int waves = std::min((a.n_units + kWave - 1) / kWave, kTensorFinal / kWave);  // no idle ones to wait for
+  hipLaunchKernelGGL(tensor_finalize_kernel, dim3(a.n_items), dim3(kWave * waves), 0, stream, a);
   return hipGetLastError();
 }
 #endif
