@@ -136,8 +136,8 @@ constexpr int64_t kSampleShots = 2048;
 constexpr int64_t kIntWaves = 4096;
 constexpr int kIntInnerDigits = 7;
 // Bytes of a polynomial permanent's exponent rows that are compared with the
-// kept plan's before anything runs (8 us).
-constexpr size_t kPolyCompareFirst = size_t{256} << 10;
+// kept plan's before anything runs (3 us).
+constexpr size_t kPolyCompareFirst = size_t{64} << 10;
 // Outputs up to which 6 and 7 particles take the subset sum.
 constexpr size_t kPolyFew6 = 64, kPolyFew7 = 4;
 // Device buffers one-shot batches may leave for the next ones, and how many
@@ -2340,44 +2340,39 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
       out[k] = 1.0;
       if (abs_sum) abs_sum[k] = 1.0;
     }
-  std::vector<TensorUnit> units;
-  for (size_t g0 = 0; g0 < order.size();) {
-    const int nk = static_cast<int>(n[order[g0]]);
-    size_t g1 = g0;
-    while (g1 < order.size() && n[order[g1]] == nk) ++g1;
+  // Passes of one order each, and flights of passes that fit the work buffer
+  // together: one copy in, one wait.
+  struct Pass {
     TensorArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.n = nk;
-    tensor_units(nk, &a.ls, &a.kt, units);
-    a.n_units = static_cast<int32_t>(units.size());
-    const TensorPass t = tensor_pass(nk, static_cast<int64_t>(g1 - g0), units.size());
-    const size_t nn = static_cast<size_t>(nk) * nk, most = static_cast<size_t>(t.items);
-    // units, overlaps, matrices and |A|^2, in one copy
-    const size_t o_x = align256(units.size() * sizeof(TensorUnit));
-    const size_t o_cols = align256(o_x + most * sizeof(double));
-    const size_t in_bytes = o_cols + t.signs;
+    TensorPass t;
+    const std::vector<TensorUnit> *units;
+    size_t first, items;               // in `order`
+    size_t o_units, o_x, o_cols, work, result;  // offsets of the flight's buffers (results in items)
+  };
+  std::vector<TensorUnit> units[kTensorMaxN + 1];
+  std::vector<Pass> flight;
+  size_t in_bytes = 0, work_bytes = 0, items = 0;
+  auto run = [&]() -> int {
+    if (flight.empty()) return PQP_OK;
+    const size_t out_bytes = items * 2 * sizeof(double);
+    const bool mapped = items <= kTensorMapped;
+    int st;
     if ((st = S.in.ensure(in_bytes)) != PQP_OK) return st;
-    if ((st = S.work.ensure(t.bytes)) != PQP_OK) return st;
-    const size_t out_bytes = most * 2 * sizeof(double);
-    const bool mapped = most <= kTensorMapped;
+    if ((st = S.work.ensure(work_bytes)) != PQP_OK) return st;
     if ((st = mapped ? S.res.ensure(out_bytes) : S.out.ensure(out_bytes)) != PQP_OK) return st;
     if ((st = S.stage.ensure(std::max(in_bytes, out_bytes))) != PQP_OK) return st;
     char *h = static_cast<char *>(S.stage.p);
     char *d = static_cast<char *>(S.in.p);
-    tensor_buffers(a, t, static_cast<char *>(S.work.p));
-    a.cols = reinterpret_cast<double *>(d + o_cols);
-    a.pw = reinterpret_cast<double *>(d + o_cols + t.pw);
-    a.units = reinterpret_cast<const TensorUnit *>(d);
-    a.x = reinterpret_cast<const double *>(d + o_x);
-    a.out = static_cast<double *>(mapped ? S.res.dev : S.out.p);
-    for (size_t p0 = g0; p0 < g1; p0 += most) {
-      const size_t m = std::min(most, g1 - p0);
-      std::memcpy(h, units.data(), units.size() * sizeof(TensorUnit));
-      for (size_t q = 0; q < m; ++q) {
-        const int64_t k = order[p0 + q];
-        reinterpret_cast<double *>(h + o_x)[q] = overlap[k];
-        double *colp = reinterpret_cast<double *>(h + o_cols) + q * nn * 2;
-        double *pwp = reinterpret_cast<double *>(h + o_cols + t.pw) + q * nn;
+    for (Pass &p : flight) {
+      TensorArgs &a = p.a;
+      const int nk = a.n;
+      const size_t nn = static_cast<size_t>(nk) * nk;
+      std::memcpy(h + p.o_units, p.units->data(), p.units->size() * sizeof(TensorUnit));
+      for (size_t q = 0; q < p.items; ++q) {
+        const int64_t k = order[p.first + q];
+        reinterpret_cast<double *>(h + p.o_x)[q] = overlap[k];
+        double *colp = reinterpret_cast<double *>(h + p.o_cols) + q * nn * 2;
+        double *pwp = reinterpret_cast<double *>(h + p.o_cols + p.t.pw) + q * nn;
         const double y = 1.0 - overlap[k];
         for (int c = 0; c < nk; ++c)
           for (int i = 0; i < nk; ++i) {
@@ -2388,23 +2383,59 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
             pwp[c * nk + i] = y * (re * re + im * im);
           }
       }
-      PQP_HIP(hipMemcpyAsync(d, h, o_cols + t.pw + m * nn * sizeof(double), hipMemcpyHostToDevice, S.stream));
-      a.n_items = static_cast<int32_t>(m);
-      PQP_HIP(launch_tensor_signs(a, S.stream));
-      PQP_HIP(launch_tensor(a, S.stream));
-      PQP_HIP(launch_tensor_finalize(a, S.stream));
-      if (!mapped)
-        PQP_HIP(hipMemcpyAsync(h, S.out.p, m * 2 * sizeof(double), hipMemcpyDeviceToHost, S.stream));
-      PQP_HIP(hipStreamSynchronize(S.stream));
-      const double *r = static_cast<const double *>(mapped ? S.res.host : static_cast<void *>(h));
-      for (size_t q = 0; q < m; ++q) {
-        out[order[p0 + q]] = r[2 * q];
-        if (abs_sum) abs_sum[order[p0 + q]] = r[2 * q + 1];
-      }
+      tensor_buffers(a, p.t, static_cast<char *>(S.work.p) + p.work);
+      a.cols = reinterpret_cast<double *>(d + p.o_cols);
+      a.pw = reinterpret_cast<double *>(d + p.o_cols + p.t.pw);
+      a.units = reinterpret_cast<const TensorUnit *>(d + p.o_units);
+      a.x = reinterpret_cast<const double *>(d + p.o_x);
+      a.out = static_cast<double *>(mapped ? S.res.dev : S.out.p) + 2 * p.result;
     }
-    g0 = g1;
+    PQP_HIP(hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, S.stream));
+    for (const Pass &p : flight) {
+      PQP_HIP(launch_tensor_signs(p.a, S.stream));
+      PQP_HIP(launch_tensor(p.a, S.stream));
+      PQP_HIP(launch_tensor_finalize(p.a, S.stream));
+    }
+    if (!mapped) PQP_HIP(hipMemcpyAsync(h, S.out.p, out_bytes, hipMemcpyDeviceToHost, S.stream));
+    PQP_HIP(hipStreamSynchronize(S.stream));
+    const double *r = static_cast<const double *>(mapped ? S.res.host : static_cast<void *>(h));
+    for (const Pass &p : flight)
+      for (size_t q = 0; q < p.items; ++q) {
+        out[order[p.first + q]] = r[2 * (p.result + q)];
+        if (abs_sum) abs_sum[order[p.first + q]] = r[2 * (p.result + q) + 1];
+      }
+    flight.clear();
+    in_bytes = work_bytes = items = 0;
+    return PQP_OK;
+  };
+  for (size_t at = 0; at < order.size();) {
+    const int nk = static_cast<int>(n[order[at]]);
+    size_t end = at;
+    while (end < order.size() && n[order[end]] == nk) ++end;
+    Pass p;
+    std::memset(&p.a, 0, sizeof(p.a));
+    p.a.n = nk;
+    if (units[nk].empty()) tensor_units(nk, &p.a.ls, &p.a.kt, units[nk]);
+    p.units = &units[nk];
+    p.a.n_units = static_cast<int32_t>(units[nk].size());
+    for (; at < end; at += p.items) {
+      p.t = tensor_pass(nk, static_cast<int64_t>(end - at), units[nk].size());
+      p.first = at;
+      p.items = static_cast<size_t>(p.t.items);
+      p.a.n_items = static_cast<int32_t>(p.items);
+      if (work_bytes + p.t.bytes > kTensorBytes && (st = run()) != PQP_OK) return st;
+      p.o_units = in_bytes;
+      p.o_x = align256(p.o_units + units[nk].size() * sizeof(TensorUnit));
+      p.o_cols = align256(p.o_x + p.items * sizeof(double));
+      in_bytes = align256(p.o_cols + p.t.signs);
+      p.work = work_bytes;
+      work_bytes = align256(work_bytes + p.t.bytes);
+      p.result = items;
+      items += p.items;
+      flight.push_back(p);
+    }
   }
-  return PQP_OK;
+  return run();
 }
 
 int pqp_overlap_table_c128(const double *matrix, int64_t modes, int64_t ld, const int32_t *input,

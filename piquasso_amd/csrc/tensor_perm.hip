@@ -42,11 +42,12 @@
 // the matrices out: 500 outputs of 6 particles 4640 -> 50 us, 2000 of 3
 // 22 ms -> 59 us (the host laid out and sent every matrix).
 //
-// A lone small permanent is bound by latency: its matrix comes in one copy,
-// short walks touch their lines first, and results of few items are written
-// to host memory.  One of 9 particles, with R_eps in every lane 38.1 us a
-// call, by sign rows at first 49.8, now 38; of 3 30.9, 35.5, 31; 30 of 7
-// particles 92, 107, 91.
+// A lone small permanent is bound by latency: the matrices of all orders come
+// in one copy, short walks touch their lines first, an only unit writes its
+// item's result, and results of few items go to host memory.  One of 9
+// particles, with R_eps in every lane 38.1 us a call, by sign rows at first
+// 49.8, now 38; of 3 30.9, 35.5, 29; 30 of 7 particles 92, 107, 91; 60 of
+// five orders 186, 240, 190.
 //
 // Compiled twice: -DPQP_TENSOR_PART=0 instantiates n = 1..12 and the other
 // kernels, =1 instantiates n = 13..20.
@@ -76,6 +77,19 @@ __device__ __forceinline__ dd wave_reduce_dd(dd v) {
     v = dd_add(v, o);
   }
   return v;
+}
+
+// An item's result from its units' sum and their |term| sum: T = hi + lo by
+// Glynn's scale 4^-(n-1) (exact), for a table the probability.
+__device__ __forceinline__ void tensor_result(const TensorArgs &a, int item, dd s, double sa) {
+  const int e = -2 * (a.n - 1);
+  const double t = ldexp(s.hi + s.lo, e);
+  if (a.prob) {
+    a.prob[item] = t / a.norm[item];
+  } else {
+    a.out[2 * item] = t;
+    a.out[2 * item + 1] = ldexp(sa, e);
+  }
 }
 
 // Every line of `bytes` bytes read as scalars, sixteen loads in flight.
@@ -247,11 +261,17 @@ __global__ __launch_bounds__(kWave) void tensor_perm_kernel(TensorArgs a) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) aabs += __shfl_xor(aabs, off);
   if (lane == 0) {
-    double *p = a.partials + 3 * (static_cast<int64_t>(item) * a.n_units + blockIdx.x);
     // twice: the sum counts each pair with its conjugate
-    p[0] = 2.0 * acc_dd.hi;
-    p[1] = 2.0 * acc_dd.lo;
-    p[2] = 2.0 * aabs;
+    acc_dd = dd{2.0 * acc_dd.hi, 2.0 * acc_dd.lo};
+    aabs *= 2.0;
+    if (a.n_units == 1) {  // the item's only unit
+      tensor_result(a, item, acc_dd, aabs);
+      return;
+    }
+    double *p = a.partials + 3 * (static_cast<int64_t>(item) * a.n_units + blockIdx.x);
+    p[0] = acc_dd.hi;
+    p[1] = acc_dd.lo;
+    p[2] = aabs;
   }
 }
 
@@ -294,10 +314,10 @@ __global__ __launch_bounds__(256) void tensor_signs_kernel(TensorArgs a) {
 }
 
 // One block per item: the dd sum of the item's unit partials (strided over
-// the threads, a fixed butterfly in each wave, then the waves in order),
-// T = hi + lo, and the sum of the units' |term| sums; for a table, the
-// probability.  Bound by the chain of loads and dd additions of one thread:
-// one wave took 21 us over the 4160 units of n = 14.
+// the threads, a fixed butterfly in each wave, then the waves in order), and
+// its result; items of one unit have written theirs.  Bound by the chain of
+// loads and dd additions of one thread: one wave took 21 us over the 4160
+// units of n = 14.
 __global__ __launch_bounds__(kTensorFinal) void tensor_finalize_kernel(TensorArgs a) {
   const int threads = static_cast<int>(blockDim.x), waves = threads / kWave;
   __shared__ double part[kTensorFinal / kWave][3];
@@ -325,15 +345,7 @@ __global__ __launch_bounds__(kTensorFinal) void tensor_finalize_kernel(TensorArg
       s = dd_add(s, dd{part[w][0], part[w][1]});
       sa += part[w][2];
     }
-    // Glynn scale 4^-(n-1) (exact)
-    const int e = -2 * (a.n - 1);
-    const double t = ldexp(s.hi + s.lo, e);
-    if (a.prob) {
-      a.prob[item] = t / a.norm[item];
-    } else {
-      a.out[2 * item] = t;
-      a.out[2 * item + 1] = ldexp(sa, e);
-    }
+    tensor_result(a, item, s, sa);
   }
 }
 #endif
@@ -373,6 +385,7 @@ hipError_t launch_tensor_signs(const TensorArgs &a, hipStream_t stream) {
 }
 
 hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream) {
+  if (a.n_units == 1) return hipSuccess;
   const int waves = std::min((a.n_units + kWave - 1) / kWave, kTensorFinal / kWave);  // no idle ones to wait for
   hipLaunchKernelGGL(tensor_finalize_kernel, dim3(a.n_items), dim3(kWave * waves), 0, stream, a);
   return hipGetLastError();

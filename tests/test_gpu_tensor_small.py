@@ -32,3 +32,16 @@ def test_short_walks_match_oracle(gpu, oracle, n):
     for a, v, g in zip(mats, x, got):
         ref, asum = oracle.tensor_perm_dd(a, v)
         assert abs(g - ref.real) <= _tol(n, asum, ref.real)
+
+
+@pytest.mark.parametrize("orders", [
+    [2, 3], [9, 2, 5, 5, 1, 0, 7, 3, 3, 4], [17] * 20 + [18] * 6,  # the last: more than one flight of buffers
+])
+def test_mixed_orders_are_the_same_alone(gpu, orders):
+    mats = [_rand(n, 7 * k + n) if n else np.zeros((0, 0), dtype=complex) for k, n in enumerate(orders)]
+    x = [0.05 * (k % 20) for k in range(len(orders))]
+    print(f"tensor orders {orders[:4]}..", flush=True)
+    got, asum = pa.tensor_permanent_batch(mats, x, with_abs_sum=True)
+    for k in sorted({0, 1, len(orders) // 2, len(orders) - 1}):
+        (one,), (s,) = pa.tensor_permanent_batch([mats[k]], [x[k]], with_abs_sum=True)
+        assert got[k] == one and asum[k] == s
