@@ -25,3 +25,14 @@ def test_streams_are_created_once():
     code = _code("capi.cpp")
     assert len(re.findall(r"hipStreamCreate", code)) == 1
     assert re.search(r"int ensure_stream\(hipStream_t &stream\) \{\s*if \(!stream\)", code)
+
+
+def test_one_shot_batches_share_no_lock():
+    """A one-shot batch runs on buffers and streams of its own: it takes no
+    lock over its work, so calls of several threads run side by side (when
+    they end also depends on the hardware queues their streams are given)."""
+    code = _code("capi.cpp")
+    at = code.index("int pqp_permanent_batch_c128(")
+    body = code[at: code.index("\n}\n", at)]
+    assert "OneShotLease lease" in body
+    assert "single_state" not in body and "lock_guard" not in body and "unique_lock" not in body
