@@ -393,9 +393,20 @@ __device__ __forceinline__ void finalize_item(const LaunchArgs &a, int item) {
 // small items, 1024 when an item has thousands of units.  Block 0 also
 // rewinds the work-queue heads for the next launch of the same plan.
 // Static launch: block b sweeps unit first_unit + b.
+//
+// The FP32 widths 9..16 keep to seven waves per SIMD by their scalar
+// registers.  Width buckets run side by side, and with eight waves of 64
+// VGPRs the register file is full: a wave that ends leaves 64, too few for
+// one of the next bucket's (80 VGPRs, and a batch's longest items), which
+// then starts when this bucket has drained.  With seven, 64 stay free and a
+// wave that ends makes room for it: 2000 items of 12 to 22 particles 307 us
+// -> 284 us, 4096 of 8 to 24 particles 251 -> 238 us; widths 9..16 alone 210
+// -> 214 us.  (A limit by VGPRs, 72 a wave, leaves no such room: 302-308 us.)
 template <int LO, int HI, typename R, bool COMP>
 __global__ __launch_bounds__(kWave)
 __attribute__((amdgpu_waves_per_eu(waves_for(HI, sizeof(R) == 4), 8))) void perm_static_kernel(LaunchArgs a, int first_unit) {
+  // more than 96 scalar registers: 112 of the SIMD's 800 a wave
+  if constexpr (HI == 16 && sizeof(R) == 4) __asm__ volatile("" ::: "s97");
   const cptr<WorkUnit> wu = as_const<WorkUnit>(a.units) + (first_unit + static_cast<int>(blockIdx.x));
   const int item = uniform(wu->item);
   const int local = uniform(wu->local);
