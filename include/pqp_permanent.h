@@ -374,9 +374,10 @@ int pqp_output_table_c128(const double *matrix, int64_t modes, int64_t ld, const
  * over the 2^n - 1 non-empty column subsets, each subset's product of row
  * factors kept as a polynomial; here on the monomials that divide some e_q
  * (the reference keeps the box of the largest exponent per variable; the
- * kept coefficients are the same).  Orders up to 12 expand the permanent row
- * by row over the column subsets instead, without an alternating sum.  Rows
- * with total degree above n give 0.
+ * kept coefficients are the same).  Orders up to 12 whose layers fit 8 GiB
+ * expand the permanent row by row over the column subsets instead, without an
+ * alternating sum (orders 6 and 7 only from 65 and 5 rows on).  Rows with total
+ * degree above n give 0.
  * info (may be null, 6 entries) describes the subset loop for these rows:
  * monomials, links, workgroups, 1 if its polynomial fits LDS, algorithmic
  * FP64 flops per subset, subsets.

@@ -389,9 +389,6 @@ __device__ __forceinline__ void finalize_item(const LaunchArgs &a, int item) {
   }
 }
 
-// One block of NT threads per item (finalize_item).  NT = 64 for batches of
-// small items, 1024 when an item has thousands of units.  Block 0 also
-// rewinds the work-queue heads for the next launch of the same plan.
 // Static launch: block b sweeps unit first_unit + b.
 //
 // The FP32 widths 9..16 keep to seven waves per SIMD by their scalar
@@ -414,6 +411,9 @@ __attribute__((amdgpu_waves_per_eu(waves_for(HI, sizeof(R) == 4), 8))) void perm
   dispatch<LO, HI, R, COMP, COMP>(a, mcp, item, local);
 }
 
+// One block of NT threads per item (finalize_item).  NT = 64 for batches of
+// small items, 1024 when an item has thousands of units.  Block 0 also
+// rewinds the work-queue heads for the next launch of the same plan.
 template <bool COMP, int NT>
 __global__ __launch_bounds__(NT) void perm_finalize_kernel(LaunchArgs a, int item0, int n_heads) {
   const int item = item0 + static_cast<int>(blockIdx.x);

@@ -30,7 +30,7 @@
 // G = 12 leaves one product per prime where G = 4 has five).  4096 waves (as
 // 2048: the start of a wave costs a third of its 32 states, but twice the
 // states leave half the waves to hide latency).  Measured, 0/1 matrices of
-// density 0.3, two primes, a call and its sweep: n = 24 153 us (87) -> 75 us
+// density 0.3, two primes, a call and its sweep: n = 24 151 us (87) -> 65 us
 // (38); n = 12 58 -> 30 us, copies, planning and two synchronisations gone.
 
 #include <hip/hip_runtime.h>
