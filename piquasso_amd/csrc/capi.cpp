@@ -2391,8 +2391,10 @@ int pqp_tensor_permanent_batch_c128(int64_t count, const double *const *matrices
       a.out = static_cast<double *>(mapped ? S.res.dev : S.out.p) + 2 * p.result;
     }
     PQP_HIP(hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, S.stream));
+    std::vector<TensorArgs> passes;
+    for (const Pass &p : flight) passes.push_back(p.a);
+    PQP_HIP(launch_tensor_signs(passes.data(), static_cast<int>(passes.size()), S.stream));
     for (const Pass &p : flight) {
-      PQP_HIP(launch_tensor_signs(p.a, S.stream));
       PQP_HIP(launch_tensor(p.a, S.stream));
       PQP_HIP(launch_tensor_finalize(p.a, S.stream));
     }
@@ -2531,7 +2533,7 @@ int pqp_overlap_table_c128(const double *matrix, int64_t modes, int64_t ld, cons
     a.norm = reinterpret_cast<const double *>(d + o_norm) + p0;
     a.prob = static_cast<double *>(S.out.p) + p0;
     PQP_HIP(launch_tensor_gather(a, S.stream));
-    PQP_HIP(launch_tensor_signs(a, S.stream));
+    PQP_HIP(launch_tensor_signs(&a, 1, S.stream));
     PQP_HIP(launch_tensor(a, S.stream));
     PQP_HIP(launch_tensor_finalize(a, S.stream));
   }

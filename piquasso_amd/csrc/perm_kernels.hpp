@@ -113,10 +113,10 @@ hipError_t launch_int(int width, const IntArgs &a, hipStream_t stream);
 hipError_t launch_int_sum(const IntArgs &a, hipStream_t stream);
 
 // Tensor permanents (tensor_perm.hip) of items of one order: the matrices
-// of a table, the rows R_eps of every sign vector, the sweep, and the
-// items' sums.
+// of a table, the rows R_eps of every sign vector (of n such passes), the
+// sweep, and the items' sums.
 hipError_t launch_tensor_gather(const TensorArgs &a, hipStream_t stream);
-hipError_t launch_tensor_signs(const TensorArgs &a, hipStream_t stream);
+hipError_t launch_tensor_signs(const TensorArgs *passes, int n, hipStream_t stream);
 hipError_t launch_tensor_p0(const TensorArgs &a, hipStream_t stream);
 hipError_t launch_tensor_p1(const TensorArgs &a, hipStream_t stream);
 hipError_t launch_tensor(const TensorArgs &a, hipStream_t stream);

@@ -46,8 +46,8 @@
 // in one copy, short walks touch their lines first, an only unit writes its
 // item's result, and results of few items go to host memory.  One of 9
 // particles, with R_eps in every lane 38.1 us a call, by sign rows at first
-// 49.8, now 38; of 3 30.9, 35.5, 29; 30 of 7 particles 92, 107, 91; 60 of
-// five orders 186, 240, 190.
+// 49.8, now 38; of 3 31, 36, 30; 30 of 7 particles 92, 107, 91; 60 of
+// 2 to 6 particles 167, 257, 174.
 //
 // Compiled twice: -DPQP_TENSOR_PART=0 instantiates n = 1..12 and the other
 // kernels, =1 instantiates n = 13..20.
@@ -292,12 +292,17 @@ __global__ __launch_bounds__(256) void tensor_gather_kernel(TensorArgs a) {
   }
 }
 
-// R_eps[i] = sum_c eps_c A[i, c] for every t and row i: a thread each.
-__global__ __launch_bounds__(256) void tensor_signs_kernel(TensorArgs a) {
-  const int item = static_cast<int>(blockIdx.y);
+// R_eps[i] = sum_c eps_c A[i, c] for every t and row i: a thread each.  The
+// items of all orders in one launch, since a launch costs small ones more than
+// its work: five orders of 1 to 5 particles 80 -> 69 us a call.
+__global__ __launch_bounds__(256) void tensor_signs_kernel(TensorSigns g) {
+  int o = 0;
+  while (o + 1 < g.n_orders && blockIdx.x >= g.orders[o + 1].first) ++o;
+  const TensorSigns::Order a = g.orders[o];
+  const uint32_t b = blockIdx.x - a.first, item = b / a.per_item;
   const int n = a.n;
   const int64_t all = static_cast<int64_t>(n) << (n - 1);
-  const int64_t at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t at = static_cast<int64_t>(b - item * a.per_item) * 256 + threadIdx.x;
   if (at >= all) return;
   const uint32_t t = static_cast<uint32_t>(at / n);
   const int i = static_cast<int>(at - static_cast<int64_t>(t) * n);
@@ -377,11 +382,24 @@ hipError_t launch_tensor_gather(const TensorArgs &a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-hipError_t launch_tensor_signs(const TensorArgs &a, hipStream_t stream) {
-  const int64_t all = static_cast<int64_t>(a.n) << (a.n - 1);
-  hipLaunchKernelGGL(tensor_signs_kernel, dim3(static_cast<unsigned>((all + 255) / 256), a.n_items), dim3(256),
-                     0, stream, a);
-  return hipGetLastError();
+hipError_t launch_tensor_signs(const TensorArgs *passes, int n, hipStream_t stream) {
+  while (n > 0) {
+    TensorSigns g{};
+    uint64_t blocks = 0;
+    for (; g.n_orders < kTensorMaxN && g.n_orders < n; ++g.n_orders) {
+      const TensorArgs &a = passes[g.n_orders];
+      const uint64_t per_item = ((static_cast<uint64_t>(a.n) << (a.n - 1)) + 255) / 256;
+      if (g.n_orders > 0 && blocks + per_item * static_cast<uint64_t>(a.n_items) > INT32_MAX) break;
+      g.orders[g.n_orders] = {a.cols, a.signs, a.n, static_cast<uint32_t>(blocks), static_cast<uint32_t>(per_item)};
+      blocks += per_item * static_cast<uint64_t>(a.n_items);
+    }
+    hipLaunchKernelGGL(tensor_signs_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, g);
+    const hipError_t st = hipGetLastError();
+    if (st != hipSuccess) return st;
+    passes += g.n_orders;
+    n -= g.n_orders;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_tensor_finalize(const TensorArgs &a, hipStream_t stream) {

@@ -46,4 +46,15 @@ struct TensorArgs {
   double *prob;          // null: no table
 };
 
+// The sign rows of items of several orders, one launch.
+struct TensorSigns {
+  struct Order {
+    const double *cols;
+    double *signs;
+    int32_t n;
+    uint32_t first, per_item;  // its first block, and blocks of an item
+  } orders[kTensorMaxN];
+  int32_t n_orders;
+};
+
 }  // namespace pqp
